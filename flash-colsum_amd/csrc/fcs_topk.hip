@@ -6,22 +6,34 @@
 // small means of long contexts that the reference's fp16 result flushes to zero
 // (reference: flash_colsum/kernel_causal.py:124).
 //
-// One workgroup of 1024 threads per batch row:
-//   1. radix select, most significant byte first: four passes over the row, each building a
-//      256-bin histogram (LDS atomics on integers) of the current byte among the elements that
-//      match the bytes fixed so far; the histogram's suffix sums fix the next byte of the k-th
-//      largest key.  Floats are ordered through the usual monotone map to unsigned integers.
-//   2. ordered compaction: tiles of 1024 elements in index order; an element is taken if it is
-//      larger than the k-th largest value, or equal to it and among the first `need` such elements
-//      (ties go to the LOWER index).  Ballot / popcount scans give every taken element its place,
-//      so the result lists the indices in ascending order and is bit-reproducible.
-//   3. optionally (k <= kTopkSortMax) a bitonic sort in LDS orders the k results by descending
-//      value, ties by ascending index.
-// The threshold form is step 2 alone with a given threshold.
+// One workgroup of 1024 threads per batch row.  Wave w owns the w-th sixteenth of the row, E elements per
+// lane, and keeps them in registers (rows of up to 32768 entries; longer ones are re-read from the L2 for
+// every sweep).  A call is a chain of sweeps over so little data that barriers and LDS round trips are what
+// it costs, so the sweeps are few and none has a barrier inside:
+//   1. smallest and largest key of the row.  Floats are ordered through the usual monotone map to unsigned
+//      integers.
+//   2. selection of the k-th largest key: 2048-bin histograms (LDS atomics on integers).  The first one spans
+//      exactly [smallest, largest], so that the entries of a row, which share their leading bits, spread over the
+//      bins instead of meeting in a few of them (a wave's atomics on one address are served one after the
+//      other); each further one spans the bin that holds the k-th key.  It ends when that bin is taken whole:
+//      two sweeps for a typical row, never more than three.
+//   3. every wave counts the entries of its part above and at the k-th key; the counts of the waves before it
+//      are its offsets.  Taken entries get their place in index order from ballots; ties at the k-th value
+//      go to the LOWER index.
+//   4. optionally (k <= kTopkSortMax) a bitonic sort by descending value, ties by ascending index, of 64-bit
+//      (key, ~index) words: exchanges over less than a wave's elements are DPP and lane swaps in registers,
+//      only the wider ones go through LDS.
+// Measured, sorted: B 4, S 8192, k 1024 14.8 us; B 1, S 32768, k 2048 31.7 us; B 1, S 262144, k 4096 181 us.  The
+// former version (four byte-wide histograms, a tile of 1024 at a time with four barriers each in the compaction,
+// every step of the sort through LDS): 46, 99.6 and 549 us.
+// The threshold form is step 3 alone with a given threshold.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "flash_colsum.h"
+#include "fcs_device.h"
 #include "fcs_kernels.h"
 
 namespace fcs {
@@ -31,6 +43,9 @@ namespace {
 constexpr int kTopkSortMax = FCS_TOPK_SORT_MAX;
 constexpr int kTopkThreads = 1024;
 constexpr int kTopkWaves = kTopkThreads / 64;
+constexpr int kTopkBins = 2048;      // two per thread
+constexpr int kTopkBinBits = 11;
+constexpr int kTopkMaxRegs = 32;     // elements per lane that stay in registers
 
 // monotone map float -> uint32: a < b  <=>  key(a) < key(b)  (-0 < +0, NaNs at the two ends)
 __device__ __forceinline__ uint32_t order_key(float v)
@@ -38,173 +53,328 @@ __device__ __forceinline__ uint32_t order_key(float v)
     const uint32_t u = __builtin_bit_cast(uint32_t, v);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
-
-// exclusive prefix count of `flag` over the workgroup in thread order, and the workgroup's total.
-// `wsum` is LDS scratch of kTopkWaves + 1 ints.  Two barriers.
-__device__ __forceinline__ int block_rank(bool flag, int *wsum, int &total)
+__device__ __forceinline__ float key_value(uint32_t key)  // its inverse
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t b = __builtin_amdgcn_ballot_w64(flag);
-    const int before = __builtin_popcountll(b & ((1ull << lane) - 1ull));
-    __syncthreads();  // the scratch may still be read from the previous use
-    if (lane == 0) wsum[wave] = __builtin_popcountll(b);
-    __syncthreads();
-    int base = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < kTopkWaves; ++w) {
-        const int c = wsum[w];
-        base += (w < wave) ? c : 0;
-        tot += c;
-    }
-    total = tot;
-    return base + before;
+    return __builtin_bit_cast(float, (key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
 }
 
-// taken elements of one row in ascending index order.  thr_key: elements with a larger key are taken;
-// `need` more with an equal key (lowest indices first).  Returns the number written (<= cap).
-// CANON: -0 counts as +0 (the value comparison `>=` of the threshold form, not the bit order of top-k).
-template <bool CANON>
-__device__ int compact_row(const float *row, int S, uint32_t thr_key, int need, int64_t *idx_out, float *val_out, int cap,
-                           int *wsum)
-{
-    int written = 0, eq_seen = 0;  // block-uniform running counts
-    for (int base = 0; base < S; base += kTopkThreads) {
-        const int i = base + threadIdx.x;
-        float v = 0.f;
-        uint32_t key = 0;
-        const bool in = i < S;
-        if (in) {
-            v = row[i];
-            key = order_key(CANON ? v + 0.0f : v);
-        }
-        const bool eq = in && key == thr_key;
-        int eq_tot;
-        const int eq_rank = block_rank(eq, wsum, eq_tot);
-        const bool take = in && (key > thr_key || (eq && eq_seen + eq_rank < need));
-        int take_tot;
-        const int pos = written + block_rank(take, wsum, take_tot);
-        if (take && pos < cap) {
-            idx_out[pos] = i;
-            if (val_out) val_out[pos] = v;
-        }
-        written += take_tot;
-        eq_seen += eq_tot;
+// This wave's part of a row: elements first + 64 j + lane for j < n_j, E of them in registers (E = 0: read again
+// by every sweep).  CANON: -0 counts as +0 (the value comparison `>=` of the threshold form, not the bit order
+// of top-k).
+template <int E, bool CANON>
+struct RowPart {
+    static constexpr int kBatch = 8;
+    const float *row;
+    int S, first, n_j;
+    uint32_t keys[E > 0 ? E : 1];
+
+    __device__ __forceinline__ uint32_t load(int i) const
+    {
+        const float v = (i < S) ? row[i] : 0.f;
+        return order_key(CANON ? v + 0.0f : v);
     }
-    return written;
+    __device__ __forceinline__ void init(const float *r, int n, int wave, int lane)
+    {
+        row = r;
+        S = n;
+        n_j = (E > 0) ? E : (n + kBatch * kTopkThreads - 1) / (kBatch * kTopkThreads) * kBatch;
+        first = wave * n_j * 64 + lane;
+        if constexpr (E > 0) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) keys[j] = load(first + 64 * j);
+        }
+    }
+    // f(index, key, exists) for every element of the lane, in ascending order; all lanes of the wave together
+    template <typename F>
+    __device__ __forceinline__ void each(F f) const
+    {
+        int at = first;
+        asm volatile("" : "+v"(at));  // every sweep forms its own comparisons: kept masks would spill
+        if constexpr (E > 0) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) f(at + 64 * j, keys[j], at + 64 * j < S);
+        } else {
+            for (int j0 = 0; j0 < n_j; j0 += kBatch, at += 64 * kBatch) {
+                uint32_t k[kBatch];  // that many loads in flight
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) k[j] = load(at + 64 * j);
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) f(at + 64 * j, k[j], at + 64 * j < S);
+            }
+        }
+    }
+};
+
+struct TopkLds {
+    int hist[kTopkBins];
+    int wsum[kTopkWaves];
+    uint32_t wmin[kTopkWaves], wmax[kTopkWaves];
+    int2 wcnt[kTopkWaves];
+    int bin, above, count;
+};
+
+// Places of the taken elements in index order.  thr: elements with a larger key are taken, and the first `need`
+// with an equal one.  put(place, index, key) is called for each; returns their number (block-uniform).  One barrier.
+template <int E, bool CANON, typename Put>
+__device__ __forceinline__ int take_in_order(const RowPart<E, CANON> &part, uint32_t thr, int need, TopkLds &lds, int wave, int lane,
+                                             Put put)
+{
+    int gt_n = 0, eq_n = 0;  // wave-uniform
+    part.each([&](int, uint32_t key, bool in) {
+        gt_n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in && key > thr));
+        eq_n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in && key == thr));
+    });
+    if (lane == 0) lds.wcnt[wave] = int2{gt_n, eq_n};
+    __syncthreads();
+    int gt = 0, eq = 0, gt_all = 0, eq_all = 0;  // above / at the threshold before this wave's part, and in the row
+#pragma unroll
+    for (int w = 0; w < kTopkWaves; ++w) {
+        const int2 c = lds.wcnt[w];
+        gt += (w < wave) ? c.x : 0;
+        eq += (w < wave) ? c.y : 0;
+        gt_all += c.x;
+        eq_all += c.y;
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+    asm volatile("" : "+v"(thr));
+    part.each([&](int i, uint32_t key, bool in) {
+        const bool is_gt = in && key > thr, is_eq = in && key == thr;
+        const uint64_t bg = __builtin_amdgcn_ballot_w64(is_gt), be = __builtin_amdgcn_ballot_w64(is_eq);
+        const int eq_before = eq + __builtin_popcountll(be & below);
+        if (is_gt || (is_eq && eq_before < need)) put(gt + __builtin_popcountll(bg & below) + min(eq_before, need), i, key);
+        gt += __builtin_popcountll(bg);
+        eq += __builtin_popcountll(be);
+    });
+    return gt_all + min(eq_all, need);
+}
+
+// the value of lane (lane ^ MASK)
+template <int MASK>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v, int lane)
+{
+    auto dpp = [](uint32_t x, auto ctrl) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xF, 0xF, false);
+    };
+    if constexpr (MASK == 1) return dpp(v, std::integral_constant<int, kDppXor1>{});
+    else if constexpr (MASK == 2) return dpp(v, std::integral_constant<int, kDppXor2>{});
+    else if constexpr (MASK == 4)  // l ^ 7, then ^ 3
+        return dpp(dpp(v, std::integral_constant<int, kDppHalfMirror>{}), std::integral_constant<int, 0x1B>{});
+    else if constexpr (MASK == 8) return dpp(v, std::integral_constant<int, 0x128>{});  // rotate a row of 16 by 8
+    else {
+        // the swap leaves, of two copies, the partner's value in one of them: which one depends on the half
+        uint32_t x = v, y = v;
+        if constexpr (MASK == 16) asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+        else asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+        return (lane & MASK) ? x : y;
+    }
+}
+
+// Bitonic sort, largest first, of n2 (a power of two, at most 1024 SE) 64-bit words in buf[0 .. n2); thread t holds
+// the words t SE .. t SE + SE - 1.  buf has two halves of kTopkSortMax words: an exchange through LDS writes one and
+// the next such exchange the other, so that each costs one barrier.  Every thread of the block calls it; the result
+// stays in `w`.
+template <int SE>
+__device__ __forceinline__ void sort_descending(uint64_t *buf, int n2, int tid, uint64_t (&w)[SE])
+{
+    const int lane = tid & 63;
+#pragma unroll
+    for (int s = 0; s < SE; ++s) w[s] = (tid * SE + s < n2) ? buf[tid * SE + s] : 0;
+    int half = 1;
+    // keep the larger word where the element comes first of its pair in a block that ends up descending
+    auto keep = [&](uint64_t mine, uint64_t other, int e, int stride, int size) {
+        const bool larger = ((e & stride) == 0) == ((e & size) == 0);
+        return ((mine > other) == larger) ? mine : other;
+    };
+    auto in_wave = [&](auto mask_c, int size) {
+        constexpr int MASK = decltype(mask_c)::value;
+#pragma unroll
+        for (int s = 0; s < SE; ++s) {
+            const uint32_t lo = lane_xor<MASK>((uint32_t)w[s], lane), hi = lane_xor<MASK>((uint32_t)(w[s] >> 32), lane);
+            w[s] = keep(w[s], ((uint64_t)hi << 32) | lo, tid * SE + s, MASK * SE, size);
+        }
+    };
+    for (int size = 2; size <= n2; size <<= 1) {
+        int stride = size >> 1;
+        for (; stride >= 64 * SE; stride >>= 1) {
+            uint64_t *b = buf + half * kTopkSortMax;
+            half ^= 1;
+#pragma unroll
+            for (int s = 0; s < SE; ++s)
+                if (tid * SE + s < n2) b[tid * SE + s] = w[s];
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < SE; ++s)
+                if (tid * SE + s < n2) w[s] = keep(w[s], b[(tid * SE + s) ^ stride], tid * SE + s, stride, size);
+        }
+        if (stride >= 32 * SE) in_wave(std::integral_constant<int, 32>{}, size);
+        if (stride >= 16 * SE) in_wave(std::integral_constant<int, 16>{}, size);
+        if (stride >= 8 * SE) in_wave(std::integral_constant<int, 8>{}, size);
+        if (stride >= 4 * SE) in_wave(std::integral_constant<int, 4>{}, size);
+        if (stride >= 2 * SE) in_wave(std::integral_constant<int, 2>{}, size);
+        if (stride >= SE) in_wave(std::integral_constant<int, 1>{}, size);
+#pragma unroll
+        for (int st = SE / 2; st > 0; st >>= 1) {
+            if (stride >= st) {
+#pragma unroll
+                for (int s = 0; s < SE; ++s)
+                    if ((s & st) == 0) {
+                        const uint64_t a = w[s], b = w[s + st];
+                        w[s] = keep(a, b, tid * SE + s, st, size);
+                        w[s + st] = keep(b, a, tid * SE + s + st, st, size);
+                    }
+            }
+        }
+    }
 }
 
 }  // namespace
 
-__global__ __launch_bounds__(kTopkThreads) void fcs_topk_kernel(const float *means, int S, int k, int64_t *idx_out,
-                                                                float *val_out, int sorted)
+template <int E>
+__global__ __launch_bounds__(kTopkThreads) void fcs_topk_kernel(const float *means, int S, int k, int64_t *idx_out, float *val_out,
+                                                                int sorted)
 {
-    __shared__ int hist[256];
-    __shared__ int wsum[kTopkWaves + 1];
-    __shared__ uint32_t sel_s[2];  // [0] the chosen byte, [1] elements still wanted among those that match the prefix
-    __shared__ float sv[kTopkSortMax];
-    __shared__ int si[kTopkSortMax];
-
-    const int tid = threadIdx.x;
-    const float *row = means + (int64_t)blockIdx.x * S;
+    __shared__ TopkLds lds;
+    __shared__ uint64_t buf[2 * kTopkSortMax];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int64_t *io = idx_out + (int64_t)blockIdx.x * k;
     float *vo = val_out ? val_out + (int64_t)blockIdx.x * k : nullptr;
+    RowPart<E, false> part;
+    part.init(means + (int64_t)blockIdx.x * S, S, wave, lane);
 
-    // ---- 1. the k-th largest key, byte by byte
-    uint32_t prefix = 0, mask = 0;
-    int want = k;  // rank (1 = largest) of the wanted key among the elements that match the prefix
-    for (int shift = 24; shift >= 0; shift -= 8) {
-        if (tid < 256) hist[tid] = 0;
-        __syncthreads();
-        for (int i = tid; i < S; i += kTopkThreads) {
-            const uint32_t key = order_key(row[i]);
-            if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1);
-        }
-        __syncthreads();
-        if (tid < 64) {
-            // lane L owns bins 4L .. 4L+3; suffix sums over lanes, then within the lane, find the bin b with
-            // count(bins > b) < want <= count(bins >= b)
-            const int c0 = hist[4 * tid], c1 = hist[4 * tid + 1], c2 = hist[4 * tid + 2], c3 = hist[4 * tid + 3];
-            const int mine = c0 + c1 + c2 + c3;
-            int above = 0;  // elements in bins of higher lanes
-            for (int l = 0; l < 64; ++l) {
-                const int o = __shfl(mine, l);
-                above += (l > tid) ? o : 0;
-            }
-            const int cs[4] = {c0, c1, c2, c3};
-            int acc = above;
+    // ---- 1. range of the row's keys
+    uint32_t kmin = 0xffffffffu, kmax = 0;
+    part.each([&](int, uint32_t key, bool in) {
+        kmin = in ? min(kmin, key) : kmin;
+        kmax = in ? max(kmax, key) : kmax;
+    });
 #pragma unroll
-            for (int j = 3; j >= 0; --j) {
-                if (acc < want && want <= acc + cs[j]) {
-                    sel_s[0] = (uint32_t)(4 * tid + j);
-                    sel_s[1] = (uint32_t)(want - acc);
-                }
-                acc += cs[j];
-            }
-        }
-        __syncthreads();
-        prefix |= sel_s[0] << shift;
-        mask |= 255u << shift;
-        want = (int)sel_s[1];
-        __syncthreads();
+    for (int m = 32; m >= 1; m >>= 1) {
+        kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, m));
+        kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, m));
     }
-    // `prefix` is the k-th largest key; `want` of the elements equal to it are taken
+    if (lane == 0) {
+        lds.wmin[wave] = kmin;
+        lds.wmax[wave] = kmax;
+    }
+    lds.hist[2 * tid] = lds.hist[2 * tid + 1] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kTopkWaves; ++w) {
+        kmin = min(kmin, lds.wmin[w]);
+        kmax = max(kmax, lds.wmax[w]);
+    }
 
-    // ---- 2. ordered compaction
-    compact_row<false>(row, S, prefix, want, io, vo ? vo : nullptr, k, wsum);
-
-    // ---- 3. descending values, ties by ascending index
-    if (sorted && k <= kTopkSortMax) {
+    // ---- 2. the k-th largest key lies in [lo, lo + span]; `want` is its rank (1 = largest) among the keys in there.
+    // Afterwards: keys above `lo` are taken, and the first `want` that equal it
+    uint32_t lo = kmin, span = kmax - kmin;
+    int want = k;
+    while (span != 0) {  // block-uniform
+        const int bits = 32 - __builtin_clz(span), shift = max(0, bits - kTopkBinBits);
+        part.each([&](int, uint32_t key, bool in) {
+            const uint32_t off = key - lo;  // wraps for keys below lo
+            if (in && off <= span) atomicAdd(&lds.hist[off >> shift], 1);
+        });
         __syncthreads();
-        int n2 = 1;
-        while (n2 < k) n2 <<= 1;
-        for (int i = tid; i < n2; i += kTopkThreads) {
-            if (i < k) {
-                si[i] = (int)io[i];
-                sv[i] = row[io[i]];
-            } else {  // padding (recognised by its index) sorts behind every real entry, negative NaNs included
-                si[i] = 0x7fffffff;
-                sv[i] = 0.f;
-            }
+        // bins 2 tid and 2 tid + 1; suffix sums over the threads
+        const int c0 = lds.hist[2 * tid], c1 = lds.hist[2 * tid + 1];
+        int run = c0 + c1;  // this lane and the higher ones of its wave
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const int o = __shfl_down(run, m);
+            run += (lane + m < 64) ? o : 0;
         }
+        if (lane == 0) lds.wsum[wave] = run;
         __syncthreads();
-        // bitonic network; "a before b"  <=>  key(a) > key(b), or equal keys and index(a) < index(b)
-        for (int size = 2; size <= n2; size <<= 1) {
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int t = tid; t < (n2 >> 1); t += kTopkThreads) {
-                    const int lo = 2 * t - (t & (stride - 1));  // index with the `stride` bit clear
-                    const int hi = lo + stride;
-                    const bool desc_block = ((lo & size) == 0);  // this block ends up in "before" order
-                    const uint32_t ka = (si[lo] == 0x7fffffff) ? 0u : order_key(sv[lo]);
-                    const uint32_t kb = (si[hi] == 0x7fffffff) ? 0u : order_key(sv[hi]);
-                    const bool a_first = ka > kb || (ka == kb && si[lo] < si[hi]);
-                    if (a_first != desc_block) {
-                        const float tv = sv[lo];
-                        sv[lo] = sv[hi];
-                        sv[hi] = tv;
-                        const int ti = si[lo];
-                        si[lo] = si[hi];
-                        si[hi] = ti;
-                    }
-                }
-                __syncthreads();
-            }
+        int above = run - c0 - c1;  // keys in the bins of higher threads
+#pragma unroll
+        for (int w = 0; w < kTopkWaves; ++w) above += (w > wave) ? lds.wsum[w] : 0;
+        if (above < want && want <= above + c1) {
+            lds.bin = 2 * tid + 1;
+            lds.above = above;
+            lds.count = c1;
+        } else if (above + c1 < want && want <= above + c1 + c0) {
+            lds.bin = 2 * tid;
+            lds.above = above + c1;
+            lds.count = c0;
         }
-        for (int i = tid; i < k; i += kTopkThreads) {
-            io[i] = si[i];
-            if (vo) vo[i] = sv[i];
+        lds.hist[2 * tid] = lds.hist[2 * tid + 1] = 0;
+        __syncthreads();
+        want -= lds.above;
+        const uint32_t bin_lo = lo + ((uint32_t)lds.bin << shift);
+        const uint32_t bin_hi_off = ((uint32_t)lds.bin << shift) + ((1u << shift) - 1u);
+        span = min(bin_hi_off, span) - ((uint32_t)lds.bin << shift);  // the last bin may be cut off
+        lo = bin_lo;
+        if (want == lds.count) {  // the bin is taken whole: every key from its lower end on
+            want = S;
+            break;
         }
     }
+
+    // ---- 3. and 4.
+    if (!sorted || k > kTopkSortMax) {
+        take_in_order(part, lo, want, lds, wave, lane, [&](int place, int i, uint32_t key) {
+            if (place < k) {
+                io[place] = i;
+                if (vo) vo[place] = key_value(key);
+            }
+        });
+        return;
+    }
+    int n2 = 1;
+    while (n2 < k) n2 <<= 1;
+    // zero words sort behind every real one (whose lower half is the complement of an index)
+    for (int i = k + tid; i < n2; i += kTopkThreads) buf[i] = 0;
+    take_in_order(part, lo, want, lds, wave, lane, [&](int place, int i, uint32_t key) {
+        if (place < k) buf[place] = ((uint64_t)key << 32) | (uint32_t)~i;
+    });
+    __syncthreads();
+    auto finish = [&](auto se_c) {
+        constexpr int SE = decltype(se_c)::value;
+        uint64_t w[SE];
+        sort_descending<SE>(buf, n2, tid, w);
+#pragma unroll
+        for (int s = 0; s < SE; ++s) {
+            const int e = tid * SE + s;
+            if (e < k) {
+                io[e] = (int)~(uint32_t)w[s];
+                if (vo) vo[e] = key_value((uint32_t)(w[s] >> 32));
+            }
+        }
+    };
+    if (n2 <= kTopkThreads) finish(std::integral_constant<int, 1>{});
+    else if (n2 <= 2 * kTopkThreads) finish(std::integral_constant<int, 2>{});
+    else finish(std::integral_constant<int, 4>{});
+    static_assert(kTopkSortMax <= 4 * kTopkThreads, "words per thread above");
 }
 
+template <int E>
 __global__ __launch_bounds__(kTopkThreads) void fcs_threshold_kernel(const float *means, int S, float tau, int64_t *idx_out,
                                                                      int32_t *count_out)
 {
-    __shared__ int wsum[kTopkWaves + 1];
-    const float *row = means + (int64_t)blockIdx.x * S;
+    __shared__ TopkLds lds;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    RowPart<E, true> part;
+    part.init(means + (int64_t)blockIdx.x * S, S, wave, lane);
+    int64_t *io = idx_out + (int64_t)blockIdx.x * S;
     // value >= tau  <=>  key(value) >= key(tau) once -0 is read as +0 on both sides (the bit order alone puts
     // -0 below +0): "larger than thr, or equal to thr with unlimited ties" with thr = key(tau + 0)
-    const int n = compact_row<true>(row, S, order_key(tau + 0.0f), 0x7fffffff, idx_out + (int64_t)blockIdx.x * S, nullptr, S, wsum);
+    const int n = take_in_order(part, order_key(tau + 0.0f), S, lds, wave, lane, [&](int place, int i, uint32_t) { io[place] = i; });
     if (threadIdx.x == 0) count_out[blockIdx.x] = n;
+}
+
+// Elements per lane for rows of S entries: the smallest power of two that holds the row in registers, 0 (re-read)
+// beyond kTopkMaxRegs.
+template <typename F>
+static void with_row_regs(int S, F f)
+{
+    const int e = (S + kTopkThreads - 1) / kTopkThreads;
+    if (e <= 1) f(std::integral_constant<int, 1>{});
+    else if (e <= 2) f(std::integral_constant<int, 2>{});
+    else if (e <= 4) f(std::integral_constant<int, 4>{});
+    else if (e <= 8) f(std::integral_constant<int, 8>{});
+    else if (e <= 16) f(std::integral_constant<int, 16>{});
+    else if (e <= kTopkMaxRegs) f(std::integral_constant<int, kTopkMaxRegs>{});
+    else f(std::integral_constant<int, 0>{});
 }
 
 }  // namespace fcs
@@ -216,8 +386,10 @@ int fcs_topk_f32(const float *means, int B, int S, int k, int64_t *idx_out, floa
     if (!means || !idx_out) return FCS_E_NULL;
     if (B < 1 || S < 1 || k < 1 || k > S) return FCS_E_DIMS;
     if (sorted && k > FCS_TOPK_SORT_MAX) return FCS_E_DIMS;
-    hipLaunchKernelGGL(fcs::fcs_topk_kernel, dim3(B), dim3(fcs::kTopkThreads), 0, reinterpret_cast<hipStream_t>(hip_stream), means, S,
-                       k, idx_out, val_out, sorted ? 1 : 0);
+    fcs::with_row_regs(S, [&](auto e) {
+        hipLaunchKernelGGL(fcs::fcs_topk_kernel<decltype(e)::value>, dim3(B), dim3(fcs::kTopkThreads), 0,
+                           reinterpret_cast<hipStream_t>(hip_stream), means, S, k, idx_out, val_out, sorted ? 1 : 0);
+    });
     return (int)hipGetLastError();
 }
 
@@ -226,8 +398,10 @@ int fcs_threshold_f32(const float *means, int B, int S, float tau, int64_t *idx_
     if (!means || !idx_out || !count_out) return FCS_E_NULL;
     if (B < 1 || S < 1) return FCS_E_DIMS;
     if (tau != tau) return FCS_E_SCALE;
-    hipLaunchKernelGGL(fcs::fcs_threshold_kernel, dim3(B), dim3(fcs::kTopkThreads), 0, reinterpret_cast<hipStream_t>(hip_stream), means,
-                       S, tau, idx_out, count_out);
+    fcs::with_row_regs(S, [&](auto e) {
+        hipLaunchKernelGGL(fcs::fcs_threshold_kernel<decltype(e)::value>, dim3(B), dim3(fcs::kTopkThreads), 0,
+                           reinterpret_cast<hipStream_t>(hip_stream), means, S, tau, idx_out, count_out);
+    });
     return (int)hipGetLastError();
 }
 

@@ -1,0 +1,42 @@
+"""Top-k and threshold selection at the sizes where the kernels change: entries per lane (1024 lanes hold 1, 2, 4, ...
+32 each, longer rows are re-read), words per thread of the sort, rows whose keys share all, many or no leading bits.
+The reference is a stable sort of the same values, so the comparison is exact."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(kind, b, s, gen):
+    x = torch.rand((b, s), generator=gen)
+    if kind == "narrow":      # a few thousand distinct values around 1e-4: long common prefix, many ties
+        x = 1e-4 + (x * 4096).round() * 2.0 ** -37
+    elif kind == "wide":      # both signs, every exponent
+        x = (x - 0.5) * torch.exp2(torch.randint(-120, 120, (b, s), generator=gen).float())
+    elif kind == "constant":
+        x = torch.full((b, s), 0.25)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["uniform", "narrow", "wide", "constant"])
+@pytest.mark.parametrize("s", [1, 63, 65, 1024, 1025, 2049, 4096, 8191, 16385, 32768, 32769, 41001])
+def test_topk_and_threshold_sizes(kind, s):
+    from flash_colsum import _hip
+
+    gen = torch.Generator().manual_seed(s)
+    x = _rows(kind, 2, s, gen)
+    print(kind, s, flush=True)
+    order = torch.sort(x, dim=1, descending=True, stable=True).indices
+    for k in sorted({k for k in (1, 2, 63, 64, 65, 1000, 1024, 1025, 2048, 2049, 4096, s // 2, s) if 1 <= k <= s}):
+        want = order[:, :k]
+        if k <= _hip.TOPK_SORT_MAX:
+            val, idx = _hip.topk_f32(x.cuda(), k, sorted=True)
+            assert torch.equal(idx.cpu(), want) and torch.equal(val.cpu(), x.gather(1, want)), k
+        asc = want.sort(dim=1).values
+        val, idx = _hip.topk_f32(x.cuda(), k, sorted=False)
+        assert torch.equal(idx.cpu(), asc) and torch.equal(val.cpu(), x.gather(1, asc)), k
+    tau = float(x[0, s // 3])
+    idx, cnt = _hip.threshold_f32(x.cuda(), tau)
+    for r in range(2):
+        want = (x[r] >= tau).nonzero().view(-1)
+        assert cnt[r].item() == want.numel() and torch.equal(idx[r, : want.numel()].cpu(), want)
