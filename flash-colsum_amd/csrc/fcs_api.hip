@@ -41,10 +41,10 @@ hipError_t static_scratch(void **ptr)
 // microseconds (more with many heads), so every thread remembers the plans of its last few
 // geometries.
 struct PlanKey {
-    int causal, B, H, Sq, Sk, D, cls_n, k_past;
+    int causal, B, H, Hk, Sq, Sk, D, cls_n, k_past;
     bool operator==(const PlanKey &o) const
     {
-        return causal == o.causal && B == o.B && H == o.H && Sq == o.Sq && Sk == o.Sk && D == o.D && cls_n == o.cls_n &&
+        return causal == o.causal && B == o.B && H == o.H && Hk == o.Hk && Sq == o.Sq && Sk == o.Sk && D == o.D && cls_n == o.cls_n &&
                k_past == o.k_past;
     }
 };
@@ -57,16 +57,16 @@ struct PlanMemo {
 };
 thread_local PlanMemo t_memo;
 
-bool cached_plan(fcs::Plan &p, int causal, int B, int H, int Sq, int Sk, int D, int cls_n, int k_past)
+bool cached_plan(fcs::Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past)
 {
-    const PlanKey key{causal, B, H, Sq, Sk, D, cls_n, k_past};
+    const PlanKey key{causal, B, H, Hk, Sq, Sk, D, cls_n, k_past};
     PlanMemo &m = t_memo;
     for (int i = 0; i < kPlanMemo; ++i)
         if (m.used[i] && m.key[i] == key) {
             p = m.plan[i];
             return true;
         }
-    if (!fcs::make_plan(p, causal, B, H, Sq, Sk, D, cls_n, k_past)) return false;
+    if (!fcs::make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return false;
     const int slot = m.next;
     m.next = (slot + 1) % kPlanMemo;
     m.key[slot] = key;
@@ -103,7 +103,7 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     // mean the same and must not reach the kernels' 32-bit row arithmetic
     if (k_past > Sk) k_past = Sk;
 
-    if (!cached_plan(p, causal, B, H, Sq, Sk, D, cls_n, k_past)) return FCS_E_DIMS;
+    if (!cached_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return FCS_E_DIMS;
     p.bf16 = bf16;
     if (need_ptrs) {
         if (ws && (reinterpret_cast<uintptr_t>(ws) & 255u)) return FCS_E_WORKSPACE;
@@ -117,9 +117,11 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     a.ks_b = ks[0]; a.ks_h = ks[1]; a.ks_s = ks[2];
     a.B = B; a.H = H; a.Sq = Sq; a.Sk = Sk;
     a.D = D;
-    a.kv_group = H / Hk;
+    a.kv_group = p.fold > 1 ? 1 : H / Hk;  // folded rows: the kernels' heads are the key heads
     a.kv_magic = (uint32_t)((0x100000000ull + (uint64_t)a.kv_group - 1) / (uint64_t)a.kv_group);  // unused when the group is 1
     a.q_rows = p.q_rows;
+    a.fold = p.fold; a.v_heads = p.v_heads; a.v_rows = p.v_rows;
+    a.fold_magic = (uint32_t)(((1ull << 31) + (uint64_t)p.q_rows - 1) / (uint64_t)p.q_rows);
     a.causal = p.causal; a.k_past = p.k_past;
     // keys j <= k_past are visible to every row; whole stages of them
     a.pre_end = p.causal ? (int)((((long)p.k_past + 1) / fcs::kStageKeys) * fcs::kStageKeys) : 0x3fffffc0;
@@ -181,8 +183,13 @@ size_t fcs_workspace_bytes(int causal, int B, int H, int Sq, int Sk, int D, int 
 {
     fcs::Plan p;
     const int k_past = (causal && Sk > Sq) ? Sk - Sq : 0;  // the layout does not depend on k_past
-    if (!cached_plan(p, causal ? 1 : 0, B, H, Sq, Sk, D, cls_n < 0 ? -1 : cls_n, k_past)) return 0;
-    return p.total;
+    const int rows = cls_n < 0 ? -1 : cls_n;
+    if (!cached_plan(p, causal ? 1 : 0, B, H, H, Sq, Sk, D, rows, k_past)) return 0;
+    size_t most = p.total;
+    // enough for any number of key heads: the two-pass path lays grouped heads out differently
+    for (int hk = 1; hk <= H / 2 && !(p.fewrows || p.small || p.fused); ++hk)
+        if (H % hk == 0 && fcs::make_plan(p, causal ? 1 : 0, B, H, hk, Sq, Sk, D, rows, k_past) && p.total > most) most = p.total;
+    return most;
 }
 
 int fcs_colsum_call(const fcs_call_t *c)
@@ -237,7 +244,7 @@ int fcs_colsum_noncausal_f16_static(const void *q, const void *k, float *out, vo
 {
     // size check first: it needs no GPU, like every other argument error
     fcs::Plan p;
-    if (!cached_plan(p, 0, B, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0)) return FCS_E_DIMS;
+    if (!cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0)) return FCS_E_DIMS;
     if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES) return FCS_E_STATIC_LIMIT;
     if (!q || !k || !out || !q_strides || !k_strides) return FCS_E_NULL;
     void *ws = nullptr;

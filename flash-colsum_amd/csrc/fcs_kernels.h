@@ -17,6 +17,10 @@ struct Args {
     int kv_group;        // query heads per key head (1 unless grouped-query): key head = head / kv_group
     uint32_t kv_magic;   // ceil(2^32 / kv_group), for the division above (unused when kv_group == 1)
     int q_rows;          // query rows that are averaged
+    // two-pass path: the averaged rows as its kernels number them.  fold == 1: row v of head h is query row v.  fold > 1:
+    // the `fold` query heads of a key head form one head of v_rows = fold * q_rows rows (then kv_group is 1)
+    int fold, v_heads, v_rows;
+    uint32_t fold_magic;  // ceil(2^31 / q_rows), for v / q_rows (unused when fold == 1)
     int causal, k_past;  // key j visible to query i  <=>  j <= k_past + i
     int pre_end;         // two-pass path, pre-scaled variant: the 64-key stages that end at or below this key (a multiple
                          // of 64) run on Q * c rounded to fp16 in both passes; the keys that every averaged row sees
@@ -24,9 +28,9 @@ struct Args {
     float c;             // |scale| * log2(e)
     // pass 1
     int n_chunks, chunk_keys, rows_pad;
-    float2 *lse;  // [B*H][rows_pad]            (m, log2 l): row maximum in score units (0 on the
+    float2 *lse;  // [B*v_heads][rows_pad]      (m, log2 l): row maximum in score units (0 on the
                   //                            unstabilised path) and log2 of sum_j 2^((s_ij - m) * c)
-    float2 *ml;   // [B*H][n_chunks][rows_pad]  (m, l) of each key split
+    float2 *ml;   // [B*v_heads][n_chunks][rows_pad]  (m, l) of each key split
     // pass 2
     int c_chunk, c_groups, c_upg, c_nrb;  // column pass: keys per block, unit groups, units per group, row blocks per head
     int c_nchunks;       // column pass: key chunks (its grid is c_nchunks x c_groups x B, launched as one dimension)
