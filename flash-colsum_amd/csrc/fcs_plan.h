@@ -82,12 +82,13 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     p.k_past = causal ? k_past : 0;
     p.q_rows = (cls_n > 0 && cls_n < Sq) ? cls_n : Sq;
 
-    // ---- grouped key heads: while a head's averaged rows leave a row block partly empty, the rows of all query heads
-    // of a key head form one head, whose keys are then streamed once instead of once per query head.  (Full
-    // blocks gain nothing from it, and a causal block that holds rows of two heads cannot stop at its own last key.)
-    // B 4, 32 query heads on 8 key heads, Q 64, K 8192, D 128: row pass 41 -> 26.5 us, column pass 60 -> 31 us.
+    // ---- grouped key heads: while a head's averaged rows fill no more than the smallest row block, the rows of all
+    // query heads of a key head form one head, whose keys are then streamed once instead of once per query head.
+    // B 4, 32 query heads on 8 key heads, K 8192, D 128 bf16, both passes: Q 64 103 -> 54 us, Q 128 103 -> 85 us.
+    // (More rows fill their own blocks, and a causal block that holds rows of several heads cannot stop at its own
+    // last key: Q 200, 32 on 4 heads, K 6000, D 64 48 us head by head, 49 us folded; Q 400, 32 on 8, K 30000 251 and 257 us.)
     const int G = H / Hk;
-    p.fold = (G > 1 && p.q_rows < 512 && (long)G * p.q_rows * p.q_rows < (1L << 31)) ? G : 1;
+    p.fold = (G > 1 && p.q_rows <= 128 && (long)G * p.q_rows * p.q_rows < (1L << 31)) ? G : 1;
     p.v_heads = H / p.fold;
     p.v_rows = p.q_rows * p.fold;
 

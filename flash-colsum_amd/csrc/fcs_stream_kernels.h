@@ -23,6 +23,11 @@
 //     global_load_lds_dwordx4 straight into an LDS ring, several stages ahead, XOR-swizzled so
 //     that the operand reads (ds_read_b128, 32 rows a row pitch apart) are conflict-free.  One
 //     workgroup barrier per stage; the DMA is waited for by hand with s_waitcnt vmcnt(n).
+//   * The stream has two loops: the stages that every row of a wave sees run in one without any test of position
+//     (unrolled over the ring), the others (diagonal, last partial stage) in a short rolled one, where a wave skips
+//     the stages it does not see.  With the masked code inlined at every tile the kernel was 2.3 times as
+//     long and needed 254 registers at D 128 (now 211).  B 1, H 32, Q 512, K 65536, D 128: 601 -> 588 us per call,
+//     B 1, H 16, S 5000, D 64 bf16 208 -> 196, causal B 1, H 32, S 900, D 128 37.5 -> 33.9.
 // A workgroup owns a chunk of keys (at most kColChunkMax, the LDS accumulator) and walks over a
 // group of (head, row block) units, re-streaming its chunk for each; at the end the waves'
 // slices are added in wave order and written as one partial slab (or the means directly, when
@@ -108,6 +113,36 @@ __device__ __forceinline__ int rows_first(const Args &a, int v, int n)
         return v;
     }
 }
+
+// Masked work on a fragment of 32 rows from row v0 on (wave-uniform): add(ahead) with ahead(i) = the rows of the heads
+// before the row of accumulator register i, which `rel` has to be raised by.  Folded rows: a fragment inside one head, the
+// usual case, raises `rel` once; only one that holds rows of several heads divides per register.
+template <bool FOLD, class F>
+__device__ __forceinline__ void mask_rows(const Args &a, int v0, int g4, int &rel, F add)
+{
+    if constexpr (FOLD) {
+        const int h0 = fold_head(v0, a.fold_magic);
+        if (h0 == fold_head(v0 + 31, a.fold_magic)) {
+            rel += h0 * a.q_rows;
+            add([](int) { return 0; });
+        } else {
+            int v = v0 + g4;
+            asm volatile("" : "+v"(v));  // formed here, not kept for every register through the stream
+            add([&](int i) { return fold_head(v + 8 * (i >> 2) + (i & 3), a.fold_magic) * a.q_rows; });
+        }
+    } else {
+        add([](int) { return 0; });
+    }
+}
+
+// How many of the nst stages from key k0 on lie within the keys up to `thr`, which all rows of a wave see
+__device__ __forceinline__ int plain_stages(int k0, int nst, int thr)
+{
+    return (thr + 1 >= k0) ? min(nst, (thr + 1 - k0) / kStageKeys) : 0;
+}
+
+// column pass: how the exponent is taken
+constexpr int kFormRaw = 0, kFormPrescaled = 1, kFormShifted = 2;
 
 // ceiling of a row's sum of exponentials in the pre-scaled variants: keeps every score of the common path
 // below 20 in the exponent's unit, which bounds what rounding Q * c to fp16 can do to it (the error of a
@@ -284,11 +319,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         const int64_t k_row_b = a.ks_s * 2;
 
         // stage `st` of the unit into ring slot `slot` (stages past the last one repeat it, so that the
-        // number of DMA instructions in flight at every wait is a compile-time constant)
+        // number of DMA instructions in flight at every wait is a compile-time constant).
         auto fetch_stage = [&](int st, int slot) {
             const int kb = c0 + min(st, nst - 1) * KT;
             char *dst = ring_w + slot * STAGE_BYTES;
-            if (kb + KT <= a.Sk && a.D == D) {  // whole stage inside the tensor, rows as wide as compiled (wave-uniform)
+            // whole stage inside the tensor, rows as wide as compiled (wave-uniform; the other case out of line)
+            if (__builtin_expect(kb + KT <= a.Sk && a.D == D, 1)) {
                 const char *src = kp + (int64_t)kb * k_row_b;
 #pragma unroll
                 for (int j = 0; j < IPW; ++j) dma16(src + g_off[j], dst + j * 1024);
@@ -352,11 +388,16 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         // rows of this wave relative to the causal diagonal; non-causal: every key below Sk is visible
         const int kp_eff = a.causal ? a.k_past : 0x3fffffff - a.Sq;
         const int thr_wave_min = a.causal ? min(a.k_past + rows_first<FOLD>(a, qw0, ROWS_W), a.Sk - 1) : a.Sk - 1;   // last key EVERY row of the wave sees
+        const int thr_wave_max = a.causal ? a.k_past + (FOLD ? a.q_rows : qw0 + ROWS_W) - 1 : a.Sk - 1;             // last key ANY row of it sees
+        // leading stages that every row of the wave sees: they run in the plain stream below
+        const int n_plain = plain_stages(c0, nst, thr_wave_min);
 
-        // One phase: the stages [s0, s1) of the unit in one form of the operand (SC: pre-scaled).  `fetched`: the
-        // phase's first NS - 1 stages are already in the ring (the unit's prologue above).
-        auto run_phase = [&](auto sc_c, const int s0, const int s1, const bool fetched) {
-            constexpr bool SC = decltype(sc_c)::value;
+        // One phase: the stages [s0, s1) of the unit in one FORM: raw operand, pre-scaled operand, or the
+        // two-constant form of a unit with a stabilised row.  `fetched`: the phase's first NS - 1 stages are already
+        // in the ring (the unit's prologue above).
+        auto run_phase = [&](auto form_c, const int s0, const int s1, const bool fetched) {
+            constexpr int FORM = decltype(form_c)::value;
+            constexpr bool SC = FORM == kFormPrescaled, SHIFTED = FORM == kFormShifted;
             if (!fetched) {
 #pragma unroll
                 for (int st = 0; st < NS - 1; ++st) fetch_stage(s0 + st, st);
@@ -364,34 +405,33 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 block_sync();
             }
             floatx16 cinit[NB];  // row constants in accumulator layout: register i <-> row 8*(i/4) + 4*g + i%4
+            int g_c = g;
+            asm volatile("" : "+v"(g_c));  // addresses are formed here, not kept from unit to unit
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
-                    floatx4 v;  // inline assembly for the same reason as the operand reads
-                    const uint32_t ad = lds_addr(SC ? np_s : nl_s) + (uint32_t)((wave * ROWS_W + nb * 32 + 8 * i4 + 4 * g) * 4);
-                    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(ad) : "memory");
+                    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+                    if (!SHIFTED) {  // inline assembly for the same reason as the operand reads
+                        const uint32_t ad = lds_addr(SC ? np_s : nl_s) + (uint32_t)((wave * ROWS_W + nb * 32 + 8 * i4 + 4 * g_c) * 4);
+                        asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(ad) : "memory");
+                    }
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) cinit[nb][4 * i4 + j] = shifted ? 0.f : v[j];
+                    for (int j = 0; j < 4; ++j) cinit[nb][4 * i4 + j] = v[j];
                 }
 
-            // ---- the stream.  A stage is NA * NB tiles of 32 rows x 32 keys; tile q = na * NB + nb uses key
-            // fragment na and accumulator q & 1.  Software pipeline inside the wave: the MFMA chain of tile q
-            // is issued BEFORE the exponent work of tile q - 1, so the matrix pipe and the VALU run together
-            // whatever the phase of the other wave on the SIMD.
+            // A stage is NA * NB tiles of 32 rows x 32 keys; tile q = na * NB + nb uses key fragment na and
+            // accumulator q & 1.
             constexpr int TILES = NA * NB;
             static_assert(TILES % 2 == 0, "two accumulators alternate");
+            static_assert(NA == 2, "fragment offsets below");
             half8 kf[NT];
-            take_frag(std::integral_constant<int, 0>{}, kf);
-            floatx16 acc[2];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
             float cp[4] = {0.f, 0.f, 0.f, 0.f};  // running column sums of the fragment being exponentiated
 
-            // Exponent work of one finished tile (kb_t: first key of its stage), split in three so that the
-            // common case can be woven between the MFMAs of the next tile:
+            // Exponent work of one finished tile (kb_t: first key of its stage):
             //   drain_begin   requests the fragment's accumulator slot (first row fragment only)
-            //   drain_slow    masked / stabilised forms, all sixteen scores at once
+            //   drain_plain   every row sees every key of the tile
+            //   drain_masked  tiles on the diagonal or past the last key
             //   drain_end     after the last row fragment: fold the half-waves, add into the wave's slice
             float col_old = 0.f;
             uint32_t col_ad = 0;
@@ -401,40 +441,55 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                     asm volatile("ds_read_b32 %0, %1" : "=v"(col_old) : "v"(col_ad) : "memory");
                 }
             };
-            auto drain_slow = [&](const floatx16 &sc, int kb_t, int na, int nb) {
+            // two-constant form (rare): the accumulators started at 0, so the scores carry the very bits pass 1 saw;
+            // m_i is subtracted before the scale and log2 l_i after it
+            auto shifted_p = [&](const floatx16 &sc, int nb, int i4, float (&pr)[4]) {
+                floatx4 l4, m4;
+                int g_o = g;
+                asm volatile("" : "+v"(g_o));  // addresses are formed here, not kept through the stream
+                const uint32_t ro = (uint32_t)((wave * ROWS_W + nb * 32 + 8 * i4 + 4 * g_o) * 4);
+                const uint32_t ad = lds_addr(lg_s) + ro, am = lds_addr(cm_s) + ro;
+                asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                             : "=&v"(l4), "=&v"(m4)
+                             : "v"(ad), "v"(am)
+                             : "memory");
+#pragma unroll
+                for (int j = 0; j < 4; ++j) pr[j] = fast_exp2(fmaf(sc[4 * i4 + j] + m4[j], cmul, -l4[j]));
+            };
+            auto drain_plain = [&](const floatx16 &sc, int nb) {
+                if constexpr (SHIFTED) {
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        float pr[4];
+                        shifted_p(sc, nb, i4, pr);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) cp[j] += pr[j];
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) cp[i & 3] += fast_exp2(SC ? sc[i] : sc[i] * cmul);
+                }
+            };
+            auto drain_masked = [&](const floatx16 &sc, int kb_t, int na, int nb) {
                 const int key = kb_t + na * 32 + n;
                 // visible  <=>  key < Sk  and  key - k_past - (row of register i) <= 0
                 int rel = (key < a.Sk) ? key - kp_eff - (qw0 + 4 * g) : 0x3fffffff;
                 asm volatile("" : "+v"(rel));
-                // FOLD: the row within its head is less by the rows of the heads before it
-                int v_first = qw0 + nb * 32 + 4 * g;
-                if (FOLD) asm volatile("" : "+v"(v_first));  // formed here, not kept for every register through the stream
-                auto ahead = [&](int i) { return FOLD ? fold_head(v_first + 8 * (i >> 2) + (i & 3), a.fold_magic) * a.q_rows : 0; };
-                if (shifted) {
-                    // rare: the accumulators started at 0, so the scores carry the very bits pass 1 saw;
-                    // m_i is subtracted before the scale and log2 l_i after it
+                auto add = [&](auto ahead) {  // ahead(i): rows of the heads before the row of register i (FOLD)
 #pragma unroll
                     for (int i4 = 0; i4 < 4; ++i4) {
-                        floatx4 l4, m4;
-                        const uint32_t ro = (uint32_t)((wave * ROWS_W + nb * 32 + 8 * i4 + 4 * g) * 4);
-                        const uint32_t ad = lds_addr(lg_s) + ro, am = lds_addr(cm_s) + ro;
-                        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-                                     : "=&v"(l4), "=&v"(m4)
-                                     : "v"(ad), "v"(am)
-                                     : "memory");
+                        float pr[4];
+                        if constexpr (SHIFTED) {
+                            shifted_p(sc, nb, i4, pr);
+                        } else {
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const float pr = fast_exp2(fmaf(sc[4 * i4 + j] + m4[j], cmul, -l4[j]));
-                            cp[j] += (rel + ahead(4 * i4 + j) <= nb * 32 + 8 * i4 + j) ? pr : 0.f;
+                            for (int j = 0; j < 4; ++j) pr[j] = fast_exp2(SC ? sc[4 * i4 + j] : sc[4 * i4 + j] * cmul);
                         }
-                    }
-                } else {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const float pr = fast_exp2(SC ? sc[i] : sc[i] * cmul);
-                        cp[i & 3] += (rel + ahead(i) <= nb * 32 + 8 * (i >> 2) + (i & 3)) ? pr : 0.f;
+                        for (int j = 0; j < 4; ++j) cp[j] += (rel + ahead(4 * i4 + j) <= nb * 32 + 8 * i4 + j) ? pr[j] : 0.f;
                     }
-                }
+                };
+                mask_rows<FOLD>(a, qw0 + nb * 32, 4 * g, rel, add);
             };
             auto drain_end = [&](int nb) {
                 if (nb == NB - 1) {
@@ -463,31 +518,34 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 for (int t = 1; t < NT; ++t) c = mfma16<BF>(qf[nb][t], kf[t], c);
                 return c;
             };
-            auto drain_fast = [&](const floatx16 &sc) {  // every key of the tile visible, no stabilised row
-#pragma unroll
-                for (int i = 0; i < 16; ++i) cp[i & 3] += fast_exp2(SC ? sc[i] : sc[i] * cmul);
-            };
 
-            // one stage, in ring slot SLOT (compile-time)
-            auto stage = [&](int st, auto slot_c) {
-                constexpr int SLOT = decltype(slot_c)::value;
-                const int kb = c0 + st * KT;
-                if (st > s0) {
-                    // stage st + 1 has landed (this wave's pieces; the barrier extends that to everyone's), and
-                    // every wave is done reading stage st - 1, whose slot takes the next fetch
-                    FCS_WAIT_VM((NS - 3) * IPW);
-                    block_barrier();
-                }
-                fetch_stage(st + NS - 1, (SLOT + NS - 1) % NS);
+            // ---- the plain stream: stages [s0, sp).  Software pipeline inside the wave: the MFMA chain of tile q is
+            // issued BEFORE the exponent work of tile q - 1, so the matrix pipe and the VALU run together whatever
+            // the phase of the other wave on the SIMD.  (Measured slower: the exponent work woven between the
+            // chain's MFMAs, and the two waves of a SIMD in opposite order.)  Nothing in here depends on where the
+            // stage lies; the waves of a block may leave it at different stages, since both loops pass one barrier
+            // and issue the same fetches per stage.
+            const int sp = min(s1, max(s0, n_plain));
+            if (sp > s0) {
+                take_frag(std::integral_constant<int, 0>{}, kf);
+                floatx16 acc[2];
 #pragma unroll
-                for (int q = 0; q < TILES; ++q) {
-                    const int na = q / NB, nb = q % NB;
-                    // the previous tile: the one before in this stage, or the last of the previous stage
-                    const int p_kb = (q > 0) ? kb : kb - KT;
-                    const int p_na = (q > 0) ? (q - 1) / NB : NA - 1, p_nb = (q > 0) ? (q - 1) % NB : NB - 1;
-                    const bool have_prev = (q > 0) || (st > s0);
-                    const bool p_fast = !shifted && !(p_kb + p_na * 32 + 31 > thr_wave_min);  // wave-uniform
-                    auto do_chain = [&]() {
+                for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+                // one stage, in ring slot SLOT (compile-time; the phase's first stage is in slot 0)
+                auto stage = [&](int st, auto slot_c) {
+                    constexpr int SLOT = decltype(slot_c)::value;
+                    const int kb = c0 + st * KT;
+                    const bool first = SLOT == 0 && st == s0;
+                    if (!first) {
+                        // stage st + 1 has landed (this wave's pieces; the barrier extends that to everyone's), and
+                        // every wave is done reading stage st - 1, whose slot takes the next fetch
+                        FCS_WAIT_VM((NS - 3) * IPW);
+                        block_barrier();
+                    }
+                    fetch_stage(st + NS - 1, (SLOT + NS - 1) % NS);
+#pragma unroll
+                    for (int q = 0; q < TILES; ++q) {
+                        const int na = q / NB, nb = q % NB;
                         if (nb == 0) frag_wait(kf);
                         acc[q & 1] = chain(nb);
                         asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));  // the chain stays where it was written
@@ -495,51 +553,81 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                             if (na == 0) take_frag(std::integral_constant<int, SLOT * STAGE_BYTES + 32 * ROW_BYTES>{}, kf);
                             else take_frag(std::integral_constant<int, ((SLOT + 1) % NS) * STAGE_BYTES>{}, kf);
                         }
-                    };
-                    auto do_drain = [&]() {
-                        if (!have_prev) return;
-                        drain_begin(p_kb, p_na, p_nb);
-                        if (p_fast) drain_fast(acc[(q - 1) & 1]);
-                        else drain_slow(acc[(q - 1) & 1], p_kb, p_na, p_nb);
-                        drain_end(p_nb);
-                        asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
-                    };
-                    // Chain first: the matrix pipe works on tile q while the VALU exponentiates tile q - 1.
-                    // (Measured slower: the exponent work woven between the chain's MFMAs, and the two waves
-                    // of a SIMD in opposite order.)
-                    do_chain();
-                    do_drain();
+                        // the tile before: in this stage, or the last one of the previous stage
+                        const int p_kb = (q > 0) ? kb : kb - KT;
+                        const int p_na = (q > 0) ? (q - 1) / NB : NA - 1, p_nb = (q > 0) ? (q - 1) % NB : NB - 1;
+                        if (q > 0 || !first) {
+                            drain_begin(p_kb, p_na, p_nb);
+                            drain_plain(acc[(q + 1) & 1], p_nb);
+                            drain_end(p_nb);
+                            asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                        }
+                    }
+                };
+                for (int st0 = s0; st0 < sp; st0 += NS) {
+                    stage(st0, std::integral_constant<int, 0>{});
+                    if (st0 + 1 < sp) stage(st0 + 1, std::integral_constant<int, 1>{});
+                    if (st0 + 2 < sp) stage(st0 + 2, std::integral_constant<int, 2>{});
+                    if (NS > 3 && st0 + 3 < sp) stage(st0 + 3, std::integral_constant<int, 3 % NS>{});
                 }
-            };
-            static_assert(NA == 2, "fragment offsets above");
-            for (int st0 = s0; st0 < s1; st0 += NS) {
-                stage(st0, std::integral_constant<int, 0>{});
-                if (st0 + 1 < s1) stage(st0 + 1, std::integral_constant<int, 1>{});
-                if (st0 + 2 < s1) stage(st0 + 2, std::integral_constant<int, 2>{});
-                if (NS > 3 && st0 + 3 < s1) stage(st0 + 3, std::integral_constant<int, 3 % NS>{});
+                static_assert(NS <= 4, "unrolled above");
+                frag_wait(kf);  // the read-back past the last stage is not used
+                drain_begin(c0 + (sp - 1) * KT, NA - 1, NB - 1);
+                drain_plain(acc[(TILES - 1) & 1], NB - 1);
+                drain_end(NB - 1);
             }
-            static_assert(NS <= 4, "unrolled above");
-            drain_begin(c0 + (s1 - 1) * KT, NA - 1, NB - 1);
-            drain_slow(acc[(TILES - 1) & 1], c0 + (s1 - 1) * KT, NA - 1, NB - 1);
-            drain_end(NB - 1);
-            // the look-ahead fetches and the operand read-back issued past the last stage must be over before
-            // the ring (and nl_s) is reused by the next phase or unit
+
+            // ---- the rest of the phase, tile by tile: stages on the diagonal or past the last key.  A stage that
+            // no row of the wave sees passes its barrier and its fetch only.
+            int slot = (sp - s0) % NS;
+            for (int st = sp; st < s1; ++st) {
+                const int kb = c0 + st * KT;
+                if (st > s0) {
+                    FCS_WAIT_VM((NS - 3) * IPW);
+                    block_barrier();
+                }
+                fetch_stage(st + NS - 1, (slot + NS - 1) % NS);
+                if (kb <= thr_wave_max) {
+#pragma unroll 1
+                    for (int na = 0; na < NA; ++na) {
+                        const uint32_t off = (uint32_t)(slot * STAGE_BYTES + na * 32 * ROW_BYTES);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) {
+                            const uint32_t ad = take[t] + off;
+                            asm volatile("ds_read_b128 %0, %1" : "=v"(kf[t]) : "v"(ad) : "memory");
+                        }
+                        frag_wait(kf);
+                        floatx16 acc[NB];
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb) acc[nb] = chain(nb);
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb) {
+                            drain_begin(kb, na, nb);
+                            drain_masked(acc[nb], kb, na, nb);
+                            drain_end(nb);
+                        }
+                    }
+                }
+                slot = (slot + 1 == NS) ? 0 : slot + 1;
+            }
+            // the look-ahead fetches issued past the last stage must be over before the ring (and nl_s) is reused by
+            // the next phase or unit
             FCS_WAIT_VM(0);
-            frag_wait(kf);
             block_sync();
         };
 
-        // (one call site per form of the operand, so that the stream's code exists twice, not three times)
+        // (one call site per form, so that the code of each exists once)
         int raw0 = 0;  // first stage of the raw phase
         if (PRE && n_pre > 0) {
             shape_q(true);
-            run_phase(std::true_type{}, 0, n_pre, true);
+            run_phase(std::integral_constant<int, kFormPrescaled>{}, 0, n_pre, true);
             raw0 = n_pre;
             if (raw0 < nst) load_q_rows();  // the unit's last stages (causal: keys that not every row sees)
         }
         if (raw0 < nst) {
             shape_q(false);
-            run_phase(std::false_type{}, raw0, nst, raw0 == 0);
+            if (shifted) run_phase(std::integral_constant<int, kFormShifted>{}, 0, nst, true);
+            else run_phase(std::integral_constant<int, kFormRaw>{}, raw0, nst, raw0 == 0);
         }
     }
 
@@ -648,11 +736,13 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     const int64_t k_row_b = a.ks_s * 2;
     const int kp_eff = a.causal ? a.k_past : 0x3fffffff - a.Sq;
     const int thr_wave_min = a.causal ? min(a.k_past + rows_first<FOLD>(a, qw0, ROWS_W), a.Sk - 1) : a.Sk - 1;
+    const int thr_wave_max = a.causal ? a.k_past + (FOLD ? a.q_rows : qw0 + ROWS_W) - 1 : a.Sk - 1;
+    const int n_plain = plain_stages(kc0, nst, thr_wave_min);
 
     auto fetch_stage = [&](int st, int slot) {
         const int kb = kc0 + min(st, nst - 1) * KT;
         char *dst = ring_w + slot * STAGE_BYTES;
-        if (kb + KT <= a.Sk && a.D == D) {
+        if (__builtin_expect(kb + KT <= a.Sk && a.D == D, 1)) {
             const char *src = kp + (int64_t)kb * k_row_b;
 #pragma unroll
             for (int j = 0; j < IPW; ++j) dma16(src + g_off[j], dst + j * 1024);
@@ -711,69 +801,101 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         for (int st = 0; st < NS - 1; ++st) fetch_stage(s0 + st, st);
         FCS_WAIT_VM((NS - 3) * IPW);
         block_sync();
-        take_frag(std::integral_constant<int, 0>{}, kf);
-        floatx16 acc[2];
+        auto drain_plain = [&](const floatx16 &sc, int nb) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
-        auto drain = [&](const floatx16 &sc, int kb_t, int na, int nb) {
-            const bool edge = kb_t + na * 32 + 31 > thr_wave_min;  // wave-uniform
-            if (!edge) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    if (MAXOP) rs[nb][i] = fmaxf(rs[nb][i], sc[i]);
-                    else rs[nb][i] += SCALED ? fast_exp2(sc[i]) : fast_exp2((SHIFT ? sc[i] + nmax[nb][i] : sc[i]) * cmul);
-                }
-            } else {
-                const int key = kb_t + na * 32 + n;
-                int rel = (key < a.Sk) ? key - kp_eff - (qw0 + 4 * g) : 0x3fffffff;
-                asm volatile("" : "+v"(rel));
-                int v_first = qw0 + nb * 32 + 4 * g;
-                if (FOLD) asm volatile("" : "+v"(v_first));  // formed here, not kept for every register through the stream
+            for (int i = 0; i < 16; ++i) {
+                if (MAXOP) rs[nb][i] = fmaxf(rs[nb][i], sc[i]);
+                else rs[nb][i] += SCALED ? fast_exp2(sc[i]) : fast_exp2((SHIFT ? sc[i] + nmax[nb][i] : sc[i]) * cmul);
+            }
+        };
+        auto drain_masked = [&](const floatx16 &sc, int kb_t, int na, int nb) {
+            const int key = kb_t + na * 32 + n;
+            int rel = (key < a.Sk) ? key - kp_eff - (qw0 + 4 * g) : 0x3fffffff;
+            asm volatile("" : "+v"(rel));
+            mask_rows<FOLD>(a, qw0 + nb * 32, 4 * g, rel, [&](auto ahead) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    // FOLD: the row within its head is less by the rows of the heads before it
-                    const int ahead = FOLD ? fold_head(v_first + 8 * (i >> 2) + (i & 3), a.fold_magic) * a.q_rows : 0;
-                    const bool vis = rel + ahead <= nb * 32 + 8 * (i >> 2) + (i & 3);
+                    const bool vis = rel + ahead(i) <= nb * 32 + 8 * (i >> 2) + (i & 3);
                     if (MAXOP) rs[nb][i] = fmaxf(rs[nb][i], vis ? sc[i] : kNegBig);
                     else rs[nb][i] += vis ? (SCALED ? fast_exp2(sc[i]) : fast_exp2((SHIFT ? sc[i] + nmax[nb][i] : sc[i]) * cmul)) : 0.f;
                 }
-            }
+            });
         };
-        auto stage = [&](int st, auto slot_c) {
-            constexpr int SLOT = decltype(slot_c)::value;
+        const floatx16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        auto chain = [&](int nb) {
+            floatx16 c = mfma16<BF>(qf[nb][0], kf[0], zero16);
+#pragma unroll
+            for (int t = 1; t < NT; ++t) c = mfma16<BF>(qf[nb][t], kf[t], c);
+            return c;
+        };
+
+        // ---- the plain stream (see the column pass): stages [s0, sp)
+        const int sp = min(s1, max(s0, n_plain));
+        if (sp > s0) {
+            take_frag(std::integral_constant<int, 0>{}, kf);
+            floatx16 acc[2];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+            auto stage = [&](int st, auto slot_c) {
+                constexpr int SLOT = decltype(slot_c)::value;
+                const bool first = SLOT == 0 && st == s0;
+                if (!first) {
+                    FCS_WAIT_VM((NS - 3) * IPW);
+                    block_barrier();
+                }
+                fetch_stage(st + NS - 1, (SLOT + NS - 1) % NS);
+#pragma unroll
+                for (int q = 0; q < TILES; ++q) {
+                    const int na = q / NB, nb = q % NB;
+                    if (nb == 0) frag_wait(kf);
+                    acc[q & 1] = chain(nb);
+                    asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                    if (nb == NB - 1) {
+                        if (na == 0) take_frag(std::integral_constant<int, SLOT * STAGE_BYTES + 32 * ROW_BYTES>{}, kf);
+                        else take_frag(std::integral_constant<int, ((SLOT + 1) % NS) * STAGE_BYTES>{}, kf);
+                    }
+                    if (q > 0 || !first) drain_plain(acc[(q + 1) & 1], (q > 0) ? (q - 1) % NB : NB - 1);
+                }
+            };
+            for (int st0 = s0; st0 < sp; st0 += NS) {
+                stage(st0, std::integral_constant<int, 0>{});
+                if (st0 + 1 < sp) stage(st0 + 1, std::integral_constant<int, 1>{});
+                if (st0 + 2 < sp) stage(st0 + 2, std::integral_constant<int, 2>{});
+                if (NS > 3 && st0 + 3 < sp) stage(st0 + 3, std::integral_constant<int, 3 % NS>{});
+            }
+            frag_wait(kf);  // the read-back past the last stage is not used
+            drain_plain(acc[(TILES - 1) & 1], NB - 1);
+        }
+
+        // ---- the rest, tile by tile; a stage that no row of the wave sees passes its barrier and its fetch only
+        int slot = (sp - s0) % NS;
+        for (int st = sp; st < s1; ++st) {
             const int kb = kc0 + st * KT;
             if (st > s0) {
                 FCS_WAIT_VM((NS - 3) * IPW);
                 block_barrier();
             }
-            fetch_stage(st + NS - 1, (SLOT + NS - 1) % NS);
+            fetch_stage(st + NS - 1, (slot + NS - 1) % NS);
+            if (kb <= thr_wave_max) {
+#pragma unroll 1
+                for (int na = 0; na < NA; ++na) {
+                    const uint32_t off = (uint32_t)(slot * STAGE_BYTES + na * 32 * ROW_BYTES);
 #pragma unroll
-            for (int q = 0; q < TILES; ++q) {
-                const int na = q / NB, nb = q % NB;
-                if (nb == 0) frag_wait(kf);
-                const floatx16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                floatx16 c = mfma16<BF>(qf[nb][0], kf[0], zero16);
+                    for (int t = 0; t < NT; ++t) {
+                        const uint32_t ad = take[t] + off;
+                        asm volatile("ds_read_b128 %0, %1" : "=v"(kf[t]) : "v"(ad) : "memory");
+                    }
+                    frag_wait(kf);
+                    floatx16 acc[NB];
 #pragma unroll
-                for (int t = 1; t < NT; ++t) c = mfma16<BF>(qf[nb][t], kf[t], c);
-                acc[q & 1] = c;
-                asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
-                if (nb == NB - 1) {
-                    if (na == 0) take_frag(std::integral_constant<int, SLOT * STAGE_BYTES + 32 * ROW_BYTES>{}, kf);
-                    else take_frag(std::integral_constant<int, ((SLOT + 1) % NS) * STAGE_BYTES>{}, kf);
+                    for (int nb = 0; nb < NB; ++nb) acc[nb] = chain(nb);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) drain_masked(acc[nb], kb, na, nb);
                 }
-                if (q > 0) drain(acc[(q - 1) & 1], kb, (q - 1) / NB, (q - 1) % NB);
-                else if (st > s0) drain(acc[(TILES - 1) & 1], kb - KT, NA - 1, NB - 1);
             }
-        };
-        for (int st0 = s0; st0 < s1; st0 += NS) {
-            stage(st0, std::integral_constant<int, 0>{});
-            if (st0 + 1 < s1) stage(st0 + 1, std::integral_constant<int, 1>{});
-            if (st0 + 2 < s1) stage(st0 + 2, std::integral_constant<int, 2>{});
-            if (NS > 3 && st0 + 3 < s1) stage(st0 + 3, std::integral_constant<int, 3 % NS>{});
+            slot = (slot + 1 == NS) ? 0 : slot + 1;
         }
-        drain(acc[(TILES - 1) & 1], kc0 + (s1 - 1) * KT, NA - 1, NB - 1);
         FCS_WAIT_VM(0);
-        frag_wait(kf);
         block_sync();  // the ring may be refilled by the next sweep
     };
 

@@ -18,7 +18,7 @@ def _check(q, k, kw, what):
     assert ((out - ref).abs() <= 1e-4).all() and ((out - ref).abs() <= 1e-3 * ref.abs()).all(), (what, (out - ref).abs().max())
 
 
-@pytest.mark.parametrize("group,q_len", [(2, 1), (8, 1), (3, 31), (4, 33), (8, 16), (5, 64), (2, 128), (8, 100), (3, 300), (2, 511), (2, 512)])
+@pytest.mark.parametrize("group,q_len", [(2, 1), (8, 1), (3, 31), (4, 33), (8, 16), (5, 64), (2, 128), (2, 129), (8, 100), (3, 300), (2, 511), (2, 512)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_rows_of_grouped_heads(group, q_len, causal):
     for dtype, d, hk, b in [(torch.bfloat16, 128, 2, 2), (torch.float16, 64, 1, 3), (torch.float16, 40, 2, 1), (torch.bfloat16, 192, 1, 1)]:
