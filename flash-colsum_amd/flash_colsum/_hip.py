@@ -93,6 +93,9 @@ def lib() -> ctypes.CDLL:
         cdll.fcs_threshold_f32.restype = ctypes.c_int
         cdll.fcs_threshold_f32.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_void_p,
                                            ctypes.c_void_p, ctypes.c_void_p]
+        cdll.fcs_round_f16.restype = ctypes.c_int
+        cdll.fcs_round_f16.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+                                       ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
         got = cdll.fcs_abi_version()
         if got != _ABI_VERSION:
             raise RuntimeError(f"libflashcolsum.so has ABI {got}, this host layer needs {_ABI_VERSION}")
@@ -287,6 +290,43 @@ def _wide_operands(q: torch.Tensor, k: torch.Tensor):
     return torch.cat([q_hi, q_hi, q_lo, q_lo], dim=-1), torch.cat([k_hi, k_lo, k_hi, k_lo], dim=-1), torch.bfloat16
 
 
+def _dense_storage(t: torch.Tensor) -> bool:
+    """The elements fill t's storage range without gaps or overlap, in (B, H, S, D) or (B, S, H, D) order."""
+    return t.is_contiguous() or t.transpose(1, 2).is_contiguous()
+
+
+def _range_flag(dev: torch.device):
+    """The calling thread's range flag for this GPU (one pinned word) and the event that says it may be read."""
+    flags = getattr(_tls, "range_flags", None)
+    if flags is None:
+        flags = _tls.range_flags = {}
+    ent = flags.get(dev.index)
+    if ent is None:
+        word = torch.zeros((1,), dtype=torch.int32, pin_memory=True)
+        ent = flags[dev.index] = (word, word.data_ptr(), ctypes.c_uint32.from_address(word.data_ptr()), torch.cuda.Event())
+    return ent
+
+
+def _rounded_operands(q: torch.Tensor, k: torch.Tensor):
+    """fp32 operands as fp16, enqueued in one launch with the range test of `_wide_operands`: (q, k, flag), or None
+    where the storage does not allow it.  The caller enqueues the column means behind it, then waits for the event of
+    `flag` (recorded right behind the rounding) and takes `_wide_operands` instead when the word is set."""
+    if (q.dtype != torch.float32 or k.dtype != torch.float32 or k.device != q.device or not _dense_storage(q) or not _dense_storage(k)
+            or q.numel() == 0 or k.numel() == 0 or q.data_ptr() % 16 or k.data_ptr() % 16
+            or torch.cuda.is_current_stream_capturing()):
+        return None
+    q_h, k_h = torch.empty_like(q, dtype=torch.float16), torch.empty_like(k, dtype=torch.float16)
+    if q_h.stride() != q.stride() or k_h.stride() != k.stride():
+        return None
+    flag = _range_flag(q.device)
+    flag[2].value = 0
+    with torch.cuda.device(q.device):
+        _check(lib().fcs_round_f16(q.data_ptr(), q_h.data_ptr(), q.numel(), k.data_ptr(), k_h.data_ptr(), k.numel(), flag[1],
+                                   _current_stream(q.device)), "fcs_round_f16")
+        flag[3].record()
+    return q_h, k_h, flag
+
+
 def _launch(causal: bool, q: torch.Tensor, k: torch.Tensor, scale: float, cls_n: int, k_past: int, want_f16: bool = False,
             f16_only: bool = False):
     """Enqueue one call; returns the fp32 means, (fp32, fp16) when `want_f16`, or the fp16 tensor alone
@@ -299,6 +339,15 @@ def _launch(causal: bool, q: torch.Tensor, k: torch.Tensor, scale: float, cls_n:
     if q.dtype in half and k.dtype in half:
         dtype = torch.bfloat16 if (q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16) else torch.float16
     else:
+        rounded = _rounded_operands(q, k)
+        if rounded is not None:
+            # the means of the rounded operands are enqueued before the range test is known, so that the GPU does not
+            # wait for the host; operands beyond the range are rare and computed again below
+            q_h, k_h, (_, _, word, event) = rounded
+            out = _launch(causal, q_h, k_h, scale, cls_n, k_past, want_f16, f16_only)
+            event.synchronize()
+            if not word.value:
+                return out
         q, k, dtype = _wide_operands(q, k)
     # The library takes head dims that are a multiple of 8 (16-byte rows) up to 256 as they are.  Only a
     # head dim that is not a multiple of 8 is padded with zero channels to the next one (a copy), which

@@ -205,6 +205,13 @@ int fcs_topk_f32(const float *means, int B, int S, int k, int64_t *idx_out, floa
 int fcs_threshold_f32(const float *means, int B, int S, float tau, int64_t *idx_out, int32_t *count_out,
                       void *hip_stream);
 
+/* fp32 operands rounded to fp16 (to nearest, ties to even), both in one launch: dst0[i] = src0[i] for i < n0,
+ * dst1[i] = src1[i] for i < n1, all four pointers 16-byte aligned.  *flag, in memory that the GPU can write and the
+ * caller can read (pinned host memory or device memory), becomes 1 when a value is a NaN or beyond +-65504 and is not
+ * touched otherwise: the caller clears it before the call and reads it after the kernel has ended. */
+int fcs_round_f16(const float *src0, void *dst0, int64_t n0, const float *src1, void *dst1, int64_t n1, uint32_t *flag,
+                  void *hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,60 @@
+"""fp32 operands: rounded to fp16 in one pass with the range test.  The result is that of the same operands rounded by torch
+beforehand, bit for bit, whatever the storage order, the element count modulo the kernel's 8-element pieces and its steps of
+1024 pieces; a value beyond the range anywhere takes the other route."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _f32(q, k, **kw):
+    from flash_colsum import flash_colsum_f32
+
+    return flash_colsum_f32(q, k, **kw)
+
+
+@pytest.mark.parametrize("b,h,s,d", [(1, 1, 1, 1), (1, 1, 3, 5), (1, 3, 7, 9), (2, 4, 33, 8), (1, 2, 511, 20), (1, 4, 2048, 2), (3, 5, 577, 64), (2, 16, 1025, 64)])
+@pytest.mark.parametrize("layout", ["heads", "tokens", "gaps", "offset"])
+def test_rounded_operands(b, h, s, d, layout):
+    g = torch.Generator().manual_seed(s * 10 + d)
+    x = []
+    for _ in range(2):
+        if layout == "tokens":
+            x.append(torch.randn((b, s, h, d), generator=g).cuda().transpose(1, 2))
+        elif layout == "gaps":  # rows with space between them
+            x.append(torch.randn((b, h, s, d + 3), generator=g).cuda()[..., :d])
+        elif layout == "offset":  # base not 16-byte aligned
+            x.append(torch.randn((b * h * s * d + 1,), generator=g).cuda()[1:].view(b, h, s, d))
+        else:
+            x.append(torch.randn((b, h, s, d), generator=g).cuda())
+    print("fp32 operands", b, h, s, d, layout, flush=True)
+    q, k = x
+    for kw in [{}, {"cls_len": 1}]:
+        assert torch.equal(_f32(q, k, **kw), _f32(q.half(), k.half(), **kw)), (b, h, s, d, layout, kw)
+    if b == 1:
+        assert torch.equal(_f32(q, k, is_causal=True), _f32(q.half(), k.half(), is_causal=True))
+
+
+@pytest.mark.parametrize("where", [0, 7, 8, 8191, 8192, -1])
+@pytest.mark.parametrize("operand", ["q", "k"])
+def test_one_value_beyond_the_range(where, operand):
+    """The first and last element, the edges of a piece and of a workgroup's step; then an in-range call: no stale flag."""
+    g = torch.Generator().manual_seed(3)
+    q, k = (torch.randn((1, 3, 301, 25), generator=g).cuda() for _ in range(2))
+    clean = _f32(q, k)
+    hurt = {"q": q, "k": k}
+    t = hurt[operand].clone()
+    hurt[operand] = t
+    for value in [float("-inf")] + [float("nan")] * (operand == "q"):
+        t.view(-1)[where] = value
+        with pytest.raises(ValueError, match="NaN or infinite"):
+            _f32(hurt["q"], hurt["k"])
+    t.view(-1)[where] = 65504.0
+    assert torch.equal(_f32(hurt["q"], hurt["k"], scale=1e-6), _f32(hurt["q"].half(), hurt["k"].half(), scale=1e-6))
+    t.view(-1)[where] = -65505.0  # would round to -65504: still the other route, whose operands keep 16 bits
+    from oracle import colsum_exact
+
+    ref = colsum_exact(hurt["q"].double(), hurt["k"].double(), scale=1e-6)
+    got = _f32(hurt["q"], hurt["k"], scale=1e-6).double()
+    assert ((got - ref).abs() <= 1e-3 * ref.abs()).all()
+    assert torch.equal(_f32(q, k), clean)
