@@ -309,10 +309,11 @@ def _range_flag(dev: torch.device):
 
 def _rounded_operands(q: torch.Tensor, k: torch.Tensor):
     """fp32 operands as fp16, enqueued in one launch with the range test of `_wide_operands`: (q, k, flag), or None
-    where the storage does not allow it.  The caller enqueues the column means behind it, then waits for the event of
-    `flag` (recorded right behind the rounding) and takes `_wide_operands` instead when the word is set."""
+    where the storage does not allow it (gaps, a misaligned base, a negation that torch has put off).  The caller
+    enqueues the column means behind it, then waits for the event of `flag` (recorded right behind the rounding) and
+    takes `_wide_operands` instead when the word is set."""
     if (q.dtype != torch.float32 or k.dtype != torch.float32 or k.device != q.device or not _dense_storage(q) or not _dense_storage(k)
-            or q.numel() == 0 or k.numel() == 0 or q.data_ptr() % 16 or k.data_ptr() % 16
+            or q.numel() == 0 or k.numel() == 0 or q.is_neg() or k.is_neg() or q.data_ptr() % 16 or k.data_ptr() % 16
             or torch.cuda.is_current_stream_capturing()):
         return None
     q_h, k_h = torch.empty_like(q, dtype=torch.float16), torch.empty_like(k, dtype=torch.float16)
@@ -344,8 +345,10 @@ def _launch(causal: bool, q: torch.Tensor, k: torch.Tensor, scale: float, cls_n:
             # the means of the rounded operands are enqueued before the range test is known, so that the GPU does not
             # wait for the host; operands beyond the range are rare and computed again below
             q_h, k_h, (_, _, word, event) = rounded
-            out = _launch(causal, q_h, k_h, scale, cls_n, k_past, want_f16, f16_only)
-            event.synchronize()
+            try:
+                out = _launch(causal, q_h, k_h, scale, cls_n, k_past, want_f16, f16_only)
+            finally:
+                event.synchronize()  # also after an error: the word is written by this call's kernel alone
             if not word.value:
                 return out
         q, k, dtype = _wide_operands(q, k)

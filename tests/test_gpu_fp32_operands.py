@@ -58,3 +58,12 @@ def test_one_value_beyond_the_range(where, operand):
     got = _f32(hurt["q"], hurt["k"], scale=1e-6).double()
     assert ((got - ref).abs() <= 1e-3 * ref.abs()).all()
     assert torch.equal(_f32(q, k), clean)
+
+
+def test_negation_that_torch_has_put_off():
+    """A tensor with torch's negative bit holds the opposite of what its storage says: it is resolved before the kernel reads it."""
+    g = torch.Generator().manual_seed(5)
+    q, k = (torch.randn((1, 3, 301, 64), generator=g).cuda() for _ in range(2))
+    lazy = torch._neg_view(q)
+    assert lazy.is_neg()
+    assert torch.equal(_f32(lazy, k), _f32((-q).half(), k.half()))
