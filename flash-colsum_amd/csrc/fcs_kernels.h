@@ -60,7 +60,7 @@ hipError_t launch_fewrows(const Plan &p, const Args &a, hipStream_t st);
 // short-sequence path (fcs_small.hip): p.small == 1
 hipError_t launch_small(const Plan &p, const Args &a, hipStream_t st);
 
-// row-statistics pass and column pass of the two-pass path (fcs_stream.hip)
+// row-statistics pass and column pass of the two-pass path (fcs_stream_kernels.h)
 hipError_t launch_rowstream(const Plan &p, const Args &a, hipStream_t st);
 hipError_t launch_colstream(const Plan &p, const Args &a, hipStream_t st);
 

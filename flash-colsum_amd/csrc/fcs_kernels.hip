@@ -1,8 +1,8 @@
 // Attention column means on gfx950 (MI355X): launch order of the paths and the final reduction.
 //
-//   pass 1 (fcs_rowstream_kernel, fcs_stream.hip)  per row (m, log2 l) with
+//   pass 1 (fcs_rowstream_kernel, fcs_stream_kernels.h)  per row (m, log2 l) with
 //          l = sum_j 2^((s_ij - m) * c), c = scale*log2(e), or (m, l) per key split.
-//   pass 2 (fcs_colstream_kernel, fcs_stream.hip)  column sums of 2^((s_ij - m_i) * c - log2 l_i),
+//   pass 2 (fcs_colstream_kernel, fcs_stream_kernels.h)  column sums of 2^((s_ij - m_i) * c - log2 l_i),
 //          one partial slab per group of (head, row block) units.
 //   fcs_finalize_kernel (here) adds the slabs in a fixed order: no atomics anywhere, every
 //          partial has exactly one writer.

@@ -17,12 +17,12 @@ constexpr int kSmallMaxTiles = 9;        // short-sequence path: one wave holds 
 // ... whose workgroups keep the keys of this many heads in an LDS ring (112 KB at most)
 constexpr int small_ring_heads(int tiles) { return 28 / tiles < 16 ? 28 / tiles : 16; }
 
-// column pass (fcs_stream.hip): ring slots of 64-key stages and keys per workgroup chunk, sized so
+// column pass (fcs_stream_kernels.h): ring slots of 64-key stages and keys per workgroup chunk, sized so
 // that the LDS ring plus one accumulator slice per wave fit (twice per compute unit for 4-wave blocks)
 constexpr int col_ring_slots(int D, int waves) { return (D == 256 || (D == 128 && waves == 4)) ? 3 : 4; }
 constexpr int col_chunk_max(int D, int waves) { return (D == 256) ? 1024 : (D == 128 && waves == 4) ? 1536 : 2048; }
 
-// row-statistics pass on the same stream (fcs_stream.hip): ring slots
+// row-statistics pass on the same stream (fcs_stream_kernels.h): ring slots
 constexpr int row_ring_slots(int D, int waves) { return (D == 256 || (D == 128 && waves == 4)) ? 3 : 4; }
 
 struct Plan {
