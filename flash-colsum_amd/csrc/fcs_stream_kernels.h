@@ -24,10 +24,17 @@
 //     that the operand reads (ds_read_b128, 32 rows a row pitch apart) are conflict-free.  One
 //     workgroup barrier per stage; the DMA is waited for by hand with s_waitcnt vmcnt(n).
 //   * The stream has two loops: the stages that every row of a wave sees run in one without any test of position
-//     (unrolled over the ring), the others (diagonal, last partial stage) in a short rolled one, where a wave skips
-//     the stages it does not see.  With the masked code inlined at every tile the kernel was 2.3 times as
-//     long and needed 254 registers at D 128 (now 211).  B 1, H 32, Q 512, K 65536, D 128: 601 -> 588 us per call,
-//     B 1, H 16, S 5000, D 64 bf16 208 -> 196, causal B 1, H 32, S 900, D 128 37.5 -> 33.9.
+//     (unrolled over the ring), the others (diagonal, last partial stage) in a short rolled one; stages that no row
+//     of a wave sees cost it a barrier and its share of the fetch.  With the masked code inlined at every tile the
+//     kernel was 2.3 times as long and needed 254 registers at D 128 (now 211).  Measured against that form, in
+//     turn: B 1, H 32, Q 512, K 65536, D 128 607 -> 599 us per call, causal B 1, H 32, S 900, D 128 38.5 -> 34.7,
+//     S 4096 bf16 233 -> 229.
+//     In the rolled loop 64-row waves take two tiles per key fragment, one after the other: the second chain runs
+//     under the first tile's exponent work, and the other waves fill the rest.  32-row waves have one tile per
+//     fragment, so there the software pipeline goes on (fragment read ahead, chain before the tile before's exponent
+//     work): a decode window has its masked stages in the last key split alone, whose workgroups end the launch.
+//     H 32, Q 128, K 16384, D 128, keys that change from call to call: 83.7 -> 81.9 us (inlined form: 82.2).  The
+//     same pipeline for 64-row waves was slower (H 32, S 2000, D 64 58.1 -> 60.0 us).
 // A workgroup owns a chunk of keys (at most kColChunkMax, the LDS accumulator) and walks over a
 // group of (head, row block) units, re-streaming its chunk for each; at the end the waves'
 // slices are added in wave order and written as one partial slab (or the means directly, when
@@ -139,6 +146,12 @@ __device__ __forceinline__ void mask_rows(const Args &a, int v0, int g4, int &re
 __device__ __forceinline__ int plain_stages(int k0, int nst, int thr)
 {
     return (thr + 1 >= k0) ? min(nst, (thr + 1 - k0) / kStageKeys) : 0;
+}
+
+// ... and how many of them hold a key up to `thr`, the last one that any row of it sees
+__device__ __forceinline__ int seen_stages(int k0, int nst, int thr)
+{
+    return (thr >= k0) ? min(nst, (thr - k0) / kStageKeys + 1) : 0;
 }
 
 // column pass: how the exponent is taken
@@ -356,6 +369,13 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(kf[t]) : "v"(ad), "n"(IMM) : "memory");
             }
         };
+        auto take_frag_at = [&](int off, half8 (&kf)[NT]) {  // the same at a run-time offset into the ring
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const uint32_t ad = take[t] + (uint32_t)off;
+                asm volatile("ds_read_b128 %0, %1" : "=v"(kf[t]) : "v"(ad) : "memory");
+            }
+        };
         auto frag_wait = [&](half8 (&kf)[NT]) {
             if constexpr (NT == 4)
                 asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(kf[0]), "+v"(kf[1]), "+v"(kf[2]), "+v"(kf[3])::"memory");
@@ -391,6 +411,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         const int thr_wave_max = a.causal ? a.k_past + (FOLD ? a.q_rows : qw0 + ROWS_W) - 1 : a.Sk - 1;             // last key ANY row of it sees
         // leading stages that every row of the wave sees: they run in the plain stream below
         const int n_plain = plain_stages(c0, nst, thr_wave_min);
+        const int n_seen = seen_stages(c0, nst, thr_wave_max);  // those that some row of it sees
 
         // One phase: the stages [s0, s1) of the unit in one FORM: raw operand, pre-scaled operand, or the
         // two-constant form of a unit with a stabilised row.  `fetched`: the phase's first NS - 1 stages are already
@@ -571,45 +592,70 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                     if (NS > 3 && st0 + 3 < sp) stage(st0 + 3, std::integral_constant<int, 3 % NS>{});
                 }
                 static_assert(NS <= 4, "unrolled above");
-                frag_wait(kf);  // the read-back past the last stage is not used
+                frag_wait(kf);  // (the first fragment of the next stage, if there is one)
                 drain_begin(c0 + (sp - 1) * KT, NA - 1, NB - 1);
                 drain_plain(acc[(TILES - 1) & 1], NB - 1);
                 drain_end(NB - 1);
             }
 
-            // ---- the rest of the phase, tile by tile: stages on the diagonal or past the last key.  A stage that
-            // no row of the wave sees passes its barrier and its fetch only.
+            // ---- the rest of the phase, in rolled loops (the ring slot is a run-time value): the stages on the diagonal or
+            // past the last key as far as some row of the wave sees them, [sp, sv), then those that none of its rows sees
+            const int sv = min(s1, max(sp, n_seen));
             int slot = (sp - s0) % NS;
-            for (int st = sp; st < s1; ++st) {
-                const int kb = c0 + st * KT;
+            auto enter_stage = [&](int st) {
                 if (st > s0) {
                     FCS_WAIT_VM((NS - 3) * IPW);
                     block_barrier();
                 }
-                fetch_stage(st + NS - 1, (slot + NS - 1) % NS);
-                if (kb <= thr_wave_max) {
+                fetch_stage(st + NS - 1, (slot == 0) ? NS - 1 : slot - 1);
+                slot = (slot + 1 == NS) ? 0 : slot + 1;
+            };
+            auto drain_one = [&](const floatx16 &sc, int kb_t, int na, int nb) {
+                drain_begin(kb_t, na, nb);
+                drain_masked(sc, kb_t, na, nb);
+                drain_end(nb);
+            };
+            if constexpr (NB == 1) {
+                if (sv > sp) {
+                    floatx16 acc[2];
+                    acc[0] = acc[1] = cinit[0];
+                    if (sp == s0) take_frag(std::integral_constant<int, 0>{}, kf);  // else the plain stream has read it
+                    frag_wait(kf);
+#pragma unroll 1
+                    for (int st = sp; st < sv; ++st) {
+                        const int kb = c0 + st * KT, here = slot * STAGE_BYTES;
+                        enter_stage(st);
+                        frag_wait(kf);
+                        acc[0] = chain(0);
+                        asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                        take_frag_at(here + 32 * ROW_BYTES, kf);
+                        if (st > sp) drain_one(acc[1], kb - KT, 1, 0);
+                        frag_wait(kf);
+                        acc[1] = chain(0);
+                        asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                        take_frag_at(slot * STAGE_BYTES, kf);
+                        drain_one(acc[0], kb, 0, 0);
+                    }
+                    frag_wait(kf);  // the read-back past the last stage is not used
+                    drain_one(acc[1], c0 + (sv - 1) * KT, 1, 0);
+                }
+            } else {
+                for (int st = sp; st < sv; ++st) {
+                    const int kb = c0 + st * KT, here = slot * STAGE_BYTES;
+                    enter_stage(st);
 #pragma unroll 1
                     for (int na = 0; na < NA; ++na) {
-                        const uint32_t off = (uint32_t)(slot * STAGE_BYTES + na * 32 * ROW_BYTES);
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) {
-                            const uint32_t ad = take[t] + off;
-                            asm volatile("ds_read_b128 %0, %1" : "=v"(kf[t]) : "v"(ad) : "memory");
-                        }
+                        take_frag_at(here + na * 32 * ROW_BYTES, kf);
                         frag_wait(kf);
                         floatx16 acc[NB];
 #pragma unroll
                         for (int nb = 0; nb < NB; ++nb) acc[nb] = chain(nb);
 #pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) {
-                            drain_begin(kb, na, nb);
-                            drain_masked(acc[nb], kb, na, nb);
-                            drain_end(nb);
-                        }
+                        for (int nb = 0; nb < NB; ++nb) drain_one(acc[nb], kb, na, nb);
                     }
                 }
-                slot = (slot + 1 == NS) ? 0 : slot + 1;
             }
+            for (int st = sv; st < s1; ++st) enter_stage(st);
             // the look-ahead fetches issued past the last stage must be over before the ring (and nl_s) is reused by
             // the next phase or unit
             FCS_WAIT_VM(0);
@@ -737,7 +783,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     const int kp_eff = a.causal ? a.k_past : 0x3fffffff - a.Sq;
     const int thr_wave_min = a.causal ? min(a.k_past + rows_first<FOLD>(a, qw0, ROWS_W), a.Sk - 1) : a.Sk - 1;
     const int thr_wave_max = a.causal ? a.k_past + (FOLD ? a.q_rows : qw0 + ROWS_W) - 1 : a.Sk - 1;
-    const int n_plain = plain_stages(kc0, nst, thr_wave_min);
+    const int n_plain = plain_stages(kc0, nst, thr_wave_min), n_seen = seen_stages(kc0, nst, thr_wave_max);
 
     auto fetch_stage = [&](int st, int slot) {
         const int kb = kc0 + min(st, nst - 1) * KT;
@@ -768,6 +814,13 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         for (int t = 0; t < NT; ++t) {
             const uint32_t ad = take[t] + (uint32_t)(OFF - IMM);
             asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst[t]) : "v"(ad), "n"(IMM) : "memory");
+        }
+    };
+    auto take_frag_at = [&](int off, half8 (&dst)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const uint32_t ad = take[t] + (uint32_t)off;
+            asm volatile("ds_read_b128 %0, %1" : "=v"(dst[t]) : "v"(ad) : "memory");
         }
     };
     auto frag_wait = [&](half8 (&dst)[NT]) {
@@ -863,28 +916,52 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
                 if (st0 + 2 < sp) stage(st0 + 2, std::integral_constant<int, 2>{});
                 if (NS > 3 && st0 + 3 < sp) stage(st0 + 3, std::integral_constant<int, 3 % NS>{});
             }
-            frag_wait(kf);  // the read-back past the last stage is not used
+            frag_wait(kf);
             drain_plain(acc[(TILES - 1) & 1], NB - 1);
         }
 
-        // ---- the rest, tile by tile; a stage that no row of the wave sees passes its barrier and its fetch only
+        // ---- the rest, as in the column pass
+        const int sv = min(s1, max(sp, n_seen));
         int slot = (sp - s0) % NS;
-        for (int st = sp; st < s1; ++st) {
-            const int kb = kc0 + st * KT;
+        auto enter_stage = [&](int st) {
             if (st > s0) {
                 FCS_WAIT_VM((NS - 3) * IPW);
                 block_barrier();
             }
-            fetch_stage(st + NS - 1, (slot + NS - 1) % NS);
-            if (kb <= thr_wave_max) {
+            fetch_stage(st + NS - 1, (slot == 0) ? NS - 1 : slot - 1);
+            slot = (slot + 1 == NS) ? 0 : slot + 1;
+        };
+        if constexpr (NB == 1) {
+            if (sv > sp) {
+                floatx16 acc[2];
+                acc[0] = acc[1] = zero16;
+                if (sp == s0) take_frag(std::integral_constant<int, 0>{}, kf);
+                frag_wait(kf);
+#pragma unroll 1
+                for (int st = sp; st < sv; ++st) {
+                    const int kb = kc0 + st * KT, here = slot * STAGE_BYTES;
+                    enter_stage(st);
+                    frag_wait(kf);
+                    acc[0] = chain(0);
+                    asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                    take_frag_at(here + 32 * ROW_BYTES, kf);
+                    if (st > sp) drain_masked(acc[1], kb - KT, 1, 0);
+                    frag_wait(kf);
+                    acc[1] = chain(0);
+                    asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                    take_frag_at(slot * STAGE_BYTES, kf);
+                    drain_masked(acc[0], kb, 0, 0);
+                }
+                frag_wait(kf);  // the read-back past the last stage is not used
+                drain_masked(acc[1], kc0 + (sv - 1) * KT, 1, 0);
+            }
+        } else {
+            for (int st = sp; st < sv; ++st) {
+                const int kb = kc0 + st * KT, here = slot * STAGE_BYTES;
+                enter_stage(st);
 #pragma unroll 1
                 for (int na = 0; na < NA; ++na) {
-                    const uint32_t off = (uint32_t)(slot * STAGE_BYTES + na * 32 * ROW_BYTES);
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        const uint32_t ad = take[t] + off;
-                        asm volatile("ds_read_b128 %0, %1" : "=v"(kf[t]) : "v"(ad) : "memory");
-                    }
+                    take_frag_at(here + na * 32 * ROW_BYTES, kf);
                     frag_wait(kf);
                     floatx16 acc[NB];
 #pragma unroll
@@ -893,8 +970,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
                     for (int nb = 0; nb < NB; ++nb) drain_masked(acc[nb], kb, na, nb);
                 }
             }
-            slot = (slot + 1 == NS) ? 0 : slot + 1;
         }
+        for (int st = sv; st < s1; ++st) enter_stage(st);
         FCS_WAIT_VM(0);
         block_sync();  // the ring may be refilled by the next sweep
     };
