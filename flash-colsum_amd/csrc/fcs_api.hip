@@ -182,7 +182,9 @@ const char *fcs_strerror(int code)
 size_t fcs_workspace_bytes(int causal, int B, int H, int Sq, int Sk, int D, int cls_n)
 {
     fcs::Plan p;
-    const int k_past = (causal && Sk > Sq) ? Sk - Sq : 0;  // the layout does not depend on k_past
+    // The layout depends on k_past only through the choice whether to lay grouped heads end to end, which a k_past of Sk
+    // (every key visible) favours most; the other choice is the layout without grouped heads.
+    const int k_past = (causal && Sk > 0) ? Sk : 0;
     const int rows = cls_n < 0 ? -1 : cls_n;
     if (!cached_plan(p, causal ? 1 : 0, B, H, H, Sq, Sk, D, rows, k_past)) return 0;
     size_t most = p.total;

@@ -82,13 +82,25 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     p.k_past = causal ? k_past : 0;
     p.q_rows = (cls_n > 0 && cls_n < Sq) ? cls_n : Sq;
 
-    // ---- grouped key heads: while a head's averaged rows fill no more than the smallest row block, the rows of all
-    // query heads of a key head form one head, whose keys are then streamed once instead of once per query head.
-    // B 4, 32 query heads on 8 key heads, K 8192, D 128 bf16, both passes: Q 64 103 -> 54 us, Q 128 103 -> 85 us.
-    // (More rows fill their own blocks, and a causal block that holds rows of several heads cannot stop at its own
-    // last key: Q 200, 32 on 4 heads, K 6000, D 64 48 us head by head, 49 us folded; Q 400, 32 on 8, K 30000 251 and 257 us.)
+    // ---- grouped key heads: the rows of all query heads of a key head can be laid end to end, as one head whose keys
+    // are then streamed once per row block of that head instead of once per query head (and row block).  For at most 128
+    // averaged rows, the smallest row block: more of them fill their own blocks, and a causal block that holds rows
+    // of several heads cannot stop at its own last key (Q 200, 32 on 4 heads, K 6000, D 64: 48 us head by head, 49
+    // folded).  Below that it pays
+    //  * where the rows of a batch entry then form a single unit of the column pass: no slabs, no final reduction
+    //    (16 on 1 head, Q 8, K 1000, D 64: 15.4 us folded, 17.8 head by head), and
+    //  * from a number of workgroups on that the call has head by head at the finest key split (visible keys / 256): one
+    //    per compute unit while half of a block's rows or more are missing (measured nearly equal or slower up to 256,
+    //    5 .. 20 % faster from 288 on, whatever the head dim), more when less is saved: ten for blocks with 65 .. 128 rows
+    //    of 128 (D 64 and 128: 0.84 .. 0.97 of the speed at 1500, 1.0 at 2500 .. 3000, 1.01 .. 1.18 at 4096), two for
+    //    256-wide heads, whose row pass has blocks of 128 rows either way (0.94 .. 1.0 at 320 .. 384, 1.0 .. 1.26 at 512).
+    // B 4, 32 on 8 heads, K 8192, D 128 bf16: Q 64 94.7 us head by head, 54.2 folded, Q 128 1.16 times as fast.
     const int G = H / Hk;
-    p.fold = (G > 1 && p.q_rows <= 128 && (long)G * p.q_rows * p.q_rows < (1L << 31)) ? G : 1;
+    const int seen_keys = p.causal ? (int)((long)p.k_past + p.q_rows < Sk ? (long)p.k_past + p.q_rows : Sk) : Sk;
+    const long head_blocks = (long)B * H * ceil_div(seen_keys, 4 * kStageKeys);
+    const long worth = (p.q_rows <= 64) ? kComputeUnits + 1 : (p.Dp == 256 ? 2 : 10) * kComputeUnits;
+    const bool one_unit = Hk == 1 && (long)G * p.q_rows <= 128;
+    p.fold = (G > 1 && p.q_rows <= 128 && (long)G * p.q_rows * p.q_rows < (1L << 31) && (one_unit || head_blocks >= worth)) ? G : 1;
     p.v_heads = H / p.fold;
     p.v_rows = p.q_rows * p.fold;
 

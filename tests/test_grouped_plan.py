@@ -1,5 +1,50 @@
-"""Which calls with grouped key heads lay the rows of a key head's query heads end to end (no GPU needed)."""
+"""Which calls with grouped key heads lay the rows of a key head's query heads end to end, and what workspace that takes
+(no GPU needed).  fcs_plan.h is plain host arithmetic: it is compiled here on its own, so that the plan of a given
+number of key heads can be looked at next to what fcs_workspace_bytes() promises for all of them."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
 from flash_colsum import _hip
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+_SOURCE = """
+#include "fcs_plan.h"
+// out: fold, total, bytes of the row statistics, of the key splits' statistics, of the column slabs and their offsets
+extern "C" int plan(int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, long *out)
+{
+    fcs::Plan p;
+    if (!fcs::make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return 0;
+    const bool two_pass = !(p.fewrows || p.small || p.fused);
+    out[0] = p.fold;
+    out[1] = (long)p.total;
+    out[2] = two_pass ? 8L * B * p.v_heads * p.rows_pad : 0;
+    out[3] = two_pass && p.n_chunks > 1 ? 8L * B * p.v_heads * p.n_chunks * p.rows_pad : 0;
+    out[4] = 4L * (two_pass ? (p.c_groups > 1 ? p.c_groups : 0) : p.n_partials) * B * Sk;
+    out[5] = (long)p.off_lse; out[6] = (long)p.off_ml; out[7] = (long)p.off_partial;
+    return 1;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    src, lib = d / "plan.cpp", d / "libplan.so"
+    src.write_text(_SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "flash-colsum_amd", "csrc"), "-o", str(lib), str(src)], check=True)
+    fn = ctypes.CDLL(str(lib)).plan
+
+    def call(causal, b, h, hk, sq, sk, d, cls_n=-1, k_past=None):
+        out = (ctypes.c_long * 8)()
+        ok = fn(int(causal), b, h, hk, sq, sk, d, cls_n, (max(0, sk - sq) if k_past is None else k_past) if causal else 0, out)
+        return dict(zip(("fold", "total", "lse", "ml", "slabs", "off_lse", "off_ml", "off_slabs"), out)) if ok else None
+
+    return call
 
 
 def test_grouped_rows_fill_row_blocks():
@@ -14,10 +59,48 @@ def test_grouped_rows_fill_row_blocks():
     assert d((2, 8, 577, 64), (2, 2, 577, 64)) == d((2, 8, 577, 64), (2, 8, 577, 64))
 
 
-def test_workspace_serves_every_number_of_key_heads():
-    """fcs_workspace_bytes() does not know the number of key heads: a multiple of 256, never less than what the
-    ungrouped call needs, still linear in the sizes."""
-    for b, h, sq, sk, d in [(1, 64, 1, 32768, 128), (4, 32, 64, 8192, 128), (2, 12, 300, 5000, 64), (1, 60, 511, 3000, 256)]:
-        n = _hip.workspace_bytes(True, b, h, sq, sk, d)
+@pytest.mark.parametrize("d,q_len,b,h,hk,s_k,kw,folds", [
+    # up to 64 rows: more than 256 blocks of 256 keys, whatever the head dim
+    (64, 64, 1, 32, 8, 2048, {}, False), (64, 64, 1, 32, 8, 2049, {}, True), (128, 4, 4, 32, 8, 300, {}, False), (256, 33, 4, 32, 8, 600, {}, True),
+    # 65 .. 128 rows: 2560 of them, 512 for heads wider than 128
+    (128, 65, 1, 32, 8, 20224, {}, False), (128, 65, 1, 32, 8, 20225, {}, True), (64, 128, 4, 32, 8, 4864, {}, False), (64, 128, 4, 32, 8, 4865, {}, True),
+    (136, 128, 4, 32, 8, 768, {}, False), (136, 128, 4, 32, 8, 769, {}, True), (64, 129, 8, 64, 8, 30000, {}, False),
+    # one unit per batch entry: no slabs
+    (64, 8, 1, 16, 1, 300, {}, True), (64, 8, 1, 17, 1, 300, {}, False), (128, 64, 3, 2, 1, 40, {}, True), (64, 1, 1, 2, 2, 300, {}, False),
+    # what counts are the keys that some row sees, and the rows that are averaged
+    (128, 64, 4, 32, 8, 8192, {"k_past": 0}, False), (128, 64, 4, 32, 8, 8192, {"k_past": 449}, True), (128, 64, 4, 32, 8, 8192, {"k_past": 448}, False),
+    (128, 300, 4, 32, 8, 8192, {"cls_n": 20}, True), (64, 64, 1, 32, 8, 2304, {"causal": False}, True),
+])
+def test_which_calls_are_laid_end_to_end(plan, d, q_len, b, h, hk, s_k, kw, folds):
+    kw = dict(kw)
+    causal = kw.pop("causal", True)
+    p = plan(causal, b, h, hk, q_len, s_k, d, **kw)
+    assert (p["fold"] > 1) == folds and p["fold"] in (1, h // hk), p
+
+
+def test_workspace_serves_every_number_of_key_heads(plan):
+    """fcs_workspace_bytes() knows neither the number of key heads nor k_past: it is at least what the plan of any of them
+    needs, a multiple of 256, and still linear in the sizes."""
+    rng = random.Random(11)
+    shapes = [(True, 1, 64, 1, 32768, 128), (True, 4, 32, 64, 8192, 128), (True, 2, 12, 300, 5000, 64), (True, 1, 60, 511, 3000, 256),
+              (True, 4, 32, 1, 32768, 128), (True, 4, 32, 100, 32768, 128)]
+    for _ in range(300):
+        causal = rng.random() < 0.7
+        shapes.append((causal, rng.choice([1, 2, 3, 8]), rng.choice([1, 2, 6, 8, 12, 32, 64]), rng.choice([1, 2, 31, 64, 65, 100, 128, 129, 600]),
+                       rng.choice([1, 40, 300, 2049, 5000, 30000]), rng.choice([64, 96, 128, 200])))
+    grouped_needs_more = 0
+    for causal, b, h, sq, sk, d in shapes:
+        n = _hip.workspace_bytes(causal, b, h, sq, sk, d)
         assert n > 0 and n % 256 == 0
         assert n <= 64 * b * h * (sq + 1024) + 4 * 4096 * (b * sk + 1024) + (1 << 20)
+        alone = plan(causal, b, h, h, sq, sk, d)["total"]
+        for hk in [x for x in range(1, h + 1) if h % x == 0]:
+            for k_past in {0, 17, sk // 2, max(0, sk - sq), sk} if causal else {0}:
+                p = plan(causal, b, h, hk, sq, sk, d, k_past=k_past)
+                assert p["total"] <= n, (causal, b, h, hk, sq, sk, d, k_past)
+                grouped_needs_more += p["total"] > alone
+                # the parts lie one behind the other inside the total, each 256-byte aligned
+                ends = [p["off_lse"] + p["lse"], p["off_ml"] + p["ml"], p["off_slabs"] + p["slabs"]]
+                assert all(p[o] % 256 == 0 for o in ("off_lse", "off_ml", "off_slabs")) and max(ends) <= p["total"]
+                assert not p["lse"] or (ends[0] <= p["off_ml"] and ends[1] <= p["off_slabs"])
+    assert grouped_needs_more > 0  # else the shapes above would not show a bound that forgets the grouped layouts
