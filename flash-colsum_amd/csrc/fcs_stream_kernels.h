@@ -29,12 +29,14 @@
 //     kernel was 2.3 times as long and needed 254 registers at D 128 (now 211).  Measured against that form, in
 //     turn: B 1, H 32, Q 512, K 65536, D 128 607 -> 599 us per call, causal B 1, H 32, S 900, D 128 38.5 -> 34.7,
 //     S 4096 bf16 233 -> 229.
-//     In the rolled loop 64-row waves take two tiles per key fragment, one after the other: the second chain runs
-//     under the first tile's exponent work, and the other waves fill the rest.  32-row waves have one tile per
-//     fragment, so there the software pipeline goes on (fragment read ahead, chain before the tile before's exponent
-//     work): a decode window has its masked stages in the last key split alone, whose workgroups end the launch.
-//     H 32, Q 128, K 16384, D 128, keys that change from call to call: 83.7 -> 81.9 us (inlined form: 82.2).  The
-//     same pipeline for 64-row waves was slower (H 32, S 2000, D 64 58.1 -> 60.0 us).
+//     In the rolled loop two chains come before their exponent work, so that the first tile's runs under the second
+//     chain: two tiles of a key fragment for 64-row waves, the two fragments of the stage for 32-row waves, which also
+//     read the next stage's first fragment ahead (not at D 256, where that was 1 .. 3 % slower).  It matters for decode windows, whose masked
+//     stages lie in the last key split alone, whose workgroups end the launch.  Against one tile at a time: H 32, Q 128,
+//     K 16384, D 128 on keys that change from call to call 83.8 -> 82.0 us (82.2 with the masked code inlined), H 8,
+//     Q 512, K 4096, D 256 37.6 -> 34.4 (34.9).  Carrying the last tile over to the next stage, as the plain loop does,
+//     was 0.1 % faster there and up to 7 % slower on short streams (H 8, Q 128, K 1000, D 64 16.3 -> 17.3 us); for
+//     64-row waves it was slower throughout (H 32, S 2000, D 64 58.0 -> 59.8).
 // A workgroup owns a chunk of keys (at most kColChunkMax, the LDS accumulator) and walks over a
 // group of (head, row block) units, re-streaming its chunk for each; at the end the waves'
 // slices are added in wave order and written as one partial slab (or the means directly, when
@@ -190,6 +192,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
     constexpr int THREADS = 64 * WAVES;
     constexpr int NT = D / 16;                 // MFMA steps along the head dim
+    constexpr int NTA = NT < 8 ? NT : 8;       // operand addresses: the swizzle stays below piece 16, step t + 8 is 256 bytes on
     constexpr int KT = kStageKeys;             // 64 keys per stage
     constexpr int NA = KT / 32;                // key fragments per stage
     constexpr int ROWS_W = 32 * NB;            // query rows per wave
@@ -234,9 +237,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
     }
     char *ring_w = ring + wave * (IPW * 1024);  // where this wave's pieces of a stage land inside a slot
     // operand read-back: lane (n, g) takes, for MFMA step t, piece 2t + g of row n (+ 32 per key fragment)
-    uint32_t take[NT];
+    uint32_t take[NTA];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NTA; ++t)
         take[t] = lds_addr(ring) + (uint32_t)(n * ROW_BYTES + (((2 * t + g) ^ row_swizzle<D>(n)) * 16));
 
     for (int u = u_begin; u < u_end; ++u) {
@@ -362,18 +365,18 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         // below is unrolled over the ring so that every slot number is a compile-time constant.
         auto take_frag = [&](auto off_c, half8 (&kf)[NT]) {
             constexpr int OFF = decltype(off_c)::value;
-            constexpr int IMM = (OFF < 65536) ? OFF : 0;  // the offset field holds 16 bits
+            constexpr int IMM = (OFF < 65536 - 256) ? OFF : 0;  // the offset field holds 16 bits
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const uint32_t ad = take[t] + (uint32_t)(OFF - IMM);
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(kf[t]) : "v"(ad), "n"(IMM) : "memory");
+                const uint32_t ad = take[t % NTA] + (uint32_t)(OFF - IMM);
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(kf[t]) : "v"(ad), "n"(IMM + t / NTA * 256) : "memory");
             }
         };
         auto take_frag_at = [&](int off, half8 (&kf)[NT]) {  // the same at a run-time offset into the ring
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const uint32_t ad = take[t] + (uint32_t)off;
-                asm volatile("ds_read_b128 %0, %1" : "=v"(kf[t]) : "v"(ad) : "memory");
+                const uint32_t ad = take[t % NTA] + (uint32_t)off;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(kf[t]) : "v"(ad), "n"(t / NTA * 256) : "memory");
             }
         };
         auto frag_wait = [&](half8 (&kf)[NT]) {
@@ -615,7 +618,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 drain_masked(sc, kb_t, na, nb);
                 drain_end(nb);
             };
-            if constexpr (NB == 1) {
+            if constexpr (NB == 1 && D <= 128) {
                 if (sv > sp) {
                     floatx16 acc[2];
                     acc[0] = acc[1] = cinit[0];
@@ -629,29 +632,32 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                         acc[0] = chain(0);
                         asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
                         take_frag_at(here + 32 * ROW_BYTES, kf);
-                        if (st > sp) drain_one(acc[1], kb - KT, 1, 0);
                         frag_wait(kf);
                         acc[1] = chain(0);
                         asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
                         take_frag_at(slot * STAGE_BYTES, kf);
                         drain_one(acc[0], kb, 0, 0);
+                        drain_one(acc[1], kb, 1, 0);
                     }
                     frag_wait(kf);  // the read-back past the last stage is not used
-                    drain_one(acc[1], c0 + (sv - 1) * KT, 1, 0);
                 }
             } else {
                 for (int st = sp; st < sv; ++st) {
                     const int kb = c0 + st * KT, here = slot * STAGE_BYTES;
                     enter_stage(st);
 #pragma unroll 1
-                    for (int na = 0; na < NA; ++na) {
-                        take_frag_at(here + na * 32 * ROW_BYTES, kf);
-                        frag_wait(kf);
-                        floatx16 acc[NB];
+                    for (int s = 0; s < TILES / 2; ++s) {
+                        floatx16 acc[2];
 #pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) acc[nb] = chain(nb);
+                        for (int q = 0; q < 2; ++q) {
+                            if (NB == 1 || q == 0) {
+                                take_frag_at(here + (NB == 1 ? q : s) * 32 * ROW_BYTES, kf);
+                                frag_wait(kf);
+                            }
+                            acc[q] = chain(NB == 1 ? 0 : q);
+                        }
 #pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) drain_one(acc[nb], kb, na, nb);
+                        for (int q = 0; q < 2; ++q) drain_one(acc[q], kb, NB == 1 ? q : s, NB == 1 ? 0 : q);
                     }
                 }
             }
@@ -713,6 +719,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
     constexpr int THREADS = 64 * WAVES;
     constexpr int NT = D / 16;
+    constexpr int NTA = NT < 8 ? NT : 8;
     constexpr int KT = kStageKeys;
     constexpr int NA = KT / 32;
     constexpr int ROWS_W = 32 * NB;
@@ -752,9 +759,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         g_off[j] = (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)((pos ^ row_swizzle<D>(row)) * 16);
     }
     char *ring_w = ring + wave * (IPW * 1024);
-    uint32_t take[NT];
+    uint32_t take[NTA];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NTA; ++t)
         take[t] = lds_addr(ring) + (uint32_t)(n * ROW_BYTES + (((2 * t + g) ^ row_swizzle<D>(n)) * 16));
 
     half8 qf[NB][NT];
@@ -809,18 +816,18 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     half8 kf[NT];
     auto take_frag = [&](auto off_c, half8 (&dst)[NT]) {
         constexpr int OFF = decltype(off_c)::value;
-        constexpr int IMM = (OFF < 65536) ? OFF : 0;
+        constexpr int IMM = (OFF < 65536 - 256) ? OFF : 0;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const uint32_t ad = take[t] + (uint32_t)(OFF - IMM);
-            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst[t]) : "v"(ad), "n"(IMM) : "memory");
+            const uint32_t ad = take[t % NTA] + (uint32_t)(OFF - IMM);
+            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst[t]) : "v"(ad), "n"(IMM + t / NTA * 256) : "memory");
         }
     };
     auto take_frag_at = [&](int off, half8 (&dst)[NT]) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const uint32_t ad = take[t] + (uint32_t)off;
-            asm volatile("ds_read_b128 %0, %1" : "=v"(dst[t]) : "v"(ad) : "memory");
+            const uint32_t ad = take[t % NTA] + (uint32_t)off;
+            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst[t]) : "v"(ad), "n"(t / NTA * 256) : "memory");
         }
     };
     auto frag_wait = [&](half8 (&dst)[NT]) {
@@ -931,7 +938,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
             fetch_stage(st + NS - 1, (slot == 0) ? NS - 1 : slot - 1);
             slot = (slot + 1 == NS) ? 0 : slot + 1;
         };
-        if constexpr (NB == 1) {
+        if constexpr (NB == 1 && D <= 128) {
             if (sv > sp) {
                 floatx16 acc[2];
                 acc[0] = acc[1] = zero16;
@@ -945,29 +952,32 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
                     acc[0] = chain(0);
                     asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
                     take_frag_at(here + 32 * ROW_BYTES, kf);
-                    if (st > sp) drain_masked(acc[1], kb - KT, 1, 0);
                     frag_wait(kf);
                     acc[1] = chain(0);
                     asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
                     take_frag_at(slot * STAGE_BYTES, kf);
                     drain_masked(acc[0], kb, 0, 0);
+                    drain_masked(acc[1], kb, 1, 0);
                 }
-                frag_wait(kf);  // the read-back past the last stage is not used
-                drain_masked(acc[1], kc0 + (sv - 1) * KT, 1, 0);
+                frag_wait(kf);
             }
         } else {
             for (int st = sp; st < sv; ++st) {
                 const int kb = kc0 + st * KT, here = slot * STAGE_BYTES;
                 enter_stage(st);
 #pragma unroll 1
-                for (int na = 0; na < NA; ++na) {
-                    take_frag_at(here + na * 32 * ROW_BYTES, kf);
-                    frag_wait(kf);
-                    floatx16 acc[NB];
+                for (int s = 0; s < TILES / 2; ++s) {
+                    floatx16 acc[2];
 #pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) acc[nb] = chain(nb);
+                    for (int q = 0; q < 2; ++q) {
+                        if (NB == 1 || q == 0) {
+                            take_frag_at(here + (NB == 1 ? q : s) * 32 * ROW_BYTES, kf);
+                            frag_wait(kf);
+                        }
+                        acc[q] = chain(NB == 1 ? 0 : q);
+                    }
 #pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) drain_masked(acc[nb], kb, na, nb);
+                    for (int q = 0; q < 2; ++q) drain_masked(acc[q], kb, NB == 1 ? q : s, NB == 1 ? 0 : q);
                 }
             }
         }
