@@ -41,7 +41,7 @@ class _Call(ctypes.Structure):
 
 
 def lib() -> ctypes.CDLL:
-    """Load the shared library once; raise loudly when it is absent or of another ABI."""
+    """Load the shared library once; raise loudly when it is absent, of another ABI or older than this file."""
     global _lib
     if _lib is None:
         if not os.path.exists(_LIB_PATH):
@@ -50,57 +50,66 @@ def lib() -> ctypes.CDLL:
                 "(hipcc, --offload-arch=gfx950). There is no fallback path."
             )
         cdll = ctypes.CDLL(_LIB_PATH)
+        # the version first: a library of another one need not have the functions below
         cdll.fcs_abi_version.restype = ctypes.c_int
         cdll.fcs_abi_version.argtypes = []
-        cdll.fcs_strerror.restype = ctypes.c_char_p
-        cdll.fcs_strerror.argtypes = [ctypes.c_int]
-        cdll.fcs_workspace_bytes.restype = ctypes.c_size_t
-        cdll.fcs_workspace_bytes.argtypes = [ctypes.c_int] * 7
-        for fn in (cdll.fcs_colsum_noncausal_f16, cdll.fcs_colsum_noncausal_bf16):
-            fn.restype = ctypes.c_int
-            fn.argtypes = [
-                ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
-                ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
-                ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
-        cdll.fcs_colsum_noncausal_f16_static.restype = ctypes.c_int
-        cdll.fcs_colsum_noncausal_f16_static.argtypes = [
-            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
-            ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
-            ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
-            ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
-        for fn in (cdll.fcs_colsum_causal_f16, cdll.fcs_colsum_causal_bf16):
-            fn.restype = ctypes.c_int
-            fn.argtypes = [
-                ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
-                ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
-                ctypes.c_float, ctypes.c_void_p]
-        cdll.fcs_colsum_general.restype = ctypes.c_int
-        cdll.fcs_colsum_general.argtypes = [
-            ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
-            ctypes.c_void_p, ctypes.c_size_t] + [ctypes.c_int] * 8 + [
-            ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64), ctypes.c_float, ctypes.c_void_p]
-        cdll.fcs_colsum_call.restype = ctypes.c_int
-        cdll.fcs_colsum_call.argtypes = [ctypes.POINTER(_Call)]
-        cdll.fcs_plan_describe.restype = ctypes.c_size_t
-        cdll.fcs_plan_describe.argtypes = [ctypes.POINTER(_Call), ctypes.c_char_p, ctypes.c_size_t]
-        cdll.fcs_static_scratch_init.restype = ctypes.c_int
-        cdll.fcs_static_scratch_init.argtypes = []
-        cdll.fcs_topk_f32.restype = ctypes.c_int
-        cdll.fcs_topk_f32.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
-                                      ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
-        cdll.fcs_threshold_f32.restype = ctypes.c_int
-        cdll.fcs_threshold_f32.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_void_p,
-                                           ctypes.c_void_p, ctypes.c_void_p]
-        cdll.fcs_round_f16.restype = ctypes.c_int
-        cdll.fcs_round_f16.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
-                                       ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
         got = cdll.fcs_abi_version()
         if got != _ABI_VERSION:
             raise RuntimeError(f"libflashcolsum.so has ABI {got}, this host layer needs {_ABI_VERSION}")
+        try:
+            _bind(cdll)
+        except AttributeError as e:  # functions are added without a new version: no caller of the older ones notices
+            raise RuntimeError(f"{_LIB_PATH} was built from older sources ({e}): rebuild it with `make -C flash-colsum_amd`") from e
         _lib = cdll
     return _lib
+
+
+def _bind(cdll: ctypes.CDLL) -> None:
+    """Argument and result types of every function that this file calls."""
+    cdll.fcs_strerror.restype = ctypes.c_char_p
+    cdll.fcs_strerror.argtypes = [ctypes.c_int]
+    cdll.fcs_workspace_bytes.restype = ctypes.c_size_t
+    cdll.fcs_workspace_bytes.argtypes = [ctypes.c_int] * 7
+    for fn in (cdll.fcs_colsum_noncausal_f16, cdll.fcs_colsum_noncausal_bf16):
+        fn.restype = ctypes.c_int
+        fn.argtypes = [
+            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+            ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+            ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
+            ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
+    cdll.fcs_colsum_noncausal_f16_static.restype = ctypes.c_int
+    cdll.fcs_colsum_noncausal_f16_static.argtypes = [
+        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
+        ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
+    for fn in (cdll.fcs_colsum_causal_f16, cdll.fcs_colsum_causal_bf16):
+        fn.restype = ctypes.c_int
+        fn.argtypes = [
+            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+            ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+            ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
+            ctypes.c_float, ctypes.c_void_p]
+    cdll.fcs_colsum_general.restype = ctypes.c_int
+    cdll.fcs_colsum_general.argtypes = [
+        ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+        ctypes.c_void_p, ctypes.c_size_t] + [ctypes.c_int] * 8 + [
+        ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64), ctypes.c_float, ctypes.c_void_p]
+    cdll.fcs_colsum_call.restype = ctypes.c_int
+    cdll.fcs_colsum_call.argtypes = [ctypes.POINTER(_Call)]
+    cdll.fcs_plan_describe.restype = ctypes.c_size_t
+    cdll.fcs_plan_describe.argtypes = [ctypes.POINTER(_Call), ctypes.c_char_p, ctypes.c_size_t]
+    cdll.fcs_static_scratch_init.restype = ctypes.c_int
+    cdll.fcs_static_scratch_init.argtypes = []
+    cdll.fcs_topk_f32.restype = ctypes.c_int
+    cdll.fcs_topk_f32.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
+                                  ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
+    cdll.fcs_threshold_f32.restype = ctypes.c_int
+    cdll.fcs_threshold_f32.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_void_p,
+                                       ctypes.c_void_p, ctypes.c_void_p]
+    cdll.fcs_round_f16.restype = ctypes.c_int
+    cdll.fcs_round_f16.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+                                   ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
 
 
 def strerror(code: int) -> str:

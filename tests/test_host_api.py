@@ -4,6 +4,7 @@ No kernel is launched here."""
 import ctypes
 import os
 import re
+import subprocess
 import types
 
 import pytest
@@ -68,6 +69,19 @@ def test_library_exports_every_declared_symbol():
     for n in names:
         assert getattr(lib, n) is not None
     assert lib.fcs_abi_version() == 5
+
+
+@pytest.mark.parametrize("version,message", [(4, "has ABI 4, this host layer needs 5"), (5, "older sources .*rebuild")])
+def test_another_library_is_refused_with_a_reason(tmp_path, monkeypatch, version, message):
+    """A library of another version, and one of this version that lacks a function added since (both know nothing but
+    their version here), end in the messages written for them."""
+    src, so = tmp_path / "other.c", tmp_path / "libflashcolsum.so"
+    src.write_text(f"int fcs_abi_version(void) {{ return {version}; }}")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(_hip, "_LIB_PATH", str(so))
+    monkeypatch.setattr(_hip, "_lib", None)
+    with pytest.raises(RuntimeError, match=message):
+        _hip.lib()
 
 
 def test_strerror_is_total():
