@@ -12,7 +12,7 @@
 //   * The per-row constant  n_i = -log2(l_i) / c  enters the matrix pipe as the INITIAL
 //     accumulator value of the row, so the scores leave the MFMAs as  s_ij + n_i  and
 //     p_ij = 2^(c * (s_ij + n_i))  costs one multiply and one v_exp_f32.  (Rows that pass 1 had
-//     to stabilise, m_i != 0, are rare: a unit that holds one starts its accumulators at 0, so
+//     to stabilise, m_i != 0, are rare: a wave that holds one starts its accumulators at 0, so
 //     that its scores carry the very bits pass 1 saw, subtracts m_i before the scale and
 //     log2 l_i after it.)
 //   * Summing p over the rows of a tile is in-lane; the two half-waves (which hold different
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 }
                 nl = (a.c == 0.f) ? -lg : -lg / a.c;
             }
-            // a stabilised row anywhere in the unit switches the whole unit to the two-constant form
+            // a stabilised row switches its wave, or the whole unit (PRE), to the two-constant form
             const bool sh = __builtin_amdgcn_ballot_w64(mm != 0.f) != 0;
             if (lane == 0) shift_s[wave] = sh ? 1 : 0;
             if (tid < BLOCK_ROWS) {
@@ -398,10 +398,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         FCS_WAIT_VM((NS - 3) * IPW);
         block_sync();  // also publishes nl_s
 
-        bool shifted = false;  // block-uniform: some row of the unit was stabilised by pass 1
+        // The two-constant form: some row of the unit was stabilised by pass 1 (PRE: block-uniform, since the forms then
+        // differ in their phases), or some row of this wave's (the flag of 64 rows: of two waves of 32).
+        bool shifted = false;
         {
             int f = 0;
-            const uint32_t ad = lds_addr(shift_s) + (uint32_t)((lane % WAVES) * 4);
+            const uint32_t ad = lds_addr(shift_s) + (uint32_t)((PRE ? lane % WAVES : wave * ROWS_W / 64) * 4);
             asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(f) : "v"(ad) : "memory");
             shifted = __builtin_amdgcn_ballot_w64(f != 0) != 0;
         }
@@ -707,12 +709,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
 // exponentials are added up per ROW: register i of a lane keeps the running sum of its row over the
 // lane's keys for the whole split, and the 32 key lanes are added once at the end through LDS.
 // Common case: 2^(c * s) without max subtraction, exact while every row sum of the split stays inside
-// [2^-80, 2^110); a block that leaves that range redoes its keys in two more sweeps (row maxima, then
-// sums of 2^((s - m) * c), the maximum subtracted before the scale).  Writes (m, log2 l) per row, or
+// [2^-80, 2^110); a wave that leaves that range redoes its keys in two more sweeps (row maxima, then
+// sums of 2^((s - m) * c), the maximum subtracted before the scale), in which the block's other waves
+// only take part in the fetches and barriers.  One row of a call out of range (K 65536, 16 on 2 heads,
+// Q 128, D 64: blocks of 512 rows laid end to end): 154 us, with none 107, with every wave of the block
+// redoing 199, with each query head in a block of its own 174.  Writes (m, log2 l) per row, or
 // (m, l) per (split, row) when the keys are split; the column pass merges the splits.
 // PRE: see the column pass.  The common sweep runs its stages below a.pre_end on Q * c rounded to fp16 (then the
 // rest on the raw operand) and accepts row sums below 2^20 only; a block that leaves the range reloads the raw
-// operand for its stabilised sweeps.
+// operand for its stabilised sweeps, all waves of it: the column pass then takes the raw operand for the whole unit.
 template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD>
 __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args a)
 {
@@ -849,7 +854,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
 #pragma unroll
             for (int i = 0; i < 16; ++i) rs[nb][i] = decltype(max_c)::value ? kNegBig : 0.f;
     };
-    auto sweep = [&](auto max_c, auto shift_c, auto scaled_c, const int s0, const int s1) {
+    // A wave that is not `active` takes part in the fetches and barriers alone.
+    auto sweep = [&](auto max_c, auto shift_c, auto scaled_c, const int s0, const int s1, const bool active) {
         constexpr bool MAXOP = decltype(max_c)::value;
         constexpr bool SHIFT = decltype(shift_c)::value;
         constexpr bool SCALED = decltype(scaled_c)::value;
@@ -890,7 +896,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         };
 
         // ---- the plain stream (see the column pass): stages [s0, sp)
-        const int sp = min(s1, max(s0, n_plain));
+        const int sp = active ? min(s1, max(s0, n_plain)) : s0;
         if (sp > s0) {
             take_frag(std::integral_constant<int, 0>{}, kf);
             floatx16 acc[2];
@@ -928,7 +934,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         }
 
         // ---- the rest, as in the column pass
-        const int sv = min(s1, max(sp, n_seen));
+        const int sv = active ? min(s1, max(sp, n_seen)) : s0;
         int slot = (sp - s0) % NS;
         auto enter_stage = [&](int st) {
             if (st > s0) {
@@ -1011,10 +1017,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     // ---- common path: no max subtraction; the pre-scaled stages first, then the raw ones
     reset_rows(std::false_type{});
     if constexpr (PRE) {
-        sweep(std::false_type{}, std::false_type{}, std::true_type{}, 0, n_pre);
+        sweep(std::false_type{}, std::false_type{}, std::true_type{}, 0, n_pre, true);
         if (n_pre > 0 && n_pre < nst) load_q(false);
     }
-    sweep(std::false_type{}, std::false_type{}, std::false_type{}, n_pre, nst);
+    sweep(std::false_type{}, std::false_type{}, std::false_type{}, n_pre, nst, true);
     float lt[NB], m_row[NB];
     fold_lanes(std::false_type{}, lt);
     bool has[NB], bad = false;
@@ -1028,6 +1034,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         m_row[nb] = has[nb] ? 0.f : kNegBig;  // an empty split must not set the merged maximum
         if (!has[nb]) lt[nb] = 0.f;
     }
+    const bool redo = PRE || __builtin_amdgcn_ballot_w64(bad) != 0;  // wave-uniform
     {
         const bool wbad = __builtin_amdgcn_ballot_w64(bad) != 0;
         if (lane == 0) bad_s[wave] = wbad ? 1 : 0;
@@ -1042,7 +1049,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     if (bad) {
         if (PRE) load_q(false);
         reset_rows(std::true_type{});
-        sweep(std::true_type{}, std::false_type{}, std::false_type{}, 0, nst);
+        sweep(std::true_type{}, std::false_type{}, std::false_type{}, 0, nst, redo);
         float mx[NB];
         fold_lanes(std::true_type{}, mx);
 #pragma unroll
@@ -1056,12 +1063,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
 #pragma unroll
             for (int i = 0; i < 16; ++i) nmax[nb][i] = -mrow[wave * ROWS_W + nb * 32 + 8 * (i >> 2) + 4 * g + (i & 3)];
         reset_rows(std::false_type{});
-        sweep(std::false_type{}, std::true_type{}, std::false_type{}, 0, nst);
-        fold_lanes(std::false_type{}, lt);
+        sweep(std::false_type{}, std::true_type{}, std::false_type{}, 0, nst, redo);
+        float ls[NB];
+        fold_lanes(std::false_type{}, ls);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
+            if (!redo) continue;  // m = 0 and the sum of the common path stand
             m_row[nb] = has[nb] ? mx[nb] : kNegBig;
-            if (!has[nb]) lt[nb] = 0.f;
+            lt[nb] = has[nb] ? ls[nb] : 0.f;
         }
     }
 

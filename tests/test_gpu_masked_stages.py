@@ -52,3 +52,26 @@ def test_rows_beyond_the_unstabilised_range():
     """Scores of several hundred: the maximum and the shifted sweep of the row pass, the two-constant form of the column pass."""
     for q_len, d in [(70, 64), (128, 128), (100, 256), (200, 64)]:
         _check(1, 2, q_len, 400, d, torch.float16, {"is_causal": True, "scale": 4.0}, d + q_len)
+
+
+@pytest.mark.parametrize("d,dtype,q_len", [(64, torch.bfloat16, 512), (64, torch.float16, 200), (128, torch.float16, 512), (128, torch.bfloat16, 250), (128, torch.float16, 128),
+                                           (256, torch.float16, 128), (256, torch.bfloat16, 300)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_one_row_beyond_the_range_in_each_wave(d, dtype, q_len, causal):
+    """A row whose scores leave the unstabilised range makes its wave redo its sums with the maximum subtracted and take the
+    two-constant form of the column pass; the block's other waves (32 or 64 rows each) keep theirs."""
+    from flash_colsum import flash_colsum_ext
+    from oracle import colsum_ext_exact
+
+    g = torch.Generator(device="cuda").manual_seed(d + q_len)
+    q = torch.randn((1, 6, q_len, d), generator=g, device="cuda").to(dtype)
+    k = torch.randn((1, 2, 2500, d), generator=g, device="cuda").to(dtype)
+    for rows in [[0], [31, 33], [64], [127], [q_len - 1], [q_len // 2, 5], list(range(0, q_len, 32))]:
+        x = q.clone()
+        x[0, 1, rows] *= 60
+        x[0, 4, rows[0]] *= -40
+        print("one row", d, dtype, q_len, causal, rows, flush=True)
+        out = flash_colsum_ext(x, k, is_causal=causal, out_dtype=torch.float32).double()
+        ref = colsum_ext_exact(x, k, is_causal=causal).double()
+        err = (out - ref).abs()
+        assert torch.isfinite(out).all() and (err <= 1e-4).all() and (err <= 1e-3 * ref.abs() + 2.0 ** -126).all(), err.max()
