@@ -68,38 +68,44 @@ struct RowPart {
     int S, first, n_j;
     uint32_t keys[E > 0 ? E : 1];
 
-    __device__ __forceinline__ uint32_t load(int i) const
+    __device__ __forceinline__ static uint32_t key_at(const float *p, int i, int n)  // of p[i], or of 0 past its n entries
     {
-        const float v = (i < S) ? row[i] : 0.f;
+        const float v = (i < n) ? p[i] : 0.f;
         return order_key(CANON ? v + 0.0f : v);
     }
     __device__ __forceinline__ void init(const float *r, int n, int wave, int lane)
     {
         row = r;
         S = n;
-        n_j = (E > 0) ? E : (n + kBatch * kTopkThreads - 1) / (kBatch * kTopkThreads) * kBatch;
+        n_j = (E > 0) ? E : ((n - 1) / (kBatch * kTopkThreads) + 1) * kBatch;
         first = wave * n_j * 64 + lane;
         if constexpr (E > 0) {
 #pragma unroll
-            for (int j = 0; j < E; ++j) keys[j] = load(first + 64 * j);
+            for (int j = 0; j < E; ++j) keys[j] = key_at(row, first + 64 * j, S);
         }
     }
     // f(index, key, exists) for every element of the lane, in ascending order; all lanes of the wave together
     template <typename F>
     __device__ __forceinline__ void each(F f) const
     {
-        int at = first;
-        asm volatile("" : "+v"(at));  // every sweep forms its own comparisons: kept masks would spill
         if constexpr (E > 0) {
+            int at = first;
+            asm volatile("" : "+v"(at));  // every sweep forms its own comparisons: kept masks would spill
 #pragma unroll
             for (int j = 0; j < E; ++j) f(at + 64 * j, keys[j], at + 64 * j < S);
         } else {
-            for (int j0 = 0; j0 < n_j; j0 += kBatch, at += 64 * kBatch) {
+            // The batch's start is wave-uniform and unsigned (a row's length rounded up to whole sweeps may pass 2^31); its
+            // entries are addressed from there.
+            const int lane = threadIdx.x & 63;
+            uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane(first - lane);
+            for (int j0 = 0; j0 < n_j; j0 += kBatch, base += 64 * kBatch) {
+                const int left = (base < (uint32_t)S) ? (int)min((uint32_t)S - base, 64u * kBatch) : 0;
+                const float *p = row + base;
                 uint32_t k[kBatch];  // that many loads in flight
 #pragma unroll
-                for (int j = 0; j < kBatch; ++j) k[j] = load(at + 64 * j);
+                for (int j = 0; j < kBatch; ++j) k[j] = key_at(p, 64 * j + lane, left);
 #pragma unroll
-                for (int j = 0; j < kBatch; ++j) f(at + 64 * j, k[j], at + 64 * j < S);
+                for (int j = 0; j < kBatch; ++j) f((int)(base + 64 * j + lane), k[j], 64 * j + lane < left);
             }
         }
     }
@@ -367,7 +373,7 @@ __global__ __launch_bounds__(kTopkThreads) void fcs_threshold_kernel(const float
 template <typename F>
 static void with_row_regs(int S, F f)
 {
-    const int e = (S + kTopkThreads - 1) / kTopkThreads;
+    const int e = (S - 1) / kTopkThreads + 1;
     if (e <= 1) f(std::integral_constant<int, 1>{});
     else if (e <= 2) f(std::integral_constant<int, 2>{});
     else if (e <= 4) f(std::integral_constant<int, 4>{});

@@ -40,3 +40,18 @@ def test_topk_and_threshold_sizes(kind, s):
     for r in range(2):
         want = (x[r] >= tau).nonzero().view(-1)
         assert cnt[r].item() == want.numel() and torch.equal(idx[r, : want.numel()].cpu(), want)
+
+
+@pytest.mark.parametrize("s", [2 ** 31 - 8193, 2 ** 31 - 1])
+def test_longest_rows(s):
+    """Rows whose length, rounded up to whole sweeps of the workgroup (8192 entries), reaches or passes 2^31."""
+    from flash_colsum import _hip
+
+    print("longest rows", s, flush=True)
+    x = torch.rand((1, s), device="cuda")
+    at = torch.tensor([0, 12345, 2 ** 30 + 1, s - 8192, s - 1], device="cuda")
+    x[0, at] = torch.tensor([2.0, 3.0, 5.0, 4.0, 6.0], device="cuda")
+    val, idx = _hip.topk_f32(x, 5, sorted=True)
+    assert val.tolist() == [[6.0, 5.0, 4.0, 3.0, 2.0]] and torch.equal(idx[0], at[[4, 2, 3, 1, 0]])
+    idx, cnt = _hip.threshold_f32(x, 2.0)
+    assert cnt.item() == 5 and torch.equal(idx[0, :5], at)
