@@ -38,7 +38,8 @@ def test_rounded_operands(b, h, s, d, layout):
 @pytest.mark.parametrize("where", [0, 7, 8, 8191, 8192, -1])
 @pytest.mark.parametrize("operand", ["q", "k"])
 def test_one_value_beyond_the_range(where, operand):
-    """The first and last element, the edges of a piece and of a workgroup's step; then an in-range call: no stale flag."""
+    """The first and last element, the edges of a piece and (of Q; K's: below) of a workgroup's step; then an in-range call:
+    no stale flag."""
     g = torch.Generator().manual_seed(3)
     q, k = (torch.randn((1, 3, 301, 25), generator=g).cuda() for _ in range(2))
     clean = _f32(q, k)
@@ -67,3 +68,43 @@ def test_negation_that_torch_has_put_off():
     lazy = torch._neg_view(q)
     assert lazy.is_neg()
     assert torch.equal(_f32(lazy, k), _f32((-q).half(), k.half()))
+
+
+def test_step_edges_of_the_second_operand():
+    """K's pieces are counted behind Q's: the last and first element on either side of each edge of a workgroup's step."""
+    g = torch.Generator().manual_seed(6)
+    q, k = (torch.randn((1, 3, 301, 25), generator=g).cuda() for _ in range(2))
+    behind_q = (q.numel() + 7) // 8
+    edges = [8 * (p - behind_q) for p in range(1024, behind_q + (k.numel() + 7) // 8, 1024) if p > behind_q]
+    assert len(edges) == 3
+    for e in [e + d for e in edges for d in (-1, 0, 7, 8)]:
+        x = k.clone()
+        x.view(-1)[e] = float("inf")
+        with pytest.raises(ValueError, match="NaN or infinite"):
+            _f32(q, x)
+        x.view(-1)[e] = 65504.0
+        assert torch.equal(_f32(q, x, scale=1e-6), _f32(q.half(), x.half(), scale=1e-6))
+
+
+@pytest.mark.parametrize("more", [-8, 0, 3])
+def test_more_elements_than_one_walk_of_the_grid(more):
+    """4096 workgroups take 1024 pieces of 8 elements each; from there on they walk.  Bit for bit torch's rounding, and a value
+    out of range in the very last element is seen."""
+    from flash_colsum import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    n0 = 8 * 1024 * 1500 + 5
+    n1 = 8 * 1024 * 4096 - (n0 + 7) // 8 * 8 + more
+    x = [torch.randn((n,), generator=g, device="cuda") * 100 for n in (n0, n1)]
+    y = [torch.full((n,), -1.0, dtype=torch.float16, device="cuda") for n in (n0, n1)]
+    flag = torch.zeros((1,), dtype=torch.int32, device="cuda")
+
+    def rounded():
+        stream = torch.cuda.current_stream().cuda_stream
+        print("rounding", n0, n1, flush=True)
+        assert _hip.lib().fcs_round_f16(x[0].data_ptr(), y[0].data_ptr(), n0, x[1].data_ptr(), y[1].data_ptr(), n1, flag.data_ptr(), stream) == 0
+        return flag.item()
+
+    assert rounded() == 0 and all(torch.equal(b, a.half()) for a, b in zip(x, y))
+    x[1][-1] = -65505.0
+    assert rounded() == 1 and torch.equal(y[1][:-1], x[1][:-1].half())

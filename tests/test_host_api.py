@@ -84,6 +84,21 @@ def test_another_library_is_refused_with_a_reason(tmp_path, monkeypatch, version
         _hip.lib()
 
 
+def test_rounding_reports_argument_errors_without_a_gpu():
+    lib = _hip.lib()
+    assert "fcs_round_f16" in _declared_symbols()
+    p, off = 4096, 4104  # never dereferenced: every call below fails its host checks
+    good = [p, p, 8, p, p, 8, p, None]
+    for i in (0, 1, 3, 4, 6):
+        assert lib.fcs_round_f16(*[None if j == i else v for j, v in enumerate(good)]) == -1
+    for i in (2, 5):
+        for n in (0, -1):
+            assert lib.fcs_round_f16(*[n if j == i else v for j, v in enumerate(good)]) == -2
+    for i in (0, 1, 3, 4):
+        assert lib.fcs_round_f16(*[off if j == i else v for j, v in enumerate(good)]) == -4
+    assert "16-byte aligned" in _hip.strerror(-4)
+
+
 def test_strerror_is_total():
     for code in range(-9, 3):
         assert isinstance(_hip.strerror(code), str) and _hip.strerror(code)
