@@ -12,9 +12,9 @@
 //   * The per-row constant  n_i = -log2(l_i) / c  enters the matrix pipe as the INITIAL
 //     accumulator value of the row, so the scores leave the MFMAs as  s_ij + n_i  and
 //     p_ij = 2^(c * (s_ij + n_i))  costs one multiply and one v_exp_f32.  (Rows that pass 1 had
-//     to stabilise, m_i != 0, are rare: a wave that holds one starts its accumulators at 0, so
-//     that its scores carry the very bits pass 1 saw, subtracts m_i before the scale and
-//     log2 l_i after it.)
+//     to stabilise, m_i != 0, are rare: a unit that holds one (FOLD: a wave) starts its
+//     accumulators at 0, so that its scores carry the very bits pass 1 saw, subtracts m_i before
+//     the scale and log2 l_i after it.)
 //   * Summing p over the rows of a tile is in-lane; the two half-waves (which hold different
 //     rows of the same keys) are added with v_permlane32_swap, and the wave adds its total for
 //     the stage's keys into ITS OWN slice of an LDS accumulator (plain read-modify-write; a slot has
@@ -156,6 +156,12 @@ __device__ __forceinline__ int seen_stages(int k0, int nst, int thr)
     return (thr >= k0) ? min(nst, (thr - k0) / kStageKeys + 1) : 0;
 }
 
+// Rows beyond the unstabilised range: rows laid end to end (FOLD) are stabilised head by head, the waves that hold such a head;
+// others with their whole block.  (PRE: the block too, since a unit with stabilised rows takes the raw operand throughout.)
+// Error against 64 bits of a call with such rows, as without folding (16 on 2 heads, Q 128, K 65536, D 64: 9.2e-7 and 9.1e-7).
+template <bool PRE, bool FOLD>
+constexpr bool kRedoHeads = FOLD && !PRE;
+
 // column pass: how the exponent is taken
 constexpr int kFormRaw = 0, kFormPrescaled = 1, kFormShifted = 2;
 
@@ -289,7 +295,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 }
                 nl = (a.c == 0.f) ? -lg : -lg / a.c;
             }
-            // a stabilised row switches its wave, or the whole unit (PRE), to the two-constant form
+            // a stabilised row switches the whole unit, or its wave (kRedoHeads), to the two-constant form
             const bool sh = __builtin_amdgcn_ballot_w64(mm != 0.f) != 0;
             if (lane == 0) shift_s[wave] = sh ? 1 : 0;
             if (tid < BLOCK_ROWS) {
@@ -398,12 +404,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         FCS_WAIT_VM((NS - 3) * IPW);
         block_sync();  // also publishes nl_s
 
-        // The two-constant form: some row of the unit was stabilised by pass 1 (PRE: block-uniform, since the forms then
-        // differ in their phases), or some row of this wave's (the flag of 64 rows: of two waves of 32).
+        // The two-constant form: some row of the unit was stabilised by pass 1 (block-uniform), or, where pass 1 redoes single
+        // heads, some row of this wave's (the flag of 64 rows: of two waves of 32).
         bool shifted = false;
         {
             int f = 0;
-            const uint32_t ad = lds_addr(shift_s) + (uint32_t)((PRE ? lane % WAVES : wave * ROWS_W / 64) * 4);
+            const uint32_t ad = lds_addr(shift_s) + (uint32_t)((kRedoHeads<PRE, FOLD> ? wave * ROWS_W / 64 : lane % WAVES) * 4);
             asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(f) : "v"(ad) : "memory");
             shifted = __builtin_amdgcn_ballot_w64(f != 0) != 0;
         }
@@ -709,11 +715,11 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
 // exponentials are added up per ROW: register i of a lane keeps the running sum of its row over the
 // lane's keys for the whole split, and the 32 key lanes are added once at the end through LDS.
 // Common case: 2^(c * s) without max subtraction, exact while every row sum of the split stays inside
-// [2^-80, 2^110); a wave that leaves that range redoes its keys in two more sweeps (row maxima, then
-// sums of 2^((s - m) * c), the maximum subtracted before the scale), in which the block's other waves
-// only take part in the fetches and barriers.  One row of a call out of range (K 65536, 16 on 2 heads,
-// Q 128, D 64: blocks of 512 rows laid end to end): 154 us, with none 107, with every wave of the block
-// redoing 199, with each query head in a block of its own 174.  Writes (m, log2 l) per row, or
+// [2^-80, 2^110); a block that leaves that range redoes its keys in two more sweeps (row maxima, then
+// sums of 2^((s - m) * c), the maximum subtracted before the scale).  FOLD: only the waves that hold rows of a
+// head with such a row redo, as when each head had a block of its own; the others take part in the fetches and barriers.
+// One row of a call out of range (K 65536, 16 on 2 heads, Q 128, D 64: blocks of 512 rows laid end to end):
+// 156 us, with none 105, with every wave of the block redoing 198, head by head 174.  Writes (m, log2 l) per row, or
 // (m, l) per (split, row) when the keys are split; the column pass merges the splits.
 // PRE: see the column pass.  The common sweep runs its stages below a.pre_end on Q * c rounded to fp16 (then the
 // rest on the raw operand) and accepts row sums below 2^20 only; a block that leaves the range reloads the raw
@@ -740,7 +746,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     __shared__ __attribute__((aligned(16))) char ring[NS * STAGE_BYTES];
     __shared__ __attribute__((aligned(16))) float red[WAVES * 32 * RP];  // wave-private [32 rows][RP]
     __shared__ __attribute__((aligned(16))) float mrow[BLOCK_ROWS];      // row maxima of the stabilised sweeps
-    __shared__ int bad_s[WAVES];
+    __shared__ int2 bad_s[WAVES];  // rows of the block that are redone: from .x to one before .y
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1023,26 +1029,39 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     sweep(std::false_type{}, std::false_type{}, std::false_type{}, n_pre, nst, true);
     float lt[NB], m_row[NB];
     fold_lanes(std::false_type{}, lt);
-    bool has[NB], bad = false;
+    bool has[NB], bad = false, redo = true;
+    uint64_t out_rows = 0;  // the wave's rows that leave the range, one bit each
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int qi = rows_first<FOLD>(a, qw0 + nb * 32 + n, 1);
         const int thr = a.causal ? min(a.k_past + qi, a.Sk - 1) : a.Sk - 1;  // last key this row sees
         has[nb] = (nst > 0) && (kc0 <= thr);
         // ceiling 2^110 rather than 2^120: up to 512 key splits of a row are added up by the column pass
-        bad = bad || (has[nb] && !(lt[nb] >= 8.2718061e-25f && lt[nb] < (n_pre > 0 ? kRowSumHiPre : 1.2980742e+33f)));
+        const bool out = has[nb] && !(lt[nb] >= 8.2718061e-25f && lt[nb] < (n_pre > 0 ? kRowSumHiPre : 1.2980742e+33f));
+        out_rows |= (uint64_t)(uint32_t)__builtin_amdgcn_ballot_w64(out) << (32 * nb);  // both half-waves hold the same rows
         m_row[nb] = has[nb] ? 0.f : kNegBig;  // an empty split must not set the merged maximum
         if (!has[nb]) lt[nb] = 0.f;
     }
-    const bool redo = PRE || __builtin_amdgcn_ballot_w64(bad) != 0;  // wave-uniform
     {
-        const bool wbad = __builtin_amdgcn_ballot_w64(bad) != 0;
-        if (lane == 0) bad_s[wave] = wbad ? 1 : 0;
+        int2 rows = {0, 0};
+        if (out_rows != 0) {
+            rows.x = qw0;
+            rows.y = qw0 + ROWS_W;
+            if constexpr (kRedoHeads<PRE, FOLD>) {
+                rows.x = fold_head(qw0 + __builtin_ctzll(out_rows), a.fold_magic) * a.q_rows;
+                rows.y = (fold_head(qw0 + 63 - __builtin_clzll(out_rows), a.fold_magic) + 1) * a.q_rows;
+            }
+        }
+        if (lane == 0) bad_s[wave] = rows;
         block_sync();
-        int any = 0;
+        if constexpr (kRedoHeads<PRE, FOLD>) redo = false;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) any |= bad_s[w];
-        bad = any != 0;  // block-uniform
+        for (int w = 0; w < WAVES; ++w) {
+            const int2 r = bad_s[w];
+            bad = bad || r.y > r.x;  // block-uniform
+            if constexpr (kRedoHeads<PRE, FOLD>) redo = redo || (r.x < qw0 + ROWS_W && r.y > qw0);
+        }
+        if constexpr (kRedoHeads<PRE, FOLD>) redo = __builtin_amdgcn_readfirstlane(redo) != 0;  // wave-uniform
     }
 
     // ---- rare: row maxima first, then sums with the maximum subtracted before the scale

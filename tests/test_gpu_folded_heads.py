@@ -135,3 +135,23 @@ def test_exact_workspace():
     assert (ws[n:] == 0xA5).all()
     ref = colsum_ext_exact(q, k, is_causal=True).double()
     assert ((out.double() - ref).abs() <= 1e-3 * ref).all()
+
+
+@pytest.mark.parametrize("group,q_len,d,dtype", [(8, 128, 64, torch.bfloat16), (4, 100, 128, torch.float16), (8, 33, 128, torch.bfloat16), (5, 16, 64, torch.float16),
+                                                 (8, 7, 256, torch.float16), (2, 120, 256, torch.bfloat16)])
+def test_one_row_beyond_the_range(group, q_len, d, dtype):
+    """A row whose scores leave the unstabilised range makes the waves that hold its head redo their sums with the maximum
+    subtracted and take the two-constant form of the column pass; the block's other waves keep theirs.  The row lies at
+    the edges of heads, of waves and of blocks."""
+    gen = torch.Generator(device="cuda").manual_seed(group * 100 + q_len)
+    hk, s_k = 2, 4200
+    b = -(-(257 if q_len <= 64 else 512 if d > 128 else 2560) // (hk * group * 16))
+    q, k = (torch.randn((b, h, s, d), generator=gen, device="cuda").to(dtype) for h, s in ((hk * group, q_len), (hk, s_k)))
+    rows = group * q_len
+    for at in [[0], [q_len - 1, q_len], [63 % rows], [64 % rows], [127 % rows, 256 % rows], [511 % rows], [rows - 1], list(range(0, rows, 64))]:
+        x = q.clone()
+        for v in at:
+            x[0, v // q_len, v % q_len] *= 60
+            x[-1, hk * group - 1 - v // q_len, v % q_len] *= -40
+        for causal in (True, False):
+            _check(x, k, {"is_causal": causal})

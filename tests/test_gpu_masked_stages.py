@@ -58,8 +58,8 @@ def test_rows_beyond_the_unstabilised_range():
                                            (256, torch.float16, 128), (256, torch.bfloat16, 300)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_one_row_beyond_the_range_in_each_wave(d, dtype, q_len, causal):
-    """A row whose scores leave the unstabilised range makes its wave redo its sums with the maximum subtracted and take the
-    two-constant form of the column pass; the block's other waves (32 or 64 rows each) keep theirs."""
+    """A row whose scores leave the unstabilised range makes its block redo its sums with the maximum subtracted and its unit
+    take the two-constant form of the column pass, whichever wave (32 or 64 rows each) holds it."""
     from flash_colsum import flash_colsum_ext
     from oracle import colsum_ext_exact
 
