@@ -23,7 +23,7 @@
 //   4. optionally (k <= kTopkSortMax) a bitonic sort by descending value, ties by ascending index, of 64-bit
 //      (key, ~index) words: exchanges over less than a wave's elements are DPP and lane swaps in registers,
 //      only the wider ones go through LDS.
-// Measured, sorted: B 4, S 8192, k 1024 14.8 us; B 1, S 32768, k 2048 31.7 us; B 1, S 262144, k 4096 181 us.  The
+// Measured, sorted: B 4, S 8192, k 1024 14.8 us; B 1, S 32768, k 2048 31.9 us; B 1, S 262144, k 4096 180 us.  The
 // former version (four byte-wide histograms, a tile of 1024 at a time with four barriers each in the compaction,
 // every step of the sort through LDS): 46, 99.6 and 549 us.
 // The threshold form is step 3 alone with a given threshold.
