@@ -318,11 +318,13 @@ def _range_flag(dev: torch.device):
 
 def _rounded_operands(q: torch.Tensor, k: torch.Tensor):
     """fp32 operands as fp16, enqueued in one launch with the range test of `_wide_operands`: (q, k, flag), or None
-    where the storage does not allow it (gaps, a misaligned base, a negation that torch has put off).  The caller
+    where the storage does not allow it (gaps, a misaligned base, a negation that torch has put off) or the library refuses
+    the head dim (after the range, which the other route looks at first).  The caller
     enqueues the column means behind it, then waits for the event of `flag` (recorded right behind the rounding) and
     takes `_wide_operands` instead when the word is set."""
     if (q.dtype != torch.float32 or k.dtype != torch.float32 or k.device != q.device or not _dense_storage(q) or not _dense_storage(k)
-            or q.numel() == 0 or k.numel() == 0 or q.is_neg() or k.is_neg() or q.data_ptr() % 16 or k.data_ptr() % 16
+            or q.numel() == 0 or k.numel() == 0 or q.shape[-1] > _MAX_HEAD_DIM
+            or q.is_neg() or k.is_neg() or q.data_ptr() % 16 or k.data_ptr() % 16
             or torch.cuda.is_current_stream_capturing()):
         return None
     q_h, k_h = torch.empty_like(q, dtype=torch.float16), torch.empty_like(k, dtype=torch.float16)

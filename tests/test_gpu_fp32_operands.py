@@ -108,3 +108,13 @@ def test_more_elements_than_one_walk_of_the_grid(more):
     assert rounded() == 0 and all(torch.equal(b, a.half()) for a, b in zip(x, y))
     x[1][-1] = -65505.0
     assert rounded() == 1 and torch.equal(y[1][:-1], x[1][:-1].half())
+
+
+def test_range_is_reported_before_the_head_dim():
+    """A head dim that the library refuses and values beyond the range at once: the range is named, as for every other storage
+    and type of fp32 operands; values within it leave the head dim."""
+    for value, error, text in [(1e6, ValueError, "beyond fp16's range"), (float("inf"), ValueError, "NaN or infinite"), (1.0, RuntimeError, "head dim")]:
+        q, k = (torch.full((1, 2, 40, 264), 0.5).cuda() for _ in range(2))
+        k[0, 1, 3, 5] = value
+        with pytest.raises(error, match=text):
+            _f32(q, k)
