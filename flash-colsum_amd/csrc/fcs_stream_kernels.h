@@ -746,7 +746,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     __shared__ __attribute__((aligned(16))) char ring[NS * STAGE_BYTES];
     __shared__ __attribute__((aligned(16))) float red[WAVES * 32 * RP];  // wave-private [32 rows][RP]
     __shared__ __attribute__((aligned(16))) float mrow[BLOCK_ROWS];      // row maxima of the stabilised sweeps
-    __shared__ int2 bad_s[WAVES];  // rows of the block that are redone: from .x to one before .y
+    __shared__ int bad_s[WAVES];
+    __shared__ int2 redo_s[kRedoHeads<PRE, FOLD> ? WAVES : 1];  // of such a wave: the rows that are redone, from .x to one before .y
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1029,43 +1030,48 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     sweep(std::false_type{}, std::false_type{}, std::false_type{}, n_pre, nst, true);
     float lt[NB], m_row[NB];
     fold_lanes(std::false_type{}, lt);
-    bool has[NB], bad = false, redo = true;
-    uint64_t out_rows = 0;  // the wave's rows that leave the range, one bit each
+    bool has[NB], out[NB], bad = false;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int qi = rows_first<FOLD>(a, qw0 + nb * 32 + n, 1);
         const int thr = a.causal ? min(a.k_past + qi, a.Sk - 1) : a.Sk - 1;  // last key this row sees
         has[nb] = (nst > 0) && (kc0 <= thr);
         // ceiling 2^110 rather than 2^120: up to 512 key splits of a row are added up by the column pass
-        const bool out = has[nb] && !(lt[nb] >= 8.2718061e-25f && lt[nb] < (n_pre > 0 ? kRowSumHiPre : 1.2980742e+33f));
-        out_rows |= (uint64_t)(uint32_t)__builtin_amdgcn_ballot_w64(out) << (32 * nb);  // both half-waves hold the same rows
+        out[nb] = has[nb] && !(lt[nb] >= 8.2718061e-25f && lt[nb] < (n_pre > 0 ? kRowSumHiPre : 1.2980742e+33f));
+        bad = bad || out[nb];
         m_row[nb] = has[nb] ? 0.f : kNegBig;  // an empty split must not set the merged maximum
         if (!has[nb]) lt[nb] = 0.f;
     }
     {
-        int2 rows = {0, 0};
-        if (out_rows != 0) {
-            rows.x = qw0;
-            rows.y = qw0 + ROWS_W;
-            if constexpr (kRedoHeads<PRE, FOLD>) {
-                rows.x = fold_head(qw0 + __builtin_ctzll(out_rows), a.fold_magic) * a.q_rows;
-                rows.y = (fold_head(qw0 + 63 - __builtin_clzll(out_rows), a.fold_magic) + 1) * a.q_rows;
+        const bool wbad = __builtin_amdgcn_ballot_w64(bad) != 0;
+        if (lane == 0) bad_s[wave] = wbad ? 1 : 0;
+        if constexpr (kRedoHeads<PRE, FOLD>) {
+            if (wbad) {  // rows of the heads from the wave's first such row to its last
+                uint64_t set = 0;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)  // both half-waves hold the same rows
+                    set |= (uint64_t)(uint32_t)__builtin_amdgcn_ballot_w64(out[nb]) << (32 * nb);
+                const int first = fold_head(qw0 + __builtin_ctzll(set), a.fold_magic) * a.q_rows;
+                const int past = (fold_head(qw0 + 63 - __builtin_clzll(set), a.fold_magic) + 1) * a.q_rows;
+                if (lane == 0) redo_s[wave] = int2{first, past};
             }
         }
-        if (lane == 0) bad_s[wave] = rows;
         block_sync();
-        if constexpr (kRedoHeads<PRE, FOLD>) redo = false;
+        int any = 0;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const int2 r = bad_s[w];
-            bad = bad || r.y > r.x;  // block-uniform
-            if constexpr (kRedoHeads<PRE, FOLD>) redo = redo || (r.x < qw0 + ROWS_W && r.y > qw0);
-        }
-        if constexpr (kRedoHeads<PRE, FOLD>) redo = __builtin_amdgcn_readfirstlane(redo) != 0;  // wave-uniform
+        for (int w = 0; w < WAVES; ++w) any |= bad_s[w];
+        bad = any != 0;  // block-uniform
     }
 
     // ---- rare: row maxima first, then sums with the maximum subtracted before the scale
     if (bad) {
+        bool redo = true;  // wave-uniform
+        if constexpr (kRedoHeads<PRE, FOLD>) {
+            redo = false;
+            for (int w = 0; w < WAVES; ++w)
+                if (bad_s[w]) redo = redo || (redo_s[w].x < qw0 + ROWS_W && redo_s[w].y > qw0);
+            redo = __builtin_amdgcn_readfirstlane(redo) != 0;
+        }
         if (PRE) load_q(false);
         reset_rows(std::true_type{});
         sweep(std::true_type{}, std::false_type{}, std::false_type{}, 0, nst, redo);
