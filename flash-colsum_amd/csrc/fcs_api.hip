@@ -90,7 +90,7 @@ bool strides_ok(const int64_t s[4], bool use_batch)
 // (H % Hk == 0; query head h reads key head h / (H / Hk)).  `need_ptrs` is false for fcs_plan_describe.
 int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, const void *k, float *out, void *out_f16, void *ws,
             size_t ws_bytes, int B, int H, int Hk, int Sq, int Sk, int D, const int64_t qs[4], const int64_t ks[4], float scale,
-            int cls_n, int k_past, uint32_t flags, bool need_ptrs)
+            int cls_n, int k_past, uint32_t flags, bool need_ptrs, bool fit_workspace = false)
 {
     if (need_ptrs && (!q || !k || !out)) return FCS_E_NULL;
     if (!qs || !ks) return FCS_E_NULL;
@@ -104,6 +104,8 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     if (k_past > Sk) k_past = Sk;
 
     if (!cached_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return FCS_E_DIMS;
+    // (a fixed workspace: the call is laid out in it where it can be)
+    if (fit_workspace && p.total > ws_bytes && !fcs::plan_within(p, ws_bytes, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return FCS_E_STATIC_LIMIT;
     p.bf16 = bf16;
     if (need_ptrs) {
         if (ws && (reinterpret_cast<uintptr_t>(ws) & 255u)) return FCS_E_WORKSPACE;
@@ -127,12 +129,14 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     a.pre_end = p.causal ? (int)((((long)p.k_past + 1) / fcs::kStageKeys) * fcs::kStageKeys) : 0x3fffffc0;
     a.negate = scale < 0.f;
     a.c = fabsf(scale) * 1.44269504088896340736f;
-    a.n_chunks = p.n_chunks; a.chunk_keys = p.chunk_keys; a.rows_pad = p.rows_pad;
+    a.r_line = p.r_line; a.r_unit = p.r_unit; a.r_seg = p.r_seg; a.r_len = p.r_len; a.r_blocks = p.r_blocks; a.r_whole = p.r_whole; a.n_qblk = p.n_qblk;
+    a.r_by_seg = p.r_by_seg; a.r_by_head = p.r_by_head; a.r_by_block = p.r_by_block; a.by_heads = p.by_heads;
     char *w = static_cast<char *>(ws);
-    a.lse = reinterpret_cast<float2 *>(w + p.off_lse);
-    a.ml = reinterpret_cast<float2 *>(w + p.off_ml);
-    a.c_chunk = p.c_chunk; a.c_groups = p.c_groups; a.c_upg = p.c_upg; a.c_nrb = p.c_nrb;
-    a.c_nchunks = p.c_nchunks; a.n_qblk = p.n_qblk;
+    a.stat = reinterpret_cast<float2 *>(w + p.off_lse);
+    a.c_chunk = p.c_chunk; a.c_nchunks = p.c_nchunks; a.c_nrb = p.c_nrb;
+    a.c_line = p.c_line; a.c_unit = p.c_unit; a.c_cs = p.c_cs; a.c_seg = p.c_seg; a.c_len = p.c_len; a.c_blocks = p.c_blocks; a.c_direct = p.c_direct;
+    a.c_by_seg = p.c_by_seg; a.c_by_batch = p.c_by_batch; a.c_by_chunks = p.c_by_chunks; a.c_by_chunk = p.c_by_chunk;
+    a.c_by_blocks = p.c_by_blocks; a.c_by_used = p.c_by_used;
     a.partial = reinterpret_cast<float *>(w + p.off_partial);
     a.out = out;
     a.out_h = static_cast<_Float16 *>(out_f16);
@@ -146,12 +150,12 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
 
 int run(int bf16, int causal, const void *q, const void *k, float *out, void *out_f16, void *ws, size_t ws_bytes, int B, int H,
         int Hk, int Sq, int Sk, int D, const int64_t qs[4], const int64_t ks[4], float scale, int cls_n,
-        int k_past, void *stream, uint32_t flags = 0)
+        int k_past, void *stream, uint32_t flags = 0, bool fit_workspace = false)
 {
     fcs::Plan p;
     fcs::Args a;
     const int rc = prepare(p, a, bf16, causal, q, k, out, out_f16, ws, ws_bytes, B, H, Hk, Sq, Sk, D, qs, ks, scale, cls_n, k_past,
-                           flags, true);
+                           flags, true, fit_workspace);
     if (rc != FCS_OK) return rc;
     return fcs::launch_colsum(p, a, stream);
 }
@@ -247,13 +251,15 @@ int fcs_colsum_noncausal_f16_static(const void *q, const void *k, float *out, vo
     // size check first: it needs no GPU, like every other argument error
     fcs::Plan p;
     if (!cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0)) return FCS_E_DIMS;
-    if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES) return FCS_E_STATIC_LIMIT;
+    if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES &&
+        !fcs::plan_within(p, FCS_STATIC_SCRATCH_BYTES, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0))
+        return FCS_E_STATIC_LIMIT;
     if (!q || !k || !out || !q_strides || !k_strides) return FCS_E_NULL;
     void *ws = nullptr;
     const hipError_t e = static_scratch(&ws);
     if (e != hipSuccess) return (int)e;
     return run(0, 0, q, k, out, out_f16, ws, FCS_STATIC_SCRATCH_BYTES, B, H, H, S, S, D, q_strides, k_strides, scale,
-               cls_n < 0 ? -1 : cls_n, 0, hip_stream);
+               cls_n < 0 ? -1 : cls_n, 0, hip_stream, 0, true);
 }
 
 int fcs_colsum_noncausal_bf16(const void *q, const void *k, float *out, void *out_f16, void *ws, size_t ws_bytes, int B, int H,

@@ -62,15 +62,19 @@ static constexpr int kDppMirror = 0x140;      // lane i <-> 15 - i within rows o
 
 // Workgroups are handed to the 8 XCDs round-robin in launch order (x fastest, then y, then z), and
 // each XCD has its own L2.  Neighbours along x usually read the same operand, so they should
-// run on one XCD and close together in time.  This returns the grid coordinates a workgroup should
-// work on instead of its own: XCD c, which receives workgroups c, c + 8, c + 16, ..., then walks a
+// run on one XCD and close together in time.  This returns the number (x fastest) of the workgroup whose work
+// a workgroup should do instead of its own: XCD c, which receives workgroups c, c + 8, c + 16, ..., then walks a
 // contiguous range of the x-fastest list of all coordinates.  A bijection for any grid size.
-// `i` is the workgroup's number in launch order, nx * ny * nz the number of workgroups.
+// `i` is the workgroup's number in launch order, n_all the number of workgroups.
+__device__ __forceinline__ int xcd_contiguous(int i, int n_all)
+{
+    const int c = i & 7, per = n_all >> 3, rem = n_all & 7;  // XCD c holds per + (c < rem) workgroups
+    return c * per + min(c, rem) + (i >> 3);
+}
+// the same as coordinates of an nx x ny x nz grid
 __device__ __forceinline__ void xcd_contiguous_block(int i, int nx, int ny, int nz, int &bx, int &by, int &bz)
 {
-    const int n_all = nx * ny * nz;
-    const int c = i & 7, per = n_all >> 3, rem = n_all & 7;  // XCD c holds per + (c < rem) workgroups
-    const int v = c * per + min(c, rem) + (i >> 3);
+    const int v = xcd_contiguous(i, nx * ny * nz);
     bx = v % nx;
     const int t = v / nx;
     by = t % ny;

@@ -27,15 +27,19 @@ struct Args {
     int negate;          // scale < 0: scores are negated by flipping the stationary operand's sign
     float c;             // |scale| * log2(e)
     // pass 1
-    int n_chunks, chunk_keys, rows_pad;
-    float2 *lse;  // [B*v_heads][rows_pad]      (m, log2 l): row maximum in score units (0 on the
-                  //                            unstabilised path) and log2 of sum_j 2^((s_ij - m) * c)
-    float2 *ml;   // [B*v_heads][n_chunks][rows_pad]  (m, l) of each key split
+    StageLine r_line;  // the stages of its row blocks in units of r_unit; workgroup w takes [w * r_seg, (w + 1) * r_seg) of all r_len
+    int r_unit, r_seg, r_len, r_blocks, r_whole, n_qblk;
+    FastDiv r_by_seg, r_by_head, r_by_block, by_heads;
+    float2 *stat;  // r_whole: [B*v_heads * n_qblk][rows of a block] (m, log2 l): row maximum in score units (0 on the
+                   //          unstabilised path) and log2 of sum_j 2^((s_ij - m) * c)
+                   // else:    set w + i holds (m, l) of share w's part of row block i (i = head * n_qblk + block); an
+                   //          empty part is (0, 0)
     // pass 2
-    int c_chunk, c_groups, c_upg, c_nrb;  // column pass: keys per block, unit groups, units per group, row blocks per head
-    int c_nchunks;       // column pass: key chunks (its grid is c_nchunks x c_groups x B, launched as one dimension)
-    int n_qblk;          // pass 1: row blocks (its grid is n_qblk x n_chunks x B*H, launched as one dimension)
-    float *partial;  // [groups][B][Sk]
+    int c_chunk, c_nchunks, c_nrb;  // keys per chunk, chunks, row blocks per head
+    StageLine c_line;               // the stages of its units, as for pass 1; chunk after chunk
+    int c_unit, c_cs, c_seg, c_len, c_blocks, c_direct;  // c_cs: units per chunk
+    FastDiv c_by_seg, c_by_batch, c_by_chunks, c_by_chunk, c_by_blocks, c_by_used;
+    float *partial;  // slabs; two-pass path: [..][c_chunk], slab w + i is share w's of chunk i (i = batch entry * c_nchunks + chunk)
     float *out;      // [B][Sk]
     _Float16 *out_h; // [B][Sk] or nullptr: the same means rounded to fp16
     float inv_norm;  // 1 / (H * q_rows)
@@ -49,6 +53,19 @@ struct Args {
     int f_nwgq;      // blocks along the query axis: ceil(f_nqblk / f_rbpw)
     int f_hg;        // head groups (fused and few-rows paths): a batch entry has f_hg * f_nwgq workgroups
 };
+
+#if defined(__HIP_DEVICE_COMPILE__) || defined(__HIPCC__)
+// First thing in a kernel: one word of every 64 bytes of its arguments, requested together.  The compiler loads arguments
+// where they are first used, and each of those loads would wait for a line of its own to come from memory, one after the
+// other; behind this they hit the scalar cache.
+__device__ __forceinline__ void fetch_args(const Args &a)
+{
+    const int *w = reinterpret_cast<const int *>(&a);
+    constexpr int N = (int)(sizeof(Args) / sizeof(int));
+    static_assert(N > 80 && N <= 96, "one word of each line");
+    asm volatile("" ::"s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[48]), "s"(w[64]), "s"(w[80]), "s"(w[N - 1]));
+}
+#endif
 
 // Enqueues every kernel of one call on `stream`; returns 0 or the hipError_t of a failed launch.
 int launch_colsum(const Plan &p, const Args &a, void *stream);

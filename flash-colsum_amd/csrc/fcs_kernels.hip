@@ -1,9 +1,9 @@
 // Attention column means on gfx950 (MI355X): launch order of the paths and the final reduction.
 //
 //   pass 1 (fcs_rowstream_kernel, fcs_stream_kernels.h)  per row (m, log2 l) with
-//          l = sum_j 2^((s_ij - m) * c), c = scale*log2(e), or (m, l) per key split.
+//          l = sum_j 2^((s_ij - m) * c), c = scale*log2(e), or (m, l) per part of a row block.
 //   pass 2 (fcs_colstream_kernel, fcs_stream_kernels.h)  column sums of 2^((s_ij - m_i) * c - log2 l_i),
-//          one partial slab per group of (head, row block) units.
+//          one partial slab per workgroup and key chunk that its share touches.
 //   fcs_finalize_kernel (here) adds the slabs in a fixed order: no atomics anywhere, every
 //          partial has exactly one writer.
 #include <hip/hip_runtime.h>
@@ -43,14 +43,34 @@ __device__ __forceinline__ float slab_lane_total(const float *p, int64_t stride,
 // usual few dozen slabs, 16 or 32 for more (slab_lanes()): a small batch can leave hundreds of
 // slabs per batch entry (B 1, H 16, S 1024 on the fused path: 512 slabs of 1024 outputs, where 8
 // lanes took longer than the kernel that wrote the slabs).
-template <int SL>
+//
+// SHARES (two-pass path): a key chunk has one slab per workgroup of the column pass whose share of the line touches it,
+// as many as its units take; the slabs of all chunks lie one behind the other.
+template <int SL, bool SHARES>
 __global__ __launch_bounds__(32 * SL) void fcs_finalize_kernel(const Args a)
 {
     __shared__ float sub[SL][32];
+    fetch_args(a);
     const int64_t n = (int64_t)a.B * a.Sk;
     const int col = threadIdx.x & 31, sl = threadIdx.x >> 5;
     const int64_t idx = (int64_t)blockIdx.x * 32 + col;
-    sub[sl][col] = (idx < n) ? slab_lane_total<SL>(a.partial + idx, n, a.n_partials, sl) : 0.f;
+    float v = 0.f;
+    if (idx < n) {
+        if constexpr (SHARES) {
+            const int b = (int)((n >> 32) == 0 ? (uint32_t)idx / (uint32_t)a.Sk : idx / a.Sk);
+            int in_chunk;
+            const int cx = a.c_by_chunk.quot((int)(idx - (int64_t)b * a.Sk), in_chunk);
+            const int before = a.c_line.chunk_places(a.c_nrb, a.c_cs, cx);
+            const int len = (a.c_line.chunk_places(a.c_nrb, a.c_cs, cx + 1) - before) * a.v_heads;
+            const int start = b * (int)a.c_by_batch.d + before * a.v_heads, w0 = a.c_by_seg.quot(start + a.c_line.start);
+            const int slabs = (len > 0) ? a.c_by_seg.quot(start + len - 1) - w0 + 1 : 0;  // 0: no row sees the chunk
+            const float *p = a.partial + (w0 + (int64_t)b * a.c_nchunks + cx) * a.c_chunk + in_chunk;
+            v = slab_lane_total<SL>(p, a.c_chunk, slabs, sl);
+        } else {
+            v = slab_lane_total<SL>(a.partial + idx, n, a.n_partials, sl);
+        }
+    }
+    sub[sl][col] = v;
     __syncthreads();
     if (sl == 0 && idx < n) {
         float t = sub[0][col];
@@ -64,17 +84,20 @@ __global__ __launch_bounds__(32 * SL) void fcs_finalize_kernel(const Args a)
 // ------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------
-hipError_t launch_finalize(const Args &a, hipStream_t st)
+template <bool SHARES>
+static hipError_t launch_finalize_t(const Args &a, hipStream_t st)
 {
     const int64_t n = (int64_t)a.B * a.Sk;
     const dim3 grid((unsigned)((n + 31) / 32));
     switch (slab_lanes(a.n_partials)) {
-    case 32: hipLaunchKernelGGL(fcs_finalize_kernel<32>, grid, dim3(1024), 0, st, a); break;
-    case 16: hipLaunchKernelGGL(fcs_finalize_kernel<16>, grid, dim3(512), 0, st, a); break;
-    default: hipLaunchKernelGGL(fcs_finalize_kernel<8>, grid, dim3(256), 0, st, a); break;
+    case 32: hipLaunchKernelGGL((fcs_finalize_kernel<32, SHARES>), grid, dim3(1024), 0, st, a); break;
+    case 16: hipLaunchKernelGGL((fcs_finalize_kernel<16, SHARES>), grid, dim3(512), 0, st, a); break;
+    default: hipLaunchKernelGGL((fcs_finalize_kernel<8, SHARES>), grid, dim3(256), 0, st, a); break;
     }
     return hipGetLastError();
 }
+
+hipError_t launch_finalize(const Args &a, hipStream_t st) { return launch_finalize_t<false>(a, st); }
 
 size_t describe_finalize(const Args &a, char *buf, size_t n)
 {
@@ -90,8 +113,7 @@ static hipError_t launch_two_pass(const Plan &p, const Args &a, hipStream_t st)
     if (e != hipSuccess) return e;
     e = launch_colstream(p, a, st);
     if (e != hipSuccess) return e;
-    if (p.c_groups > 1) return launch_finalize(a, st);
-    return hipSuccess;
+    return p.c_direct ? hipSuccess : launch_finalize_t<true>(a, st);
 }
 
 int launch_colsum(const Plan &p, const Args &a, void *stream)

@@ -22,8 +22,93 @@ constexpr int small_ring_heads(int tiles) { return 28 / tiles < 16 ? 28 / tiles 
 constexpr int col_ring_slots(int D, int waves) { return (D == 256 || (D == 128 && waves == 4)) ? 3 : 4; }
 constexpr int col_chunk_max(int D, int waves) { return (D == 256) ? 1024 : (D == 128 && waves == 4) ? 1536 : 2048; }
 
+// The shares of a pass (64-key stages): the shortest, and what starting on a row block or unit costs
+constexpr int kMinShare = 4;
+constexpr int start_places(int D, int rows_per_wave) { return D == 256 ? 1 : (D == 64 && rows_per_wave == 32) ? 3 : 2; }
+
 // row-statistics pass on the same stream (fcs_stream_kernels.h): ring slots
-constexpr int row_ring_slots(int D, int waves) { return (D == 256 || (D == 128 && waves == 4)) ? 3 : 4; }
+constexpr int row_ring_slots(int D, int waves) { return (D == 256 || waves > 8) ? 3 : 4; }
+
+#if defined(__HIPCC__)
+#define FCS_HD __host__ __device__ inline
+#else
+#define FCS_HD inline
+#endif
+
+// Division of 0 <= n < 2^32 by a number that the host knows: a multiply-high and one correction (the estimate is the
+// quotient or one less).
+struct FastDiv {
+    uint32_t d, magic;
+    void set(int64_t by)
+    {
+        d = (uint32_t)by;
+        magic = by <= 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d);
+    }
+    FCS_HD int quot(int n, int &rest) const
+    {
+        int q = (int)(((uint64_t)(uint32_t)n * magic) >> 32);
+        rest = n - q * (int)d;
+        if ((uint32_t)rest >= d) {
+            rest -= (int)d;
+            ++q;
+        }
+        return q;
+    }
+    FCS_HD int quot(int n) const
+    {
+        int rest;
+        return quot(n, rest);
+    }
+};
+
+// The two-pass path lays the work of a pass out as a line of 64-key stages, head after head and row block after row
+// block, and gives every workgroup an equal share of it.  Row block rb of any head has
+//     n(rb) = min(last, first + (rb + 1) * step)    stages:
+// the stages up to the last key that one of its rows sees.  step is 0 where all row blocks count the same (the line may
+// then be counted in units of several stages), else a power of two.  Every row block takes `start` places of the line in front
+// of its stages, for what starting on it costs a workgroup.  A line has fewer than 2^31 places.
+struct StageLine {
+    int first, step, last, log_step, start;
+    FCS_HD int n(int rb) const
+    {
+        const int v = first + (rb + 1) * step;
+        return v < last ? v : last;
+    }
+    // how many of the row blocks before rb have `cap` stages at most
+    FCS_HD int up_to(int rb, int cap) const
+    {
+        if (cap >= last) return rb;
+        const int m = (step == 0 || cap < first) ? 0 : (cap - first) >> log_step;
+        return m < rb ? m : rb;
+    }
+    // stages of the row blocks before rb that are among the first `cap` of their block
+    FCS_HD int sum(int rb, int cap) const
+    {
+        const int c = cap < last ? cap : last;
+        if (step == 0) return rb * c;
+        int m = c > first ? (c - first) >> log_step : 0;  // row blocks that end at or below the cap
+        if (m > rb) m = rb;
+        return m * first + step * (m * (m + 1) / 2) + (rb - m) * c;
+    }
+    // places of the row blocks before rb
+    FCS_HD int places(int rb) const { return sum(rb, last) + rb * start; }
+    // stages lo .. hi-1 of row block rb
+    FCS_HD int between(int rb, int lo, int hi) const
+    {
+        int v = n(rb);
+        v = (v < hi ? v : hi) - lo;
+        return v > 0 ? v : 0;
+    }
+    // column pass: places of the first `chunks` chunks of cs stages of a head with nrb row blocks; each row block takes
+    // `start` places in each chunk that it sees
+    FCS_HD int chunk_places(int nrb, int cs, int chunks) const
+    {
+        int seen = 0;  // (row block, chunk) pairs
+        if (step == 0) seen = nrb * (chunks < (last + cs - 1) / cs ? chunks : (last + cs - 1) / cs);
+        else for (int c = 0; c < chunks; ++c) seen += nrb - up_to(nrb, c * cs);
+        return sum(nrb, chunks * cs) + seen * start;
+    }
+};
 
 struct Plan {
     int B, H, Sq, Sk, D;
@@ -34,19 +119,30 @@ struct Plan {
     // two-pass path: query heads of a key head whose rows are laid end to end (1: none), and the heads and rows per
     // head that come of it; everything below up to the single-kernel paths counts in those
     int fold, v_heads, v_rows;
-    // pass 1: row statistics.  grid = (n_qblk, n_chunks, B*v_heads)
+    // pass 1: row statistics.  Workgroup w takes the stages [w * r_seg, (w + 1) * r_seg) of the line
+    // (batch entry, head, row block)
     int qw;          // query rows per wave (32 or 64)
     int k1_waves;    // waves per block (4 or 8); a block covers k1_waves*qw rows
-    int n_qblk;      // blocks along the query axis
-    int n_chunks;    // key-axis splits (partial (max,sum) per chunk when > 1)
-    int chunk_keys;  // keys per split, multiple of kStageKeys
-    int rows_pad;    // n_qblk * 4 * qw  (row pitch of the statistics arrays)
-    // column pass: grid = (c_nchunks, c_groups, B); a block owns c_chunk keys and walks over c_upg
-    // (head, row block) units
+    int n_qblk;      // row blocks per head
+    int rows_pad;    // n_qblk * k1_waves * qw
+    StageLine r_line;
+    int r_unit, r_seg, r_len, r_blocks;  // stages per unit of the line, units per share and in all, workgroups
+    int r_whole;     // every row block lies within one share
+    int r_one;       // every share is one (part of a) row block
+    FastDiv r_by_seg, r_by_head, r_by_block, by_heads;  // divisions by r_seg, a head's units, a row block's (step 0), v_heads
+    int n_chunks;    // shares per row block, rounded down
+    // column pass: the same over (batch entry, key chunk, head, row block); a (head, row block) is a unit of the chunk, whose
+    // column sums a block keeps in LDS
     int c_nb, c_waves; // 32-row fragments per wave, waves per block: a unit has 32 * c_nb * c_waves rows
     int c_nrb;         // row blocks per head
     int c_chunk, c_nchunks;
-    int c_groups, c_upg;
+    StageLine c_line;
+    int c_unit, c_cs;                      // stages per unit of the line, units per chunk
+    int c_seg, c_len, c_blocks, c_direct;  // c_direct: block w computes all of chunk w and writes the means
+    int c_one;                             // every share is one chunk of one unit
+    FastDiv c_by_seg, c_by_batch, c_by_chunks, c_by_chunk;  // divisions by c_seg, a batch entry's units, c_nchunks, c_chunk
+    FastDiv c_by_blocks, c_by_used;        // divisions by c_nrb, the chunks that some row sees
+    int c_groups;      // slabs per chunk, rounded down (1: none)
     // fused single-kernel path: non-causal, all keys of a row block fit in one
     // workgroup's registers.  grid = (f_nwgq * B, f_hg)
     int fewrows;     // 1: few-rows path (non-causal, q_rows <= 4): grid = B * f_hg, slabs = f_hg
@@ -59,12 +155,13 @@ struct Plan {
     int f_hg, f_hpg; // head groups, heads per group
     int f_rbpw;      // adjacent query blocks per workgroup (fused path; 1 on the few-rows path)
     int f_nwgq;      // workgroups along the query axis: ceil(f_nqblk / f_rbpw)
-    int n_partials;  // slabs summed by the finalize kernel
+    int n_partials;  // slabs summed by the finalize kernel (two-pass path: at most)
     int gen_blocks;  // two-pass path: resident workgroups of one generation (what the GPU holds at once)
     // workspace layout (byte offsets, each 256-byte aligned)
-    size_t off_lse;      // float2 [B*v_heads][rows_pad]            row maximum and log2 of the row sum
-    size_t off_ml;       // float2 [B*v_heads][n_chunks][rows_pad]  only when n_chunks > 1
-    size_t off_partial;  // float  [c_groups][B][Sk]          only when c_groups > 1
+    size_t off_lse;      // float2 [B*v_heads][rows_pad]  r_whole: row maximum and log2 of the row sum; else the first
+                         //                               B*v_heads*n_qblk of the sets of row statistics (row maximum and row sum)
+    size_t off_ml;       // float2 [shares][rows of a block]  the rest of them: set w + i is share w's of row block i
+    size_t off_partial;  // float  [c_chunk] slabs: w + i is share w's of chunk i (none with c_direct)
     size_t total;
 };
 
@@ -72,7 +169,9 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Returns false for invalid dimensions.  cls_n <= 0 means all rows.  Hk: key heads, a divisor of H.
-inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past)
+// tight_stages > 0: the two-pass path with as little workspace as it can do with: row blocks are not cut, chunks are not longer
+// than that (see plan_within).
+inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight_stages = 0)
 {
     if (B < 1 || H < 1 || Hk < 1 || H % Hk != 0 || Sq < 1 || Sk < 1 || D < 1 || k_past < 0) return false;
     p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
@@ -120,20 +219,70 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     const int qblk = p.k1_waves * p.qw;
     p.n_qblk = ceil_div(p.v_rows, qblk);
     p.rows_pad = p.n_qblk * qblk;
-    const long base1 = (long)p.n_qblk * B * p.v_heads;
-    // One generation of workgroups: an 8-wave block fills a compute unit's registers, the 4-wave
-    // blocks fit twice.  Every further generation pays the block start (Q fragments, first key
-    // stage: ~5 us) again, which nothing overlaps.
-    // (256-wide heads: the kernels' registers and LDS allow one block per compute unit whatever its waves)
-    const int target1 = (p.k1_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
-    p.gen_blocks = target1;
-    // as many splits as still fit one generation (rounding up could start a second one for a few blocks)
-    int want = (base1 >= target1) ? 1 : (int)(target1 / base1);
-    int max_chunks = ceil_div(Sk, 4 * kStageKeys);  // at least 256 keys per split
-    if (want > max_chunks) want = max_chunks;
-    if (want < 1) want = 1;
-    p.chunk_keys = ceil_div(ceil_div(Sk, want), kStageKeys) * kStageKeys;
-    p.n_chunks = ceil_div(Sk, p.chunk_keys);
+    // ---- the stages of a pass.  A causal row block ends at the last key that one of its rows sees; of a call with a
+    // single row block per head (or rows laid end to end: every block holds a head's last row) that is the same for all.
+    const int seen_stages = ceil_div(seen_keys, kStageKeys);
+    const int whole_past = p.causal ? ceil_div(p.k_past < Sk ? p.k_past : Sk, kStageKeys) : 0;
+    auto line_of = [&](int rows, int blocks) {
+        if (!p.causal || p.fold > 1 || blocks == 1) return StageLine{seen_stages, 0, seen_stages, 0, 0};
+        const int step = rows / kStageKeys;  // 2, 4 or 8
+        return StageLine{whole_past, step, seen_stages, step == 8 ? 3 : step == 4 ? 2 : 1, 0};
+    };
+    // One generation of workgroups: an 8-wave block fills a compute unit's registers, the 4-wave blocks fit twice
+    // (256-wide heads: the kernels' registers and LDS allow one block per compute unit whatever its waves).
+    p.gen_blocks = (p.k1_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
+
+    // A pass of 2^31 places or more (days of them) is counted in row blocks and chunks.
+    const auto stages_of = [&](const StageLine &l, int blocks) {
+        double t = 0.;
+        for (int rb = 0; l.step && rb < blocks; ++rb) t += l.n(rb);
+        return (l.step ? t : (double)l.last * blocks) * B * p.v_heads;
+    };
+    constexpr double kHuge = 1e9;
+
+    // ---- pass 1: equal shares of the line, at least kMinShare stages each.  A share that crosses into another row block
+    // pays that block's start (Q fragments, first key stages) on top, so where all row blocks are equal it is also
+    // priced to cut each of them into equal parts, or to give a workgroup whole ones.
+    {
+        const long blocks = (long)p.n_qblk * B * p.v_heads;
+        if (blocks >= (1L << 31)) return false;
+        const int start = start_places(p.Dp, p.qw);
+        p.r_line = line_of(qblk, p.n_qblk);
+        p.r_unit = 1;
+        const double all = stages_of(p.r_line, p.n_qblk) + (double)blocks * start;
+        const bool huge = all >= kHuge || tight_stages > 0;
+        int seg = huge ? 0 : (int)(((int64_t)all + p.gen_blocks - 1) / p.gen_blocks);
+        if (seg < kMinShare + start) seg = kMinShare + start;
+        p.r_whole = p.r_one = 0;
+        p.r_line.start = start;
+        const int best = seg + start;  // (a share that starts inside a row block pays its start unasked)
+        {
+            const int n = p.r_line.last;
+            const long per = (blocks + p.gen_blocks - 1) / p.gen_blocks;  // whole row blocks per workgroup
+            const int most = ceil_div(n, kMinShare);
+            const long fit = p.gen_blocks / blocks;
+            const int parts = (per > 1 || fit < 2 || tight_stages > 0) ? 1 : (int)(fit < most ? fit : most);
+            const int part = ceil_div(n, parts);
+            // (row blocks that see different numbers of keys: parts of the longest one's length)
+            if (huge || ((p.r_line.step == 0 || per == 1) && per * (part + start) <= best)) {
+                seg = (int)per;
+                p.r_unit = part;
+                const int units = ceil_div(n, part);
+                p.r_whole = units == 1;
+                p.r_one = per == 1;
+                p.r_line = StageLine{units, 0, units, 0, 0};
+            }
+        }
+        p.r_len = B * p.v_heads * p.r_line.places(p.n_qblk);
+        if (seg > p.r_len) seg = p.r_len;
+        p.r_seg = seg;
+        p.r_blocks = ceil_div(p.r_len, seg);
+        p.n_chunks = (!p.r_whole && p.r_blocks / blocks > 1) ? (int)(p.r_blocks / blocks) : 1;
+        p.r_by_seg.set(seg);
+        p.r_by_head.set(p.r_line.places(p.n_qblk));
+        p.r_by_block.set(p.r_line.last + p.r_line.start);
+        p.by_heads.set(p.v_heads);
+    }
 
     // ---- column pass (streaming kernel)
     {
@@ -141,51 +290,80 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         else if (block_rows > 128) { p.c_nb = 2; p.c_waves = 4; }
         else { p.c_nb = 1; p.c_waves = 4; }
         if (p.Dp == 256) { p.c_nb = 1; p.c_waves = (block_rows > 128) ? 8 : 4; }
-        const int block_rows = 32 * p.c_nb * p.c_waves;
-        p.c_nrb = ceil_div(p.v_rows, block_rows);
-        const long units = (long)p.v_heads * p.c_nrb;
-        const int chunk_max = col_chunk_max(p.Dp, p.c_waves);
+        const int rows = 32 * p.c_nb * p.c_waves;
+        p.c_nrb = ceil_div(p.v_rows, rows);
+        const int start = start_places(p.Dp, 32 * p.c_nb);
+        const long units = (long)p.v_heads * p.c_nrb;  // per batch entry
+        int most = col_chunk_max(p.Dp, p.c_waves) / kStageKeys;
+        if (tight_stages > 0 && tight_stages < most) most = tight_stages;
         const long target = (p.c_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
-        int chunk = ceil_div(Sk, kStageKeys) * kStageKeys;
-        if (chunk > chunk_max) chunk = chunk_max;
-        int nchunks = ceil_div(Sk, chunk);
-        long groups = (target + (long)B * nchunks - 1) / ((long)B * nchunks);
-        if (groups > units) {
-            // one unit per block is still too few blocks: shorter chunks (at least four stages each)
-            groups = units;
-            const long want_c = target / ((long)B * units);  // rounded down: stay within one generation
-            int c = ceil_div(ceil_div(Sk, (int)(want_c < 1 ? 1 : want_c)), kStageKeys) * kStageKeys;
-            if (c < 4 * kStageKeys) c = 4 * kStageKeys;
-            if (c < chunk) chunk = c;
-            nchunks = ceil_div(Sk, chunk);
-        } else {
-            // Blocks run in generations of `target` (what the GPU holds at once); a launch takes
-            // generations x units per block.  Among a few group counts around whole generations take
-            // the cheapest: one block over a generation would double the time of the launch.
-            const long per = (long)B * nchunks;
-            long cand[6] = {groups, target / per, 2 * target / per, 3 * target / per, 4 * target / per, units};
-            double best = 0.;
-            long best_g = groups;
-            for (int ci = 0; ci < 6; ++ci) {
-                long gcnt = cand[ci];
-                if (gcnt < 1) gcnt = 1;
-                if (gcnt > units) gcnt = units;
-                const long upg = (units + gcnt - 1) / gcnt;
-                const long g_eff = (units + upg - 1) / upg;
-                const long gens = (per * g_eff + target - 1) / target;
-                const double cost = (double)gens * ((double)upg + 0.15) + 0.0005 * (double)g_eff;
-                if (ci == 0 || cost < best) {
-                    best = cost;
-                    best_g = g_eff;
-                }
+        const StageLine stages = line_of(rows, p.c_nrb);
+        const int n = seen_stages;
+        const double all = stages_of(stages, p.c_nrb);
+        const bool huge = all * (1. + start) >= kHuge;
+        // what the final reduction takes, in stages: a launch, and the slabs, written and read
+        const auto reduce = [&](long shares, int c) { return 2.5 + (double)shares * c * 1e-4; };
+        const int parts0 = ceil_div(n, most), parts_end = ceil_div(n, kMinShare);
+        int cs = 1, seg = 1;
+        enum { kShares, kUnits, kDirect } how = kDirect;
+        double best = 1e300;
+        for (int parts = parts0; parts <= parts_end && parts < parts0 + 128; ++parts) {
+            const int c = ceil_div(n, parts);
+            if (ceil_div(n, c) != parts) continue;
+            const long pieces = (long)B * parts * units;  // chunks of the units
+            if (!huge) {
+                StageLine l = stages;
+                l.start = start;
+                int sg = (int)(((int64_t)B * p.v_heads * l.chunk_places(p.c_nrb, c, parts) + target - 1) / target);
+                if (sg < kMinShare + start) sg = kMinShare + start;
+                const double cost = sg + start + reduce(target, c);
+                if (cost < best) { best = cost; cs = c; seg = sg; how = kShares; }
             }
-            groups = best_g;
+            // whole ones per workgroup where all units are equal, or a workgroup for each
+            const long per = (pieces + target - 1) / target;
+            if (!huge && (stages.step == 0 || per == 1)) {
+                const double cost = (double)per * (c + start) + reduce(pieces / per, c);
+                if (cost < best) { best = cost; cs = c; seg = (int)per; how = kUnits; }
+            }
+            // a workgroup per chunk, which writes the means itself: no slabs, no final reduction
+            const double cost = (double)((B * (long)parts + target - 1) / target) * (double)units * (c + start);
+            if (cost <= best) { best = cost; cs = c; how = kDirect; }
+            if (pieces > 4 * target && parts > parts0 + 8) break;
         }
-        if (groups < 1) groups = 1;
-        p.c_chunk = chunk;
-        p.c_nchunks = nchunks;
-        p.c_upg = (int)((units + groups - 1) / groups);
-        p.c_groups = (int)((units + p.c_upg - 1) / p.c_upg);
+        const int used = ceil_div(n, cs);  // chunks that some row sees
+        p.c_chunk = cs * kStageKeys;
+        p.c_nchunks = ceil_div(Sk, p.c_chunk);
+        p.c_line = stages;
+        p.c_line.start = start;
+        p.c_unit = 1;
+        p.c_cs = cs;
+        if (how != kShares) {  // counted in chunks (the kernel stops a unit at the last key that it sees)
+            p.c_line = StageLine{used, 0, used, 0, 0};
+            p.c_unit = cs;
+            p.c_cs = 1;
+        }
+        const long chunks = (long)B * p.c_nchunks;
+        if (chunks >= (1L << 31)) return false;
+        p.c_direct = how == kDirect;
+        p.c_one = how == kUnits && seg == 1;
+        p.c_by_blocks.set(p.c_nrb);
+        p.c_by_used.set(used);
+        p.c_len = p.c_seg = p.c_groups = p.n_partials = 1;
+        p.c_blocks = (int)chunks;
+        p.c_by_batch.set(1);
+        if (how != kDirect) {
+            const int per_batch = p.v_heads * p.c_line.chunk_places(p.c_nrb, p.c_cs, used);
+            p.c_len = B * per_batch;
+            if (seg > p.c_len) seg = p.c_len;
+            p.c_seg = seg;
+            p.c_blocks = ceil_div(p.c_len, seg);
+            p.c_groups = (int)(1 + p.c_blocks / chunks);
+            p.n_partials = p.v_heads * p.c_line.chunk_places(p.c_nrb, p.c_cs, 1) / seg + 2;  // of the first chunk, the most seen
+            p.c_by_batch.set(per_batch);
+        }
+        p.c_by_seg.set(p.c_seg);
+        p.c_by_chunks.set(p.c_nchunks);
+        p.c_by_chunk.set(p.c_chunk);
     }
 
     // ---- few-rows path: a batch of matrix-vector products, one workgroup per (batch entry, head group)
@@ -257,7 +435,6 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     }
 
     // ---- fused path
-    p.n_partials = p.c_groups;
     // (at least one whole key tile: the kernel moves a tile that reaches past the last key back to end there)
     // (64-wide kernels for head dims up to 64, 128-wide ones up to 128; wider heads take the two-pass path)
     // (Heads of 72 .. 120 channels: the 128-wide kernel's variant for narrower heads runs out of registers at seven
@@ -317,17 +494,35 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         return (long)p.f_nwgq * B * p.f_hg < (1L << 31);
     }
 
-    // ---- workspace
+    // ---- workspace.  Its size must not depend on k_past (fcs_workspace_bytes does not know it), so the parts that the shares
+    // need are sized for the most that any k_past gives: a workgroup leaves one set of row statistics per row block
+    // that it touches (with a block that is cut, one more than the cuts), and one slab per chunk.
+    const int64_t stages = ceil_div(Sk, kStageKeys);
+    const int64_t row_blocks = (int64_t)B * p.v_heads * p.n_qblk, units = (int64_t)B * p.v_heads * p.c_nrb;
+    const int64_t r_most = row_blocks * ceil_div((int)stages, kMinShare);
+    const int64_t c_slots = (p.c_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
+    const int64_t chunk_most = tight_stages > 0 ? p.c_chunk / kStageKeys : col_chunk_max(p.Dp, p.c_waves) / kStageKeys;
+    const int64_t c_most = stages < chunk_most ? stages : chunk_most;
+    const int64_t c_shares = units * ceil_div((int)stages, kMinShare);
+    const int64_t slab_stages = (c_slots < c_shares ? c_slots : c_shares) * c_most + B * (stages + c_most);
     size_t off = 0;
     p.off_lse = off;
     off = align256(off + 2 * sizeof(float) * (size_t)B * p.v_heads * p.rows_pad);
     p.off_ml = off;
-    if (p.n_chunks > 1) off = align256(off + 2 * sizeof(float) * (size_t)B * p.v_heads * p.n_chunks * p.rows_pad);
+    if (tight_stages == 0) off = align256(off + 2 * sizeof(float) * (size_t)qblk * (size_t)(r_most < p.gen_blocks ? r_most : p.gen_blocks));
     p.off_partial = off;
-    if (p.c_groups > 1) off = align256(off + sizeof(float) * (size_t)p.c_groups * B * Sk);
+    if (tight_stages == 0 || !p.c_direct) off = align256(off + sizeof(float) * kStageKeys * (size_t)slab_stages);
     p.total = off;
-    // both passes launch one-dimensional grids
-    return (long)p.n_qblk * p.n_chunks * B * p.v_heads < (1L << 31) && (long)p.c_nchunks * p.c_groups * B < (1L << 31);
+    return true;
+}
+
+// The plan for a workspace of `bytes`: the usual one, or one that needs less.  False if none fits.
+inline bool plan_within(Plan &p, size_t bytes, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past)
+{
+    if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return false;
+    for (int stages = 32; p.total > bytes && stages >= 1; stages /= 2)
+        if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, stages)) return false;
+    return p.total <= bytes;
 }
 
 }  // namespace fcs

@@ -15,14 +15,16 @@ size_t describe_two_pass(const Plan &p, const Args &a, char *buf, size_t n)
     const bool pre = stream_prescaled(p, a);
     const int nb1 = p.qw / 32;
     const char *fold = p.fold > 1 ? ",true" : "";  // query heads of a key head in one unit
+    const char *bf = p.bf16 ? "true" : "false", *ps = pre ? "true" : "false";
+    const long heads = (long)p.B * p.v_heads;
     int r = snprintf(buf, n,
-                     "fcs_rowstream_kernel<%d,%d,%d,%s,%s%s> grid %d x %d x %d + fcs_colstream_kernel<%d,%d,%d,%s,%s%s> grid %d x %d x %d, "
-                     "%d units per workgroup",
-                     p.Dp, nb1, p.k1_waves, p.bf16 ? "true" : "false", pre ? "true" : "false", fold, p.n_qblk, p.n_chunks, p.B * p.v_heads, p.Dp,
-                     p.c_nb, p.c_waves, p.bf16 ? "true" : "false", pre ? "true" : "false", fold, p.c_nchunks, p.c_groups, p.B, p.c_upg);
+                     "fcs_rowstream_kernel<%d,%d,%d,%s,%s%s> grid %d x %d x %ld, %d shares of %d places + fcs_colstream_kernel<%d,%d,%d,%s,%s%s> "
+                     "grid %d, shares of %d places, chunks of %d keys%s",
+                     p.Dp, nb1, p.k1_waves, bf, ps, fold, p.n_qblk, p.n_chunks, heads, p.r_blocks, p.r_seg * p.r_unit, p.Dp, p.c_nb, p.c_waves, bf, ps, fold,
+                     p.c_blocks, p.c_seg * p.c_unit, p.c_chunk, p.c_direct ? ", direct" : "");
     if (r < 0) return 0;
     const size_t len = (size_t)r;
-    if (p.c_groups > 1) return len + describe_finalize(a, len < n ? buf + len : nullptr, len < n ? n - len : 0);
+    if (!p.c_direct) return len + describe_finalize(a, len < n ? buf + len : nullptr, len < n ? n - len : 0);
     return len;
 }
 

@@ -37,10 +37,18 @@
 //     Q 512, K 4096, D 256 37.6 -> 34.4 (34.9).  Carrying the last tile over to the next stage, as the plain loop does,
 //     was 0.1 % faster there and up to 7 % slower on short streams (H 8, Q 128, K 1000, D 64 16.3 -> 17.3 us); for
 //     64-row waves it was slower throughout (H 32, S 2000, D 64 58.0 -> 59.8).
-// A workgroup owns a chunk of keys (at most kColChunkMax, the LDS accumulator) and walks over a
-// group of (head, row block) units, re-streaming its chunk for each; at the end the waves'
-// slices are added in wave order and written as one partial slab (or the means directly, when
-// there is a single group).  Causal alignment  j <= k_past + i  (reference:
+// The keys are cut into chunks (at most col_chunk_max(), the LDS accumulator).  The work is a line of stages: batch
+// entry, chunk, head, row block, stage; every workgroup takes an equal share of it (StageLine in fcs_plan.h), walks over the
+// (head, row block) units of its share, re-streaming the chunk for each, and leaves one partial slab per chunk that it
+// touched: the waves' slices added in wave order.  What bounds a call that is cut unit by unit is its longest
+// workgroup: of a causal prompt the row blocks see 8, 16, .. 64 stages, and of 144 or 304 equal units every second or the
+// last compute units have nothing to do.  Both passes on the line, against whole units (this pass and pass 1, us per
+// call): causal H 32, S 4096, D 128 bf16 229 -> 163; H 12, S 5242, D 64 178 -> 124; H 12, S 4491, D 64 bf16 146 -> 102;
+// H 16, S 9459, D 64 571 -> 467; H 8, S 4435, D 128 bf16 causal 97 -> 69.  Where whole units of one length fill
+// the chip evenly the plan keeps to them, one to a workgroup (ONE: the walk and its state are compiled out; a small call spends
+// half its time before the first stage, and cold instructions are a good part of that: H 8, S 2219, D 64 18.2 -> 16.3 us).
+// At a unit's start the first stages, the row statistics and the query rows are requested together, and nothing is
+// requested past a unit's last stage.  Causal alignment  j <= k_past + i  (reference:
 // flash_colsum/kernel_causal.py:39,57,113): the stage loop stops at the last key any row of the
 // unit sees, only stages on the diagonal (or past the last key) take the masked code path.
 #pragma once
@@ -51,6 +59,7 @@
 
 #include "fcs_device.h"
 #include "fcs_kernels.h"
+#include "fcs_rowfold.h"
 
 namespace fcs {
 
@@ -105,6 +114,85 @@ __device__ __forceinline__ const _Float16 *q_row_ptr(const Args &a, int b, int h
     }
 }
 
+// Which 16-byte piece of its row a lane of half-wave g takes for MFMA step t (the contraction may run in any order, as long as
+// both operands take the same one): four steps take 64 consecutive bytes of a row.
+template <int NTA>
+__host__ __device__ constexpr int piece_of(int t, int g)
+{
+    return t % NTA + NTA * g + 2 * NTA * (t / NTA);
+}
+
+// The stationary rows.  A lane needs pieces of its own row, but four neighbouring lanes first read 64 consecutive bytes of one
+// of their four rows after the other: an access of four lanes to four rows takes the address path four times as long (a block of
+// 512 rows of 128 channels had its rows 5 .. 9 us after its start, the first stages long before).  Row pass with 32 bytes of a
+// row per access, then with this, against the same kernel on the same box: H 32, Q 512, K 65536, D 128 0.985 and 0.977 of its
+// time, H 16, S 8192, D 64 0.978 and 0.967.  load_quads leaves row
+// (lane & ~3) + j in f[nb][4 * i + j], pieces 4 * i ..; quad_transpose then hands every lane its own row.
+template <int D, int NB, bool FOLD>
+__device__ __forceinline__ void load_quads(const Args &a, int b, int h, int first_row, int lane, half8 (&f)[NB][D / 16])
+{
+    constexpr int NT = D / 16, NTA = NT < 8 ? NT : 8;
+    const int n4 = lane & 28, q = lane & 3, g = lane >> 5;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const _Float16 *row = q_row_ptr<FOLD>(a, b, h, first_row + nb * 32 + n4 + j);
+#pragma unroll
+            for (int i = 0; i < NT / 4; ++i) {
+                // (narrower heads: the row's last piece again in the place of those past it, see zero_past_dim)
+                const int at = (piece_of<NTA>(4 * i, g) + q) * 8;
+                f[nb][4 * i + j] = load8(row + min(at, a.D - 8));
+            }
+        }
+}
+// 4 x 4 transposes within four neighbouring lanes: two rounds of exchanges, with the lane 1 away and with the lane 2 away.
+// v_cndmask_b32 with the quad permutation on its first source does select and exchange in one; a register that a vector
+// instruction wrote may be read through a permutation two wait states later.
+#define FCS_QUAD_PICK(DST, OTHER, OWN, PERM) "v_cndmask_b32_dpp " DST ", " OTHER ", " OWN ", vcc quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"
+template <int NT>
+__device__ __forceinline__ void quad_transpose(half8 (&f)[NT])
+{
+    const uint64_t even = 0x5555555555555555ull, low = 0x3333333333333333ull;
+#pragma unroll
+    for (int i = 0; i < NT; i += 4) {
+        uint4v x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = __builtin_bit_cast(uint4v, f[i + j]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            uint32_t p0 = x[0][c], p1 = x[1][c], p2 = x[2][c], p3 = x[3][c], y0, y1, y2, y3;
+            asm("s_mov_b64 vcc, %8\n\ts_nop 1\n\t"                            // even lanes keep rows 0 and 2
+                FCS_QUAD_PICK("%4", "%1", "%0", "[1,0,3,2]") FCS_QUAD_PICK("%6", "%3", "%2", "[1,0,3,2]")
+                "s_not_b64 vcc, vcc\n\t"                                        // odd lanes rows 1 and 3
+                FCS_QUAD_PICK("%5", "%0", "%1", "[1,0,3,2]") FCS_QUAD_PICK("%7", "%2", "%3", "[1,0,3,2]")
+                "s_mov_b64 vcc, %9\n\ts_nop 1\n\t"                            // then the same two lanes apart
+                FCS_QUAD_PICK("%0", "%6", "%4", "[2,3,0,1]") FCS_QUAD_PICK("%1", "%7", "%5", "[2,3,0,1]")
+                "s_not_b64 vcc, vcc\n\t"
+                FCS_QUAD_PICK("%2", "%4", "%6", "[2,3,0,1]") FCS_QUAD_PICK("%3", "%5", "%7", "[2,3,0,1]")
+                : "+v"(p0), "+v"(p1), "+v"(p2), "+v"(p3), "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3)
+                : "s"(even), "s"(low)
+                : "vcc", "scc");
+            x[0][c] = p0;
+            x[1][c] = p1;
+            x[2][c] = p2;
+            x[3][c] = p3;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f[i + j] = __builtin_bit_cast(half8, x[j]);
+    }
+}
+#undef FCS_QUAD_PICK
+// channels past the tensor's head dim are zeros
+template <int NT>
+__device__ __forceinline__ void zero_past_dim(half8 (&f)[NT], int dim, int g)
+{
+    constexpr int NTA = NT < 8 ? NT : 8;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        if (piece_of<NTA>(t, g) * 8 >= dim) f[t] = kZero8;
+}
+
 // causal calls: one past the last row (within its head) of the rows [v0, v1) that see the most keys, and the row that
 // sees the fewest of the wave's `n` rows from v on
 template <bool FOLD>
@@ -142,6 +230,15 @@ __device__ __forceinline__ void mask_rows(const Args &a, int v0, int g4, int &re
     } else {
         add([](int) { return 0; });
     }
+}
+
+// A stage with n - 1 more behind it in its stream is entered (n > 0): the one behind it has landed once at most the stages
+// requested after that are outstanding, NS - 3 of them, or none at the stream's end.  (Other loads in flight make it wait longer.)
+template <int NS, int IPW>
+__device__ __forceinline__ void wait_stages(int n)
+{
+    if (NS > 3 && n >= NS - 1) FCS_WAIT_VM((NS - 3) * IPW);
+    else FCS_WAIT_VM(0);
 }
 
 // How many of the nst stages from key k0 on lie within the keys up to `thr`, which all rows of a wave see
@@ -192,7 +289,8 @@ __device__ __forceinline__ half8 prescale(half8 v, float cs)
 // are averaged over few rows and keep the raw operand).  A unit therefore streams in up to two phases, the
 // pre-scaled stages first, then the raw ones after reloading Q.  Units with a stabilised row keep the raw operand
 // and the two-constant form throughout.
-template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD>
+// ONE: a workgroup has one chunk of one unit (see the plan).
+template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD, bool ONE>
 __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args a)
 {
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
@@ -207,6 +305,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
     constexpr int PPR = D / 8;                 // 16-byte pieces per row
     constexpr int STAGE_BYTES = KT * ROW_BYTES;
     constexpr int IPW = KT * PPR / THREADS;    // DMA instructions per wave per stage
+    constexpr int ROWS1 = D == 256 ? 128 : BLOCK_ROWS;  // pass 1's row blocks
     constexpr int NS = col_ring_slots(D, WAVES);
     constexpr int CHUNK = col_chunk_max(D, WAVES);
     static_assert(IPW >= 1 && KT * PPR == IPW * THREADS, "a stage is a whole number of DMA instructions per wave");
@@ -221,16 +320,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int cx, grp, b;  // chunks of one (group, batch entry) stream the same Q: neighbours in launch order
-    xcd_contiguous_block((int)blockIdx.x, a.c_nchunks, a.c_groups, a.B, cx, grp, b);  // a one-dimensional grid: no axis limit
-    const int c0 = cx * a.c_chunk;                     // first key of the chunk
-    const int c1 = min(a.Sk, c0 + a.c_chunk);          // one past its last key
-    const int u_begin = grp * a.c_upg, u_end = min(a.v_heads * a.c_nrb, u_begin + a.c_upg);
+    fetch_args(a);
+    int share = xcd_contiguous((int)blockIdx.x, a.c_blocks);  // neighbours on the line run on one XCD
     const float cmul = (a.c == 0.f) ? 1.f : a.c;       // scale 0: Q is zeroed instead and n_i = -log2 l_i
 
-    // ---- this wave's slice of the column accumulator
-    float *colw_w = colw + wave * CHUNK;
-    for (int i = lane * 4; i < CHUNK; i += 256) *reinterpret_cast<floatx4 *>(colw_w + i) = floatx4{0.f, 0.f, 0.f, 0.f};
+    const float inv_c = __builtin_amdgcn_rcpf(cmul);
+    float *colw_w = colw + wave * CHUNK;  // this wave's slice of the column accumulator
 
     // ---- DMA geometry: piece P of a stage goes to LDS byte 16 * P; it is piece pos ^ swizzle(row)
     // of stage row `row`, so that row r keeps piece p at position p ^ swizzle(r)
@@ -242,68 +337,86 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         g_off[j] = (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)((pos ^ row_swizzle<D>(row)) * 16);
     }
     char *ring_w = ring + wave * (IPW * 1024);  // where this wave's pieces of a stage land inside a slot
-    // operand read-back: lane (n, g) takes, for MFMA step t, piece 2t + g of row n (+ 32 per key fragment)
+    // operand read-back: lane (n, g) takes, for MFMA step t, piece piece_of(t, g) of row n (+ 32 per key fragment)
     uint32_t take[NTA];
 #pragma unroll
     for (int t = 0; t < NTA; ++t)
-        take[t] = lds_addr(ring) + (uint32_t)(n * ROW_BYTES + (((2 * t + g) ^ row_swizzle<D>(n)) * 16));
+        take[t] = lds_addr(ring) + (uint32_t)(n * ROW_BYTES + ((piece_of<NTA>(t, g) ^ row_swizzle<D>(n)) * 16));
 
-    for (int u = u_begin; u < u_end; ++u) {
-        const int h = u / a.c_nrb, rb = u - h * a.c_nrb;
+    // ---- where this workgroup's share of the line starts: batch entry, chunk, head, row block, place in it
+    int b, cx, h = 0, rb = 0, at = 0, left = 0x7fffffff;  // left: places of the share that are still to do
+    if constexpr (ONE) {
+        // The chunks of a unit side by side: of causal units the last ones are empty, and every XCD gets its part of them
+        // (H 32, Q = K 634, D 128: 15.6 us with a chunk's units side by side).
+        b = a.by_heads.quot(a.c_by_blocks.quot(a.c_by_used.quot(share, cx), rb), h);
+        share = ((b * (int)a.c_by_used.d + cx) * a.v_heads + h) * a.c_nrb + rb;
+    } else if (a.c_direct) {
+        b = a.c_by_chunks.quot(share, cx);
+    } else if (a.c_unit > 1) {  // counted in chunks of units
+        const int pos = share * a.c_seg;
+        left = min(a.c_seg, a.c_len - pos);
+        b = a.c_by_used.quot(a.by_heads.quot(a.c_by_blocks.quot(pos, rb), h), cx);
+    } else {
+        int pos = share * a.c_seg;
+        left = min(a.c_seg, a.c_len - pos);
+        b = a.c_by_batch.quot(pos, pos);
+        int lo = 0, hi;
+        for (cx = 0;; ++cx, lo = hi) {
+            hi = a.c_line.chunk_places(a.c_nrb, a.c_cs, cx + 1);
+            if (pos < a.v_heads * hi) break;
+        }
+        pos -= a.v_heads * lo;
+        const int per_h = hi - lo;
+        h = (int)((float)pos * __builtin_amdgcn_rcpf((float)per_h));  // the head or a neighbour of it
+        h = __builtin_amdgcn_readfirstlane(h);
+        for (pos -= h * per_h; pos < 0; --h) pos += per_h;
+        for (; pos >= per_h; ++h) pos -= per_h;
+        for (;; ++rb) {
+            const int n_rb = a.c_line.between(rb, cx * a.c_cs, (cx + 1) * a.c_cs), len = n_rb > 0 ? n_rb + a.c_line.start : 0;
+            if (pos < len) break;
+            pos -= len;
+        }
+        at = pos;
+    }
+
+    for (;;) {  // the chunks that the share touches
+    const int ck0 = cx * a.c_chunk;                    // first key of the chunk
+    const int c1 = min(a.Sk, ck0 + a.c_chunk);         // one past its last key
+    bool cleared = false;
+    auto clear_slice = [&]() {
+        const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
+        for (int i = lane * 4; i < a.c_chunk; i += 256)
+            asm volatile("ds_write_b128 %0, %1" ::"v"(lds_addr(colw_w) + (uint32_t)(i * 4)), "v"(zero4) : "memory");
+        cleared = true;
+    };
+
+    for (; left > 0 && h < a.v_heads; at = 0, rb = (rb + 1 == a.c_nrb) ? 0 : rb + 1, h += (rb == 0)) {
+        // the part of the row block's stages that belongs to the share
+        int c0 = ck0, c_past = c1;  // its first key, and one past its last
+        if constexpr (!ONE) {
+            const int all = a.c_line.between(rb, cx * a.c_cs, (cx + 1) * a.c_cs);
+            if (all <= 0) continue;  // no row of it sees the chunk
+            const int first = max(0, at - a.c_line.start), past = max(0, min(all, at + min(left, 0x3fffffff) - a.c_line.start));
+            left -= all + a.c_line.start - at;
+            if (past <= first) break;  // the share ends with places for its start
+            c0 += first * a.c_unit * KT;
+            c_past = min(c1, ck0 + past * a.c_unit * KT);
+        }
         const int row0 = rb * BLOCK_ROWS;                        // first query row of the unit
-        // keys of the chunk that some row of the unit sees
-        int kend = c1;
+        // keys of these stages that some row of the unit sees
+        int kend = c_past;
         if (a.causal) kend = min(kend, a.k_past + rows_past<FOLD>(a, row0 + BLOCK_ROWS));
         const int nst = (kend > c0) ? (kend - c0 + KT - 1) / KT : 0;
-        if (nst == 0) continue;  // block-uniform
-
-        // ---- per-row constants, merged over the key splits of pass 1
-        {
-            const int qi = row0 + tid;
-            float nl = -INFINITY;  // a row that is not averaged: every p comes out as 2^-inf = 0
-            float mm = 0.f, lg = 0.f;
-            if (tid < BLOCK_ROWS && qi < a.v_rows) {
-                const int64_t bh = (int64_t)b * a.v_heads + h;
-                if (a.n_chunks == 1) {
-                    const float2 v = a.lse[bh * a.rows_pad + qi];
-                    mm = v.x;
-                    lg = v.y;
-                } else {
-                    const float2 *p = a.ml + bh * a.n_chunks * a.rows_pad + qi;
-                    mm = kNegBig * 4.f;
-                    float ll = 0.f;
-                    for (int ch0 = 0; ch0 < a.n_chunks; ch0 += 8) {  // eight loads in flight; folded in split order
-                        float2 v[8];
+        if (nst == 0) {  // block-uniform
+            if constexpr (ONE) break;
+            else continue;
+        }
+        const int n_whole = (a.D == D) ? min(nst, (a.Sk - c0) / KT) : 0;  // stages inside the tensor, of rows as wide as compiled
+        if constexpr (!ONE) {  // what derives from these is formed anew, not kept from unit to unit
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) {
-                            v[j].x = kNegBig * 4.f;
-                            v[j].y = 0.f;
-                            if (ch0 + j < a.n_chunks) v[j] = p[(int64_t)(ch0 + j) * a.rows_pad];
-                        }
+            for (int t = 0; t < NTA; ++t) asm volatile("" : "+v"(take[t]));
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) {  // fixed order: bit-reproducible
-                            // A split that pass 1 left unstabilised reports m = 0 and a sum of up to 2^110;
-                            // next to a stabilised split its weight 2^((0 - m) * c) alone underflows although
-                            // the product does not: the weights are applied as two square roots.
-                            const float mn = fmaxf(mm, v[j].x);
-                            const float wa = fast_exp2((mm - mn) * (0.5f * a.c)), wb = fast_exp2((v[j].x - mn) * (0.5f * a.c));
-                            ll = (ll * wa) * wa + (v[j].y * wb) * wb;
-                            mm = mn;
-                        }
-                    }
-                    lg = fast_log2(ll);
-                }
-                nl = (a.c == 0.f) ? -lg : -lg / a.c;
-            }
-            // a stabilised row switches the whole unit, or its wave (kRedoHeads), to the two-constant form
-            const bool sh = __builtin_amdgcn_ballot_w64(mm != 0.f) != 0;
-            if (lane == 0) shift_s[wave] = sh ? 1 : 0;
-            if (tid < BLOCK_ROWS) {
-                nl_s[tid] = nl;
-                if (PRE) np_s[tid] = (nl == -INFINITY) ? -INFINITY : -lg;
-                lg_s[tid] = lg;
-                cm_s[tid] = (nl == -INFINITY) ? -INFINITY : -mm;
-            }
+            for (int j = 0; j < IPW; ++j) asm volatile("" : "+v"(g_off[j]));
         }
 
         // ---- stationary operand: this wave's query rows of head h, as they are in memory
@@ -312,17 +425,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         auto load_q_rows = [&]() {
             int lane_o = lane;
             asm volatile("" : "+v"(lane_o));  // addresses are formed here, not kept for a second call
-            const int n_o = lane_o & 31, g_o = lane_o >> 5;
+            load_quads<D, NB, FOLD>(a, b, h, qw0, lane_o, qf);
+        };
+        auto take_q_rows = [&]() {  // once they have come
+            int lane_o = lane;
+            asm volatile("" : "+v"(lane_o));
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
-                const _Float16 *row = q_row_ptr<FOLD>(a, b, h, qw0 + nb * 32 + n_o) + g_o * 8;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    half8 v = kZero8;  // channels past the tensor's head dim are zeros
-                    if (t * 16 + g_o * 8 < a.D) v = load8(row + t * 16);
-                    if (a.c == 0.f) v = kZero8;
-                    qf[nb][t] = v;
-                }
+                quad_transpose(qf[nb]);
+                if (a.D != D) zero_past_dim(qf[nb], a.D, lane_o >> 5);
             }
         };
         // the form the matrix pipe takes: pre-scaled (sign included), or raw with the scale's sign
@@ -332,25 +443,29 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     if (PRE && scaled) qf[nb][t] = prescale(qf[nb][t], a.negate ? -a.c : a.c);
+                    else if (a.c == 0.f) qf[nb][t] = kZero8;
                     else if (a.negate) qf[nb][t] = flip_sign(qf[nb][t]);
                 }
         };
-        load_q_rows();
         const char *kp = reinterpret_cast<const char *>(a.k + (int64_t)b * a.ks_b +
                                                         (int64_t)kv_head(h, a.kv_group, a.kv_magic) * a.ks_h);
         const int64_t k_row_b = a.ks_s * 2;
 
-        // stage `st` of the unit into ring slot `slot` (stages past the last one repeat it, so that the
-        // number of DMA instructions in flight at every wait is a compile-time constant).
-        auto fetch_stage = [&](int st, int slot) {
-            const int kb = c0 + min(st, nst - 1) * KT;
+        // stage `st` of the unit into ring slot `slot`
+        // The stages of a stream are requested in order; k_src is where the next one starts.
+        const char *k_src;
+        auto fetch_whole = [&](int slot) __attribute__((always_inline)) {  // a stage inside the tensor, of rows as wide as compiled
             char *dst = ring_w + slot * STAGE_BYTES;
-            // whole stage inside the tensor, rows as wide as compiled (wave-uniform; the other case out of line)
-            if (__builtin_expect(kb + KT <= a.Sk && a.D == D, 1)) {
-                const char *src = kp + (int64_t)kb * k_row_b;
 #pragma unroll
-                for (int j = 0; j < IPW; ++j) dma16(src + g_off[j], dst + j * 1024);
-            } else {  // rows past the last key re-read it; the consumer masks them
+            for (int j = 0; j < IPW; ++j) dma16(k_src + g_off[j], dst + j * 1024);
+            k_src += KT * k_row_b;
+        };
+        auto fetch_stage = [&](int st, int slot) __attribute__((always_inline)) {
+            if (__builtin_expect(st < n_whole, 1)) {
+                fetch_whole(slot);
+            } else {  // rows past the last key re-read it (the consumer masks them), pieces past the head dim are zeros
+                const int kb = c0 + st * KT;
+                char *dst = ring_w + slot * STAGE_BYTES;
                 int lane_o = lane;
                 asm volatile("" : "+v"(lane_o));  // formed here, not kept in registers through the stream
 #pragma unroll
@@ -359,10 +474,19 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                     const int row = P / PPR, pos = P % PPR;
                     const int piece = pos ^ row_swizzle<D>(row);
                     const char *src = kp + (int64_t)min(kb + row, a.Sk - 1) * k_row_b + piece * 16;
-                    if (piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_zero_piece);  // past the head dim: zeros
+                    if (piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_zero_piece);
                     dma16(src, dst + j * 1024);
                 }
             }
+        };
+        // Stage `st` of the stream [.., s1) is entered: the one behind it has landed (this wave's pieces; the barrier extends that
+        // to everyone's), and every wave is done reading the stage before it, whose slot takes the next fetch.
+        auto enter = [&](int st, int s1) __attribute__((always_inline)) {
+            wait_stages<NS, IPW>(s1 - st);
+            block_barrier();
+        };
+        auto fetch_ahead = [&](int st, int s1, int slot) __attribute__((always_inline)) {
+            if (st + NS - 1 < s1) fetch_stage(st + NS - 1, slot);
         };
 
         // key fragment `na` of the stage in `slot` as MFMA B operand.  Inline assembly: the compiler
@@ -397,11 +521,101 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             }
         };
 
-        // ---- prologue of the unit's first phase: NS - 1 stages in flight; stages 0 and 1 must have landed
-        // before the first barrier
+        // ---- prologue of the unit's first phase: NS - 1 stages in flight, then the statistics, then the query rows, which
+        // share their latency; the statistics are worked on while the query rows come
+        auto fetch_first = [&](int s0, int s1) __attribute__((always_inline)) {
+            k_src = kp + (int64_t)(c0 + s0 * KT) * k_row_b;
 #pragma unroll
-        for (int st = 0; st < NS - 1; ++st) fetch_stage(st, st);
-        FCS_WAIT_VM((NS - 3) * IPW);
+            for (int st = 0; st < NS - 1; ++st)
+                if (s0 + st < s1) fetch_stage(s0 + st, st);
+        };
+        const int n_pre_most = PRE ? min(nst, max(0, (a.pre_end - c0) / KT)) : 0;
+        fetch_first(0, nst);
+
+        // ---- the row statistics that pass 1 left: (m, log2 l), or the parts' (m, l)
+        const int qi = row0 + tid;
+        const bool real = tid < BLOCK_ROWS && qi < a.v_rows;
+        int parts = 1;
+        const float2 *stat = a.stat;
+        {
+            const int rb1 = (row0 + wave * 64) / ROWS1;  // pass 1's row block (ROWS1 rows: those of a wave lie in one)
+            const int i1 = (b * a.v_heads + h) * a.n_qblk + rb1;
+            int w0 = 0;
+            if (!a.r_whole) {
+                const int start = (b * a.v_heads + h) * (int)a.r_by_head.d + a.r_line.places(rb1) + a.r_line.start;
+                w0 = a.r_by_seg.quot(start);
+                parts = a.r_by_seg.quot(start + a.r_line.n(rb1) - 1) - w0 + 1;
+            }
+            stat += ((int64_t)w0 + i1) * ROWS1 + (min(qi, a.v_rows - 1) - rb1 * ROWS1);
+        }
+        constexpr int PB = (NB == 1 && D < 256) ? 16 : D < 256 ? 8 : 4;  // parts in flight
+        float2 part[PB];
+        auto load_parts = [&](int ch0) {  // (past the last one: that one again, for nothing)
+#pragma unroll
+            for (int j = 0; j < PB; ++j) part[j] = stat[(int64_t)min(ch0 + j, parts - 1) * ROWS1];
+        };
+        if ((BLOCK_ROWS >= THREADS || wave * 64 < BLOCK_ROWS) && row0 + wave * 64 < a.v_rows) load_parts(0);
+        load_q_rows();
+
+        // ---- meanwhile: the accumulator slice of a new chunk; the per-row constants, merged over the parts of pass 1.  (Inline
+        // assembly: the compiler could make ordinary LDS accesses wait for the DMA.)
+        if (!cleared) clear_slice();
+        {
+            float nl = -INFINITY;  // a row that is not averaged: every p comes out as 2^-inf = 0
+            float mm = 0.f, lg = 0.f;
+            if (real) {
+                // Added up in split order: bit-reproducible.  The usual parts are unstabilised (m = 0) or empty (both 0), and
+                // the row's sum is the sum of theirs.
+                float ll = 0.f;
+                uint32_t stab = 0;  // a bit of any m
+                auto add_parts = [&](int ch0) {
+#pragma unroll
+                    for (int j = 0; j < PB; ++j) {
+                        ll += (ch0 + j < parts) ? part[j].y : 0.f;
+                        stab |= __float_as_uint(part[j].x);
+                    }
+                };
+                add_parts(0);
+                for (int ch0 = PB; ch0 < parts; ch0 += PB) {
+                    load_parts(ch0);
+                    add_parts(ch0);
+                }
+                lg = a.r_whole ? part[0].y : fast_log2(ll);
+                mm = part[0].x;
+                if (__builtin_expect((stab & 0x7fffffffu) != 0 && !a.r_whole, 0)) {
+                    // A split that pass 1 left unstabilised reports m = 0 and a sum of up to 2^110;
+                    // next to a stabilised split its weight 2^((0 - m) * c) alone underflows although
+                    // the product does not: the weights are applied as two square roots.
+                    mm = kNegBig * 4.f;
+                    ll = 0.f;
+                    for (int ch = 0; ch < parts; ++ch) {
+                        const float2 v = stat[(int64_t)ch * ROWS1];
+                        if (v.y == 0.f) continue;  // empty
+                        const float mn = fmaxf(mm, v.x);
+                        const float wa = fast_exp2((mm - mn) * (0.5f * a.c)), wb = fast_exp2((v.x - mn) * (0.5f * a.c));
+                        ll = (ll * wa) * wa + (v.y * wb) * wb;
+                        mm = mn;
+                    }
+                    lg = fast_log2(ll);
+                }
+                // -lg / c: the reciprocal's quotient and one correction by its remainder
+                const float q = lg * inv_c;
+                nl = -fmaf(fmaf(-q, cmul, lg), inv_c, q);
+            }
+            // a stabilised row switches the whole unit, or its wave (kRedoHeads), to the two-constant form
+            const int sh = __builtin_amdgcn_ballot_w64(mm != 0.f) != 0 ? 1 : 0;
+            asm volatile("ds_write_b32 %0, %1" ::"v"(lds_addr(shift_s) + (uint32_t)(wave * 4)), "v"(sh) : "memory");
+            if (tid < BLOCK_ROWS) {
+                const uint32_t at = (uint32_t)(tid * 4);
+                const float np = (nl == -INFINITY) ? -INFINITY : -lg, cm = (nl == -INFINITY) ? -INFINITY : -mm;
+                asm volatile("ds_write_b32 %0, %1" ::"v"(lds_addr(nl_s) + at), "v"(nl) : "memory");
+                if (PRE) asm volatile("ds_write_b32 %0, %1" ::"v"(lds_addr(np_s) + at), "v"(np) : "memory");
+                asm volatile("ds_write_b32 %0, %1" ::"v"(lds_addr(lg_s) + at), "v"(lg) : "memory");
+                asm volatile("ds_write_b32 %0, %1" ::"v"(lds_addr(cm_s) + at), "v"(cm) : "memory");
+            }
+        }
+        take_q_rows();
+        wait_stages<NS, IPW>(nst);
         block_sync();  // also publishes nl_s
 
         // The two-constant form: some row of the unit was stabilised by pass 1 (block-uniform), or, where pass 1 redoes single
@@ -414,7 +628,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             shifted = __builtin_amdgcn_ballot_w64(f != 0) != 0;
         }
         // leading stages of the unit that run on the pre-scaled operand (block-uniform)
-        const int n_pre = (!PRE || shifted) ? 0 : min(nst, max(0, (a.pre_end - c0) / KT));
+        const int n_pre = (!PRE || shifted) ? 0 : n_pre_most;
 
         // rows of this wave relative to the causal diagonal; non-causal: every key below Sk is visible
         const int kp_eff = a.causal ? a.k_past : 0x3fffffff - a.Sq;
@@ -431,9 +645,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             constexpr int FORM = decltype(form_c)::value;
             constexpr bool SC = FORM == kFormPrescaled, SHIFTED = FORM == kFormShifted;
             if (!fetched) {
-#pragma unroll
-                for (int st = 0; st < NS - 1; ++st) fetch_stage(s0 + st, st);
-                FCS_WAIT_VM((NS - 3) * IPW);
+                fetch_first(s0, s1);
+                wait_stages<NS, IPW>(s1 - s0);
                 block_sync();
             }
             floatx16 cinit[NB];  // row constants in accumulator layout: register i <-> row 8*(i/4) + 4*g + i%4
@@ -469,7 +682,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             uint32_t col_ad = 0;
             auto drain_begin = [&](int kb_t, int na, int nb) {
                 if (nb == 0) {
-                    col_ad = lds_addr(colw_w) + (uint32_t)((kb_t - c0 + na * 32 + n) * 4);
+                    col_ad = lds_addr(colw_w) + (uint32_t)((kb_t - ck0 + na * 32 + n) * 4);
                     asm volatile("ds_read_b32 %0, %1" : "=v"(col_old) : "v"(col_ad) : "memory");
                 }
             };
@@ -568,19 +781,16 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                     constexpr int SLOT = decltype(slot_c)::value;
                     const int kb = c0 + st * KT;
                     const bool first = SLOT == 0 && st == s0;
-                    if (!first) {
-                        // stage st + 1 has landed (this wave's pieces; the barrier extends that to everyone's), and
-                        // every wave is done reading stage st - 1, whose slot takes the next fetch
-                        FCS_WAIT_VM((NS - 3) * IPW);
-                        block_barrier();
-                    }
-                    fetch_stage(st + NS - 1, (SLOT + NS - 1) % NS);
+                    if (!first) enter(st, s1);
+                    if (NS == 3) fetch_ahead(st, s1, (SLOT + NS - 1) % NS);
 #pragma unroll
                     for (int q = 0; q < TILES; ++q) {
                         const int na = q / NB, nb = q % NB;
                         if (nb == 0) frag_wait(kf);
                         acc[q & 1] = chain(nb);
                         asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));  // the chain stays where it was written
+                        // (a ring of four: the fetch, which has time, does not stand between the barrier and the chain)
+                        if (NS > 3 && q == 0) fetch_ahead(st, s1, (SLOT + NS - 1) % NS);
                         if (nb == NB - 1) {  // this fragment's last chain has been issued: read back the next one
                             if (na == 0) take_frag(std::integral_constant<int, SLOT * STAGE_BYTES + 32 * ROW_BYTES>{}, kf);
                             else take_frag(std::integral_constant<int, ((SLOT + 1) % NS) * STAGE_BYTES>{}, kf);
@@ -614,11 +824,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             const int sv = min(s1, max(sp, n_seen));
             int slot = (sp - s0) % NS;
             auto enter_stage = [&](int st) {
-                if (st > s0) {
-                    FCS_WAIT_VM((NS - 3) * IPW);
-                    block_barrier();
-                }
-                fetch_stage(st + NS - 1, (slot == 0) ? NS - 1 : slot - 1);
+                if (st > s0) enter(st, s1);
+                fetch_ahead(st, s1, (slot == 0) ? NS - 1 : slot - 1);
                 slot = (slot + 1 == NS) ? 0 : slot + 1;
             };
             auto drain_one = [&](const floatx16 &sc, int kb_t, int na, int nb) {
@@ -670,10 +877,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 }
             }
             for (int st = sv; st < s1; ++st) enter_stage(st);
-            // the look-ahead fetches issued past the last stage must be over before the ring (and nl_s) is reused by
-            // the next phase or unit
-            FCS_WAIT_VM(0);
-            block_sync();
+            block_sync();  // the ring (and nl_s) is reused by the next phase or unit
         };
 
         // (one call site per form, so that the code of each exists once)
@@ -682,49 +886,66 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             shape_q(true);
             run_phase(std::integral_constant<int, kFormPrescaled>{}, 0, n_pre, true);
             raw0 = n_pre;
-            if (raw0 < nst) load_q_rows();  // the unit's last stages (causal: keys that not every row sees)
+            if (raw0 < nst) {  // the unit's last stages (causal: keys that not every row sees)
+                load_q_rows();
+                take_q_rows();
+            }
         }
         if (raw0 < nst) {
             shape_q(false);
             if (shifted) run_phase(std::integral_constant<int, kFormShifted>{}, 0, nst, true);
             else run_phase(std::integral_constant<int, kFormRaw>{}, raw0, nst, raw0 == 0);
         }
+        if constexpr (ONE) break;
     }
 
     // ---- add the waves' slices in wave order and store
+    if (!cleared) clear_slice();  // no row of any unit sees the keys
     block_sync();
-    const bool direct = (a.c_groups == 1);
-    for (int i = tid; i < c1 - c0; i += THREADS) {
+    float *slab = a.partial + ((int64_t)share + (int64_t)b * a.c_nchunks + cx) * a.c_chunk;
+    for (int i = tid; i < c1 - ck0; i += THREADS) {
         float v = colw[i];
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) v += colw[w * CHUNK + i];
-        const int64_t o = (int64_t)b * a.Sk + c0 + i;
-        if (direct) {
+        if (!ONE && a.c_direct) {
+            const int64_t o = (int64_t)b * a.Sk + ck0 + i;
             a.out[o] = v * a.inv_norm;
             if (a.out_h) a.out_h[o] = (_Float16)(v * a.inv_norm);
         } else {
-            a.partial[(int64_t)grp * a.B * a.Sk + o] = v;
+            slab[i] = v;
         }
+    }
+    if (ONE || a.c_direct || left <= a.c_line.start) break;
+    block_sync();  // the accumulators are cleared again
+    h = rb = at = 0;
+    // the next chunk that some row sees
+    do {
+        if (++cx == a.c_nchunks) {
+            cx = 0;
+            ++b;
+        }
+    } while (cx * a.c_cs >= a.c_line.last);
     }
 }
 
 // ------------------------------------------------------------------------------------
-// pass 1 on the same machinery: row maximum and sum of exponentials of one (row block, head, key split)
+// pass 1 on the same machinery: row maximum and sum of exponentials of the row blocks that a share of the line touches
 // ------------------------------------------------------------------------------------
 // Same orientation and stream as the column pass (Q stationary, K through the LDS-DMA ring), but the
 // exponentials are added up per ROW: register i of a lane keeps the running sum of its row over the
-// lane's keys for the whole split, and the 32 key lanes are added once at the end through LDS.
+// lane's keys for the part of the row block that the share has, and the 32 key lanes are added once at its end, in
+// registers (fcs_rowfold.h; through LDS it took 1.2 us and the space of a fourth ring slot at D 128).
 // Common case: 2^(c * s) without max subtraction, exact while every row sum of the split stays inside
 // [2^-80, 2^110); a block that leaves that range redoes its keys in two more sweeps (row maxima, then
 // sums of 2^((s - m) * c), the maximum subtracted before the scale).  FOLD: only the waves that hold rows of a
 // head with such a row redo, as when each head had a block of its own; the others take part in the fetches and barriers.
 // One row of a call out of range (K 65536, 16 on 2 heads, Q 128, D 64: blocks of 512 rows laid end to end):
 // 156 us, with none 105, with every wave of the block redoing 198, head by head 174.  Writes (m, log2 l) per row, or
-// (m, l) per (split, row) when the keys are split; the column pass merges the splits.
+// (m, l) per row and part when row blocks are cut; the column pass merges the parts.
 // PRE: see the column pass.  The common sweep runs its stages below a.pre_end on Q * c rounded to fp16 (then the
 // rest on the raw operand) and accepts row sums below 2^20 only; a block that leaves the range reloads the raw
 // operand for its stabilised sweeps, all waves of it: the column pass then takes the raw operand for the whole unit.
-template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD>
+template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD, bool ONE>
 __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args a)
 {
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
@@ -740,28 +961,28 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     constexpr int STAGE_BYTES = KT * ROW_BYTES;
     constexpr int IPW = KT * PPR / THREADS;
     constexpr int NS = row_ring_slots(D, WAVES);
-    constexpr int RP = 33;  // floats per row of the transpose buffer
     static_assert(IPW >= 1 && KT * PPR == IPW * THREADS, "a stage is a whole number of DMA instructions per wave");
     static_assert(NS >= 3 && NS <= 4, "ring depth");
     __shared__ __attribute__((aligned(16))) char ring[NS * STAGE_BYTES];
-    __shared__ __attribute__((aligned(16))) float red[WAVES * 32 * RP];  // wave-private [32 rows][RP]
     __shared__ __attribute__((aligned(16))) float mrow[BLOCK_ROWS];      // row maxima of the stabilised sweeps
     __shared__ int bad_s[WAVES];
     __shared__ int2 redo_s[kRedoHeads<PRE, FOLD> ? WAVES : 1];  // of such a wave: the rows that are redone, from .x to one before .y
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int bx, chunk, bh;  // row blocks of one (key split, head) read the same keys: same XCD
-    xcd_contiguous_block((int)blockIdx.x, a.n_qblk, a.n_chunks, a.B * a.v_heads, bx, chunk, bh);  // a one-dimensional grid: no axis limit
-    const int b = bh / a.v_heads, h = bh - b * a.v_heads;
-    const int row0 = bx * BLOCK_ROWS, qw0 = row0 + wave * ROWS_W;
     const float cmul = a.c;
 
-    // key range of this block: its split, cut at the last key any of its rows may see
-    const int kc0 = chunk * a.chunk_keys;
-    int kc1 = min(a.Sk, kc0 + a.chunk_keys);
-    if (a.causal) kc1 = min(kc1, a.k_past + rows_past<FOLD>(a, row0 + BLOCK_ROWS));
-    const int nst = (kc1 > kc0) ? (kc1 - kc0 + KT - 1) / KT : 0;
+    // ---- where this workgroup's share of the line starts: (batch entry, head), row block, stage
+    fetch_args(a);
+    const int share = xcd_contiguous((int)blockIdx.x, a.r_blocks);  // neighbours on the line run on one XCD
+    int pos = ONE ? share : share * a.r_seg;
+    int left = ONE ? 1 : min(a.r_seg, a.r_len - pos);  // places of the share that are still to do
+    const int bh = a.r_by_head.quot(pos, pos);
+    int bx = 0;
+    if (ONE || a.r_line.step == 0) bx = a.r_by_block.quot(pos);
+    else for (int sum = 0; pos >= (sum += a.r_line.n(bx) + a.r_line.start); ++bx) {}
+    int at = pos - a.r_line.places(bx);  // place in the row block
+    int h, b = a.by_heads.quot(bh, h);
 
     uint32_t g_off[IPW];
 #pragma unroll
@@ -774,46 +995,84 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     uint32_t take[NTA];
 #pragma unroll
     for (int t = 0; t < NTA; ++t)
-        take[t] = lds_addr(ring) + (uint32_t)(n * ROW_BYTES + (((2 * t + g) ^ row_swizzle<D>(n)) * 16));
+        take[t] = lds_addr(ring) + (uint32_t)(n * ROW_BYTES + ((piece_of<NTA>(t, g) ^ row_swizzle<D>(n)) * 16));
 
-    half8 qf[NB][NT];
-    auto load_q = [&](bool scaled) {  // this wave's query rows: pre-scaled, or raw with the scale's sign
-        int lane_o = lane;
-        asm volatile("" : "+v"(lane_o));  // addresses are formed here, not kept for a second call
-        const int n_o = lane_o & 31, g_o = lane_o >> 5;
+    // what derives from these is formed anew behind the call, not kept in registers from row block to row block or (the
+    // rare sweeps' addresses) through the common sweep
+    int lane_i = lane;
+    auto form_anew = [&]() {
+        asm volatile("" : "+v"(lane_i));
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const _Float16 *row = q_row_ptr<FOLD>(a, b, h, qw0 + nb * 32 + n_o) + g_o * 8;
+        for (int t = 0; t < NTA; ++t) asm volatile("" : "+v"(take[t]));
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                half8 v = kZero8;
-                if (t * 16 + g_o * 8 < a.D) v = load8(row + t * 16);
-                if (PRE && scaled) qf[nb][t] = prescale(v, a.negate ? -a.c : a.c);
-                else qf[nb][t] = a.negate ? flip_sign(v) : v;
-            }
-        }
+        for (int j = 0; j < IPW; ++j) asm volatile("" : "+v"(g_off[j]));
     };
-    // leading stages of the block that run on the pre-scaled operand in the common sweep (block-uniform)
-    const int n_pre = PRE ? min(nst, max(0, (a.pre_end - kc0) / KT)) : 0;
-    load_q(n_pre > 0);
-    const char *kp = reinterpret_cast<const char *>(a.k + (int64_t)b * a.ks_b +
-                                                    (int64_t)kv_head(h, a.kv_group, a.kv_magic) * a.ks_h);
+
+    // ---- the row block at hand: which of its stages belong to the share
     const int64_t k_row_b = a.ks_s * 2;
     const int kp_eff = a.causal ? a.k_past : 0x3fffffff - a.Sq;
-    const int thr_wave_min = a.causal ? min(a.k_past + rows_first<FOLD>(a, qw0, ROWS_W), a.Sk - 1) : a.Sk - 1;
-    const int thr_wave_max = a.causal ? a.k_past + (FOLD ? a.q_rows : qw0 + ROWS_W) - 1 : a.Sk - 1;
-    const int n_plain = plain_stages(kc0, nst, thr_wave_min), n_seen = seen_stages(kc0, nst, thr_wave_max);
+    int row0, qw0, kc0, nst, n_whole, n_plain, n_seen, n_pre;
+    const char *kp;
+    auto set_block = [&]() {
+        const int first = ONE ? at : max(0, at - a.r_line.start), past = ONE ? at + 1 : min(a.r_line.n(bx), at + left - a.r_line.start);
+        row0 = bx * BLOCK_ROWS;
+        qw0 = row0 + wave * ROWS_W;
+        // the keys of these stages, cut at the last key any of the block's rows may see
+        kc0 = first * a.r_unit * KT;
+        int kc1 = min(a.Sk, kc0 + (past - first) * a.r_unit * KT);
+        if (a.causal) kc1 = min(kc1, a.k_past + rows_past<FOLD>(a, row0 + BLOCK_ROWS));
+        nst = (kc1 > kc0) ? (kc1 - kc0 + KT - 1) / KT : 0;
+        n_whole = (a.D == D) ? min(nst, (a.Sk - kc0) / KT) : 0;  // stages inside the tensor, of rows as wide as compiled
+        // leading stages that run on the pre-scaled operand in the common sweep (block-uniform)
+        n_pre = PRE ? min(nst, max(0, (a.pre_end - kc0) / KT)) : 0;
+        const int thr_wave_min = a.causal ? min(a.k_past + rows_first<FOLD>(a, qw0, ROWS_W), a.Sk - 1) : a.Sk - 1;
+        const int thr_wave_max = a.causal ? a.k_past + (FOLD ? a.q_rows : qw0 + ROWS_W) - 1 : a.Sk - 1;
+        n_plain = plain_stages(kc0, nst, thr_wave_min);
+        n_seen = seen_stages(kc0, nst, thr_wave_max);
+        if (qw0 >= a.v_rows) n_plain = n_seen = 0;  // none of the wave's rows exists
+        kp = reinterpret_cast<const char *>(a.k + (int64_t)b * a.ks_b + (int64_t)kv_head(h, a.kv_group, a.kv_magic) * a.ks_h);
+    };
 
-    auto fetch_stage = [&](int st, int slot) {
-        const int kb = kc0 + min(st, nst - 1) * KT;
-        char *dst = ring_w + slot * STAGE_BYTES;
-        if (__builtin_expect(kb + KT <= a.Sk && a.D == D, 1)) {
-            const char *src = kp + (int64_t)kb * k_row_b;
+    half8 qf[NB][NT];
+    auto load_q = [&]() {  // this wave's query rows
+        int lane_o = lane;
+        asm volatile("" : "+v"(lane_o));  // addresses are formed here, not kept for a second call
+        load_quads<D, NB, FOLD>(a, b, h, qw0, lane_o, qf);
+    };
+    // the form the matrix pipe takes: pre-scaled (sign included), or raw with the scale's sign
+    auto shape_q = [&](bool scaled) {
+        int lane_o = lane;
+        asm volatile("" : "+v"(lane_o));
 #pragma unroll
-            for (int j = 0; j < IPW; ++j) dma16(src + g_off[j], dst + j * 1024);
-        } else {
+        for (int nb = 0; nb < NB; ++nb) {
+            quad_transpose(qf[nb]);
+            if (a.D != D) zero_past_dim(qf[nb], a.D, lane_o >> 5);
+        }
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                if (PRE && scaled) qf[nb][t] = prescale(qf[nb][t], a.negate ? -a.c : a.c);
+                else if (a.negate) qf[nb][t] = flip_sign(qf[nb][t]);
+            }
+    };
+
+    // The stages of a stream are requested in order; k_src is where the next one starts.
+    const char *k_src;
+    auto fetch_whole = [&](int slot) __attribute__((always_inline)) {  // a stage inside the tensor, of rows as wide as compiled
+        char *dst = ring_w + slot * STAGE_BYTES;
+#pragma unroll
+        for (int j = 0; j < IPW; ++j) dma16(k_src + g_off[j], dst + j * 1024);
+        k_src += KT * k_row_b;
+    };
+    auto fetch_stage = [&](int st, int slot) __attribute__((always_inline)) {
+        if (__builtin_expect(st < n_whole, 1)) {
+            fetch_whole(slot);
+        } else {  // rows past the last key re-read it (the consumer masks them), pieces past the head dim are zeros
+            const int kb = kc0 + st * KT;
+            char *dst = ring_w + slot * STAGE_BYTES;
             int lane_o = lane;
-            asm volatile("" : "+v"(lane_o));
+            asm volatile("" : "+v"(lane_o));  // formed here, not kept in registers through the stream
 #pragma unroll
             for (int j = 0; j < IPW; ++j) {
                 const int P = (wave * IPW + j) * 64 + lane_o;
@@ -824,6 +1083,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
                 dma16(src, dst + j * 1024);
             }
         }
+    };
+    // Stage `st` of the stream [.., s1) is entered: the one behind it has landed (this wave's pieces; the barrier extends that
+    // to everyone's), and every wave is done reading the stage before it, whose slot takes the next fetch.
+    auto enter = [&](int st, int s1) __attribute__((always_inline)) {
+        wait_stages<NS, IPW>(s1 - st);
+        block_barrier();
+    };
+    auto fetch_ahead = [&](int st, int s1, int slot) __attribute__((always_inline)) {
+        if (st + NS - 1 < s1) fetch_stage(st + NS - 1, slot);
     };
     half8 kf[NT];
     auto take_frag = [&](auto off_c, half8 (&dst)[NT]) {
@@ -861,8 +1129,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
 #pragma unroll
             for (int i = 0; i < 16; ++i) rs[nb][i] = decltype(max_c)::value ? kNegBig : 0.f;
     };
-    // A wave that is not `active` takes part in the fetches and barriers alone.
-    auto sweep = [&](auto max_c, auto shift_c, auto scaled_c, const int s0, const int s1, const bool active) {
+    // A wave that is not `active` takes part in the fetches and barriers alone.  `fetched`: the first NS - 1 stages have been
+    // requested already.
+    auto fetch_first = [&](int s0, int s1) __attribute__((always_inline)) {
+        k_src = kp + (int64_t)(kc0 + s0 * KT) * k_row_b;
+#pragma unroll
+        for (int st = 0; st < NS - 1; ++st)
+            if (s0 + st < s1) fetch_stage(s0 + st, st);
+    };
+    auto sweep = [&](auto max_c, auto shift_c, auto scaled_c, const int s0, const int s1, const bool active, const bool fetched) {
         constexpr bool MAXOP = decltype(max_c)::value;
         constexpr bool SHIFT = decltype(shift_c)::value;
         constexpr bool SCALED = decltype(scaled_c)::value;
@@ -870,10 +1145,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         constexpr int TILES = NA * NB;
         static_assert(NA == 2 && TILES % 2 == 0, "fragment offsets and the two alternating accumulators");
         if (s1 <= s0) return;  // block-uniform
-#pragma unroll
-        for (int st = 0; st < NS - 1; ++st) fetch_stage(s0 + st, st);
-        FCS_WAIT_VM((NS - 3) * IPW);
+        if (!fetched) fetch_first(s0, s1);
+        wait_stages<NS, IPW>(s1 - s0);
         block_sync();
+        const int n = lane_i & 31, g = lane_i >> 5;
         auto drain_plain = [&](const floatx16 &sc, int nb) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
@@ -912,17 +1187,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
             auto stage = [&](int st, auto slot_c) {
                 constexpr int SLOT = decltype(slot_c)::value;
                 const bool first = SLOT == 0 && st == s0;
-                if (!first) {
-                    FCS_WAIT_VM((NS - 3) * IPW);
-                    block_barrier();
-                }
-                fetch_stage(st + NS - 1, (SLOT + NS - 1) % NS);
+                if (!first) enter(st, s1);
+                if (NS == 3) fetch_ahead(st, s1, (SLOT + NS - 1) % NS);
 #pragma unroll
                 for (int q = 0; q < TILES; ++q) {
                     const int na = q / NB, nb = q % NB;
                     if (nb == 0) frag_wait(kf);
                     acc[q & 1] = chain(nb);
                     asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+                    if (NS > 3 && q == 0) fetch_ahead(st, s1, (SLOT + NS - 1) % NS);
                     if (nb == NB - 1) {
                         if (na == 0) take_frag(std::integral_constant<int, SLOT * STAGE_BYTES + 32 * ROW_BYTES>{}, kf);
                         else take_frag(std::integral_constant<int, ((SLOT + 1) % NS) * STAGE_BYTES>{}, kf);
@@ -944,11 +1217,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         const int sv = active ? min(s1, max(sp, n_seen)) : s0;
         int slot = (sp - s0) % NS;
         auto enter_stage = [&](int st) {
-            if (st > s0) {
-                FCS_WAIT_VM((NS - 3) * IPW);
-                block_barrier();
-            }
-            fetch_stage(st + NS - 1, (slot == 0) ? NS - 1 : slot - 1);
+            if (st > s0) enter(st, s1);
+            fetch_ahead(st, s1, (slot == 0) ? NS - 1 : slot - 1);
             slot = (slot + 1 == NS) ? 0 : slot + 1;
         };
         if constexpr (NB == 1 && D <= 128) {
@@ -995,125 +1265,161 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
             }
         }
         for (int st = sv; st < s1; ++st) enter_stage(st);
-        FCS_WAIT_VM(0);
         block_sync();  // the ring may be refilled by the next sweep
     };
 
-    // rs[nb][*] over the 32 key lanes: every lane gets the value of row nb * 32 + (lane % 32) of this wave.
-    // Fixed order of additions.  (No DMA is in flight here, so these are ordinary LDS accesses.)
-    float *red_w = red + wave * (32 * RP);
-    auto fold_lanes = [&](auto max_c, float (&tot)[NB]) {
-        constexpr bool MAXOP = decltype(max_c)::value;
+    // ---- the row blocks that the share touches.  The next one's rows and first stages are requested as soon as the sweep
+    // over this one has left the ring, ahead of its row sums.
+    set_block();
+    load_q();
+    fetch_first(0, PRE && n_pre > 0 ? n_pre : nst);
+    for (;;) {
+        form_anew();
+        if (nst == 0) block_sync();  // (in the place of the sweep's barriers: bad_s is written again)
+        shape_q(n_pre > 0);
+        // ---- common path: no max subtraction; the pre-scaled stages first, then the raw ones
+        reset_rows(std::false_type{});
+        if constexpr (PRE) {
+            sweep(std::false_type{}, std::false_type{}, std::true_type{}, 0, n_pre, true, true);
+            if (n_pre > 0 && n_pre < nst) {
+                load_q();
+                shape_q(false);
+            }
+        }
+        sweep(std::false_type{}, std::false_type{}, std::false_type{}, n_pre, nst, true, n_pre == 0);
+
+        const int c_b = b, c_h = h, c_bx = bx, c_at = at, c_left = left, c_kc0 = kc0, c_qw0 = qw0, c_nst = nst;
+        const bool c_pre = n_pre > 0;
+        left -= a.r_line.n(bx) + a.r_line.start - at;
+        const bool more = !ONE && left > a.r_line.start;  // (not more than places for the next one's start: nothing to do there)
+        if (more) {
+            at = 0;
+            if (++bx == a.n_qblk) {
+                bx = 0;
+                if (++h == a.v_heads) {
+                    h = 0;
+                    ++b;
+                }
+            }
+            set_block();
+            load_q();
+            fetch_first(0, PRE && n_pre > 0 ? n_pre : nst);
+        }
+
+        // ---- row sums over the 32 key lanes, in registers: a lane is left with row `rw` of each fragment, like its neighbour
+        const int lane_r = lane_i;
+        const int rw = 16 * ((lane_r >> 4) & 1) + 8 * ((lane_r >> 3) & 1) + 4 * (lane_r >> 5) + 2 * ((lane_r >> 2) & 1) + ((lane_r >> 1) & 1);
+        float lt[NB], m_row[NB];
+        bool has[NB], out[NB], bad = false;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) red_w[(8 * (i >> 2) + 4 * g + (i & 3)) * RP + n] = rs[nb][i];
-            __builtin_amdgcn_wave_barrier();
-            float v = MAXOP ? kNegBig : 0.f;  // each half-wave takes 16 of the row's 32 lanes' values
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const float x = red_w[n * RP + g * 16 + j];
-                v = MAXOP ? fmaxf(v, x) : v + x;
-            }
-            const float o = __shfl_xor(v, 32);
-            tot[nb] = MAXOP ? fmaxf(v, o) : (g == 0 ? v + o : o + v);  // lower half first in both halves
-            __builtin_amdgcn_wave_barrier();
+            lt[nb] = fold_lanes_sum(rs[nb], lane_r);
+            const int v = c_qw0 + nb * 32 + rw, qi = rows_first<FOLD>(a, v, 1);
+            const int thr = a.causal ? min(a.k_past + qi, a.Sk - 1) : a.Sk - 1;  // last key this row sees
+            has[nb] = c_nst > 0 && c_kc0 <= thr && v < a.v_rows;
+            // ceiling 2^110 rather than 2^120: up to 512 key splits of a row are added up by the column pass
+            out[nb] = has[nb] && !(lt[nb] >= 8.2718061e-25f && lt[nb] < (c_pre ? kRowSumHiPre : 1.2980742e+33f));
+            bad = bad || out[nb];
+            m_row[nb] = 0.f;
+            if (!has[nb]) lt[nb] = 0.f;  // an empty split
         }
-    };
-
-    // ---- common path: no max subtraction; the pre-scaled stages first, then the raw ones
-    reset_rows(std::false_type{});
-    if constexpr (PRE) {
-        sweep(std::false_type{}, std::false_type{}, std::true_type{}, 0, n_pre, true);
-        if (n_pre > 0 && n_pre < nst) load_q(false);
-    }
-    sweep(std::false_type{}, std::false_type{}, std::false_type{}, n_pre, nst, true);
-    float lt[NB], m_row[NB];
-    fold_lanes(std::false_type{}, lt);
-    bool has[NB], out[NB], bad = false;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const int qi = rows_first<FOLD>(a, qw0 + nb * 32 + n, 1);
-        const int thr = a.causal ? min(a.k_past + qi, a.Sk - 1) : a.Sk - 1;  // last key this row sees
-        has[nb] = (nst > 0) && (kc0 <= thr);
-        // ceiling 2^110 rather than 2^120: up to 512 key splits of a row are added up by the column pass
-        out[nb] = has[nb] && !(lt[nb] >= 8.2718061e-25f && lt[nb] < (n_pre > 0 ? kRowSumHiPre : 1.2980742e+33f));
-        bad = bad || out[nb];
-        m_row[nb] = has[nb] ? 0.f : kNegBig;  // an empty split must not set the merged maximum
-        if (!has[nb]) lt[nb] = 0.f;
-    }
-    {
         const bool wbad = __builtin_amdgcn_ballot_w64(bad) != 0;
-        if (lane == 0) bad_s[wave] = wbad ? 1 : 0;
         if constexpr (kRedoHeads<PRE, FOLD>) {
             if (wbad) {  // rows of the heads from the wave's first such row to its last
-                uint64_t set = 0;
+                int lo = 0x7fffffff, hi = -1;
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb)  // both half-waves hold the same rows
-                    set |= (uint64_t)(uint32_t)__builtin_amdgcn_ballot_w64(out[nb]) << (32 * nb);
-                const int first = fold_head(qw0 + __builtin_ctzll(set), a.fold_magic) * a.q_rows;
-                const int past = (fold_head(qw0 + 63 - __builtin_clzll(set), a.fold_magic) + 1) * a.q_rows;
-                if (lane == 0) redo_s[wave] = int2{first, past};
+                for (int nb = 0; nb < NB; ++nb)
+                    if (out[nb]) {
+                        lo = min(lo, nb * 32 + rw);
+                        hi = max(hi, nb * 32 + rw);
+                    }
+#pragma unroll
+                for (int m = 1; m < 64; m *= 2) {
+                    lo = min(lo, __shfl_xor(lo, m));
+                    hi = max(hi, __shfl_xor(hi, m));
+                }
+                const int from = fold_head(c_qw0 + lo, a.fold_magic) * a.q_rows;
+                const int past = (fold_head(c_qw0 + hi, a.fold_magic) + 1) * a.q_rows;
+                if (lane == 0) redo_s[wave] = int2{from, past};
             }
         }
-        block_sync();
-        int any = 0;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) any |= bad_s[w];
-        bad = any != 0;  // block-uniform
-    }
+        // (inline assembly: an ordinary LDS access would wait for the requested stages)
+        {
+            const int f = wbad ? 1 : 0;
+            const uint32_t at = lds_addr(bad_s) + (uint32_t)(wave * 4);
+            asm volatile("ds_write_b32 %0, %1" ::"v"(at), "v"(f) : "memory");
+            block_sync();
+            int any = 0;
+            const uint32_t from = lds_addr(bad_s) + (uint32_t)((lane % WAVES) * 4);
+            asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(any) : "v"(from) : "memory");
+            bad = __builtin_amdgcn_ballot_w64(any != 0) != 0;  // block-uniform
+        }
 
-    // ---- rare: row maxima first, then sums with the maximum subtracted before the scale
-    if (bad) {
-        bool redo = true;  // wave-uniform
-        if constexpr (kRedoHeads<PRE, FOLD>) {
-            redo = false;
-            for (int w = 0; w < WAVES; ++w)
-                if (bad_s[w]) redo = redo || (redo_s[w].x < qw0 + ROWS_W && redo_s[w].y > qw0);
-            redo = __builtin_amdgcn_readfirstlane(redo) != 0;
-        }
-        if (PRE) load_q(false);
-        reset_rows(std::true_type{});
-        sweep(std::true_type{}, std::false_type{}, std::false_type{}, 0, nst, redo);
-        float mx[NB];
-        fold_lanes(std::true_type{}, mx);
+        // ---- rare: row maxima first, then sums with the maximum subtracted before the scale
+        if (bad) {
+            const int n_b = b, n_h = h, n_bx = bx, n_at = at, n_left = left;
+            b = c_b;
+            h = c_h;
+            bx = c_bx;
+            at = c_at;
+            left = c_left;
+            form_anew();
+            set_block();
+            FCS_WAIT_VM(0);  // the next row block's stages: requested again below
+            block_sync();
+            bool redo = true;  // wave-uniform
+            if constexpr (kRedoHeads<PRE, FOLD>) {
+                redo = false;
+                for (int w = 0; w < WAVES; ++w)
+                    if (bad_s[w]) redo = redo || (redo_s[w].x < qw0 + ROWS_W && redo_s[w].y > qw0);
+                redo = __builtin_amdgcn_readfirstlane(redo) != 0;
+            }
+            load_q();
+            shape_q(false);
+            reset_rows(std::true_type{});
+            sweep(std::true_type{}, std::false_type{}, std::false_type{}, 0, nst, redo, false);
+            float mx[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            if (!has[nb]) mx[nb] = 0.f;  // no visible key in this split: every exponential is masked anyway
-            if (g == 0) mrow[wave * ROWS_W + nb * 32 + n] = mx[nb];
-        }
-        __builtin_amdgcn_wave_barrier();
+            for (int nb = 0; nb < NB; ++nb) {
+                mx[nb] = fold_lanes_max(rs[nb], lane_r);
+                if (!has[nb]) mx[nb] = 0.f;  // no visible key in this split: every exponential is masked anyway
+                mrow[wave * ROWS_W + nb * 32 + rw] = mx[nb];
+            }
+            __builtin_amdgcn_wave_barrier();
+            const int g = lane_i >> 5;
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) nmax[nb][i] = -mrow[wave * ROWS_W + nb * 32 + 8 * (i >> 2) + 4 * g + (i & 3)];
-        reset_rows(std::false_type{});
-        sweep(std::false_type{}, std::true_type{}, std::false_type{}, 0, nst, redo);
-        float ls[NB];
-        fold_lanes(std::false_type{}, ls);
+                for (int i = 0; i < 16; ++i) nmax[nb][i] = -mrow[wave * ROWS_W + nb * 32 + 8 * (i >> 2) + 4 * g + (i & 3)];
+            reset_rows(std::false_type{});
+            sweep(std::false_type{}, std::true_type{}, std::false_type{}, 0, nst, redo, false);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            if (!redo) continue;  // m = 0 and the sum of the common path stand
-            m_row[nb] = has[nb] ? mx[nb] : kNegBig;
-            lt[nb] = has[nb] ? ls[nb] : 0.f;
-        }
-    }
-
-    // ---- store: the lower half-wave holds one row per lane
-    if (g == 0) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const int qi = qw0 + nb * 32 + n;  // < rows_pad by construction
-            float2 v;
-            v.x = m_row[nb];
-            if (a.n_chunks == 1) {
-                v.y = fast_log2(lt[nb]);
-                a.lse[(int64_t)bh * a.rows_pad + qi] = v;
-            } else {
-                v.y = lt[nb];
-                a.ml[((int64_t)bh * a.n_chunks + chunk) * a.rows_pad + qi] = v;
+            for (int nb = 0; nb < NB; ++nb) {
+                const float ls = fold_lanes_sum(rs[nb], lane_r);
+                if (!redo) continue;  // m = 0 and the sum of the common path stand
+                m_row[nb] = mx[nb];  // (0 where the split is empty)
+                lt[nb] = has[nb] ? ls : 0.f;
+            }
+            b = n_b;
+            h = n_h;
+            bx = n_bx;
+            at = n_at;
+            left = n_left;
+            if (more) {
+                set_block();
+                load_q();
+                fetch_first(0, PRE && n_pre > 0 ? n_pre : nst);
             }
         }
+
+        // ---- store: one of the two lanes that hold a row
+        if ((lane_r & 1) == 0) {
+            const int64_t i = ((int64_t)c_b * a.v_heads + c_h) * a.n_qblk + c_bx;
+            float2 *dst = a.stat + (a.r_whole ? i : i + share) * BLOCK_ROWS + wave * ROWS_W + rw;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) dst[nb * 32] = float2{m_row[nb], a.r_whole ? fast_log2(lt[nb]) : lt[nb]};
+        }
+        if (!more) break;
     }
 }
 
@@ -1138,14 +1444,16 @@ inline bool stream_prescaled(const Plan &p, const Args &a)
 template <int D, int NB, int WAVES, bool BF, bool FOLD>
 static hipError_t launch_cfg(const Plan &p, const Args &a, hipStream_t st)
 {
-    const dim3 grid((unsigned)((long)p.c_nchunks * p.c_groups * p.B));
+    const dim3 grid((unsigned)p.c_blocks);
     if constexpr (D == 64 && !BF) {
         if (stream_prescaled(p, a)) {
-            hipLaunchKernelGGL((fcs_colstream_kernel<D, NB, WAVES, BF, true, FOLD>), grid, dim3(64 * WAVES), 0, st, a);
+            if (p.c_one) hipLaunchKernelGGL((fcs_colstream_kernel<D, NB, WAVES, BF, true, FOLD, true>), grid, dim3(64 * WAVES), 0, st, a);
+            else hipLaunchKernelGGL((fcs_colstream_kernel<D, NB, WAVES, BF, true, FOLD, false>), grid, dim3(64 * WAVES), 0, st, a);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((fcs_colstream_kernel<D, NB, WAVES, BF, false, FOLD>), grid, dim3(64 * WAVES), 0, st, a);
+    if (p.c_one) hipLaunchKernelGGL((fcs_colstream_kernel<D, NB, WAVES, BF, false, FOLD, true>), grid, dim3(64 * WAVES), 0, st, a);
+    else hipLaunchKernelGGL((fcs_colstream_kernel<D, NB, WAVES, BF, false, FOLD, false>), grid, dim3(64 * WAVES), 0, st, a);
     return hipGetLastError();
 }
 
@@ -1166,14 +1474,16 @@ static hipError_t launch_colstream_d(const Plan &p, const Args &a, hipStream_t s
 template <int D, int NB, int WAVES, bool BF, bool FOLD>
 static hipError_t launch_rows_cfg(const Plan &p, const Args &a, hipStream_t st)
 {
-    const dim3 grid((unsigned)((long)p.n_qblk * p.n_chunks * p.B * p.v_heads));
+    const dim3 grid((unsigned)p.r_blocks);
     if constexpr (D == 64 && !BF) {
         if (stream_prescaled(p, a)) {
-            hipLaunchKernelGGL((fcs_rowstream_kernel<D, NB, WAVES, BF, true, FOLD>), grid, dim3(64 * WAVES), 0, st, a);
+            if (p.r_one) hipLaunchKernelGGL((fcs_rowstream_kernel<D, NB, WAVES, BF, true, FOLD, true>), grid, dim3(64 * WAVES), 0, st, a);
+            else hipLaunchKernelGGL((fcs_rowstream_kernel<D, NB, WAVES, BF, true, FOLD, false>), grid, dim3(64 * WAVES), 0, st, a);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((fcs_rowstream_kernel<D, NB, WAVES, BF, false, FOLD>), grid, dim3(64 * WAVES), 0, st, a);
+    if (p.r_one) hipLaunchKernelGGL((fcs_rowstream_kernel<D, NB, WAVES, BF, false, FOLD, true>), grid, dim3(64 * WAVES), 0, st, a);
+    else hipLaunchKernelGGL((fcs_rowstream_kernel<D, NB, WAVES, BF, false, FOLD, false>), grid, dim3(64 * WAVES), 0, st, a);
     return hipGetLastError();
 }
 

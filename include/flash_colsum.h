@@ -83,11 +83,13 @@ int fcs_colsum_noncausal_f16(const void *q, const void *k, float *out, void *out
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): same arguments minus
  * the workspace, which is a static device array of FCS_STATIC_SCRATCH_BYTES that every GPU
  * the library runs on holds until the process ends.  Has no counterpart in the reference.
- * Calls no hipMalloc / hipFree or any allocating routine.  Returns FCS_E_STATIC_LIMIT when
+ * Calls no hipMalloc / hipFree or any allocating routine.  A call for which
  * fcs_workspace_bytes(0, B, H, S, S, D, cls_n) exceeds FCS_STATIC_SCRATCH_BYTES (8 MiB: enough
- * for B=8 H=16 S=2048 D=64, which needs 2 MiB).  All calls on one GPU share that GPU's array:
+ * for B=8 H=16 S=2048 D=64, which needs 2 MiB) is laid out with less workspace where that makes
+ * it fit, and returns FCS_E_STATIC_LIMIT otherwise.  All calls on one GPU share that GPU's array:
  * calls that overlap in time on one GPU (different streams or threads) race; calls on one
- * stream are ordered and safe.  Results are bit-identical to fcs_colsum_noncausal_f16.
+ * stream are ordered and safe.  Results are bit-identical to fcs_colsum_noncausal_f16, except
+ * that a call laid out with less workspace adds up the same terms in another grouping.
  * The first call on a GPU looks up the array's device address (hipGetSymbolAddress), which may
  * load the code object: make that call, or fcs_static_scratch_init(), outside stream capture.  A
  * failed look-up is not remembered; the next call tries again. */

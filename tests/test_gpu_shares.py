@@ -1,0 +1,86 @@
+"""Two-pass path: workgroups whose equal share of a pass crosses into other row blocks, units, key chunks, heads and batch
+entries, or ends inside one (GPU).  Error bar as everywhere: max 1e-4, element-wise relative 1e-3, of the fp32 means against float64."""
+import ctypes
+
+import pytest
+import torch
+
+from flash_colsum import _hip, flash_colsum_ext
+from oracle import colsum_ext_exact
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, ref):
+    err = (got.double() - ref).abs()
+    assert err.max().item() <= 1e-4 and (err / ref.abs().clamp_min(1e-12)).max().item() <= 1e-3, (err.max().item(), (err / ref).max().item())
+
+
+def _call(b, h, hk, q_len, k_len, d, dtype=torch.float16, causal=True, seed=0, prepare=None, **kw):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q = torch.randn(b, h, q_len, d, generator=g, device="cuda")
+    k = torch.randn(b, hk, k_len, d, generator=g, device="cuda")
+    if prepare:
+        prepare(q, k)
+    q, k = q.to(dtype), k.to(dtype)
+    print((b, h, hk, q_len, k_len, d, dtype, causal, kw), flush=True)
+    return flash_colsum_ext(q, k, is_causal=causal, out_dtype=torch.float32, **kw), colsum_ext_exact(q, k, is_causal=causal, **kw), q, k
+
+
+# several row blocks per share and several shares per row block; a last key stage of one key; head dims of every kernel width
+SHAPES = [(1, 12, 12, 2400, 2400, 128, True), (1, 8, 8, 4097, 4097, 64, True), (3, 5, 5, 1537, 1537, 64, True), (1, 16, 4, 2600, 3000, 80, True),
+          (1, 12, 12, 4500, 4500, 64, False), (2, 7, 7, 2305, 2305, 128, False), (1, 6, 6, 2900, 2900, 256, True), (40, 3, 3, 200, 2113, 64, False),
+          (2, 24, 24, 513, 700, 64, True)]
+
+
+@pytest.mark.parametrize("b,h,hk,q_len,k_len,d,causal", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_shares_that_cross(b, h, hk, q_len, k_len, d, causal, dtype):
+    t = _hip.plan_description((b, h, q_len, d), (b, hk, k_len, d), causal=causal, bf16=dtype == torch.bfloat16)
+    assert "places" in t
+    got, ref, q, k = _call(b, h, hk, q_len, k_len, d, dtype, causal)
+    _check(got, ref)
+    assert torch.equal(got, flash_colsum_ext(q, k, is_causal=causal, out_dtype=torch.float32))  # fixed order of additions
+
+
+@pytest.mark.parametrize("d,h,s", [(64, 16, 3000), (128, 8, 2500)])
+@pytest.mark.parametrize("which", ["one_row", "late_keys", "one_head"])
+def test_rows_out_of_range_in_some_parts(d, h, s, which):
+    """A part of a row block that leaves the unstabilised range is redone while the next one's rows and stages are on their way;
+    the parts of a row are then of both kinds."""
+    def scale_up(q, k):
+        if which == "one_row":
+            q[:, 0, 777] *= 40.0
+        elif which == "late_keys":
+            k[:, :, s - 300:] *= 30.0
+        else:
+            q[:, h // 2] *= 25.0
+    got, ref, _, _ = _call(1, h, h, s, s, d, prepare=scale_up)
+    _check(got, ref)
+
+
+def test_rows_that_see_nothing_and_few_averaged_rows():
+    # k_past well below K_len - Q_len: the last chunks are seen by no row, their means are 0
+    got, ref, _, _ = _call(2, 6, 6, 1100, 9000, 64, k_past=100)
+    _check(got, ref)
+    assert (got[:, 1200:] == 0).all()
+    got, ref, _, _ = _call(1, 16, 16, 3000, 3000, 64, cls_len=1030)
+    _check(got, ref)
+
+
+def test_static_scratch_lays_out_what_the_usual_plan_does_not_fit():
+    """Accepted before the parts of row blocks had workspace of their own: 12 heads of 55565 keys."""
+    b, h, s, d = 1, 12, 55565, 64
+    assert _hip.workspace_bytes(False, b, h, s, s, d) > 8 << 20
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randn(b, h, s, d, generator=g, device="cuda").half()
+    k = torch.randn(b, h, s, d, generator=g, device="cuda").half()
+    out = torch.empty(b, s, device="cuda")
+    strides = (ctypes.c_int64 * 4)(*q.stride())
+    lib = _hip.lib()
+    torch.cuda.synchronize()
+    rc = lib.fcs_colsum_noncausal_f16_static(ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(out.data_ptr()), None, b, h, s, d,
+                                             strides, strides, ctypes.c_float(d ** -0.5), -1, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    usual = flash_colsum_ext(q, k, is_causal=False, out_dtype=torch.float32)
+    assert ((out - usual).abs() <= 2e-6 * usual).all()  # the same terms in another grouping: 12 x 109 fp32 partial sums

@@ -1,0 +1,190 @@
+"""Two-pass path: the equal shares that its workgroups take of a pass's stages (no GPU needed).  fcs_plan.h is plain host
+arithmetic: it is compiled here on its own, and the walk of every workgroup is followed as the kernels do it."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+from flash_colsum import _hip
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+_SOURCE = r"""
+#include <algorithm>
+#include <map>
+#include <set>
+#include <vector>
+#include "fcs_plan.h"
+using namespace fcs;
+
+// keys of a row block's rows [v0, v1) that at least one of them sees
+static int seen(const Plan &p, int v1)
+{
+    if (!p.causal) return p.Sk;
+    const long rows = p.fold > 1 ? p.q_rows : std::min(v1, p.q_rows);
+    return (int)std::min<long>(p.Sk, p.k_past + rows);
+}
+
+// 0: every stage is in exactly one share, and what the shares leave behind fits the workspace; else the check that failed
+extern "C" int check(int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, long *two_pass)
+{
+    Plan p;
+    *two_pass = 0;
+    if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return 1;
+    if (p.fewrows || p.small || p.fused) return 0;
+    *two_pass = 1;
+    const long heads = (long)B * p.v_heads;
+
+    // pass 1
+    const int rows1 = p.k1_waves * p.qw;
+    std::vector<std::set<long>> sets(heads * p.n_qblk);
+    std::vector<int> done1(heads * p.n_qblk);
+    for (long share = 0; share < p.r_blocks; ++share) {
+        int pos = (int)share * p.r_seg, left = std::min(p.r_seg, p.r_len - pos), bx = 0;
+        if (left <= 0) return 2;
+        long bh = p.r_by_head.quot(pos, pos);
+        if (p.r_line.step == 0) bx = p.r_by_block.quot(pos);
+        else for (int sum = 0; pos >= (sum += p.r_line.n(bx) + p.r_line.start); ++bx) {}
+        for (int at = pos - p.r_line.places(bx); left > p.r_line.start || at >= 0; at = 0) {
+            if (bh >= heads || bx >= p.n_qblk) return 3;
+            const int first = std::max(0, at - p.r_line.start), past = std::min(p.r_line.n(bx), at + left - p.r_line.start);
+            const long i = bh * p.n_qblk + bx, set = p.r_whole ? i : share + i;
+            if (past <= first || done1[i] != first) return 4;  // in order, none left out
+            done1[i] = past;
+            sets[i].insert(set);
+            if ((size_t)(set + 1) * rows1 * 8 > p.off_partial) return 5;
+            left -= p.r_line.n(bx) + p.r_line.start - at;
+            if (left <= p.r_line.start) break;
+            if (++bx == p.n_qblk) { bx = 0; ++bh; }
+        }
+    }
+    std::set<long> all;
+    for (long i = 0; i < heads * p.n_qblk; ++i) {
+        if ((long)done1[i] * p.r_unit * 64 < seen(p, (int)(i % p.n_qblk + 1) * rows1)) return 6;
+        // the sets as the column pass looks for them
+        long w0 = 0, parts = 1;
+        if (!p.r_whole) {
+            const int start = (int)(i / p.n_qblk) * p.r_line.places(p.n_qblk) + p.r_line.places((int)(i % p.n_qblk)) + p.r_line.start;
+            w0 = p.r_by_seg.quot(start);
+            parts = p.r_by_seg.quot(start + p.r_line.n((int)(i % p.n_qblk)) - 1) - w0 + 1;
+        }
+        if ((long)sets[i].size() != parts || *sets[i].begin() != w0 + i || *sets[i].rbegin() != w0 + i + parts - 1) return 7;
+        for (long s : sets[i]) if (!all.insert(s).second) return 8;  // a single writer each
+    }
+
+    // column pass
+    const int rows2 = 32 * p.c_nb * p.c_waves, cs = p.c_cs;
+    if (p.c_chunk > col_chunk_max(p.Dp, p.c_waves) || p.c_cs * p.c_unit * kStageKeys != p.c_chunk) return 10;
+    std::vector<std::set<long>> slabs((long)B * p.c_nchunks);
+    std::vector<int> done2((long)B * p.c_nchunks * p.v_heads * p.c_nrb);
+    for (long share = 0; share < p.c_blocks; ++share) {
+        long b;
+        int cx, h = 0, rb = 0, at = 0, left = 0x7fffffff;
+        if (p.c_direct) {
+            b = p.c_by_chunks.quot((int)share, cx);
+        } else {
+            int pos = (int)share * p.c_seg;
+            left = std::min(p.c_seg, p.c_len - pos);
+            if (left <= 0) return 11;
+            b = p.c_by_batch.quot(pos, pos);
+            for (cx = 0; pos >= p.v_heads * p.c_line.chunk_places(p.c_nrb, cs, cx + 1); ++cx) {}
+            pos -= p.v_heads * p.c_line.chunk_places(p.c_nrb, cs, cx);
+            const int per_h = p.c_line.chunk_places(p.c_nrb, cs, cx + 1) - p.c_line.chunk_places(p.c_nrb, cs, cx);
+            for (; pos >= per_h; ++h) pos -= per_h;
+            for (;; ++rb) {
+                const int n = p.c_line.between(rb, cx * cs, cx * cs + cs), len = n > 0 ? n + p.c_line.start : 0;
+                if (pos < len) break;
+                pos -= len;
+            }
+            at = pos;
+        }
+        for (;;) {
+            if (b >= B || cx >= p.c_nchunks) return 12;
+            const long chunk = b * p.c_nchunks + cx;
+            bool any = p.c_direct;
+            for (; left > 0 && h < p.v_heads; at = 0, rb = (rb + 1 == p.c_nrb) ? 0 : rb + 1, h += (rb == 0)) {
+                const int n = p.c_line.between(rb, cx * cs, cx * cs + cs);
+                if (n <= 0) continue;
+                const int first = std::max(0, at - p.c_line.start), past = std::max(0, std::min(n, at + std::min(left, 0x3fffffff) - p.c_line.start));
+                left -= n + p.c_line.start - at;
+                if (past <= first) break;
+                int &d = done2[(chunk * p.v_heads + h) * p.c_nrb + rb];
+                if (d != first) return 13;
+                d = past;
+                any = true;
+            }
+            if (!any) return 19;  // a chunk is entered for at least one stage
+            slabs[chunk].insert(share + chunk);
+            if (!p.c_direct && p.off_partial + (size_t)(share + chunk + 1) * p.c_chunk * 4 > p.total) return 14;
+            if (p.c_direct || left <= p.c_line.start) break;
+            h = rb = at = 0;
+            do {
+                if (++cx == p.c_nchunks) { cx = 0; ++b; }
+            } while (cx * cs >= p.c_line.last);
+        }
+    }
+    all.clear();
+    for (long chunk = 0; chunk < (long)B * p.c_nchunks; ++chunk) {
+        const int cx = (int)(chunk % p.c_nchunks);
+        for (int h = 0; h < p.v_heads; ++h)
+            for (int rb = 0; rb < p.c_nrb; ++rb) {
+                const int end = std::min(seen(p, (rb + 1) * rows2), std::min(Sk, (cx + 1) * p.c_chunk));
+                if ((long)(cx * cs + done2[(chunk * p.v_heads + h) * p.c_nrb + rb]) * p.c_unit * 64 < end) return 15;
+            }
+        if (p.c_direct) continue;
+        // the slabs as the final reduction looks for them
+        const int before = p.c_line.chunk_places(p.c_nrb, cs, cx), len = (p.c_line.chunk_places(p.c_nrb, cs, cx + 1) - before) * p.v_heads;
+        const int start = (int)(chunk / p.c_nchunks) * (int)p.c_by_batch.d + before * p.v_heads;
+        const long w0 = p.c_by_seg.quot(start + p.c_line.start), n = len > 0 ? p.c_by_seg.quot(start + len - 1) - w0 + 1 : 0;
+        if ((long)slabs[chunk].size() != n || n > p.n_partials) return 16;
+        if (n && (*slabs[chunk].begin() != w0 + chunk || *slabs[chunk].rbegin() != w0 + chunk + n - 1)) return 17;
+        for (long s : slabs[chunk]) if (!all.insert(s).second) return 18;
+    }
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shares")
+    src, lib = d / "shares.cpp", d / "libshares.so"
+    src.write_text(_SOURCE)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "flash-colsum_amd", "csrc"), "-o", str(lib), str(src)], check=True)
+    fn = ctypes.CDLL(str(lib)).check
+
+    def call(causal, b, h, hk, sq, sk, d, cls_n, k_past):
+        two_pass = ctypes.c_long()
+        return fn(int(causal), b, h, hk, sq, sk, d, cls_n, k_past, ctypes.byref(two_pass)), two_pass.value
+
+    return call
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_every_stage_is_in_one_share(check, seed):
+    rng = random.Random(seed)
+    fixed = [(False, 1, 16, 16, 8192, 8192, 64, -1, 0), (False, 1, 16, 16, 9289, 9289, 64, -1, 0), (True, 1, 32, 32, 4096, 4096, 128, -1, 0),
+             (True, 1, 32, 32, 512, 65536, 128, -1, 65024), (True, 4, 32, 8, 64, 8192, 128, -1, 8128), (True, 1, 8, 8, 512, 4096, 256, -1, 3584),
+             (True, 257, 1, 1, 128, 250, 64, -1, 122), (True, 3, 5, 1, 1, 1, 64, -1, 0), (True, 1, 2, 2, 20000, 300, 128, -1, 0),
+             (False, 300, 3, 3, 5, 3000, 64, -1, 0), (True, 2, 3, 3, 700, 5000, 200, 100, 10)]
+    shapes, n_two_pass = fixed if seed == 0 else [], 0
+    for _ in range(400):
+        causal = rng.random() < 0.75
+        hk = rng.choice([1, 2, 3, 8, 12])
+        sq = rng.choice([1, 2, 63, 64, 65, 128, 129, 256, 257, 511, 512, 513, 700, 1025, rng.randint(1, 9000)])
+        sk = rng.choice([1, 40, 64, 65, 300, 2047, 2049, rng.randint(1, 12000), rng.randint(1, 40000)])
+        shapes.append((causal, rng.choice([1, 1, 2, 3, 8, 40, 300]), hk * rng.choice([1, 1, 2, 4, 8]), hk, sq, sk, rng.choice([64, 80, 128, 200]),
+                       rng.choice([-1, -1, -1, 20, 300]), rng.choice([max(0, sk - sq), max(0, sk - sq), 0, sk // 2, sk])))
+    for s in shapes:
+        rc, two_pass = check(*s)
+        assert rc == 0, (rc, s)
+        n_two_pass += two_pass
+    assert n_two_pass > 100
+
+
+def test_shares_of_uneven_row_blocks_are_equal():
+    """The triangle of a prompt against itself: 32 heads x (8 + 16 + .. + 64) stages over 256 workgroups."""
+    t = _hip.plan_description((1, 32, 4096, 128), (1, 32, 4096, 128), causal=True)
+    assert "256 shares of 38 places + " in t and "grid 256, shares of 39 places" in t, t
