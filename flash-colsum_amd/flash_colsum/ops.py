@@ -48,10 +48,14 @@ def flash_colsum_f32(
     cls_len: Optional[int] = None,
 ) -> torch.Tensor:
     """Same as `flash_colsum` but returns the kernels' fp32 means (no fp16 rounding)."""
+    call = _hip.call_key(1, query, key, scale, is_causal, cls_len)
+    out = _hip.repeated_call(call, query, key)
+    if out is not None:
+        return out
     scale, cls_n = _validated(query, key, scale, is_causal, cls_len)
     if is_causal:
-        return _hip.colsum_causal_f32(query, key, scale)
-    return _hip.colsum_noncausal_f32(query, key, scale, cls_n)
+        return _hip.colsum_causal_f32(query, key, scale, key=call)
+    return _hip.colsum_noncausal_f32(query, key, scale, cls_n, key=call)
 
 
 def flash_colsum(
@@ -70,12 +74,16 @@ def flash_colsum(
     cls_len: non-causal only; average over the first min(cls_len, S) query rows.
     Returns fp16 (B, S), or (1, K_len) for causal.  Raises ValueError for invalid input.
     """
+    call = _hip.call_key(0, query, key, scale, is_causal, cls_len)
+    out = _hip.repeated_call(call, query, key)
+    if out is not None:
+        return out
     scale, cls_n = _validated(query, key, scale, is_causal, cls_len)
     if is_causal:
-        return _hip._flash_colsum_causal(query, key, scale)
+        return _hip._flash_colsum_causal(query, key, scale, key=call)
     if query.shape[0] == 1:
-        return _hip._flash_colsum_non_batched(query, key, scale, CLS_N=cls_n)
-    return _hip._flash_colsum_batched(query, key, scale, CLS_N=cls_n)
+        return _hip._flash_colsum_non_batched(query, key, scale, CLS_N=cls_n, key=call)
+    return _hip._flash_colsum_batched(query, key, scale, CLS_N=cls_n, key=call)
 
 
 def flash_colsum_ext(
@@ -99,6 +107,10 @@ def flash_colsum_ext(
     * non-causal with S_q != S_k (cross-attention shape).
     Returns (B, S_k) in `out_dtype` (torch.float16 like the reference, or torch.float32).
     """
+    call = _hip.call_key(2, query, key, scale, is_causal, cls_len, k_past) if out_dtype is torch.float32 else None
+    out = _hip.repeated_call(call, query, key) if call is not None else None
+    if out is not None:
+        return out
     if query.ndim != 4 or key.ndim != 4:
         raise ValueError(f"Expected 4D tensors, got query.ndim={query.ndim}, key.ndim={key.ndim}")
     if query.device.type != "cuda":
@@ -119,7 +131,7 @@ def flash_colsum_ext(
         scale = dq ** -0.5
     cls_n = -1 if cls_len is None else int(cls_len)
     if out_dtype == torch.float32:
-        return _hip.colsum_general(query, key, float(scale), is_causal, cls_n, k_past)
+        return _hip.colsum_general(query, key, float(scale), is_causal, cls_n, k_past, key=call)
     return _hip.colsum_general(query, key, float(scale), is_causal, cls_n, k_past, want_f16=True)[1]
 
 

@@ -1,0 +1,103 @@
+"""Calls whose geometry the thread has had before go straight to the library: they see the tensors they are given, and whatever
+the geometry does not decide is looked at again."""
+import numpy as np
+import pytest
+import torch
+
+from flash_colsum import _hip, flash_colsum, flash_colsum_ext, flash_colsum_f32
+from oracle import colsum_exact
+
+
+def test_only_plain_arguments_are_recognised():
+    q = torch.zeros(1, 2, 8, 64, dtype=torch.float16)
+    assert _hip.call_key(0, q, q, None, False, None) is not None and _hip.call_key(0, q, q, 0.5, True, 3) is not None
+    for args in [(0, torch.nn.Parameter(q), q, None, False, None), (0, q, q, torch.tensor(0.5), False, None), (0, q, q, np.float32(0.5), False, None),
+                 (0, q, q, None, 1, None), (0, q, q, None, False, torch.tensor(3)), (0, None, q, None, False, None), (0, q, q, None, False, 1.5)]:
+        assert _hip.call_key(*args) is None
+    # kinds, dtypes and storage orders are told apart
+    t = torch.zeros(1, 8, 2, 64, dtype=torch.float16).transpose(1, 2)
+    keys = [_hip.call_key(kind, a, b, None, False, None) for kind in (0, 1, 2) for a, b in ((q, q), (t, q), (q.bfloat16(), q), (q, t))]
+    assert len(set(keys)) == len(keys)
+    assert _hip.repeated_call(keys[0], q, q) is None  # nothing known, and not on a GPU
+    with pytest.raises(ValueError, match="only supports CUDA tensors"):
+        flash_colsum(q, q)
+
+
+def _pair(seed, shape=(2, 4, 100, 64), dtype=torch.float16):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return tuple(torch.randn(shape, generator=g, device="cuda").to(dtype) for _ in range(2))
+
+
+def _good(out, q, k, **kw):
+    ref = colsum_exact(q, k, **kw)
+    rel = 1e-3 if out.dtype == torch.float32 else 2e-3  # one rounding to fp16 on top
+    assert out.shape == ref.shape and ((out.double() - ref).abs() <= rel * ref.abs() + 1e-7).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_repeated_calls_see_their_own_tensors(dtype):
+    for seed in range(4):
+        q, k = _pair(seed, dtype=dtype)
+        _good(flash_colsum(q, k), q, k)
+        _good(flash_colsum_f32(q, k, 0.3), q, k, scale=0.3)
+        _good(flash_colsum(q, k, cls_len=2), q, k, cls_len=2)
+        _good(flash_colsum_ext(q, k, out_dtype=torch.float32), q, k)
+        assert flash_colsum_ext(q, k).dtype == torch.float16
+        a, b = flash_colsum(q, k), flash_colsum(k, q)  # results of their own
+        assert a.data_ptr() != b.data_ptr()
+        _good(a, q, k)
+
+
+@pytest.mark.gpu
+def test_what_the_geometry_does_not_decide():
+    shape = (2, 4, 100, 64)
+    q, k = _pair(0, shape)
+    for _ in range(2):
+        flash_colsum(q, k)
+    # a base that is not 16-byte aligned
+    odd = torch.empty(q.numel() + 8, dtype=torch.float16, device="cuda")[1:1 + q.numel()].view(shape)
+    odd.copy_(q)
+    assert odd.stride() == q.stride() and odd.data_ptr() % 16 != 0
+    _good(flash_colsum(odd, k), q, k)
+    # the other operand elsewhere
+    with pytest.raises(ValueError):
+        flash_colsum(q, k.cpu())
+    with pytest.raises(ValueError):
+        flash_colsum(q.cpu(), k)
+    # another stream
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        out = flash_colsum(q, k)
+    s.synchronize()
+    _good(out, q, k)
+    # fp32: out of fp16's range after a call that was not, not finite, and in range again
+    q32, k32 = _pair(1, shape, torch.float32)
+    for _ in range(2):
+        _good(flash_colsum(q32, k32), q32, k32)
+    big = q32.clone()
+    big[0, 1, 7] *= 1e6
+    _good(flash_colsum_f32(big, k32, 1e-5), big, k32, scale=1e-5)
+    _good(flash_colsum_f32(q32, k32, 1e-5), q32, k32, scale=1e-5)
+    _good(flash_colsum_f32(big, k32, 1e-5), big, k32, scale=1e-5)
+    big[0, 0, 0, 0] = float("nan")
+    with pytest.raises(ValueError, match="NaN"):
+        flash_colsum_f32(big, k32, 1e-5)
+    neg = torch._neg_view(q32)
+    _good(flash_colsum(neg, k32), -q32, k32)
+
+
+@pytest.mark.gpu
+def test_repeated_call_in_a_graph():
+    q, k = _pair(2)
+    for _ in range(3):
+        eager = flash_colsum(q, k)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = flash_colsum(q, k)
+    for i in range(4):
+        q.copy_(q.flip(2))
+        g.replay()
+        assert torch.equal(out, flash_colsum(q, k))
+    assert eager.shape == out.shape
