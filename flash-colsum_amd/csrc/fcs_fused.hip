@@ -1,11 +1,11 @@
 // Attention column means on gfx950 (MI355X): fused single-kernel path for non-causal
-// calls whose whole key range fits in one workgroup's registers (32 <= S_k <= 2048, head dims up to 128:
+// calls whose whole key range fits in one workgroup's registers (32 <= S_k <= 2560, head dims up to 128:
 // 64 channels natively, 128 as two 64-channel chunks, anything narrower on one of those two with zeros in Q).
 //
 // One workgroup = 8 waves.  The waves form a (query group) x (key group) grid; a wave
 // computes the 32 x (32 * tiles) block of scores  S = Q_tile * K_tile^T  for its 32 query
 // rows and its keys with v_mfma_f32_32x32x16_f16 and KEEPS it in registers (up to 8
-// accumulator tiles = 128 VGPRs), so the scores are computed once and exponentiated
+// accumulator tiles = 128 VGPRs, 10 in the shared-Q variants), so the scores are computed once and exponentiated
 // once.  In this orientation a lane owns one key (column l % 32) and 16 query rows, so the
 // column sums  sum_i e_ij / L_i  are in-lane FMAs; only the row sums L_i cross lanes and
 // waves, once per (head, row block): lanes are folded in registers (DPP and lane-swap
@@ -138,7 +138,7 @@ __device__ __forceinline__ floatx4 row_values(const RowRed &rr, int i4, int g)
 // RAGGED = false: S_k is exactly (key groups) x TPW x 32, S_q a multiple of the block's rows and
 //                 the rows of Q and K are dense (row stride == D): every operand tile is whole,
 //                 no padding keys anywhere, and tile addresses need no per-lane arithmetic.
-// RAGGED = true : anything else (any 32 <= S_k <= 2048, any S_q, any 16-byte aligned row pitch).  Key
+// RAGGED = true : anything else (any 32 <= S_k <= 2560, any S_q, any 16-byte aligned row pitch).  Key
 //                 tiles still need no per-lane arithmetic and no branch: a tile that would reach
 //                 past the last key is moved back to end there, and the columns that then repeat
 //                 the tile before it are given no weight.  Q rows are clamped per lane, once per unit.
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
     // first chunk's four steps, then the second chunk's, into the same accumulators.
     constexpr int DC = D / 64;
     constexpr int NT = 4;                  // MFMA steps (and 16-byte pieces per lane) per (half) tile
-    // KEEP (shared-Q variants with five to eight key tiles per wave): the Q item of those variants is
+    // KEEP (shared-Q variants with five to ten key tiles per wave): the Q item of those variants is
     // a plain load that needs no ring slot, so the ring holds key tiles only, tile k of every unit in
     // slot k % NS.  The row blocks of a head, which a workgroup walks one after the other, use the
     // same key tiles: a unit leaves its last NS key tiles in the ring and the next unit of the same
@@ -178,7 +178,8 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
     //     always uses slot t % NS, a compile-time value;
     //   * otherwise (NS = 4, or 3 with two key groups): 0 .. TPW-1 and TPW-1 .. 0; the slot of a step depends on
     //     the order and is added to the read-back addresses at run time.
-    // Each order has its own column sums; they are added at the end.
+    // Phase 3 is written once per order, so that both add into the same column sums under compile-time indices (a
+    // set of sums per order cost the eight to ten registers that nine and ten tiles per wave need: they spilled).
     // (With two key groups there are four query groups: their Q tiles take 32 KB and leave room for
     // three slots per wave, so eight tiles walk ascending / descending too.)
     constexpr bool KEEP_ROT = PRE && (TPW == 6 || (TPW == 8 && PRE != 2));
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
     // ring holds four, which leaves the fourth in flight)
     constexpr int NS = KEEP_ROT ? TPW / 2 : KEEP_REV ? (PRE == 2 ? 3 : 4) : (DC == 2 ? 4 : 3);  // ring slots per wave
     constexpr int QV = (PRE == 2) ? 2 : 1;  // load instructions of a wave's share of the raw Q rows
-    static_assert(!PRE || (TPW >= 5 && TPW <= 8), "the shared-Q variants are written for five to eight key tiles per wave");
+    static_assert(!PRE || (TPW >= 5 && TPW <= 10), "the shared-Q variants are written for five to ten key tiles per wave");
     constexpr int ITEMS = DC * (TPW + 1);  // per (head, row block): the Q tile, then TPW key tiles (chunk by chunk)
     constexpr int SLOT_BYTES = NT * 1024;  // one item: NT pieces x 64 lanes x 16 bytes
     constexpr bool STATIC_SLOTS = KEEP_ROT || (!KEEP_REV && ITEMS % NS == 0);  // then an item's slot is a compile-time value
@@ -354,11 +355,8 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
     };
 
     float col_acc[TPW];
-    float col_rot[KEEP ? TPW : 1];  // KEEP: sums of the units that ran in the second order: col_rot[t] belongs to tile tile_of(t)
 #pragma unroll
     for (int t = 0; t < TPW; ++t) col_acc[t] = 0.f;
-#pragma unroll
-    for (int t = 0; t < (KEEP ? TPW : 1); ++t) col_rot[t] = 0.f;
     int rot = 0;  // KEEP: 1 while the current unit runs in the second order
     // KEEP: the key tile of step t (compile-time) of the current unit, and its ring slot
     auto tile_of = [&](int t) { return !rot ? t : KEEP_ROT ? (t + NS) % TPW : TPW - 1 - t; };
@@ -704,9 +702,13 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
 #pragma unroll
-                    for (int t = 0; t < (KEEP ? TPW : 1); ++t) col_rot[t] = fmaf(acc[t][4 * i4 + j], w4[j], col_rot[t]);
+                    for (int t = 0; t < TPW; ++t) {
+                        float &sum = col_acc[KEEP_ROT ? (t + NS) % TPW : TPW - 1 - t];
+                        sum = fmaf(acc[t][4 * i4 + j], w4[j], sum);
+                    }
                 }
             }
+            asm volatile("" ::: "memory");
         } else if (!slow) {
             // ---------------- phase 3: column sums of e * w
 #pragma unroll
@@ -812,16 +814,14 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
     float *dst = a.partial + ((int64_t)slab * a.B + b) * a.Sk;
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
-        // KEEP: tile t was held by step (t + NS) % TPW (rotated order) or TPW - 1 - t (reversed order) of the units in the second order
-        const float both = KEEP ? col_acc[t] + col_rot[KEEP_ROT ? (t + NS) % TPW : KEEP_REV ? TPW - 1 - t : 0] : col_acc[t];
-        const float v = both + __shfl_xor(both, 32);
+        const float v = col_acc[t] + __shfl_xor(col_acc[t], 32);
         if (g == 0 && t <= tmax_lane) dst[tile_first(t) + n] = v;
     }
 }
 
 // Which instantiation serves a call with TPW key tiles per wave (shared by the launcher and the plan description).
 struct FusedVariant {
-    int tpw;      // template TPW (the shared-Q variants exist for five to eight tiles)
+    int tpw;      // template TPW (the shared-Q variants exist for five to ten tiles, and nine and ten only as those)
     bool ragged;
     int pre;      // 8, 4, 2: shared Q tile with that many key groups; 0: private rings
     bool qs;      // shared Q tile pre-scaled
@@ -833,17 +833,38 @@ static FusedVariant pick_fused(const Plan &p, const Args &a, bool bf)
     // the head dim read as zeros)
     if (p.D != 64) return {TPW, true, 0, true};
     const bool whole = p.Sk == p.f_kg * TPW * 32 && p.Sq % (32 * p.f_qg) == 0 && a.qs_s == 64 && a.ks_s == 64;
-    // shared-Q variants: five to eight tiles per wave and 8, 4 or 2 key groups (S 257 .. 2048)
+    // shared-Q variants: five to ten tiles per wave and 8, 4 or 2 key groups (S 257 .. 2560)
     const bool shared_q = TPW >= 5 && (p.f_kg == 8 || p.f_kg == 4 || p.f_kg == 2);
     // ... pre-scaled when the rounding of Q*c to fp16 cannot show in the means
-    const bool pre = shared_q && !bf && (long)p.H * p.q_rows >= 4096 && fabsf(a.c) <= 0.1251f * 1.44269504f;
+    // (beyond 2048 keys from the number of pairs on from which the two-pass path takes its pre-scaled operand)
+    const bool pre = shared_q && !bf && (long)p.H * p.q_rows >= (p.Sk > 2048 ? 16384 : 4096) && fabsf(a.c) <= 0.1251f * 1.44269504f;
     if (pre && whole && TPW == 8 && (p.f_kg == 8 || p.f_kg == 4)) return {8, false, p.f_kg, true};
     if (pre) return {TPW, true, p.f_kg, true};
     // ... else Q shared through LDS as it is (8 or 4 key groups).  (Two key groups that cannot be
     // pre-scaled stay on the private rings: sharing the Q tile as it is was measured 4 % slower there,
-    // B 64 H 16 S 512 bf16 67.2 -> 69.9 us.)
-    if (shared_q && p.f_kg != 2) return {TPW, true, p.f_kg, false};
+    // B 64 H 16 S 512 bf16 67.2 -> 69.9 us.  Nine and ten tiles fit the registers only with a shared Q.)
+    if (shared_q && (p.f_kg != 2 || TPW > 8)) return {TPW, true, p.f_kg, false};
     return {TPW, !whole, 0, true};
+}
+
+// nine or ten key tiles per wave: shared-Q variants only
+template <int TPW, bool BF>
+static void launch_wide(const Plan &p, const Args &a, hipStream_t st)
+{
+    const dim3 grid(p.f_nwgq * p.B, p.f_hg);
+    const FusedVariant v = pick_fused(p, a, BF);
+    if (v.pre == 8 && v.qs)
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 8, false>), grid, dim3(512), 0, st, a);
+    else if (v.pre == 4 && v.qs)
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 4, false>), grid, dim3(512), 0, st, a);
+    else if (v.pre == 2 && v.qs)
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 2, false>), grid, dim3(512), 0, st, a);
+    else if (v.pre == 8)
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 8, BF, false>), grid, dim3(512), 0, st, a);
+    else if (v.pre == 4)
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 4, BF, false>), grid, dim3(512), 0, st, a);
+    else
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 2, BF, false>), grid, dim3(512), 0, st, a);
 }
 
 template <int TPW, bool BF>
@@ -902,6 +923,8 @@ static bool launch_fused_t(const Plan &p, const Args &a, hipStream_t st)
     case 6: launch_tpw<6, BF>(p, a, st); break;
     case 7: launch_tpw<7, BF>(p, a, st); break;
     case 8: launch_tpw<8, BF>(p, a, st); break;
+    case 9: launch_wide<9, BF>(p, a, st); break;
+    case 10: launch_wide<10, BF>(p, a, st); break;
     default: return false;
     }
     return true;

@@ -11,6 +11,7 @@ constexpr int kWavesPerBlock = 4;   // 256 threads
 constexpr int kStageKeys = 64;      // keys staged in LDS per step of either pass
 constexpr int kComputeUnits = 256;  // MI355X
 constexpr int kFusedMaxKeys = 2048; // 8 waves x 8 tiles x 32 keys of fp32 scores per 32 query rows
+constexpr int kFusedMaxKeys64 = 2560; // 64-wide heads: ten tiles per wave
 constexpr int kFewRowsMaxRows = 4;      // few-rows path: at most this many averaged query rows per head ...
 constexpr int kFewRowsMaxScores = 12288; // ... and rows * Sk scores (48 KB of LDS)
 constexpr int kSmallMaxTiles = 9;        // short-sequence path: one wave holds the scores of 32 rows x (32 x 9) keys
@@ -440,50 +441,78 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // (Heads of 72 .. 120 channels: the 128-wide kernel's variant for narrower heads runs out of registers at seven
     // and eight key tiles per wave, so it takes at most six, i.e. 1536 keys; longer calls take the two-pass path.)
     const bool narrow128 = D > 64 && D < 128;
-    if (!causal && Sk >= 32 && Sk <= (narrow128 ? 8 * 6 * 32 : kFusedMaxKeys) && D <= 128) {
+    // (64-wide heads: the shared-Q variants hold ten tiles per wave, so calls of up to 2560 keys are served too, unless grouped
+    // heads are laid end to end, whose keys are streamed once for the whole group.  us per call, two passes -> here:
+    // B 1 H 16 S 2500 47.9 -> 32.4, B 4 H 16 S 2300 212.8 -> 83.9, H 1 S 2500 14.6 -> 10.6, 5 averaged rows of B 8 H 16
+    // S 2300 30.2 -> 12.8, 128 of them 29.9 -> 17.2; no size in between was slower.)
+    const bool wide = D == 64 && tight_stages == 0;
+    const int fused_max = narrow128 ? 8 * 6 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
+    if (!causal && Sk >= 32 && Sk <= fused_max && D <= 128) {
         p.fused = 1;
         p.fold = 1;
         const int tiles = ceil_div(Sk, 32);
-        p.f_kg = 1;
-        while (p.f_kg * 8 < tiles) p.f_kg *= 2;  // <= 8 tiles per wave
-        if (narrow128) while (p.f_kg * 6 < tiles) p.f_kg *= 2;  // <= 6 there
-        p.f_qg = 8 / p.f_kg;
-        p.f_tpw = ceil_div(tiles, p.f_kg);
-        p.f_nqblk = ceil_div(p.q_rows, 32 * p.f_qg);
-        // Units per workgroup: a unit is one (query block, head); a workgroup takes f_rbpw adjacent
-        // query blocks times f_hpg heads.  One workgroup is resident per compute unit, so the launch
-        // runs in generations of kComputeUnits workgroups, each as long as its units plus about 0.7 of
-        // a unit for starting and finishing.  Fewer units per workgroup fill the last generation
-        // better (528 workgroups of 16 units take three generations, 2112 of 4 take nine quarter-
-        // length ones) at the price of more starts and more partial slabs; more units per workgroup
-        // save starts (512 workgroups of 16 units take two generations, 256 of 32 one).
-        p.f_hpg = H;
-        p.f_rbpw = 1;
-        double best = 0.;
-        bool first = true;
-        for (int rbpw = 1; rbpw <= 16 && (rbpw == 1 || rbpw <= p.f_nqblk); ++rbpw) {
-            const int nwgq = ceil_div(p.f_nqblk, rbpw);
-            if (ceil_div(p.f_nqblk, nwgq) != rbpw) continue;  // same grouping as a smaller rbpw
-            // heads per workgroup, descending, one value per distinct grouping: hpg = ceil(H / hg) for
-            // hg = 1, then the next hg that lowers it (about 2 sqrt(H) values)
-            for (int hg = 1, hpg = H; hpg >= 1; hg = (hpg > 1) ? ceil_div(H, hpg - 1) : H + 1, hpg = (hg <= H) ? ceil_div(H, hg) : 0) {
-                const long gens = ((long)nwgq * B * hg + kComputeUnits - 1) / kComputeUnits;
-                // a unit that follows another row block of the same head finds half of its key tiles in
-                // the LDS ring (the shared-Q kernels; measured 4 % of a unit): row blocks per head count
-                // a little less than heads
-                double cost = (double)gens * ((double)hpg * (rbpw - 0.04 * (rbpw - 1)) + 0.7) + 0.01 * hg + 0.002 * rbpw;
-                // The 32 workgroups that an XCD runs at a time are neighbours in launch order: nwgq of
-                // them share a batch entry, i.e. one head's keys.  When the key heads they stream at
-                // the same time outgrow the XCD's 4 MiB L2, the re-reads of a head's keys by its row
-                // blocks miss (measured +6 % at B 256, S 1024 with 32 batch entries per XCD).
-                const long streams = (nwgq >= 32) ? 1 : (32 + nwgq - 1) / nwgq;
-                if (streams * (long)Sk * (2 * p.Dp) > (5L << 19)) cost *= 1.08;
-                if (first || cost < best) {
-                    first = false;
-                    best = cost;
-                    p.f_hpg = hpg;
-                    p.f_rbpw = rbpw;
+        int usual = 1;  // key groups: the fewest that hold the keys with eight tiles per wave
+        while (usual * 8 < tiles && usual < 8) usual *= 2;
+        if (narrow128) while (usual * 6 < tiles) usual *= 2;  // six there
+        // Other splits over the key groups are priced too; tight_stages keeps the usual one, whose slabs are what such a
+        // caller has always had room for.
+        //  * Half as many groups of nine or ten tiles (64-wide heads): half the barriers, row sums and exchanges, but the last
+        //    generation is coarser, and a unit of ten tiles takes 1.9 times one of five, not 1.6 as eight do.  us per call,
+        //    usual -> half: B 8 H 16 S 1100 50.2 -> 44.0, B 32 H 16 S 577 57.2 -> 52.8, S 1040 173.6 -> 156.4, but B 32 H 12
+        //    S 640 44.4 -> 48.4 and B 1 H 12 S 1100 12.7 -> 14.0: both sides of the price below.
+        //  * More groups of fewer tiles where the workgroups get two units at most, i.e. where most of the chip is idle or a
+        //    unit's chain of tiles is all there is: B 2 H 4 S 512 9.3 -> 7.3, B 1 H 16 S 1024 bf16 14.1 -> 12.3, D 128
+        //    18.2 -> 15.1, B 8 H 8 S 197 D 128 11.3 -> 8.7.  With three units or more it was up to 9 % slower.
+        double best_kg = 0.;
+        bool any = false;
+        for (int kg = (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {
+            const int tpw = ceil_div(tiles, kg), nqblk = ceil_div(p.q_rows, 32 * (8 / kg));
+            if (kg > usual && (tight_stages > 0 || (long)B * H * nqblk > 2 * kComputeUnits)) break;
+            // Units per workgroup: a unit is one (query block, head); a workgroup takes f_rbpw adjacent
+            // query blocks times f_hpg heads.  One workgroup is resident per compute unit, so the launch
+            // runs in generations of kComputeUnits workgroups, each as long as its units plus about 0.7 of
+            // a unit for starting and finishing.  Fewer units per workgroup fill the last generation
+            // better (528 workgroups of 16 units take three generations, 2112 of 4 take nine quarter-
+            // length ones) at the price of more starts and more partial slabs; more units per workgroup
+            // save starts (512 workgroups of 16 units take two generations, 256 of 32 one).
+            int best_hpg = H, best_rbpw = 1;
+            double best = 0.;
+            bool first = true;
+            for (int rbpw = 1; rbpw <= 16 && (rbpw == 1 || rbpw <= nqblk); ++rbpw) {
+                const int nwgq = ceil_div(nqblk, rbpw);
+                if (ceil_div(nqblk, nwgq) != rbpw) continue;  // same grouping as a smaller rbpw
+                // heads per workgroup, descending, one value per distinct grouping: hpg = ceil(H / hg) for
+                // hg = 1, then the next hg that lowers it (about 2 sqrt(H) values)
+                for (int hg = 1, hpg = H; hpg >= 1; hg = (hpg > 1) ? ceil_div(H, hpg - 1) : H + 1, hpg = (hg <= H) ? ceil_div(H, hg) : 0) {
+                    const long gens = ((long)nwgq * B * hg + kComputeUnits - 1) / kComputeUnits;
+                    // a unit that follows another row block of the same head finds half of its key tiles in
+                    // the LDS ring (the shared-Q kernels; measured 4 % of a unit): row blocks per head count
+                    // a little less than heads
+                    double cost = (double)gens * ((double)hpg * (rbpw - 0.04 * (rbpw - 1)) + 0.7) + 0.01 * hg + 0.002 * rbpw;
+                    // The 32 workgroups that an XCD runs at a time are neighbours in launch order: nwgq of
+                    // them share a batch entry, i.e. one head's keys.  When the key heads they stream at
+                    // the same time outgrow the XCD's 4 MiB L2, the re-reads of a head's keys by its row
+                    // blocks miss (measured +6 % at B 256, S 1024 with 32 batch entries per XCD).
+                    const long streams = (nwgq >= 32) ? 1 : (32 + nwgq - 1) / nwgq;
+                    if (streams * (long)Sk * (2 * p.Dp) > (5L << 19)) cost *= 1.08;
+                    if (first || cost < best) {
+                        first = false;
+                        best = cost;
+                        best_hpg = hpg;
+                        best_rbpw = rbpw;
+                    }
                 }
+            }
+            best *= tpw > 8 ? 1.03 * (tpw + 3) : tpw + 2;  // a unit's time: its tiles, and its reduction
+            if (!any || best < best_kg) {
+                any = true;
+                best_kg = best;
+                p.f_kg = kg;
+                p.f_qg = 8 / kg;
+                p.f_tpw = tpw;
+                p.f_nqblk = nqblk;
+                p.f_hpg = best_hpg;
+                p.f_rbpw = best_rbpw;
             }
         }
         p.f_hg = ceil_div(H, p.f_hpg);

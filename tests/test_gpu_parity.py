@@ -278,7 +278,7 @@ def test_prescaled_shared_q_variant(shape, same, kw, boost):
 @pytest.mark.parametrize("qs,ks,kw,same,boost", [
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {}, False, 0.0),                        # non-causal, keys split in pass 1
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {"scale": -0.125}, False, 0.0),         # the sign rides on the operand
-    ((2, 8, 2100, 64), (2, 8, 2100, 64), {}, False, 0.0),                        # ragged, just past the fused kernel's range
+    ((2, 8, 2100, 64), (2, 8, 2100, 64), {}, False, 0.0),                        # ragged, just past 2048 keys
     ((1, 16, 700, 64), (1, 16, 5000, 64), {"is_causal": True}, False, 0.0),      # causal, 11200 pairs: the exact variant
     ((1, 16, 1100, 64), (1, 16, 5000, 64), {"is_causal": True}, False, 0.0),     # causal, 17600 pairs: pre-scaled below key 3840
     ((1, 16, 1100, 64), (1, 16, 5000, 64), {"is_causal": True}, False, 6.0),     # ... with rows that leave the 2^20 range

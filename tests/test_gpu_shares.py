@@ -29,7 +29,7 @@ def _call(b, h, hk, q_len, k_len, d, dtype=torch.float16, causal=True, seed=0, p
 
 # several row blocks per share and several shares per row block; a last key stage of one key; head dims of every kernel width
 SHAPES = [(1, 12, 12, 2400, 2400, 128, True), (1, 8, 8, 4097, 4097, 64, True), (3, 5, 5, 1537, 1537, 64, True), (1, 16, 4, 2600, 3000, 80, True),
-          (1, 12, 12, 4500, 4500, 64, False), (2, 7, 7, 2305, 2305, 128, False), (1, 6, 6, 2900, 2900, 256, True), (40, 3, 3, 200, 2113, 64, False),
+          (1, 12, 12, 4500, 4500, 64, False), (2, 7, 7, 2305, 2305, 128, False), (1, 6, 6, 2900, 2900, 256, True), (40, 3, 3, 200, 2113, 48, False),
           (2, 24, 24, 513, 700, 64, True)]
 
 
