@@ -20,12 +20,15 @@
 //   3. every wave counts the entries of its part above and at the k-th key; the counts of the waves before it
 //      are its offsets.  Taken entries get their place in index order from ballots; ties at the k-th value
 //      go to the LOWER index.
-//   4. optionally (k <= kTopkSortMax) a bitonic sort by descending value, ties by ascending index, of 64-bit
-//      (key, ~index) words: exchanges over less than a wave's elements are DPP and lane swaps in registers,
-//      only the wider ones go through LDS.
-// Measured, sorted: B 4, S 8192, k 1024 14.8 us; B 1, S 32768, k 2048 31.9 us; B 1, S 262144, k 4096 180 us.  The
-// former version (four byte-wide histograms, a tile of 1024 at a time with four barriers each in the compaction,
-// every step of the sort through LDS): 46, 99.6 and 549 us.
+//   4. optionally (k <= kTopkSortMax) the order by descending value, ties by ascending index, of 64-bit
+//      (key, ~index) words: counted in 2048 bins that span them, each word's place then is the number of words in higher
+//      bins plus those of its own bin that are larger (four barriers, about one comparison per word).  Up to a
+//      wave of words, and where more than 64 share a bin (ties, a few outliers in several parts of the row), a bitonic
+//      sort: exchanges over less than a wave's elements are DPP and lane swaps in registers, only the wider ones go through
+//      LDS.  Its 55 steps on 1024 words were 4 us of the 15, all VALU work of a single compute unit.
+// Measured, sorted, B 4, bitonic sort -> counting: S 8192, k 128 11.1 -> 10.1 us, 512 13.0 -> 10.8, 1024 14.9 -> 11.3,
+// 4096 31.0 -> 17.0; S 32768, k 2048 32.1 -> 26.5; S 131072, k 4096 103.8 -> 94.1.  k 64 is equal either way.  Rows with a
+// crowded bin pay for the count and the sort (S 8192, k 1024, 16.0 -> 16.8).
 // The threshold form is step 3 alone with a given threshold.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -46,6 +49,8 @@ constexpr int kTopkWaves = kTopkThreads / 64;
 constexpr int kTopkBins = 2048;      // two per thread
 constexpr int kTopkBinBits = 11;
 constexpr int kTopkMaxRegs = 32;     // elements per lane that stay in registers
+constexpr int kTopkCountMin = 64;    // more than this many are ordered by counting
+constexpr int kTopkCrowd = 64;       // ... if no bin holds more than this many of them
 
 // monotone map float -> uint32: a < b  <=>  key(a) < key(b)  (-0 < +0, NaNs at the two ends)
 __device__ __forceinline__ uint32_t order_key(float v)
@@ -117,7 +122,25 @@ struct TopkLds {
     uint32_t wmin[kTopkWaves], wmax[kTopkWaves];
     int2 wcnt[kTopkWaves];
     int bin, above, count;
+    int crowded;
 };
+
+// How many of the counted keys lie in the bins of higher threads; c: those in this thread's two.  One barrier.
+__device__ __forceinline__ int in_higher_bins(int c, TopkLds &lds, int wave, int lane)
+{
+    int run = c;  // this lane and the higher ones of its wave
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        const int o = __shfl_down(run, m);
+        run += (lane + m < 64) ? o : 0;
+    }
+    if (lane == 0) lds.wsum[wave] = run;
+    __syncthreads();
+    int above = run - c;
+#pragma unroll
+    for (int w = 0; w < kTopkWaves; ++w) above += (w > wave) ? lds.wsum[w] : 0;
+    return above;
+}
 
 // Places of the taken elements in index order.  thr: elements with a larger key are taken, and the first `need`
 // with an equal one.  put(place, index, key) is called for each; returns their number (block-uniform).  One barrier.
@@ -233,6 +256,46 @@ __device__ __forceinline__ void sort_descending(uint64_t *buf, int n2, int tid, 
     }
 }
 
+// The same order by counting, for k words in buf[0 .. k) whose keys are lo or more and are counted in lds.hist by
+// count_bin: every word goes to its bin's part of buf's second half, takes its place from the words of its bin that
+// are larger (all words differ, so the places do not depend on the order in which a bin was filled), and buf[0 .. k) ends up
+// in order.  False, with buf as it was, where a bin is crowded: a word is compared with all of its bin.  Block-uniform.
+__device__ __forceinline__ int count_bin(uint32_t key, uint32_t lo, int shift)
+{
+    return (int)min((key - lo) >> shift, (uint32_t)(kTopkBins - 1));
+}
+template <int SE>
+__device__ __forceinline__ bool count_descending(uint64_t *buf, int k, uint32_t lo, int shift, TopkLds &lds, int tid, int wave, int lane)
+{
+    const int c0 = lds.hist[2 * tid], c1 = lds.hist[2 * tid + 1];
+    if (max(c0, c1) > kTopkCrowd) lds.crowded = 1;
+    const int above = in_higher_bins(c0 + c1, lds, wave, lane);
+    if (lds.crowded) return false;
+    lds.hist[2 * tid + 1] = above;  // where a bin's words begin; where they end once they are all in
+    lds.hist[2 * tid] = above + c1;
+    __syncthreads();
+    uint64_t w[SE], *binned = buf + kTopkSortMax;
+#pragma unroll
+    for (int s = 0; s < SE; ++s) {
+        const int i = tid + s * kTopkThreads;
+        w[s] = (i < k) ? buf[i] : 0;
+        if (i < k) binned[atomicAdd(&lds.hist[count_bin((uint32_t)(w[s] >> 32), lo, shift)], 1)] = w[s];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < SE; ++s) {
+        if (tid + s * kTopkThreads < k) {
+            const int bin = count_bin((uint32_t)(w[s] >> 32), lo, shift), end = lds.hist[bin];
+            const int start = (bin + 1 < kTopkBins) ? lds.hist[bin + 1] : 0;
+            int place = start;
+            for (int j = start; j < end; ++j) place += (binned[j] > w[s]) ? 1 : 0;
+            buf[place] = w[s];
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
 }  // namespace
 
 template <int E>
@@ -263,11 +326,16 @@ __global__ __launch_bounds__(kTopkThreads) void fcs_topk_kernel(const float *mea
         lds.wmax[wave] = kmax;
     }
     lds.hist[2 * tid] = lds.hist[2 * tid + 1] = 0;
+    if (tid == 0) lds.crowded = 0;
     __syncthreads();
+    uint32_t kmax2 = 0;  // of the waves' largest keys the second
+    kmax = 0;
 #pragma unroll
     for (int w = 0; w < kTopkWaves; ++w) {
+        const uint32_t v = lds.wmax[w];
         kmin = min(kmin, lds.wmin[w]);
-        kmax = max(kmax, lds.wmax[w]);
+        kmax2 = max(kmax2, min(kmax, v));
+        kmax = max(kmax, v);
     }
 
     // ---- 2. the k-th largest key lies in [lo, lo + span]; `want` is its rank (1 = largest) among the keys in there.
@@ -283,17 +351,7 @@ __global__ __launch_bounds__(kTopkThreads) void fcs_topk_kernel(const float *mea
         __syncthreads();
         // bins 2 tid and 2 tid + 1; suffix sums over the threads
         const int c0 = lds.hist[2 * tid], c1 = lds.hist[2 * tid + 1];
-        int run = c0 + c1;  // this lane and the higher ones of its wave
-#pragma unroll
-        for (int m = 1; m < 64; m <<= 1) {
-            const int o = __shfl_down(run, m);
-            run += (lane + m < 64) ? o : 0;
-        }
-        if (lane == 0) lds.wsum[wave] = run;
-        __syncthreads();
-        int above = run - c0 - c1;  // keys in the bins of higher threads
-#pragma unroll
-        for (int w = 0; w < kTopkWaves; ++w) above += (w > wave) ? lds.wsum[w] : 0;
+        const int above = in_higher_bins(c0 + c1, lds, wave, lane);
         if (above < want && want <= above + c1) {
             lds.bin = 2 * tid + 1;
             lds.above = above;
@@ -330,22 +388,34 @@ __global__ __launch_bounds__(kTopkThreads) void fcs_topk_kernel(const float *mea
     while (n2 < k) n2 <<= 1;
     // zero words sort behind every real one (whose lower half is the complement of an index)
     for (int i = k + tid; i < n2; i += kTopkThreads) buf[i] = 0;
+    const bool equal = kmax == lo;  // all that are taken: in order as they are
+    const bool count = k > kTopkCountMin && !equal;
+    // The bins span the taken keys, or without those of one wave where these (a context's first tokens) would leave the
+    // others an eighth of the bins: they meet in the last one.
+    const uint32_t top = (kmax2 > lo && (kmax - lo) >> 3 > kmax2 - lo) ? kmax2 : kmax;
+    const int shift = (top == lo) ? 0 : max(0, 32 - __builtin_clz(top - lo) - kTopkBinBits);
     take_in_order(part, lo, want, lds, wave, lane, [&](int place, int i, uint32_t key) {
-        if (place < k) buf[place] = ((uint64_t)key << 32) | (uint32_t)~i;
+        if (place < k) {
+            buf[place] = ((uint64_t)key << 32) | (uint32_t)~i;
+            if (count) atomicAdd(&lds.hist[count_bin(key, lo, shift)], 1);
+        }
     });
     __syncthreads();
+    auto put = [&](int e, uint64_t w) {
+        io[e] = (int)~(uint32_t)w;
+        if (vo) vo[e] = key_value((uint32_t)(w >> 32));
+    };
     auto finish = [&](auto se_c) {
         constexpr int SE = decltype(se_c)::value;
+        if (equal || (count && count_descending<SE>(buf, k, lo, shift, lds, tid, wave, lane))) {
+            for (int e = tid; e < k; e += kTopkThreads) put(e, buf[e]);
+            return;
+        }
         uint64_t w[SE];
         sort_descending<SE>(buf, n2, tid, w);
 #pragma unroll
-        for (int s = 0; s < SE; ++s) {
-            const int e = tid * SE + s;
-            if (e < k) {
-                io[e] = (int)~(uint32_t)w[s];
-                if (vo) vo[e] = key_value((uint32_t)(w[s] >> 32));
-            }
-        }
+        for (int s = 0; s < SE; ++s)
+            if (tid * SE + s < k) put(tid * SE + s, w[s]);
     };
     if (n2 <= kTopkThreads) finish(std::integral_constant<int, 1>{});
     else if (n2 <= 2 * kTopkThreads) finish(std::integral_constant<int, 2>{});

@@ -55,3 +55,28 @@ def test_longest_rows(s):
     assert val.tolist() == [[6.0, 5.0, 4.0, 3.0, 2.0]] and torch.equal(idx[0], at[[4, 2, 3, 1, 0]])
     idx, cnt = _hip.threshold_f32(x, 2.0)
     assert cnt.item() == 5 and torch.equal(idx[0, :5], at)
+
+
+@pytest.mark.parametrize("k", [64, 65, 513, 1024, 1025, 2048, 4095, 4096])
+@pytest.mark.parametrize("shape", ["full", "crowded", "outlier", "outliers", "spread"])
+def test_order_by_counting(shape, k):
+    """More than 64 taken entries are ordered by counting in 2048 bins between the smallest and the largest of them (without
+    those of one wave where they lie far above the others), unless a bin holds more than 64."""
+    from flash_colsum import _hip
+
+    print(shape, k, flush=True)
+    gen = torch.Generator().manual_seed(k)
+    if shape in ("full", "crowded"):  # bins of 2^10 keys, each with 64 or 65 entries; the row is taken whole
+        m = 64 if shape == "full" else 65
+        n = torch.arange(k)
+        bits = 0x3F000000 + (n // m) * 1024 + n % m
+        bits[-1] = 0x3F000000 + 2 ** 21 - 1
+        x = bits[torch.randperm(k, generator=gen)].to(torch.int32).view(torch.float32)[None]
+    else:
+        x = torch.randn((3, 2 * k), generator=gen)
+        if shape != "spread":  # all but the outliers, of one wave or of two, lie close together
+            x = 1.0 + 1e-3 * x
+            x[:, [0, 1] if shape == "outlier" else [0, -1]] = 3e38
+    order = torch.sort(x, dim=1, descending=True, stable=True).indices[:, :k]
+    val, idx = _hip.topk_f32(x.cuda(), k, sorted=True)
+    assert torch.equal(idx.cpu(), order) and torch.equal(val.cpu(), x.gather(1, order))
