@@ -836,8 +836,9 @@ static FusedVariant pick_fused(const Plan &p, const Args &a, bool bf)
     // shared-Q variants: five to ten tiles per wave and 8, 4 or 2 key groups (S 257 .. 2560)
     const bool shared_q = TPW >= 5 && (p.f_kg == 8 || p.f_kg == 4 || p.f_kg == 2);
     // ... pre-scaled when the rounding of Q*c to fp16 cannot show in the means
-    // (beyond 2048 keys from the number of pairs on from which the two-pass path takes its pre-scaled operand)
-    const bool pre = shared_q && !bf && (long)p.H * p.q_rows >= (p.Sk > 2048 ? 16384 : 4096) && fabsf(a.c) <= 0.1251f * 1.44269504f;
+    // (up to 2048 keys.  Longer calls took their exact operand from a row sum of 2^20 on while they ran in two passes, not from
+    // 2^28: the scores' rounding would reach rows that it did not reach then.)
+    const bool pre = shared_q && !bf && p.Sk <= kFusedMaxKeys && (long)p.H * p.q_rows >= 4096 && fabsf(a.c) <= 0.1251f * 1.44269504f;
     if (pre && whole && TPW == 8 && (p.f_kg == 8 || p.f_kg == 4)) return {8, false, p.f_kg, true};
     if (pre) return {TPW, true, p.f_kg, true};
     // ... else Q shared through LDS as it is (8 or 4 key groups).  (Two key groups that cannot be
@@ -853,14 +854,12 @@ static void launch_wide(const Plan &p, const Args &a, hipStream_t st)
 {
     const dim3 grid(p.f_nwgq * p.B, p.f_hg);
     const FusedVariant v = pick_fused(p, a, BF);
-    if (v.pre == 8 && v.qs)
-        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 8, false>), grid, dim3(512), 0, st, a);
+    if (v.pre == 8)  // more than 2048 keys: never pre-scaled
+        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 8, BF, false>), grid, dim3(512), 0, st, a);
     else if (v.pre == 4 && v.qs)
         hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 4, false>), grid, dim3(512), 0, st, a);
     else if (v.pre == 2 && v.qs)
         hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 2, false>), grid, dim3(512), 0, st, a);
-    else if (v.pre == 8)
-        hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 8, BF, false>), grid, dim3(512), 0, st, a);
     else if (v.pre == 4)
         hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 4, BF, false>), grid, dim3(512), 0, st, a);
     else

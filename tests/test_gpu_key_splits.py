@@ -47,7 +47,7 @@ WIDE = [(24, 513, 2, 9), (24, 545, 2, 9), (24, 576, 2, 9), (32, 577, 2, 10), (32
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_nine_and_ten_tiles(b, s, kg, tiles, dtype):
     q, k = _make(b, 16, 16, s, s, 64, dtype, layout="tokens" if s % 2 else "heads")
-    _check(q, k, {}, (tiles, kg, dtype == torch.float16))
+    _check(q, k, {}, (tiles, kg, dtype == torch.float16 and s <= 2048))
 
 
 @pytest.mark.parametrize("which", ["row", "head", "keys"])
@@ -61,17 +61,32 @@ def test_rows_out_of_range(b, s, kg, tiles, which):
         q[:, 5] *= 40
     else:
         k[:, 7, s - 40:] *= 50
-    _check(q, k, {}, (tiles, kg, True))
+    _check(q, k, {}, (tiles, kg, s <= 2048))
+
+
+@pytest.mark.parametrize("std", [1.0, 2.5, 3.5, 5.0])
+@pytest.mark.parametrize("b,h,s", [(1, 16, 2300), (2, 8, 2560), (1, 8, 2049)])
+def test_logits_beyond_2048_keys_are_not_rounded(b, h, s, std):
+    """More than 2048 keys take the operand as it is whatever the number of pairs: rows of widely spread logits (row sums of 2^20 and
+    more) had it when such calls ran in two passes.  Bound: an fp32 score of up to 6 std is off by 1e-6 of itself at most, and with
+    it its exponential; a mean adds 16000 and more of them, of either sign.  With Q * c rounded to fp16 it is 6.5e-6 at std 1
+    and 2e-4 at std 3.5."""
+    g = torch.Generator(device="cuda").manual_seed(int(10 * std))
+    q, k = ((torch.randn((b, h, s, 64), generator=g, device="cuda") * std ** 0.5).half() for _ in range(2))
+    print((b, h, s), std, flush=True)
+    assert _variant(q, k, {})[1:] == (8, False)
+    ref = torch.cat([colsum_ext_exact(q[i:i + 1], k[i:i + 1]) for i in range(b)])
+    got = flash_colsum_ext(q, k, out_dtype=torch.float32)
+    assert ((got.double() - ref).abs() / ref).max().item() <= 3e-6
 
 
 @pytest.mark.parametrize("kw", [{"scale": -0.1}, {"scale": 0.3}, {"cls_len": 300}])
 @pytest.mark.parametrize("s,kg", [(2100, 8), (2400, 8)])
 def test_beyond_2048_keys(s, kg, kw):
-    """Grouped heads (key tiles kept from one query head to the next), other scales, fewer rows than keys; few pairs take the
-    operand as it is."""
+    """Grouped heads (key tiles kept from one query head to the next), other scales, fewer rows than keys."""
     tiles = 9 if s <= 2304 else 10
     q, k = _make(2, 16, 4, s, s, 64, torch.float16, seed=2)
-    _check(q, k, kw, (tiles, kg, "cls_len" not in kw and kw.get("scale") != 0.3))
+    _check(q, k, kw, (tiles, kg, False))
     q, k = _make(3, 2, 1, 150, s, 64, torch.bfloat16, seed=3)
     _check(q, k, {k_: v for k_, v in kw.items() if k_ != "cls_len"}, (tiles, kg, False))
 
