@@ -296,7 +296,7 @@ def repeated_call(key, q, k):
         return None
     c, c_ref, n_ws, shape, f16, n_q, n_k = ent
     if n_q:  # fp32 operands
-        return _repeated_rounded(ent, q, k, q_ptr, k_ptr, index)
+        return _repeated_rounded(key, ent, q, k, q_ptr, k_ptr, index)
     return _run_known(c, c_ref, n_ws, shape, f16, q_ptr, k_ptr, q.device, index)
 
 
@@ -313,8 +313,9 @@ def _run_known(c, c_ref, n_ws, shape, f16, q_ptr, k_ptr, dev, index):
     return out
 
 
-def _repeated_rounded(ent, q, k, q_ptr, k_ptr, index):
-    """The route of `_rounded_operands`, both rounded operands in one allocation; None for the full path."""
+def _repeated_rounded(key, ent, q, k, q_ptr, k_ptr, index):
+    """The route of `_rounded_operands`, both rounded operands in one allocation; None for the full path.  Operands beyond
+    the range go on from there, and their geometry is forgotten: the next call may be as they are."""
     c, c_ref, n_ws, shape, f16, n_q, n_k = ent
     if q.is_neg() or k.is_neg() or torch.cuda.is_current_stream_capturing():
         return None
@@ -330,7 +331,10 @@ def _repeated_rounded(ent, q, k, q_ptr, k_ptr, index):
         out = _run_known(c, c_ref, n_ws, shape, f16, r_ptr, r_ptr + at_k, dev, index)
     finally:
         event.synchronize()  # also after an error: the word is written by this call's kernel alone
-    return None if word.value else out  # (out of range: the full path works it out)
+    if not word.value:
+        return out
+    _tls.known.pop(key, None)
+    return _launch(bool(c.causal), q, k, c.scale, c.cls_n, c.k_past, f16_only=f16, beyond=True)
 
 
 def _remember(key, causal, q, k, scale, cls_n, k_past, f16, rounded):
@@ -424,9 +428,10 @@ def _rounded_operands(q: torch.Tensor, k: torch.Tensor):
 
 
 def _launch(causal: bool, q: torch.Tensor, k: torch.Tensor, scale: float, cls_n: int, k_past: int, want_f16: bool = False,
-            f16_only: bool = False, key=None, rounded: bool = False):
+            f16_only: bool = False, key=None, beyond: bool = False):
     """Enqueue one call; returns the fp32 means, (fp32, fp16) when `want_f16`, or the fp16 tensor alone
-    when `f16_only` (which implies `want_f16`).  `key`: what a repeated call will be recognised by."""
+    when `f16_only` (which implies `want_f16`).  `key`: what a repeated call will be recognised by.  `beyond`: fp32 operands
+    that are known to leave fp16's range."""
     want_f16 = want_f16 or f16_only
     if q.device.type != "cuda" or k.device != q.device:
         raise ValueError(f"query and key must live on the same GPU, got {q.device} and {k.device}")
@@ -435,16 +440,19 @@ def _launch(causal: bool, q: torch.Tensor, k: torch.Tensor, scale: float, cls_n:
     if q.dtype in half and k.dtype in half:
         dtype = torch.bfloat16 if (q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16) else torch.float16
     else:
-        both = _rounded_operands(q, k)
+        both = None if beyond else _rounded_operands(q, k)
         if both is not None:
             # the means of the rounded operands are enqueued before the range test is known, so that the GPU does not
             # wait for the host; operands beyond the range are rare and computed again below
             q_h, k_h, (_, _, word, event) = both
             try:
-                out = _launch(causal, q_h, k_h, scale, cls_n, k_past, want_f16, f16_only, key, True)
+                out = _launch(causal, q_h, k_h, scale, cls_n, k_past, want_f16, f16_only)
             finally:
                 event.synchronize()  # also after an error: the word is written by this call's kernel alone
             if not word.value:
+                if (key is not None and q.shape[-1] % 8 == 0 and q.device.index == torch.cuda.current_device()
+                        and _as_kernel_input(q_h) is q_h and _as_kernel_input(k_h) is k_h):
+                    _remember(key, causal, q_h, k_h, float(scale), cls_n, min(int(k_past), k.shape[2]), f16_only, True)
                 return out
         q, k, dtype = _wide_operands(q, k)
         key = None
@@ -464,7 +472,7 @@ def _launch(causal: bool, q: torch.Tensor, k: torch.Tensor, scale: float, cls_n:
     if q.device.index == torch.cuda.current_device():
         out = _enqueue(causal, q, k, float(scale), cls_n, k_past, want_f16, f16_only)
         if key is not None and q is given[0] and k is given[1]:
-            _remember(key, causal, q, k, float(scale), cls_n, k_past, f16_only, rounded)
+            _remember(key, causal, q, k, float(scale), cls_n, k_past, f16_only, False)
         return out
     with torch.cuda.device(q.device):
         return _enqueue(causal, q, k, float(scale), cls_n, k_past, want_f16, f16_only)

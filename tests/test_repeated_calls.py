@@ -101,3 +101,40 @@ def test_repeated_call_in_a_graph():
         g.replay()
         assert torch.equal(out, flash_colsum(q, k))
     assert eager.shape == out.shape
+
+
+class _Counted:
+    """The library, with a count of its calls."""
+
+    def __init__(self, lib):
+        self.lib, self.n = lib, {}
+
+    def __getattr__(self, name):
+        fn = getattr(self.lib, name)
+
+        def call(*args):
+            self.n[name] = self.n.get(name, 0) + 1
+            return fn(*args)
+
+        return call
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fn", [flash_colsum, flash_colsum_f32])
+def test_operands_beyond_fp16_are_computed_once_more_only(fn, monkeypatch):
+    """fp32 operands that leave fp16's range: one rounding, one discarded computation and that of the split operands, also on
+    repeated calls; a geometry is remembered by calls that stayed inside the range."""
+    q, k = _pair(3, (2, 3, 90, 64), torch.float32)
+    big = q.clone()
+    big[1, 2, 5] *= 1e6
+    counted = _Counted(_hip.lib())
+    monkeypatch.setattr(_hip, "_lib", counted)
+    monkeypatch.setattr(_hip._tls, "known", {}, raising=False)
+
+    def calls(a):
+        counted.n.clear()
+        _good(fn(a, k, 1e-5), a, k, scale=1e-5)
+        return counted.n.get("fcs_round_f16", 0), counted.n["fcs_colsum_call"]
+
+    for a, n, known in [(big, (1, 2), 0), (big, (1, 2), 0), (q, (1, 1), 1), (q, (1, 1), 1), (big, (1, 2), 0), (big, (1, 2), 0), (q, (1, 1), 1)]:
+        assert calls(a) == n and len(_hip._tls.known) == known
