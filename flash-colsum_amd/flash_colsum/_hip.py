@@ -126,6 +126,8 @@ def _as_kernel_input(t: torch.Tensor, dtype: torch.dtype = torch.float16) -> tor
     """`dtype` (fp16 or bf16), unit last stride, 16-byte aligned rows/heads/base; copies only when it must."""
     if t.dtype != dtype:
         t = t.to(dtype)
+    if t.is_neg():  # a negation that torch has put off: the memory holds the opposite values
+        t = t.resolve_neg()
     if t.is_contiguous() and t.shape[-1] % 8 == 0 and t.data_ptr() % 16 == 0 and t.shape[1] > 1 and t.shape[2] > 1:
         # the common case, decided without looking at the strides one by one (a dimension of size 1 may carry
         # any stride and still count as contiguous: those tensors take the checks below)
@@ -292,7 +294,7 @@ def repeated_call(key, q, k):
     if index < 0 or k.get_device() != index or _get_device() != index:
         return None
     q_ptr, k_ptr = q.data_ptr(), k.data_ptr()
-    if (q_ptr | k_ptr) & 15:
+    if (q_ptr | k_ptr) & 15 or q.is_neg() or k.is_neg():
         return None
     c, c_ref, n_ws, shape, f16, n_q, n_k = ent
     if n_q:  # fp32 operands
@@ -317,7 +319,7 @@ def _repeated_rounded(key, ent, q, k, q_ptr, k_ptr, index):
     """The route of `_rounded_operands`, both rounded operands in one allocation; None for the full path.  Operands beyond
     the range go on from there, and their geometry is forgotten: the next call may be as they are."""
     c, c_ref, n_ws, shape, f16, n_q, n_k = ent
-    if q.is_neg() or k.is_neg() or torch.cuda.is_current_stream_capturing():
+    if torch.cuda.is_current_stream_capturing():
         return None
     dev = q.device
     at_k = (2 * n_q + 255) & ~255

@@ -138,3 +138,18 @@ def test_operands_beyond_fp16_are_computed_once_more_only(fn, monkeypatch):
 
     for a, n, known in [(big, (1, 2), 0), (big, (1, 2), 0), (q, (1, 1), 1), (q, (1, 1), 1), (big, (1, 2), 0), (big, (1, 2), 0), (q, (1, 1), 1)]:
         assert calls(a) == n and len(_hip._tls.known) == known
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(2, 4, 100, 64), (2, 4, 100, 36)])  # (36 channels are padded, by a copy)
+def test_pending_negations(shape, dtype):
+    """A view whose negation torch has put off, as the first call of a geometry and as a repeated one."""
+    q, k = _pair(4, shape, dtype)
+    for _ in range(2):
+        for a, b in ((torch._neg_view(q), k), (q, torch._neg_view(k)), (torch._neg_view(q), torch._neg_view(k))):
+            assert a.is_neg() or b.is_neg()
+            _good(flash_colsum(a, b), a.resolve_neg(), b.resolve_neg())
+            t = a.transpose(1, 2).contiguous().transpose(1, 2) if not a.is_neg() else torch._neg_view(q.transpose(1, 2).contiguous()).transpose(1, 2)
+            _good(flash_colsum(t, b), t.resolve_neg(), b.resolve_neg())
+        _good(flash_colsum(q, k), q, k)
