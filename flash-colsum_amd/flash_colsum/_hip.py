@@ -280,7 +280,10 @@ def call_key(kind: int, q, k, scale, is_causal, cls_len, k_past=None):
     """What a repeated call is recognised by, or None where the arguments are of other than the plain types."""
     if (type(q) is torch.Tensor and type(k) is torch.Tensor and (scale is None or type(scale) is float) and type(is_causal) is bool
             and (cls_len is None or type(cls_len) is int) and (k_past is None or type(k_past) is int)):
-        return kind, q.shape, k.shape, q.stride(), k.stride(), q.dtype, k.dtype, scale, is_causal, cls_len, k_past
+        try:
+            return kind, q.shape, k.shape, q.stride(), k.stride(), q.dtype, k.dtype, scale, is_causal, cls_len, k_past
+        except RuntimeError:  # tensors without sizes or strides (nested, compressed): refused by the checks of the full path
+            pass
     return None
 
 

@@ -23,6 +23,17 @@ def test_only_plain_arguments_are_recognised():
         flash_colsum(q, q)
 
 
+@pytest.mark.filterwarnings("ignore")  # nested and compressed tensors warn that they are prototypes
+def test_tensors_without_sizes_or_strides_are_refused_as_others_are():
+    nested = torch.nested.nested_tensor([torch.zeros(2, 3, 8), torch.zeros(2, 5, 8)])
+    compressed = torch.zeros(2, 3, 8, 8).to_sparse_csr()
+    for t in (nested, compressed):
+        assert t.ndim == 4 and _hip.call_key(0, t, t, None, False, None) is None
+        for fn in (flash_colsum, flash_colsum_f32, flash_colsum_ext):
+            with pytest.raises(ValueError, match="only supports CUDA tensors"):
+                fn(t, t)
+
+
 def _pair(seed, shape=(2, 4, 100, 64), dtype=torch.float16):
     g = torch.Generator(device="cuda").manual_seed(seed)
     return tuple(torch.randn(shape, generator=g, device="cuda").to(dtype) for _ in range(2))
