@@ -136,7 +136,7 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     a.c_chunk = p.c_chunk; a.c_nchunks = p.c_nchunks; a.c_nrb = p.c_nrb;
     a.c_line = p.c_line; a.c_unit = p.c_unit; a.c_cs = p.c_cs; a.c_seg = p.c_seg; a.c_len = p.c_len; a.c_blocks = p.c_blocks; a.c_direct = p.c_direct;
     a.c_by_seg = p.c_by_seg; a.c_by_batch = p.c_by_batch; a.c_by_chunks = p.c_by_chunks; a.c_by_chunk = p.c_by_chunk;
-    a.c_by_blocks = p.c_by_blocks; a.c_by_used = p.c_by_used;
+    a.c_by_blocks = p.c_by_blocks; a.c_every = p.c_every;
     a.partial = reinterpret_cast<float *>(w + p.off_partial);
     a.out = out;
     a.out_h = static_cast<_Float16 *>(out_f16);

@@ -37,8 +37,8 @@ struct Args {
     // pass 2
     int c_chunk, c_nchunks, c_nrb;  // keys per chunk, chunks, row blocks per head
     StageLine c_line;               // the stages of its units, as for pass 1; chunk after chunk
-    int c_unit, c_cs, c_seg, c_len, c_blocks, c_direct;  // c_cs: units per chunk
-    FastDiv c_by_seg, c_by_batch, c_by_chunks, c_by_chunk, c_by_blocks, c_by_used;
+    int c_unit, c_cs, c_seg, c_len, c_blocks, c_direct, c_every;  // c_cs: units per chunk
+    FastDiv c_by_seg, c_by_batch, c_by_chunks, c_by_chunk, c_by_blocks;
     float *partial;  // slabs; two-pass path: [..][c_chunk], slab w + i is share w's of chunk i (i = batch entry * c_nchunks + chunk)
     float *out;      // [B][Sk]
     _Float16 *out_h; // [B][Sk] or nullptr: the same means rounded to fp16

@@ -60,8 +60,9 @@ __global__ __launch_bounds__(32 * SL) void fcs_finalize_kernel(const Args a)
             const int b = (int)((n >> 32) == 0 ? (uint32_t)idx / (uint32_t)a.Sk : idx / a.Sk);
             int in_chunk;
             const int cx = a.c_by_chunk.quot((int)(idx - (int64_t)b * a.Sk), in_chunk);
-            const int before = a.c_line.chunk_places(a.c_nrb, a.c_cs, cx);
-            const int len = (a.c_line.chunk_places(a.c_nrb, a.c_cs, cx + 1) - before) * a.v_heads;
+            const int pairs = a.c_line.pairs(a.c_nrb, a.c_cs, cx, a.c_every), at = a.c_line.sum(a.c_nrb, cx * a.c_cs);
+            const int before = at + pairs * a.c_line.start;
+            const int len = (a.c_line.sum(a.c_nrb, (cx + 1) * a.c_cs) - at + a.c_line.sees(a.c_nrb, a.c_cs, cx) * a.c_line.start) * a.v_heads;
             const int start = b * (int)a.c_by_batch.d + before * a.v_heads, w0 = a.c_by_seg.quot(start + a.c_line.start);
             const int slabs = (len > 0) ? a.c_by_seg.quot(start + len - 1) - w0 + 1 : 0;  // 0: no row sees the chunk
             const float *p = a.partial + (w0 + (int64_t)b * a.c_nchunks + cx) * a.c_chunk + in_chunk;

@@ -100,15 +100,19 @@ struct StageLine {
         v = (v < hi ? v : hi) - lo;
         return v > 0 ? v : 0;
     }
-    // column pass: places of the first `chunks` chunks of cs stages of a head with nrb row blocks; each row block takes
-    // `start` places in each chunk that it sees
-    FCS_HD int chunk_places(int nrb, int cs, int chunks) const
+    // column pass, chunks of cs stages of a head with nrb row blocks: the row blocks that see chunk c
+    FCS_HD int sees(int nrb, int cs, int c) const { return nrb - up_to(nrb, c * cs); }
+    // how many chunks every row block sees
+    FCS_HD int every(int cs) const { return (n(0) + cs - 1) / cs; }
+    // (row block, chunk) pairs among the first `chunks` chunks, of which `all` = every(cs) go without looking
+    FCS_HD int pairs(int nrb, int cs, int chunks, int all) const
     {
-        int seen = 0;  // (row block, chunk) pairs
-        if (step == 0) seen = nrb * (chunks < (last + cs - 1) / cs ? chunks : (last + cs - 1) / cs);
-        else for (int c = 0; c < chunks; ++c) seen += nrb - up_to(nrb, c * cs);
-        return sum(nrb, chunks * cs) + seen * start;
+        int seen = nrb * (chunks < all ? chunks : all);
+        for (int c = all; c < chunks && c * cs < last; ++c) seen += sees(nrb, cs, c);
+        return seen;
     }
+    // places of the first `chunks` chunks; each row block takes `start` places in each chunk that it sees
+    FCS_HD int chunk_places(int nrb, int cs, int chunks) const { return sum(nrb, chunks * cs) + pairs(nrb, cs, chunks, every(cs)) * start; }
 };
 
 struct Plan {
@@ -141,8 +145,10 @@ struct Plan {
     int c_unit, c_cs;                      // stages per unit of the line, units per chunk
     int c_seg, c_len, c_blocks, c_direct;  // c_direct: block w computes all of chunk w and writes the means
     int c_one;                             // every share is one chunk of one unit
-    FastDiv c_by_seg, c_by_batch, c_by_chunks, c_by_chunk;  // divisions by c_seg, a batch entry's units, c_nchunks, c_chunk
-    FastDiv c_by_blocks, c_by_used;        // divisions by c_nrb, the chunks that some row sees
+    int c_every;                           // chunks that every row block sees
+    FastDiv c_by_seg, c_by_batch, c_by_chunk, c_by_blocks;  // divisions by c_seg, a batch entry's units, c_chunk, c_nrb
+    FastDiv c_by_chunks;  // by c_nchunks (c_direct), the chunks that some row sees (c_unit > 1 or c_one), or the places of a
+                          // chunk that all row blocks see to its end
     int c_groups;      // slabs per chunk, rounded down (1: none)
     // fused single-kernel path: non-causal, all keys of a row block fit in one
     // workgroup's registers.  grid = (f_nwgq * B, f_hg)
@@ -348,7 +354,6 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         p.c_direct = how == kDirect;
         p.c_one = how == kUnits && seg == 1;
         p.c_by_blocks.set(p.c_nrb);
-        p.c_by_used.set(used);
         p.c_len = p.c_seg = p.c_groups = p.n_partials = 1;
         p.c_blocks = (int)chunks;
         p.c_by_batch.set(1);
@@ -363,7 +368,8 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
             p.c_by_batch.set(per_batch);
         }
         p.c_by_seg.set(p.c_seg);
-        p.c_by_chunks.set(p.c_nchunks);
+        p.c_every = p.c_line.every(p.c_cs);
+        p.c_by_chunks.set(p.c_direct ? p.c_nchunks : (p.c_unit > 1 || p.c_one) ? used : (int64_t)units * (p.c_cs + p.c_line.start));
         p.c_by_chunk.set(p.c_chunk);
     }
 

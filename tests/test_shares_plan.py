@@ -78,6 +78,7 @@ extern "C" int check(int causal, int B, int H, int Hk, int Sq, int Sk, int D, in
     const int rows2 = 32 * p.c_nb * p.c_waves, cs = p.c_cs;
     if (p.c_chunk > col_chunk_max(p.Dp, p.c_waves) || p.c_cs * p.c_unit * kStageKeys != p.c_chunk) return 10;
     std::vector<std::set<long>> slabs((long)B * p.c_nchunks);
+    std::set<long> numbers;
     std::vector<int> done2((long)B * p.c_nchunks * p.v_heads * p.c_nrb);
     for (long share = 0; share < p.c_blocks; ++share) {
         long b;
@@ -88,6 +89,7 @@ extern "C" int check(int causal, int B, int H, int Hk, int Sq, int Sk, int D, in
             int pos = (int)share * p.c_seg;
             left = std::min(p.c_seg, p.c_len - pos);
             if (left <= 0) return 11;
+            // the line in order: batch entry, chunk, head, row block
             b = p.c_by_batch.quot(pos, pos);
             for (cx = 0; pos >= p.v_heads * p.c_line.chunk_places(p.c_nrb, cs, cx + 1); ++cx) {}
             pos -= p.v_heads * p.c_line.chunk_places(p.c_nrb, cs, cx);
@@ -99,6 +101,32 @@ extern "C" int check(int causal, int B, int H, int Hk, int Sq, int Sk, int D, in
                 pos -= len;
             }
             at = pos;
+            // the kernel's three ways to the same place
+            int k_cx, k_h, k_rb;
+            if (p.c_one) {  // chunks of a unit side by side: another place, and the share that belongs there
+                long k_b = p.by_heads.quot(p.c_by_blocks.quot(p.c_by_chunks.quot((int)share, k_cx), k_rb), k_h);
+                const long number = ((k_b * (int)p.c_by_chunks.d + k_cx) * p.v_heads + k_h) * p.c_nrb + k_rb;
+                if (number < 0 || number >= p.c_blocks || !numbers.insert(number).second) return 20;
+                // that share, by the line: its slab is the one that the walk below gives it
+                int q = (int)number * p.c_seg, q_cx, q_h, q_rb;
+                const long q_b = p.c_by_batch.quot(q, q);
+                q_rb = q % p.c_nrb, q_h = q / p.c_nrb % p.v_heads, q_cx = q / p.c_nrb / p.v_heads;
+                if (p.c_seg != 1 || p.c_line.start || q_b != k_b || q_cx != k_cx || q_h != k_h || q_rb != k_rb) return 21;
+            } else if (p.c_unit > 1) {
+                const long k_b = p.c_by_chunks.quot(p.by_heads.quot(p.c_by_blocks.quot((int)share * p.c_seg, k_rb), k_h), k_cx);
+                if (k_b != b || k_cx != cx || k_h != h || k_rb != rb || at != 0) return 22;
+            } else {
+                p.c_by_batch.quot((int)share * p.c_seg, pos);
+                k_cx = std::min(p.c_by_chunks.quot(pos), p.c_every - (p.c_every * cs > p.c_line.n(0) ? 1 : 0));
+                int pairs = k_cx * p.c_nrb, steps = 0;
+                for (;; ++k_cx, ++steps) {
+                    pairs += p.c_line.sees(p.c_nrb, cs, k_cx);
+                    if (pos < p.v_heads * (p.c_line.sum(p.c_nrb, (k_cx + 1) * cs) + pairs * p.c_line.start)) break;
+                }
+                if (k_cx != cx || pairs != p.c_line.pairs(p.c_nrb, cs, cx + 1, p.c_every)) return 23;
+                // only chunks that not every row block sees to its end are walked over
+                if (steps > (p.c_line.last - p.c_line.n(0)) / cs + 1) return 24;
+            }
         }
         for (;;) {
             if (b >= B || cx >= p.c_nchunks) return 12;
@@ -168,6 +196,7 @@ def test_every_stage_is_in_one_share(check, seed):
     fixed = [(False, 1, 16, 16, 8192, 8192, 64, -1, 0), (False, 1, 16, 16, 9289, 9289, 64, -1, 0), (True, 1, 32, 32, 4096, 4096, 128, -1, 0),
              (True, 1, 32, 32, 512, 65536, 128, -1, 65024), (True, 4, 32, 8, 64, 8192, 128, -1, 8128), (True, 1, 8, 8, 512, 4096, 256, -1, 3584),
              (True, 257, 1, 1, 128, 250, 64, -1, 122), (True, 3, 5, 1, 1, 1, 64, -1, 0), (True, 1, 2, 2, 20000, 300, 128, -1, 0),
+             (True, 1, 8, 8, 1024, 262144, 128, -1, 261120), (True, 1, 3, 3, 1100, 90000, 64, -1, 50000), (True, 1, 1, 1, 65536, 65536, 64, -1, 0),
              (False, 300, 3, 3, 5, 3000, 64, -1, 0), (True, 2, 3, 3, 700, 5000, 200, 100, 10)]
     shapes, n_two_pass = fixed if seed == 0 else [], 0
     for _ in range(400):
