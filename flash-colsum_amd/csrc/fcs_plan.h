@@ -310,6 +310,11 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         const bool huge = all * (1. + start) >= kHuge;
         // what the final reduction takes, in stages: a launch, and the slabs, written and read
         const auto reduce = [&](long shares, int c) { return 2.5 + (double)shares * c * 1e-4; };
+        // Causal row blocks that see almost the same keys (the last rows of a long context) are quicker whole, four of one head
+        // re-reading its chunk, than in shares that straddle two heads at every workgroup (us per call, shares -> whole: H 8, Q 4096,
+        // K 65536, D 64 693 -> 653; H 32, Q 1500, K 32768, D 64 538 -> 496; H 4, Q 2048, K 65536, D 128 291 -> 279), up to
+        // about 3 % of the line's length (H 12, Q 4096, K 12288, D 128, where whole ones are 14 % longer: 280 in shares, 301).
+        const double uneven = stages.step ? 1.03 : 1.;
         const int parts0 = ceil_div(n, most), parts_end = ceil_div(n, kMinShare);
         int cs = 1, seg = 1;
         enum { kShares, kUnits, kDirect } how = kDirect;
@@ -323,12 +328,12 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
                 l.start = start;
                 int sg = (int)(((int64_t)B * p.v_heads * l.chunk_places(p.c_nrb, c, parts) + target - 1) / target);
                 if (sg < kMinShare + start) sg = kMinShare + start;
-                const double cost = sg + start + reduce(target, c);
+                const double cost = uneven * (sg + start) + reduce(target, c);
                 if (cost < best) { best = cost; cs = c; seg = sg; how = kShares; }
             }
-            // whole ones per workgroup where all units are equal, or a workgroup for each
+            // whole ones per workgroup, priced as if all were as long as the longest
             const long per = (pieces + target - 1) / target;
-            if (!huge && (stages.step == 0 || per == 1)) {
+            if (!huge) {
                 const double cost = (double)per * (c + start) + reduce(pieces / per, c);
                 if (cost < best) { best = cost; cs = c; seg = (int)per; how = kUnits; }
             }

@@ -217,3 +217,13 @@ def test_shares_of_uneven_row_blocks_are_equal():
     """The triangle of a prompt against itself: 32 heads x (8 + 16 + .. + 64) stages over 256 workgroups."""
     t = _hip.plan_description((1, 32, 4096, 128), (1, 32, 4096, 128), causal=True)
     assert "256 shares of 38 places + " in t and "grid 256, shares of 39 places" in t, t
+
+
+@pytest.mark.parametrize("h,q_len,k_len,d,places", [(8, 4096, 65536, 64, 256), (4, 2048, 65536, 128, 64), (16, 2048, 32768, 64, 128), (12, 1000, 65536, 128, 96)])
+def test_almost_equal_row_blocks_stay_whole(h, q_len, k_len, d, places):
+    """The last rows of a long context: whole units of 32 stages per workgroup, two to eight of them."""
+    t = _hip.plan_description((1, h, q_len, d), (1, h, k_len, d), causal=True)
+    assert f"grid 256, shares of {places} places, chunks of 2048 keys" in t, t
+    # ... and not where the longest is much longer than the others
+    t = _hip.plan_description((1, 12, 4096, 128), (1, 12, 12288, 128), causal=True)
+    assert "shares of 66 places" in t, t
