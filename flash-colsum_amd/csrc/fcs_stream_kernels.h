@@ -267,6 +267,9 @@ constexpr int kFormRaw = 0, kFormPrescaled = 1, kFormShifted = 2;
 // score grows with the spread of the scores; peaked rows, whose few large probabilities are not averaged
 // with thousands of others, are the ones this sends to the exact sweeps)
 constexpr float kRowSumHiPre = 1048576.f;  // 2^20
+// Column pass: log2 of a row's sum in score units, log2(l) / c, overflows below a scale of 1e-37; from here on down the form without
+// it is taken (bf16 scores reach 2^127, so that such a scale still tells keys apart).
+constexpr float kTinyScale = 1e-30f;
 
 // Pre-scaled stationary operand: q * cs in fp32, rounded to fp16 (cs = c with the scale's sign).  The
 // scores then leave the matrix pipe in the exponent's unit and the per-score multiply disappears.  Both
@@ -325,6 +328,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
     const float cmul = (a.c == 0.f) ? 1.f : a.c;       // scale 0: Q is zeroed instead and n_i = -log2 l_i
 
     const float inv_c = __builtin_amdgcn_rcpf(cmul);
+    const bool tiny = cmul < kTinyScale;
     float *colw_w = colw + wave * CHUNK;  // this wave's slice of the column accumulator
 
     // ---- DMA geometry: piece P of a stage goes to LDS byte 16 * P; it is piece pos ^ swizzle(row)
@@ -604,10 +608,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 }
                 // -lg / c: the reciprocal's quotient and one correction by its remainder
                 const float q = lg * inv_c;
-                nl = -fmaf(fmaf(-q, cmul, lg), inv_c, q);
+                nl = tiny ? 0.f : -fmaf(fmaf(-q, cmul, lg), inv_c, q);
             }
             // a stabilised row switches the whole unit, or its wave (kRedoHeads), to the two-constant form
-            const int sh = __builtin_amdgcn_ballot_w64(mm != 0.f) != 0 ? 1 : 0;
+            const int sh = (tiny || __builtin_amdgcn_ballot_w64(mm != 0.f) != 0) ? 1 : 0;
             asm volatile("ds_write_b32 %0, %1" ::"v"(lds_addr(shift_s) + (uint32_t)(wave * 4)), "v"(sh) : "memory");
             if (tid < BLOCK_ROWS) {
                 const uint32_t at = (uint32_t)(tid * 4);

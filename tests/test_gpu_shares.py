@@ -84,3 +84,19 @@ def test_static_scratch_lays_out_what_the_usual_plan_does_not_fit():
     assert rc == 0
     usual = flash_colsum_ext(q, k, is_causal=False, out_dtype=torch.float32)
     assert ((out - usual).abs() <= 2e-6 * usual).all()  # the same terms in another grouping: 12 x 109 fp32 partial sums
+
+
+@pytest.mark.parametrize("scale", [1e-45, 5e-39, 2e-38, 1e-37, 9e-31, 1.1e-30, 1e-20, -2e-38, 0.0])
+@pytest.mark.parametrize("d,dtype,causal", [(64, torch.float16, True), (64, torch.float16, False), (128, torch.float16, False), (64, torch.bfloat16, True),
+                                            (200, torch.bfloat16, True)])
+def test_scales_next_to_zero(d, dtype, causal, scale):
+    """Every row is uniform; log2(row sum) / scale is beyond fp32 for the first of them."""
+    got, ref, _, _ = _call(1, 4, 4, 4096, 4100, d, dtype, causal, scale=scale)
+    _check(got, ref)
+
+
+def test_scale_next_to_zero_on_scores_next_to_the_largest():
+    """bf16 scores of standard deviation 2^124, a scale of 2^-125: logits of one half."""
+    got, ref, _, _ = _call(1, 4, 4, 40, 4096, 64, torch.bfloat16, True, scale=2.0 ** -125, prepare=lambda q, k: (q.mul_(2.0 ** 61), k.mul_(2.0 ** 60)))
+    assert ref.max() / ref.median() > 1.1
+    _check(got, ref)
