@@ -239,13 +239,14 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // (256-wide heads: the kernels' registers and LDS allow one block per compute unit whatever its waves).
     p.gen_blocks = (p.k1_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
 
-    // A pass of 2^31 places or more (days of them) is counted in row blocks and chunks.
+    // A line of 2^31 places (20 s of a pass on 512 rows of 128 channels) or more has no shares: a workgroup per row block in pass 1
+    // (or, where all are equal, whole ones), and per chunk in the column pass.  The limit leaves room for rounding up to whole shares.
     const auto stages_of = [&](const StageLine &l, int blocks) {
         double t = 0.;
         for (int rb = 0; l.step && rb < blocks; ++rb) t += l.n(rb);
         return (l.step ? t : (double)l.last * blocks) * B * p.v_heads;
     };
-    constexpr double kHuge = 1e9;
+    constexpr double kMostPlaces = 2.1e9;
 
     // ---- pass 1: equal shares of the line, at least kMinShare stages each.  A share that crosses into another row block
     // pays that block's start (Q fragments, first key stages) on top, so where all row blocks are equal it is also
@@ -257,7 +258,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         p.r_line = line_of(qblk, p.n_qblk);
         p.r_unit = 1;
         const double all = stages_of(p.r_line, p.n_qblk) + (double)blocks * start;
-        const bool huge = all >= kHuge || tight_stages > 0;
+        const bool huge = all >= kMostPlaces || tight_stages > 0;
         int seg = huge ? 0 : (int)(((int64_t)all + p.gen_blocks - 1) / p.gen_blocks);
         if (seg < kMinShare + start) seg = kMinShare + start;
         p.r_whole = p.r_one = 0;
@@ -265,7 +266,8 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         const int best = seg + start;  // (a share that starts inside a row block pays its start unasked)
         {
             const int n = p.r_line.last;
-            const long per = (blocks + p.gen_blocks - 1) / p.gen_blocks;  // whole row blocks per workgroup
+            // whole row blocks per workgroup (uneven ones without shares: one, and the hardware hands them out)
+            const long per = (huge && p.r_line.step) ? 1 : (blocks + p.gen_blocks - 1) / p.gen_blocks;
             const int most = ceil_div(n, kMinShare);
             const long fit = p.gen_blocks / blocks;
             const int parts = (per > 1 || fit < 2 || tight_stages > 0) ? 1 : (int)(fit < most ? fit : most);
@@ -307,7 +309,6 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         const StageLine stages = line_of(rows, p.c_nrb);
         const int n = seen_stages;
         const double all = stages_of(stages, p.c_nrb);
-        const bool huge = all * (1. + start) >= kHuge;
         // what the final reduction takes, in stages: a launch, and the slabs, written and read
         const auto reduce = [&](long shares, int c) { return 2.5 + (double)shares * c * 1e-4; };
         // Causal row blocks that see almost the same keys (the last rows of a long context) are quicker whole, four of one head
@@ -323,6 +324,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
             const int c = ceil_div(n, parts);
             if (ceil_div(n, c) != parts) continue;
             const long pieces = (long)B * parts * units;  // chunks of the units
+            const bool huge = all + (double)pieces * start >= kMostPlaces;
             if (!huge) {
                 StageLine l = stages;
                 l.start = start;
