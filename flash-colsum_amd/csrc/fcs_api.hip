@@ -42,10 +42,11 @@ hipError_t static_scratch(void **ptr)
 // geometries.
 struct PlanKey {
     int causal, B, H, Hk, Sq, Sk, D, cls_n, k_past;
+    size_t within;  // non-causal: the plan for a workspace of this many bytes (0: the usual one)
     bool operator==(const PlanKey &o) const
     {
         return causal == o.causal && B == o.B && H == o.H && Hk == o.Hk && Sq == o.Sq && Sk == o.Sk && D == o.D && cls_n == o.cls_n &&
-               k_past == o.k_past;
+               k_past == o.k_past && within == o.within;
     }
 };
 constexpr int kPlanMemo = 8;
@@ -57,16 +58,16 @@ struct PlanMemo {
 };
 thread_local PlanMemo t_memo;
 
-bool cached_plan(fcs::Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past)
+bool cached_plan(fcs::Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, size_t within = 0)
 {
-    const PlanKey key{causal, B, H, Hk, Sq, Sk, D, cls_n, k_past};
+    const PlanKey key{causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, within};
     PlanMemo &m = t_memo;
     for (int i = 0; i < kPlanMemo; ++i)
         if (m.used[i] && m.key[i] == key) {
             p = m.plan[i];
             return true;
         }
-    if (!fcs::make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return false;
+    if (!(within ? fcs::plan_within(p, within, B, H, Hk, Sq, Sk, D, cls_n) : fcs::make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past))) return false;
     const int slot = m.next;
     m.next = (slot + 1) % kPlanMemo;
     m.key[slot] = key;
@@ -104,8 +105,8 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     if (k_past > Sk) k_past = Sk;
 
     if (!cached_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return FCS_E_DIMS;
-    // (a fixed workspace: the call is laid out in it where it can be)
-    if (fit_workspace && p.total > ws_bytes && !fcs::plan_within(p, ws_bytes, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return FCS_E_STATIC_LIMIT;
+    // (a fixed workspace, of non-causal calls: the call is laid out in it where it can be)
+    if (fit_workspace && p.total > ws_bytes && !cached_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, ws_bytes)) return FCS_E_STATIC_LIMIT;
     p.bf16 = bf16;
     if (need_ptrs) {
         if (ws && (reinterpret_cast<uintptr_t>(ws) & 255u)) return FCS_E_WORKSPACE;
@@ -252,8 +253,7 @@ int fcs_colsum_noncausal_f16_static(const void *q, const void *k, float *out, vo
     // size check first: it needs no GPU, like every other argument error
     fcs::Plan p;
     if (!cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0)) return FCS_E_DIMS;
-    if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES &&
-        !fcs::plan_within(p, FCS_STATIC_SCRATCH_BYTES, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0))
+    if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES && !cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0, FCS_STATIC_SCRATCH_BYTES))
         return FCS_E_STATIC_LIMIT;
     if (!q || !k || !out || !q_strides || !k_strides) return FCS_E_NULL;
     void *ws = nullptr;

@@ -177,7 +177,7 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Returns false for invalid dimensions.  cls_n <= 0 means all rows.  Hk: key heads, a divisor of H.
 // tight_stages > 0: the two-pass path with as little workspace as it can do with: row blocks are not cut, chunks are not longer
-// than that (see plan_within).
+// than that; < 0: not even slabs, a workgroup computes all of a chunk (see plan_within).
 inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight_stages = 0)
 {
     if (B < 1 || H < 1 || Hk < 1 || H % Hk != 0 || Sq < 1 || Sk < 1 || D < 1 || k_past < 0) return false;
@@ -258,7 +258,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         p.r_line = line_of(qblk, p.n_qblk);
         p.r_unit = 1;
         const double all = stages_of(p.r_line, p.n_qblk) + (double)blocks * start;
-        const bool huge = all >= kMostPlaces || tight_stages > 0;
+        const bool huge = all >= kMostPlaces || tight_stages != 0;
         int seg = huge ? 0 : (int)(((int64_t)all + p.gen_blocks - 1) / p.gen_blocks);
         if (seg < kMinShare + start) seg = kMinShare + start;
         p.r_whole = p.r_one = 0;
@@ -270,7 +270,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
             const long per = (huge && p.r_line.step) ? 1 : (blocks + p.gen_blocks - 1) / p.gen_blocks;
             const int most = ceil_div(n, kMinShare);
             const long fit = p.gen_blocks / blocks;
-            const int parts = (per > 1 || fit < 2 || tight_stages > 0) ? 1 : (int)(fit < most ? fit : most);
+            const int parts = (per > 1 || fit < 2 || tight_stages != 0) ? 1 : (int)(fit < most ? fit : most);
             const int part = ceil_div(n, parts);
             // (row blocks that see different numbers of keys: parts of the longest one's length)
             if (huge || ((p.r_line.step == 0 || per == 1) && per * (part + start) <= best)) {
@@ -324,7 +324,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
             const int c = ceil_div(n, parts);
             if (ceil_div(n, c) != parts) continue;
             const long pieces = (long)B * parts * units;  // chunks of the units
-            const bool huge = all + (double)pieces * start >= kMostPlaces;
+            const bool huge = all + (double)pieces * start >= kMostPlaces || tight_stages < 0;
             if (!huge) {
                 StageLine l = stages;
                 l.start = start;
@@ -480,7 +480,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         bool any = false;
         for (int kg = (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {
             const int tpw = ceil_div(tiles, kg), nqblk = ceil_div(p.q_rows, 32 * (8 / kg));
-            if (kg > usual && (tight_stages > 0 || (long)B * H * nqblk > 2 * kComputeUnits)) break;
+            if (kg > usual && (tight_stages != 0 || (long)B * H * nqblk > 2 * kComputeUnits)) break;
             // Units per workgroup: a unit is one (query block, head); a workgroup takes f_rbpw adjacent
             // query blocks times f_hpg heads.  One workgroup is resident per compute unit, so the launch
             // runs in generations of kComputeUnits workgroups, each as long as its units plus about 0.7 of
@@ -539,32 +539,41 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // ---- workspace.  Its size must not depend on k_past (fcs_workspace_bytes does not know it), so the parts that the shares
     // need are sized for the most that any k_past gives: a workgroup leaves one set of row statistics per row block
     // that it touches (with a block that is cut, one more than the cuts), and one slab per chunk.
+    // A non-causal call has no k_past: what its own plan needs.
     const int64_t stages = ceil_div(Sk, kStageKeys);
     const int64_t row_blocks = (int64_t)B * p.v_heads * p.n_qblk, units = (int64_t)B * p.v_heads * p.c_nrb;
     const int64_t r_most = row_blocks * ceil_div((int)stages, kMinShare);
     const int64_t c_slots = (p.c_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
-    const int64_t chunk_most = tight_stages > 0 ? p.c_chunk / kStageKeys : col_chunk_max(p.Dp, p.c_waves) / kStageKeys;
+    const int64_t chunk_most = col_chunk_max(p.Dp, p.c_waves) / kStageKeys;
     const int64_t c_most = stages < chunk_most ? stages : chunk_most;
     const int64_t c_shares = units * ceil_div((int)stages, kMinShare);
-    const int64_t slab_stages = (c_slots < c_shares ? c_slots : c_shares) * c_most + B * (stages + c_most);
+    int64_t slab_stages = (c_slots < c_shares ? c_slots : c_shares) * c_most + B * (stages + c_most);
+    int64_t row_sets = r_most < p.gen_blocks ? r_most : p.gen_blocks;
+    if (!p.causal) {
+        slab_stages = p.c_direct ? 0 : ((int64_t)p.c_blocks + (int64_t)B * p.c_nchunks) * (p.c_chunk / kStageKeys);
+        row_sets = p.r_whole ? 0 : p.r_blocks;
+    }
     size_t off = 0;
     p.off_lse = off;
     off = align256(off + 2 * sizeof(float) * (size_t)B * p.v_heads * p.rows_pad);
     p.off_ml = off;
-    if (tight_stages == 0) off = align256(off + 2 * sizeof(float) * (size_t)qblk * (size_t)(r_most < p.gen_blocks ? r_most : p.gen_blocks));
+    off = align256(off + 2 * sizeof(float) * (size_t)qblk * (size_t)row_sets);
     p.off_partial = off;
-    if (tight_stages == 0 || !p.c_direct) off = align256(off + sizeof(float) * kStageKeys * (size_t)slab_stages);
+    off = align256(off + sizeof(float) * kStageKeys * (size_t)slab_stages);
     p.total = off;
     return true;
 }
 
-// The plan for a workspace of `bytes`: the usual one, or one that needs less.  False if none fits.
-inline bool plan_within(Plan &p, size_t bytes, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past)
+// The plan of a non-causal call for a workspace of `bytes`: the usual one, or one that needs less.  False if none fits, i.e. if the
+// row statistics alone (or the slabs of a single-kernel path) do not.
+inline bool plan_within(Plan &p, size_t bytes, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n)
 {
-    if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return false;
-    for (int stages = 32; p.total > bytes && stages >= 1; stages /= 2)
-        if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, stages)) return false;
-    return p.total <= bytes;
+    const int tight[] = {0, 32, 16, 8, 4, 2, 1, -1};
+    for (const int stages : tight) {
+        if (!make_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, stages)) return false;
+        if (p.total <= bytes) return true;
+    }
+    return false;
 }
 
 }  // namespace fcs

@@ -68,6 +68,25 @@ def test_rows_that_see_nothing_and_few_averaged_rows():
     _check(got, ref)
 
 
+def _static(q, k):
+    b, h, s, d = q.shape
+    out = torch.empty(b, s, device="cuda")
+    strides = (ctypes.c_int64 * 4)(*q.stride())
+    rc = _hip.lib().fcs_colsum_noncausal_f16_static(
+        ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(out.data_ptr()), None, b, h, s, d, strides, strides,
+        ctypes.c_float(d ** -0.5), -1, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    return out
+
+
+@pytest.mark.parametrize("b,h,s,d", [(352, 23, 27, 256), (568, 14, 2, 72), (172, 47, 13, 200)])
+def test_static_scratch_without_room_for_slabs(b, h, s, d):
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k = (torch.randn(b, h, s, d, generator=g, device="cuda").half() for _ in range(2))
+    out, usual = _static(q, k), flash_colsum_ext(q, k, is_causal=False, out_dtype=torch.float32)
+    assert ((out - usual).abs() <= 2e-6 * usual).all()  # the same terms in another grouping: up to 47 x 13 of them
+
+
 def test_static_scratch_lays_out_what_the_usual_plan_does_not_fit():
     """Accepted before the parts of row blocks had workspace of their own: 12 heads of 55565 keys."""
     b, h, s, d = 1, 12, 55565, 64
@@ -75,13 +94,7 @@ def test_static_scratch_lays_out_what_the_usual_plan_does_not_fit():
     g = torch.Generator(device="cuda").manual_seed(1)
     q = torch.randn(b, h, s, d, generator=g, device="cuda").half()
     k = torch.randn(b, h, s, d, generator=g, device="cuda").half()
-    out = torch.empty(b, s, device="cuda")
-    strides = (ctypes.c_int64 * 4)(*q.stride())
-    lib = _hip.lib()
-    torch.cuda.synchronize()
-    rc = lib.fcs_colsum_noncausal_f16_static(ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(out.data_ptr()), None, b, h, s, d,
-                                             strides, strides, ctypes.c_float(d ** -0.5), -1, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-    assert rc == 0
+    out = _static(q, k)
     usual = flash_colsum_ext(q, k, is_causal=False, out_dtype=torch.float32)
     assert ((out - usual).abs() <= 2e-6 * usual).all()  # the same terms in another grouping: 12 x 109 fp32 partial sums
 

@@ -28,14 +28,17 @@ static int seen(const Plan &p, int v1)
 }
 
 // 0: every stage is in exactly one share, and what the shares leave behind fits the workspace; else the check that failed
-extern "C" int check(int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, long *two_pass)
+extern "C" int check(int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight, long *two_pass)
 {
     Plan p;
     *two_pass = 0;
-    if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return 1;
+    if (!make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, tight)) return 1;
     if (p.fewrows || p.small || p.fused) return 0;
     *two_pass = 1;
     const long heads = (long)B * p.v_heads;
+    // the tightest layout: the row statistics alone
+    if (tight < 0 && (!p.c_direct || p.total != align256((size_t)8 * heads * p.rows_pad))) return 25;
+    if (tight > 0 && (!p.r_whole || p.c_chunk > std::min(tight, 32) * kStageKeys)) return 26;
 
     // pass 1
     const int rows1 = p.k1_waves * p.qw;
@@ -251,9 +254,9 @@ def check(tmp_path_factory):
     dll = ctypes.CDLL(str(lib))
     fn = dll.check
 
-    def call(causal, b, h, hk, sq, sk, d, cls_n, k_past):
+    def call(causal, b, h, hk, sq, sk, d, cls_n, k_past, tight=0):
         two_pass = ctypes.c_long()
-        return fn(int(causal), b, h, hk, sq, sk, d, cls_n, k_past, ctypes.byref(two_pass)), two_pass.value
+        return fn(int(causal), b, h, hk, sq, sk, d, cls_n, k_past, tight, ctypes.byref(two_pass)), two_pass.value
 
     call.dll = dll
     return call
@@ -279,7 +282,21 @@ def test_every_stage_is_in_one_share(check, seed):
         rc, two_pass = check(*s)
         assert rc == 0, (rc, s)
         n_two_pass += two_pass
+        if not s[0]:  # the layouts for a given workspace
+            for tight in (32, 16, 8, 4, 2, 1, -1):
+                assert check(*s[:3], s[2], *s[4:], tight)[0] == 0, (tight, s)
     assert n_two_pass > 100
+
+
+@pytest.mark.parametrize("b,h,s,d", [(352, 23, 27, 256), (446, 18, 12, 256), (157, 51, 17, 128), (568, 14, 2, 72), (467, 17, 1, 96), (172, 47, 13, 200),
+                                     (1, 12, 55565, 64), (64, 1, 16384, 256)])
+def test_static_scratch_takes_calls_whose_row_statistics_fit(b, h, s, d):
+    """8 MiB hold them in each of these; slabs beside them do not fit in most.  The size is looked at before the pointers."""
+    lib = _hip.lib()
+    rc = lib.fcs_colsum_noncausal_f16_static(None, None, None, None, b, h, s, d, None, None, ctypes.c_float(0.1), -1, None)
+    assert lib.fcs_strerror(rc) == b"a required pointer is NULL"
+    rc = lib.fcs_colsum_noncausal_f16_static(None, None, None, None, 2 * b, 2 * h, s, d, None, None, ctypes.c_float(0.1), -1, None)
+    assert b"static scratch" in lib.fcs_strerror(rc)
 
 
 def test_shares_of_uneven_row_blocks_are_equal():
