@@ -228,12 +228,11 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     p.rows_pad = p.n_qblk * qblk;
     // ---- the stages of a pass.  A causal row block ends at the last key that one of its rows sees; of a call with a
     // single row block per head (or rows laid end to end: every block holds a head's last row) that is the same for all.
-    const int seen_stages = ceil_div(seen_keys, kStageKeys);
-    const int whole_past = p.causal ? ceil_div(p.k_past < Sk ? p.k_past : Sk, kStageKeys) : 0;
-    auto line_of = [&](int rows, int blocks) {
-        if (!p.causal || p.fold > 1 || blocks == 1) return StageLine{seen_stages, 0, seen_stages, 0, 0};
+    const auto line_of = [&](int rows, int blocks, int past) {
+        const int seen = p.causal ? (int)((long)past + p.q_rows < Sk ? (long)past + p.q_rows : Sk) : Sk, n = ceil_div(seen, kStageKeys);
+        if (!p.causal || p.fold > 1 || blocks == 1) return StageLine{n, 0, n, 0, 0};
         const int step = rows / kStageKeys;  // 2, 4 or 8
-        return StageLine{whole_past, step, seen_stages, step == 8 ? 3 : step == 4 ? 2 : 1, 0};
+        return StageLine{ceil_div(past < Sk ? past : Sk, kStageKeys), step, n, step == 8 ? 3 : step == 4 ? 2 : 1, 0};
     };
     // One generation of workgroups: an 8-wave block fills a compute unit's registers, the 4-wave blocks fit twice
     // (256-wide heads: the kernels' registers and LDS allow one block per compute unit whatever its waves).
@@ -255,7 +254,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         const long blocks = (long)p.n_qblk * B * p.v_heads;
         if (blocks >= (1L << 31)) return false;
         const int start = start_places(p.Dp, p.qw);
-        p.r_line = line_of(qblk, p.n_qblk);
+        p.r_line = line_of(qblk, p.n_qblk, p.k_past);
         p.r_unit = 1;
         const double all = stages_of(p.r_line, p.n_qblk) + (double)blocks * start;
         const bool huge = all >= kMostPlaces || tight_stages != 0;
@@ -294,6 +293,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     }
 
     // ---- column pass (streaming kernel)
+    int64_t slab_stages = 0;  // what the call's slabs take of the workspace, in stages of 64 floats
     {
         if (block_rows > 256) { p.c_nb = 2; p.c_waves = 8; }
         else if (block_rows > 128) { p.c_nb = 2; p.c_waves = 4; }
@@ -306,44 +306,77 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         int most = col_chunk_max(p.Dp, p.c_waves) / kStageKeys;
         if (tight_stages > 0 && tight_stages < most) most = tight_stages;
         const long target = (p.c_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
-        const StageLine stages = line_of(rows, p.c_nrb);
-        const int n = seen_stages;
-        const double all = stages_of(stages, p.c_nrb);
-        // what the final reduction takes, in stages: a launch, and the slabs, written and read
-        const auto reduce = [&](long shares, int c) { return 2.5 + (double)shares * c * 1e-4; };
-        // Causal row blocks that see almost the same keys (the last rows of a long context) are quicker whole, four of one head
-        // re-reading its chunk, than in shares that straddle two heads at every workgroup (us per call, shares -> whole: H 8, Q 4096,
-        // K 65536, D 64 693 -> 653; H 32, Q 1500, K 32768, D 64 538 -> 496; H 4, Q 2048, K 65536, D 128 291 -> 279), up to
-        // about 3 % of the line's length (H 12, Q 4096, K 12288, D 128, where whole ones are 14 % longer: 280 in shares, 301).
-        const double uneven = stages.step ? 1.03 : 1.;
-        const int parts0 = ceil_div(n, most), parts_end = ceil_div(n, kMinShare);
-        int cs = 1, seg = 1;
-        enum { kShares, kUnits, kDirect } how = kDirect;
-        double best = 1e300;
-        for (int parts = parts0; parts <= parts_end && parts < parts0 + 128; ++parts) {
-            const int c = ceil_div(n, parts);
-            if (ceil_div(n, c) != parts) continue;
-            const long pieces = (long)B * parts * units;  // chunks of the units
-            const bool huge = all + (double)pieces * start >= kMostPlaces || tight_stages < 0;
-            if (!huge) {
-                StageLine l = stages;
-                l.start = start;
-                int sg = (int)(((int64_t)B * p.v_heads * l.chunk_places(p.c_nrb, c, parts) + target - 1) / target);
-                if (sg < kMinShare + start) sg = kMinShare + start;
-                const double cost = uneven * (sg + start) + reduce(target, c);
-                if (cost < best) { best = cost; cs = c; seg = sg; how = kShares; }
+        enum { kShares, kUnits, kDirect };
+        struct Split { int cs, seg, how; int64_t slabs; };
+        // the cheapest split of a line among those whose slabs take `room` stages at most
+        const auto cheapest = [&](const StageLine &stages, int64_t room) {
+            const int n = stages.last;
+            const double all = stages_of(stages, p.c_nrb);
+            // what the final reduction takes, in stages: a launch, and the slabs (one per workgroup and chunk that it touches), written
+            // and read.  (With the workgroups alone, calls of many batch entries got a slab per chunk where a workgroup per chunk is as
+            // fast without: B 594, H 2, S 189291, 1 row 436 MiB of them.)
+            const auto reduce = [&](long slabs, int c) { return 2.5 + (double)slabs * c * 1e-4; };
+            // Causal row blocks that see almost the same keys (the last rows of a long context) are quicker whole, four of one head
+            // re-reading its chunk, than in shares that straddle two heads at every workgroup (us per call, shares -> whole: H 8, Q 4096,
+            // K 65536, D 64 693 -> 653; H 32, Q 1500, K 32768, D 64 538 -> 496; H 4, Q 2048, K 65536, D 128 291 -> 279), up to
+            // about 3 % of the line's length (H 12, Q 4096, K 12288, D 128, where whole ones are 14 % longer: 280 in shares, 301).
+            const double uneven = stages.step ? 1.03 : 1.;
+            const int parts0 = ceil_div(n, most), parts_end = ceil_div(n, kMinShare);
+            Split s{1, 1, kDirect, 0};
+            double best = 1e300;
+            for (int parts = parts0; parts <= parts_end && parts < parts0 + 128; ++parts) {
+                const int c = ceil_div(n, parts);
+                if (ceil_div(n, c) != parts) continue;
+                const long pieces = (long)B * parts * units;  // chunks of the units
+                const bool huge = all + (double)pieces * start >= kMostPlaces || tight_stages < 0;
+                const auto slabs = [&](long shares) { return (shares + (int64_t)B * ceil_div(Sk, c * kStageKeys)) * c; };
+                if (!huge) {
+                    StageLine l = stages;
+                    l.start = start;
+                    const int64_t len = (int64_t)B * p.v_heads * l.chunk_places(p.c_nrb, c, parts);
+                    int sg = (int)((len + target - 1) / target);
+                    if (sg < kMinShare + start) sg = kMinShare + start;
+                    const int64_t need = slabs((len + sg - 1) / sg);
+                    const double cost = uneven * (sg + start) + reduce(target + (long)B * parts, c);
+                    if (cost < best && need <= room) { best = cost; s = Split{c, sg, kShares, need}; }
+                }
+                // whole ones per workgroup, priced as if all were as long as the longest
+                const long per = (pieces + target - 1) / target;
+                if (!huge) {
+                    const int64_t need = slabs((pieces + per - 1) / per);
+                    const double cost = (double)per * (c + start) + reduce(pieces / per + (units % per ? (long)B * parts : 0), c);
+                    if (cost < best && need <= room) { best = cost; s = Split{c, (int)per, kUnits, need}; }
+                }
+                // a workgroup per chunk, which writes the means itself: no slabs, no final reduction
+                const double cost = (double)((B * (long)parts + target - 1) / target) * (double)units * (c + start);
+                if (cost <= best) { best = cost; s = Split{c, 1, kDirect, 0}; }
+                if (pieces > 4 * target && parts > parts0 + 8) break;
             }
-            // whole ones per workgroup, priced as if all were as long as the longest
-            const long per = (pieces + target - 1) / target;
-            if (!huge) {
-                const double cost = (double)per * (c + start) + reduce(pieces / per, c);
-                if (cost < best) { best = cost; cs = c; seg = (int)per; how = kUnits; }
-            }
-            // a workgroup per chunk, which writes the means itself: no slabs, no final reduction
-            const double cost = (double)((B * (long)parts + target - 1) / target) * (double)units * (c + start);
-            if (cost <= best) { best = cost; cs = c; how = kDirect; }
-            if (pieces > 4 * target && parts > parts0 + 8) break;
+            return s;
+        };
+        const StageLine stages = line_of(rows, p.c_nrb, p.k_past);
+        Split split;
+        if (!p.causal) {
+            split = cheapest(stages, INT64_MAX);
+            slab_stages = split.slabs;
+        } else {
+            // The workspace's size must not depend on k_past (fcs_workspace_bytes does not know it).  There is room for what the call takes
+            // with the usual k_past and with every key visible, and for slabs of up to 8 MiB if one for each chunk fits in there; with
+            // another k_past it is split so that it fits.
+            const auto same = [](const StageLine &a, const StageLine &b) { return a.first == b.first && a.step == b.step && a.last == b.last; };
+            const StageLine usual = line_of(rows, p.c_nrb, Sk > Sq ? Sk - Sq : 0), whole = line_of(rows, p.c_nrb, Sk);
+            const Split of_usual = cheapest(usual, INT64_MAX), of_whole = same(usual, whole) ? of_usual : cheapest(whole, INT64_MAX);
+            const int64_t all_stages = ceil_div(Sk, kStageKeys), c_most = all_stages < most ? all_stages : most;
+            const int64_t shares = B * units * ceil_div((int)all_stages, kMinShare);
+            slab_stages = (target < shares ? target : shares) * c_most + B * (all_stages + c_most);  // the most that any k_past takes
+            const int64_t small = (8 << 20) / (int64_t)(sizeof(float) * kStageKeys);
+            if (slab_stages > small) slab_stages = B * all_stages <= small ? small : 0;
+            if (slab_stages < of_usual.slabs) slab_stages = of_usual.slabs;
+            if (slab_stages < of_whole.slabs) slab_stages = of_whole.slabs;
+            split = same(stages, usual) ? of_usual : same(stages, whole) ? of_whole : cheapest(stages, slab_stages);
         }
+        const int n = stages.last, cs = split.cs, how = split.how;
+        int seg = split.seg;
         const int used = ceil_div(n, cs);  // chunks that some row sees
         p.c_chunk = cs * kStageKeys;
         p.c_nchunks = ceil_div(Sk, p.c_chunk);
@@ -536,23 +569,10 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         return (long)p.f_nwgq * B * p.f_hg < (1L << 31);
     }
 
-    // ---- workspace.  Its size must not depend on k_past (fcs_workspace_bytes does not know it), so the parts that the shares
-    // need are sized for the most that any k_past gives: a workgroup leaves one set of row statistics per row block
-    // that it touches (with a block that is cut, one more than the cuts), and one slab per chunk.
-    // A non-causal call has no k_past: what its own plan needs.
-    const int64_t stages = ceil_div(Sk, kStageKeys);
-    const int64_t row_blocks = (int64_t)B * p.v_heads * p.n_qblk, units = (int64_t)B * p.v_heads * p.c_nrb;
-    const int64_t r_most = row_blocks * ceil_div((int)stages, kMinShare);
-    const int64_t c_slots = (p.c_waves == 8 || p.Dp == 256) ? kComputeUnits : 2 * kComputeUnits;
-    const int64_t chunk_most = col_chunk_max(p.Dp, p.c_waves) / kStageKeys;
-    const int64_t c_most = stages < chunk_most ? stages : chunk_most;
-    const int64_t c_shares = units * ceil_div((int)stages, kMinShare);
-    int64_t slab_stages = (c_slots < c_shares ? c_slots : c_shares) * c_most + B * (stages + c_most);
-    int64_t row_sets = r_most < p.gen_blocks ? r_most : p.gen_blocks;
-    if (!p.causal) {
-        slab_stages = p.c_direct ? 0 : ((int64_t)p.c_blocks + (int64_t)B * p.c_nchunks) * (p.c_chunk / kStageKeys);
-        row_sets = p.r_whole ? 0 : p.r_blocks;
-    }
+    // ---- workspace.  A causal call's parts of row blocks, too, are given room for the most that any k_past leaves: a workgroup
+    // leaves one set of row statistics per row block that it touches (with a block that is cut, one more than the cuts).
+    const int64_t r_most = (int64_t)B * p.v_heads * p.n_qblk * ceil_div(ceil_div(Sk, kStageKeys), kMinShare);
+    const int64_t row_sets = p.causal ? (r_most < p.gen_blocks ? r_most : p.gen_blocks) : p.r_whole ? 0 : p.r_blocks;
     size_t off = 0;
     p.off_lse = off;
     off = align256(off + 2 * sizeof(float) * (size_t)B * p.v_heads * p.rows_pad);
