@@ -95,6 +95,7 @@ __device__ __forceinline__ int row_swizzle(int row)
 
 // source of the 16-byte pieces that lie past the tensor's head dim (kernels compiled for a wider head)
 __device__ unsigned int g_zero_piece[4];
+constexpr uint32_t kPastDim = 0xffffffffu;  // in the place of such a piece's offset
 
 // FOLD: the rows of a unit are those of ALL query heads that share a key head, laid end to end: row v of key head hk
 // is row v % q_rows of query head hk * fold + v / q_rows.  v / q_rows through a multiply-high; fold_magic is
@@ -338,7 +339,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
     for (int j = 0; j < IPW; ++j) {
         const int P = (wave * IPW + j) * 64 + lane;
         const int row = P / PPR, pos = P % PPR;
-        g_off[j] = (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)((pos ^ row_swizzle<D>(row)) * 16);
+        const int piece = pos ^ row_swizzle<D>(row);
+        g_off[j] = (D < 256 || piece * 8 < a.D) ? (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)(piece * 16) : kPastDim;
     }
     char *ring_w = ring + wave * (IPW * 1024);  // where this wave's pieces of a stage land inside a slot
     // operand read-back: lane (n, g) takes, for MFMA step t, piece piece_of(t, g) of row n (+ 32 per key fragment)
@@ -471,9 +473,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         auto fetch_stage = [&](int st, int slot) __attribute__((always_inline)) {
             if (__builtin_expect(st < n_whole, 1)) {
                 fetch_whole(slot);
+                return;
+            }
+            const int kb = c0 + st * KT;
+            char *dst = ring_w + slot * STAGE_BYTES;
+            if (D == 256 && kb + KT <= a.Sk) {  // narrower rows, as in the row pass (the smaller kernels are no faster with it)
+                const char *base = kp + kb * k_row_b;
+#pragma unroll
+                for (int j = 0; j < IPW; ++j) dma16(g_off[j] == kPastDim ? reinterpret_cast<const char *>(g_zero_piece) : base + g_off[j], dst + j * 1024);
             } else {  // rows past the last key re-read it (the consumer masks them), pieces past the head dim are zeros
-                const int kb = c0 + st * KT;
-                char *dst = ring_w + slot * STAGE_BYTES;
                 int lane_o = lane;
                 asm volatile("" : "+v"(lane_o));  // formed here, not kept in registers through the stream
 #pragma unroll
@@ -997,7 +1005,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     for (int j = 0; j < IPW; ++j) {
         const int P = (wave * IPW + j) * 64 + lane;
         const int row = P / PPR, pos = P % PPR;
-        g_off[j] = (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)((pos ^ row_swizzle<D>(row)) * 16);
+        const int piece = pos ^ row_swizzle<D>(row);
+        g_off[j] = (piece * 8 < a.D) ? (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)(piece * 16) : kPastDim;
     }
     char *ring_w = ring + wave * (IPW * 1024);
     uint32_t take[NTA];
@@ -1076,9 +1085,17 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     auto fetch_stage = [&](int st, int slot) __attribute__((always_inline)) {
         if (__builtin_expect(st < n_whole, 1)) {
             fetch_whole(slot);
+            return;
+        }
+        const int kb = kc0 + st * KT;
+        char *dst = ring_w + slot * STAGE_BYTES;
+        // Narrower rows: zeros past their end, nothing but the base formed anew.  (Every piece's row and channel formed for each
+        // stage: B 16, H 8, S 4096, D 96 584 us against 556, B 8, S 2048, D 200 245 against 207.)
+        if (kb + KT <= a.Sk) {
+            const char *base = kp + kb * k_row_b;
+#pragma unroll
+            for (int j = 0; j < IPW; ++j) dma16(g_off[j] == kPastDim ? reinterpret_cast<const char *>(g_zero_piece) : base + g_off[j], dst + j * 1024);
         } else {  // rows past the last key re-read it (the consumer masks them), pieces past the head dim are zeros
-            const int kb = kc0 + st * KT;
-            char *dst = ring_w + slot * STAGE_BYTES;
             int lane_o = lane;
             asm volatile("" : "+v"(lane_o));  // formed here, not kept in registers through the stream
 #pragma unroll

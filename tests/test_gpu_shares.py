@@ -113,3 +113,17 @@ def test_scale_next_to_zero_on_scores_next_to_the_largest():
     got, ref, _, _ = _call(1, 4, 4, 40, 4096, 64, torch.bfloat16, True, scale=2.0 ** -125, prepare=lambda q, k: (q.mul_(2.0 ** 61), k.mul_(2.0 ** 60)))
     assert ref.max() / ref.median() > 1.1
     _check(got, ref)
+
+
+@pytest.mark.parametrize("d", [8, 40, 56, 72, 96, 120, 136, 200, 248])
+@pytest.mark.parametrize("causal", [True, False])
+def test_channels_past_the_head_dim_are_not_read(d, causal):
+    """Heads narrower than the kernels are compiled for, in rows that go on with NaN: whole key stages and the last one."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    wide = [torch.full((2, 3, s, 256), float("nan"), device="cuda", dtype=torch.float16) for s in (700, 2900 if not causal else 1000)]
+    q, k = (w[..., :d] for w in wide)
+    for t in (q, k):
+        t.copy_(torch.randn(t.shape, generator=g, device="cuda"))
+    print((d, causal), flush=True)
+    got = flash_colsum_ext(q, k, is_causal=causal, out_dtype=torch.float32)
+    _check(got, colsum_ext_exact(q.contiguous(), k.contiguous(), is_causal=causal))
