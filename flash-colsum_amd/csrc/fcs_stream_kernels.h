@@ -979,6 +979,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
     constexpr int NS = row_ring_slots(D, WAVES);
     static_assert(IPW >= 1 && KT * PPR == IPW * THREADS, "a stage is a whole number of DMA instructions per wave");
     static_assert(NS >= 3 && NS <= 4, "ring depth");
+    constexpr bool NARROW = D > 64 && !FOLD;  // stages of rows narrower than compiled have a path of their own
     __shared__ __attribute__((aligned(16))) char ring[NS * STAGE_BYTES];
     __shared__ __attribute__((aligned(16))) float mrow[BLOCK_ROWS];      // row maxima of the stabilised sweeps
     __shared__ int bad_s[WAVES];
@@ -1006,7 +1007,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         const int P = (wave * IPW + j) * 64 + lane;
         const int row = P / PPR, pos = P % PPR;
         const int piece = pos ^ row_swizzle<D>(row);
-        g_off[j] = (piece * 8 < a.D) ? (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)(piece * 16) : kPastDim;
+        g_off[j] = (!NARROW || piece * 8 < a.D) ? (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)(piece * 16) : kPastDim;
     }
     char *ring_w = ring + wave * (IPW * 1024);
     uint32_t take[NTA];
@@ -1090,8 +1091,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_rowstream_kernel(const Args
         const int kb = kc0 + st * KT;
         char *dst = ring_w + slot * STAGE_BYTES;
         // Narrower rows: zeros past their end, nothing but the base formed anew.  (Every piece's row and channel formed for each
-        // stage: B 16, H 8, S 4096, D 96 584 us against 556, B 8, S 2048, D 200 245 against 207.)
-        if (kb + KT <= a.Sk) {
+        // stage: B 16, H 8, S 4096, D 96 584 us against 556, B 8, S 2048, D 200 245 against 207.  Not for rows laid end to end, whose
+        // kernels are out of scalar registers: B 4, 32 on 8 heads, Q 64, K 8192, D 128 with the selection 60.3 -> 61.1.)
+        if (NARROW && kb + KT <= a.Sk) {
             const char *base = kp + kb * k_row_b;
 #pragma unroll
             for (int j = 0; j < IPW; ++j) dma16(g_off[j] == kPastDim ? reinterpret_cast<const char *>(g_zero_piece) : base + g_off[j], dst + j * 1024);
