@@ -174,7 +174,7 @@ size_t describe_fewrows(const Plan &p, const Args &a, char *buf, size_t n)
                            p.bf16 ? "true" : "false", p.B * p.f_hg, p.f_hpg, p.n_partials);
     if (r < 0) return 0;
     const size_t len = (size_t)r;
-    return len + describe_finalize(a, len < n ? buf + len : nullptr, len < n ? n - len : 0);
+    return len + describe_finalize(a, false, len < n ? buf + len : nullptr, len < n ? n - len : 0);
 }
 
 }  // namespace fcs

@@ -907,7 +907,7 @@ size_t describe_fused(const Plan &p, const Args &a, char *buf, size_t n)
                      p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
     if (r < 0) return 0;
     const size_t len = (size_t)r;
-    return len + describe_finalize(a, len < n ? buf + len : nullptr, len < n ? n - len : 0);
+    return len + describe_finalize(a, false, len < n ? buf + len : nullptr, len < n ? n - len : 0);
 }
 
 template <bool BF>

@@ -90,6 +90,6 @@ size_t describe_fused(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_fewrows(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_small(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_two_pass(const Plan &p, const Args &a, char *buf, size_t n);
-size_t describe_finalize(const Args &a, char *buf, size_t n);
+size_t describe_finalize(const Args &a, bool shares, char *buf, size_t n);
 
 }  // namespace fcs

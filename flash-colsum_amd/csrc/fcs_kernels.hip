@@ -100,9 +100,9 @@ static hipError_t launch_finalize_t(const Args &a, hipStream_t st)
 
 hipError_t launch_finalize(const Args &a, hipStream_t st) { return launch_finalize_t<false>(a, st); }
 
-size_t describe_finalize(const Args &a, char *buf, size_t n)
+size_t describe_finalize(const Args &a, bool shares, char *buf, size_t n)
 {
-    const int r = snprintf(buf, n, " + fcs_finalize_kernel<%d> grid %lld", slab_lanes(a.n_partials),
+    const int r = snprintf(buf, n, " + fcs_finalize_kernel<%d%s> grid %lld", slab_lanes(a.n_partials), shares ? ",true" : "",
                            (long long)(((int64_t)a.B * a.Sk + 31) / 32));
     return r < 0 ? 0 : (size_t)r;
 }

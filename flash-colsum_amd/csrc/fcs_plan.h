@@ -135,7 +135,6 @@ struct Plan {
     int r_whole;     // every row block lies within one share
     int r_one;       // every share is one (part of a) row block
     FastDiv r_by_seg, r_by_head, r_by_block, by_heads;  // divisions by r_seg, a head's units, a row block's (step 0), v_heads
-    int n_chunks;    // shares per row block, rounded down
     // column pass: the same over (batch entry, key chunk, head, row block); a (head, row block) is a unit of the chunk, whose
     // column sums a block keeps in LDS
     int c_nb, c_waves; // 32-row fragments per wave, waves per block: a unit has 32 * c_nb * c_waves rows
@@ -149,7 +148,6 @@ struct Plan {
     FastDiv c_by_seg, c_by_batch, c_by_chunk, c_by_blocks;  // divisions by c_seg, a batch entry's units, c_chunk, c_nrb
     FastDiv c_by_chunks;  // by c_nchunks (c_direct), the chunks that some row sees (c_unit > 1 or c_one), or the places of a
                           // chunk that all row blocks see to its end
-    int c_groups;      // slabs per chunk, rounded down (1: none)
     // fused single-kernel path: non-causal, all keys of a row block fit in one
     // workgroup's registers.  grid = (f_nwgq * B, f_hg)
     int fewrows;     // 1: few-rows path (non-causal, q_rows <= 4): grid = B * f_hg, slabs = f_hg
@@ -285,7 +283,6 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         if (seg > p.r_len) seg = p.r_len;
         p.r_seg = seg;
         p.r_blocks = ceil_div(p.r_len, seg);
-        p.n_chunks = (!p.r_whole && p.r_blocks / blocks > 1) ? (int)(p.r_blocks / blocks) : 1;
         p.r_by_seg.set(seg);
         p.r_by_head.set(p.r_line.places(p.n_qblk));
         p.r_by_block.set(p.r_line.last + p.r_line.start);
@@ -394,7 +391,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         p.c_direct = how == kDirect;
         p.c_one = how == kUnits && seg == 1;
         p.c_by_blocks.set(p.c_nrb);
-        p.c_len = p.c_seg = p.c_groups = p.n_partials = 1;
+        p.c_len = p.c_seg = p.n_partials = 1;
         p.c_blocks = (int)chunks;
         p.c_by_batch.set(1);
         if (how != kDirect) {
@@ -403,7 +400,6 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
             if (seg > p.c_len) seg = p.c_len;
             p.c_seg = seg;
             p.c_blocks = ceil_div(p.c_len, seg);
-            p.c_groups = (int)(1 + p.c_blocks / chunks);
             p.n_partials = p.v_heads * p.c_line.chunk_places(p.c_nrb, p.c_cs, 1) / seg + 2;  // of the first chunk, the most seen
             p.c_by_batch.set(per_batch);
         }

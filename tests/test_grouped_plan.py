@@ -14,7 +14,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 _SOURCE = """
 #include "fcs_plan.h"
-// out: fold, total, bytes of the row statistics, of the key splits' statistics, of the column slabs and their offsets
+// out: fold, total, where the row statistics and the column slabs begin and where the last one written ends
 extern "C" int plan(int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, long *out)
 {
     fcs::Plan p;
@@ -22,10 +22,10 @@ extern "C" int plan(int causal, int B, int H, int Hk, int Sq, int Sk, int D, int
     const bool two_pass = !(p.fewrows || p.small || p.fused);
     out[0] = p.fold;
     out[1] = (long)p.total;
-    out[2] = two_pass ? 8L * B * p.v_heads * p.rows_pad : 0;
-    out[3] = two_pass && p.n_chunks > 1 ? 8L * B * p.v_heads * p.n_chunks * p.rows_pad : 0;
-    out[4] = 4L * (two_pass ? (p.c_groups > 1 ? p.c_groups : 0) : p.n_partials) * B * Sk;
-    out[5] = (long)p.off_lse; out[6] = (long)p.off_ml; out[7] = (long)p.off_partial;
+    const long blocks = (long)B * p.v_heads * p.n_qblk;
+    out[2] = (long)p.off_lse; out[3] = (long)p.off_partial;
+    out[4] = out[2] + (two_pass ? 8L * p.k1_waves * p.qw * (blocks + (p.r_whole ? 0 : p.r_blocks - 1)) : 0);
+    out[5] = out[3] + 4L * (!two_pass ? (long)p.n_partials * B * Sk : p.c_direct ? 0 : ((long)p.c_blocks + (long)B * p.c_nchunks - 1) * p.c_chunk);
     return 1;
 }
 """
@@ -40,9 +40,9 @@ def plan(tmp_path_factory):
     fn = ctypes.CDLL(str(lib)).plan
 
     def call(causal, b, h, hk, sq, sk, d, cls_n=-1, k_past=None):
-        out = (ctypes.c_long * 8)()
+        out = (ctypes.c_long * 6)()
         ok = fn(int(causal), b, h, hk, sq, sk, d, cls_n, (max(0, sk - sq) if k_past is None else k_past) if causal else 0, out)
-        return dict(zip(("fold", "total", "lse", "ml", "slabs", "off_lse", "off_ml", "off_slabs"), out)) if ok else None
+        return dict(zip(("fold", "total", "stats", "slabs", "stats_end", "slabs_end"), out)) if ok else None
 
     return call
 
@@ -51,9 +51,9 @@ def test_grouped_rows_fill_row_blocks():
     d = _hip.plan_description
     # 4 query heads x 64 rows per key head: one block of 256 rows instead of four of 128 half empty ones
     t = d((4, 32, 64, 128), (4, 8, 8192, 128), causal=True, bf16=True)
-    assert "fcs_rowstream_kernel<128,2,4,true,false,true> grid 1 x 16 x 32" in t and "fcs_colstream_kernel<128,2,4,true,false,true>" in t, t
+    assert "fcs_rowstream_kernel<128,2,4,true,false,true> grid 512, shares of 8 places, one piece each" in t and "fcs_colstream_kernel<128,2,4,true,false,true>" in t, t
     # full blocks of 512 rows, and ungrouped heads, stay head by head
-    assert "fcs_rowstream_kernel<128,2,8,false,false> grid 1 x" in d((1, 32, 512, 128), (1, 8, 8192, 128), causal=True)
+    assert "fcs_rowstream_kernel<128,2,8,false,false> grid 256, " in d((1, 32, 512, 128), (1, 8, 8192, 128), causal=True)
     assert "fcs_rowstream_kernel<128,1,4,false,false> " in d((1, 8, 64, 128), (1, 8, 8192, 128), causal=True)
     # the single-pass kernels are unchanged by grouping
     assert d((2, 8, 577, 64), (2, 2, 577, 64)) == d((2, 8, 577, 64), (2, 8, 577, 64))
@@ -100,7 +100,6 @@ def test_workspace_serves_every_number_of_key_heads(plan):
                 assert p["total"] <= n, (causal, b, h, hk, sq, sk, d, k_past)
                 grouped_needs_more += p["total"] > alone
                 # the parts lie one behind the other inside the total, each 256-byte aligned
-                ends = [p["off_lse"] + p["lse"], p["off_ml"] + p["ml"], p["off_slabs"] + p["slabs"]]
-                assert all(p[o] % 256 == 0 for o in ("off_lse", "off_ml", "off_slabs")) and max(ends) <= p["total"]
-                assert not p["lse"] or (ends[0] <= p["off_ml"] and ends[1] <= p["off_slabs"])
+                assert p["stats"] % 256 == 0 and p["slabs"] % 256 == 0
+                assert p["stats"] <= p["stats_end"] <= p["slabs"] <= p["slabs_end"] <= p["total"]
     assert grouped_needs_more > 0  # else the shapes above would not show a bound that forgets the grouped layouts

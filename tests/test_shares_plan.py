@@ -302,7 +302,7 @@ def test_static_scratch_takes_calls_whose_row_statistics_fit(b, h, s, d):
 def test_shares_of_uneven_row_blocks_are_equal():
     """The triangle of a prompt against itself: 32 heads x (8 + 16 + .. + 64) stages over 256 workgroups."""
     t = _hip.plan_description((1, 32, 4096, 128), (1, 32, 4096, 128), causal=True)
-    assert "256 shares of 38 places + " in t and "grid 256, shares of 39 places" in t, t
+    assert "grid 256, shares of 38 places + " in t and "grid 256, shares of 39 places" in t, t
 
 
 @pytest.mark.parametrize("h,q_len,k_len,d,places", [(8, 4096, 65536, 64, 256), (4, 2048, 65536, 128, 64), (16, 2048, 32768, 64, 128), (12, 1000, 65536, 128, 96)])
@@ -327,5 +327,5 @@ def test_long_lines_have_equal_shares(check, h, q_len, k_len, d):
 def test_lines_beyond_the_limit_are_handed_out_by_the_hardware(check):
     """4.3e9 places: a workgroup per row block of uneven ones, which the hardware starts one after the other."""
     t = _hip.plan_description((1, 64, 1 << 21, 128), (1, 64, 1 << 21, 128), causal=True)
-    assert f"{64 * 4096} shares of {1 << 15} places" in t and "direct" in t, t
+    assert f"grid {64 * 4096}, shares of {1 << 15} places, one piece each" in t and "direct" in t, t
     assert check(True, 1, 64, 64, 1 << 17, 1 << 17, 64, -1, 0)[0] == 0
