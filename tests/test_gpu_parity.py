@@ -278,7 +278,8 @@ def test_prescaled_shared_q_variant(shape, same, kw, boost):
 @pytest.mark.parametrize("qs,ks,kw,same,boost", [
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {}, False, 0.0),                        # non-causal, keys split in pass 1
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {"scale": -0.125}, False, 0.0),         # the sign rides on the operand
-    ((2, 8, 2100, 64), (2, 8, 2100, 64), {}, False, 0.0),                        # ragged, just past 2048 keys
+    ((2, 8, 2100, 64), (2, 8, 2100, 64), {}, False, 0.0),                        # up to 2560 keys: the single-pass kernel, on the operand as it is
+    ((2, 8, 2600, 64), (2, 8, 2600, 64), {}, False, 0.0),                        # ragged
     ((1, 16, 700, 64), (1, 16, 5000, 64), {"is_causal": True}, False, 0.0),      # causal, 11200 pairs: the exact variant
     ((1, 16, 1100, 64), (1, 16, 5000, 64), {"is_causal": True}, False, 0.0),     # causal, 17600 pairs: pre-scaled below key 3840
     ((1, 16, 1100, 64), (1, 16, 5000, 64), {"is_causal": True}, False, 6.0),     # ... with rows that leave the 2^20 range
@@ -292,7 +293,8 @@ def test_prescaled_shared_q_variant(shape, same, kw, boost):
     ((1, 4, 3000, 64), (1, 4, 3000, 64), {"cls_len": 1500}, False, 0.0),         # 6000 averaged pairs: the exact variant
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {}, False, 6.0),                        # some rows leave the 2^20 range: raw-operand sweeps
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {}, True, 40.0),                        # ... far out, Q == K
-    ((3, 8, 2304, 64), (3, 8, 2304, 64), {}, False, 8.0),                        # ... batched
+    ((3, 8, 2304, 64), (3, 8, 2304, 64), {}, False, 8.0),                        # (single pass)
+    ((3, 8, 2816, 64), (3, 8, 2816, 64), {}, False, 8.0),                        # ... batched
     ((1, 4, 4096, 64), (1, 4, 4096, 64), {"scale": 0.2}, False, 0.0),            # scale above 1/8: the exact variant
     ((1, 2, 4096, 64), (1, 2, 4096, 64), {}, False, 0.0),                        # fewer than 16384 pairs: the exact variant
 ])
