@@ -340,7 +340,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         const int P = (wave * IPW + j) * 64 + lane;
         const int row = P / PPR, pos = P % PPR;
         const int piece = pos ^ row_swizzle<D>(row);
-        g_off[j] = (D < 256 || piece * 8 < a.D) ? (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)(piece * 16) : kPastDim;
+        g_off[j] = (D == 128 || piece * 8 < a.D) ? (uint32_t)row * (uint32_t)(a.ks_s * 2) + (uint32_t)(piece * 16) : kPastDim;
     }
     char *ring_w = ring + wave * (IPW * 1024);  // where this wave's pieces of a stage land inside a slot
     // operand read-back: lane (n, g) takes, for MFMA step t, piece piece_of(t, g) of row n (+ 32 per key fragment)
@@ -421,7 +421,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             if constexpr (ONE) break;
             else continue;
         }
-        const int n_whole = (a.D == D) ? min(nst, (a.Sk - c0) / KT) : 0;  // stages inside the tensor, of rows as wide as compiled
+        const int n_whole = (D == 64 || a.D == D) ? min(nst, (a.Sk - c0) / KT) : 0;  // stages inside the tensor, of rows as wide as compiled (64: or not)
         if constexpr (!ONE) {  // what derives from these is formed anew, not kept from unit to unit
 #pragma unroll
             for (int t = 0; t < NTA; ++t) asm volatile("" : "+v"(take[t]));
@@ -464,10 +464,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         // stage `st` of the unit into ring slot `slot`
         // The stages of a stream are requested in order; k_src is where the next one starts.
         const char *k_src;
-        auto fetch_whole = [&](int slot) __attribute__((always_inline)) {  // a stage inside the tensor, of rows as wide as compiled
+        auto fetch_whole = [&](int slot) __attribute__((always_inline)) {  // such a stage
             char *dst = ring_w + slot * STAGE_BYTES;
+            if (D != 64 || __builtin_expect(a.D == D, 1)) {
 #pragma unroll
-            for (int j = 0; j < IPW; ++j) dma16(k_src + g_off[j], dst + j * 1024);
+                for (int j = 0; j < IPW; ++j) dma16(k_src + g_off[j], dst + j * 1024);
+            } else {
+#pragma unroll
+                for (int j = 0; j < IPW; ++j) dma16(g_off[j] == kPastDim ? reinterpret_cast<const char *>(g_zero_piece) : k_src + g_off[j], dst + j * 1024);
+            }
             k_src += KT * k_row_b;
         };
         auto fetch_stage = [&](int st, int slot) __attribute__((always_inline)) {
