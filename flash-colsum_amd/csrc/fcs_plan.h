@@ -485,8 +485,8 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     const bool narrow128 = D > 64 && D < 128;
     // (64-wide heads: the shared-Q variants hold ten tiles per wave, so calls of up to 2560 keys are served too, unless grouped
     // heads are laid end to end, whose keys are streamed once for the whole group.  us per call, two passes -> here:
-    // B 1 H 16 S 2500 47.9 -> 32.4, B 4 H 16 S 2300 212.8 -> 83.9, H 1 S 2500 14.6 -> 10.6, 5 averaged rows of B 8 H 16
-    // S 2300 30.2 -> 12.8, 128 of them 29.9 -> 17.2; no size in between was slower.)
+    // B 1 H 16 S 2500 47.9 -> 33.5, B 4 H 16 S 2300 212.8 -> 88.0, H 1 S 2500 14.6 -> 10.9, 5 averaged rows of B 8 H 16
+    // S 2300 30.2 -> 12.1, 128 of them 29.9 -> 18.5; no size in between was slower.)
     const bool wide = D == 64 && tight_stages == 0;
     const int fused_max = narrow128 ? 8 * 6 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
     if (!causal && Sk >= 32 && Sk <= fused_max && D <= 128) {

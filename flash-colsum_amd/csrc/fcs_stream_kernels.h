@@ -46,7 +46,9 @@
 // call): causal H 32, S 4096, D 128 bf16 229 -> 163; H 12, S 5242, D 64 178 -> 124; H 12, S 4491, D 64 bf16 146 -> 102;
 // H 16, S 9459, D 64 571 -> 467; H 8, S 4435, D 128 bf16 causal 97 -> 69.  Where whole units of one length fill
 // the chip evenly the plan keeps to them, one to a workgroup (ONE: the walk and its state are compiled out; a small call spends
-// half its time before the first stage, and cold instructions are a good part of that: H 8, S 2219, D 64 18.2 -> 16.3 us).
+// half its time before the first stage, and cold instructions are a good part of that).  us per call, the same shares with the
+// walk -> without: causal H 32, Q 128, K 4096, D 128 29.1 -> 22.9, K 16384 60.1 -> 57.6; H 32, S 634 30.8 -> 25.7; H 8, Q 512,
+// K 4096, D 256 35.1 -> 31.0; H 16, S 4096, D 64 90.9 -> 86.7; 32 on 8 heads laid end to end, Q 64, K 8192 53.3 -> 53.1.
 // At a unit's start the first stages, the row statistics and the query rows are requested together, and nothing is
 // requested past a unit's last stage.  Causal alignment  j <= k_past + i  (reference:
 // flash_colsum/kernel_causal.py:39,57,113): the stage loop stops at the last key any row of the
