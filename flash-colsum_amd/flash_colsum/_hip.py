@@ -178,8 +178,12 @@ _WS_MAX_ENTRIES = 16
 _CALLS_MAX_ENTRIES = 256
 
 
+# (asked on every call, without the Python frame around it: B 2, H 4, S 512, D 64 11.1 -> 10.4 us per call, median of ten processes)
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None) or torch.cuda.is_current_stream_capturing
+
+
 def _workspace(device: torch.device, stream: int, n_bytes: int) -> torch.Tensor:
-    if n_bytes > _WS_MAX_CACHED_BYTES or torch.cuda.is_current_stream_capturing():
+    if n_bytes > _WS_MAX_CACHED_BYTES or _capturing():
         return torch.empty((max(n_bytes, 256),), dtype=torch.uint8, device=device)
     cache = getattr(_tls, "workspaces", None)
     if cache is None:
@@ -322,7 +326,7 @@ def _repeated_rounded(key, ent, q, k, q_ptr, k_ptr, index):
     """The route of `_rounded_operands`, both rounded operands in one allocation; None for the full path.  Operands beyond
     the range go on from there, and their geometry is forgotten: the next call may be as they are."""
     c, c_ref, n_ws, shape, f16, n_q, n_k = ent
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing():
         return None
     dev = q.device
     at_k = (2 * n_q + 255) & ~255
@@ -368,7 +372,7 @@ def _wide_operands(q: torch.Tensor, k: torch.Tensor):
     [hi, lo, hi, lo], so that one dot product over 4 D channels adds up all four partial products.  That needs
     4 D <= 256; wider heads raise.  The range test reads one number back from the GPU; while a stream is
     capturing a graph it is skipped and the operands are rounded to fp16 unseen."""
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing():
         return q.to(torch.float16), k.to(torch.float16), torch.float16
     amax = max(float(t.detach().abs().max()) if t.dtype not in (torch.float16, torch.bfloat16) else 0.0 for t in (q, k))
     if amax <= _FP16_MAX:  # (a NaN or an infinity fails this test too)
@@ -418,7 +422,7 @@ def _rounded_operands(q: torch.Tensor, k: torch.Tensor):
     if (q.dtype != torch.float32 or k.dtype != torch.float32 or k.device != q.device or not _dense_storage(q) or not _dense_storage(k)
             or q.numel() == 0 or k.numel() == 0 or q.shape[-1] > _MAX_HEAD_DIM
             or q.is_neg() or k.is_neg() or q.data_ptr() % 16 or k.data_ptr() % 16
-            or torch.cuda.is_current_stream_capturing()):
+            or _capturing()):
         return None
     q_h, k_h = torch.empty_like(q, dtype=torch.float16), torch.empty_like(k, dtype=torch.float16)
     if q_h.stride() != q.stride() or k_h.stride() != k.stride():
