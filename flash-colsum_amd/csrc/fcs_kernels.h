@@ -72,6 +72,7 @@ int launch_colsum(const Plan &p, const Args &a, void *stream);
 
 // fused path, defined in fcs_fused.hip
 hipError_t launch_fused(const Plan &p, const Args &a, hipStream_t st);
+hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st);
 // few-rows path (fcs_fewrows.hip): p.fewrows == 1
 hipError_t launch_fewrows(const Plan &p, const Args &a, hipStream_t st);
 // short-sequence path (fcs_small.hip): p.small == 1
@@ -87,6 +88,7 @@ hipError_t launch_finalize(const Args &a, hipStream_t st);
 // Text description of what launch_colsum(p, a, .) launches; snprintf semantics.
 size_t describe_colsum(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_fused(const Plan &p, const Args &a, char *buf, size_t n);
+size_t describe_tall(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_fewrows(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_small(const Plan &p, const Args &a, char *buf, size_t n);
 size_t describe_two_pass(const Plan &p, const Args &a, char *buf, size_t n);

@@ -154,6 +154,7 @@ struct Plan {
     int small;       // 1: short-sequence path (non-causal, Sk <= 288, D <= 64): grid = B * f_hg, slabs = f_hg,
                      //    f_tpw key tiles, f_nqblk row tiles of 32 rows per head
     int fused;       // 1: use it (then the two-pass fields above are unused)
+    int tall;        // with fused: 64 query rows per wave (fcs_tall.hip) in place of 32 rows with this many key tiles; else 0
     int f_kg, f_qg;  // waves along keys / along queries, f_kg * f_qg == 8
     int f_tpw;       // 32-key tiles per wave
     int f_nqblk;     // query blocks of 32 * f_qg rows
@@ -413,6 +414,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     p.fewrows = 0;
     p.small = 0;
     p.fused = 0;
+    p.tall = 0;
     // (One workgroup streams a whole key head and computes its R x Sk scores on the VALU.  The fused
     // path, which splits a head's keys over eight waves and uses the matrix pipe, is quicker when
     // there are fewer (batch entry, head) pairs than compute units and a thousand keys or more per
@@ -505,11 +507,18 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         //  * More groups of fewer tiles where the workgroups get two units at most, i.e. where most of the chip is idle or a
         //    unit's chain of tiles is all there is: B 2 H 4 S 512 9.3 -> 7.3, B 1 H 16 S 1024 bf16 14.1 -> 12.3, D 128
         //    18.2 -> 15.1, B 8 H 8 S 197 D 128 11.3 -> 8.7.  With three units or more it was up to 9 % slower.
+        // Heads of 65 .. 128 channels and 449 (narrower than 128: 385) .. 1024 keys: 64 query rows per wave, eight key groups (fcs_tall.hip).
+        // us per call, 32 rows -> 64: B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5; S 768 41.1 -> 36.6, S 640 32.1 -> 31.0; with two
+        // tiles per wave S 512 B 32 76.3 -> 68.2, S 480 B 16 40.2 -> 35.6, but S 448 B 8 20.2 -> 20.8, S 384 B 32 47.3 -> 54.2 (D 128; D 96,
+        // S 400 62.1 -> 51.6).  A call that leaves half of the chip idle takes the shorter blocks:
+        // B 2 H 4 S 1024 10.4 against 11.1.  So do calls of up to 32 averaged rows.
+        const bool tall = D > 64 && tiles > (narrow128 ? 12 : 14) && tiles <= 32 && tight_stages == 0 && p.q_rows > 32 &&
+                          (long)B * H * ceil_div(p.q_rows, 64) > kComputeUnits / 2;
         double best_kg = 0.;
         bool any = false;
-        for (int kg = (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {
-            const int tpw = ceil_div(tiles, kg), nqblk = ceil_div(p.q_rows, 32 * (8 / kg));
-            if (kg > usual && (tight_stages != 0 || (long)B * H * nqblk > 2 * kComputeUnits)) break;
+        for (int kg = tall ? 8 : (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {
+            const int tpw = ceil_div(tiles, kg), nqblk = ceil_div(p.q_rows, tall ? 64 : 32 * (8 / kg));
+            if (!tall && kg > usual && (tight_stages != 0 || (long)B * H * nqblk > 2 * kComputeUnits)) break;
             // Units per workgroup: a unit is one (query block, head); a workgroup takes f_rbpw adjacent
             // query blocks times f_hpg heads.  One workgroup is resident per compute unit, so the launch
             // runs in generations of kComputeUnits workgroups, each as long as its units plus about 0.7 of
@@ -557,6 +566,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
                 p.f_rbpw = best_rbpw;
             }
         }
+        p.tall = tall ? ceil_div(tiles, usual) : 0;
         p.f_hg = ceil_div(H, p.f_hpg);
         p.f_nwgq = ceil_div(p.f_nqblk, p.f_rbpw);
         p.n_partials = p.f_hg * p.f_nwgq * p.f_qg;

@@ -1,0 +1,479 @@
+// Attention column means on gfx950 (MI355X): single-pass path for wide heads (65 .. 128 channels) of 513 .. 1024 keys,
+// non-causal.  A wave owns 64 query rows x up to 128 keys, where the waves of fcs_fused.hip own 32 rows x up to 256.
+//
+// What bounds the 32-row tile at these head dims is moving operands, not arithmetic: every wave brings its own copy of its keys,
+// so that a row block of 64 rows x 1024 keys of 128 channels takes 576 KB through the L2 -> LDS path (about 65 B/clk
+// per compute unit: 8.9 k cycles of the 15.5 k that the block took at B 8, H 16, S 1024) and as much through the LDS read port.
+// With 64 rows to a wave
+//   * no key tile is fetched twice by a workgroup (eight key groups, one group of rows), and an operand fragment that has been read
+//     back serves two MFMA chains: half of both streams;
+//   * the 64 query rows come once per workgroup, by DMA into an LDS tile that all waves read;
+//   * the ring's last three items stay for the next row block of the same key head, which walks them in the opposite order.
+// us per call, 32 rows -> 64: B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5, B 16 H 16 S 800 120.7 -> 85.1.  What is left: without
+// the key fetches it would be 7 % faster, without three of four MFMAs 14 %, without phase 3 5 %.
+//
+// The scores of a wave (2 x 4 tiles) fill 128 registers as there.  Both chunks of 64 channels of the query rows would take another
+// 64, which is more than there is: all tiles take the first chunk's products, then all take the second's, and only one
+// chunk of the rows is held at a time.  The exponents run under the second chunk's MFMAs.  The row sums are added up behind
+// them: running sums in phase 1 would be 32 registers more and were 4 % slower; and the rare path is marked as such,
+// since the register allocator otherwise spilled a tile's exponentials to spare it (67 us at B 8, H 16, S 1024).
+//
+// The rest is fcs_fused.hip's: e = 2^(c s) without max subtraction while every row sum lands in [2^-80, 2^120), in-lane
+// column sums, one barrier per row block, a slab of column sums per workgroup; a row block outside the range is redone
+// with the row maxima subtracted.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <stdio.h>
+
+#include "fcs_device.h"
+#include "fcs_kernels.h"
+#include "fcs_rowfold.h"
+
+namespace fcs {
+
+namespace {
+
+constexpr float kSumLo = 8.2718061e-25f;  // 2^-80
+constexpr float kSumHi = 1.3292280e+36f;  // 2^120
+
+__device__ __attribute__((aligned(16))) unsigned int g_tall_zeros[4];  // the pieces of query rows past the head dim
+
+#define FCS_WAIT_VM(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
+#define FCS_OPAQUE_V(x) asm volatile("" : "+v"(x))
+
+__device__ __forceinline__ void pin16(float (&v)[16])
+{
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]), "+v"(v[8]), "+v"(v[9]),
+                 "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
+}
+
+// Four operand pieces of a row from LDS: those at `at`, and 2, 4 and 6 pieces on (the swizzles below only exchange bits of
+// the piece number).  Only issued here: take_wait stands between this and the first use.  (Inline assembly: the
+// compiler would make an ordinary LDS read wait for all DMA.)
+template <int OFF>
+__device__ __forceinline__ void take_issue(uint32_t at, half8 (&dst)[4])
+{
+    const uint32_t a1 = at ^ 32u, a2 = at ^ 64u, a3 = at ^ 96u;
+    asm volatile("ds_read_b128 %0, %4 offset:%8\n\tds_read_b128 %1, %5 offset:%8\n\tds_read_b128 %2, %6 offset:%8\n\tds_read_b128 %3, %7 offset:%8"
+                 : "=&v"(dst[0]), "=&v"(dst[1]), "=&v"(dst[2]), "=&v"(dst[3])
+                 : "v"(at), "v"(a1), "v"(a2), "v"(a3), "n"(OFF)
+                 : "memory");
+}
+__device__ __forceinline__ void take_wait(half8 (&dst)[4])
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(dst[0]), "+v"(dst[1]), "+v"(dst[2]), "+v"(dst[3])::"memory");
+}
+
+}  // namespace
+
+// TPW: 32-key tiles per wave.  NARROW: the head dim is less than 128.
+template <int TPW, bool BF, bool NARROW>
+__global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
+{
+    constexpr int NT = 4;                // MFMA steps per chunk of 64 channels
+    constexpr int STEPS = 2 * TPW;       // ring items of a row block: half tiles, 32 keys x 64 channels; chunk by chunk
+    constexpr int NS = 3;                // ring slots per wave; item j of every row block lives in slot j % NS
+    constexpr int ITEM = 4096;
+    constexpr int QTILE = 64 * 256;
+    static_assert(STEPS > NS, "the waits below count on a request at the first step");
+    __shared__ __attribute__((aligned(256))) char ring[8 * NS * ITEM];
+    __shared__ __attribute__((aligned(256))) char qtile[2 * QTILE];  // 64 rows x 128 channels, double-buffered
+    __shared__ __attribute__((aligned(16))) float part[2 * 64 * 8];  // row sums per (row, wave), double-buffered
+    __shared__ __attribute__((aligned(16))) float wv[8 * 64];        // per wave: a value per row
+
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int hgi, b, qwg;
+    {
+        int bx, by, bz;
+        xcd_contiguous_block(bx, by, bz);
+        qwg = bx % a.f_nwgq;
+        b = bx / a.f_nwgq;
+        hgi = by;
+    }
+    // the walk over units (head, row block of 64 rows), row blocks innermost
+    const int h_begin = hgi * a.f_hpg, n_heads = min(a.H, h_begin + a.f_hpg) - h_begin;
+    const int rb_first = qwg * a.f_rbpw, rb_n = min(a.f_rbpw, a.f_nqblk - rb_first);
+    const int n_units = rb_n * n_heads;
+    // key tile t of the wave holds keys [kbase + 32 t, ..), moved back to end at the last key where it would reach past it; its
+    // columns then repeat keys of the tile before and count for nothing: those of a lane are t > tmax_lane
+    const int kbase = wave * TPW * 32;
+    auto tile_first = [&](int t) { return min(kbase + t * 32, a.Sk - 32); };
+    const int tmax_lane = (n + a.Sk - 32 - kbase) >> 5;
+
+    const uint32_t q_row_b = (uint32_t)a.qs_s * 2u, k_row_b = (uint32_t)a.ks_s * 2u;
+    const char *q_batch = reinterpret_cast<const char *>(a.q + (int64_t)b * a.qs_b);
+    const char *k_batch = reinterpret_cast<const char *>(a.k + (int64_t)b * a.ks_b);
+    const int64_t q_head_b = a.qs_h * 2, k_head_b = a.ks_h * 2;
+    char *my_ring = ring + wave * (NS * ITEM);
+
+    // ---- DMA.  A key item is 32 rows x 128 bytes; an instruction brings 8 rows, lane L piece (16 bytes) L % 8 of row L / 8,
+    // stored XOR-swizzled (position p of row r holds piece p ^ ((r >> 1) & 7)).  Instructions 0 and 2, and 1 and 3, have the same
+    // lane offsets, 16 rows apart.
+    uint32_t k_voff[2], k_voff_n[NARROW ? 2 : 1];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t piece_b = (uint32_t)(((lane & 7) ^ ((i * 4 + (lane >> 4)) & 7)) * 16);
+        const uint32_t row = (uint32_t)((lane >> 3) + 8 * i) * k_row_b;
+        k_voff[i] = row + piece_b;
+        // (second chunk of a narrower head: a piece past the head dim is replaced by the row's first of the chunk; the query
+        // rows hold zeros there)
+        if (NARROW) k_voff_n[i % (NARROW ? 2 : 1)] = row + ((int)(64 + (piece_b >> 1)) < a.D ? piece_b : 0u);
+    }
+    auto dma = [](const char *src, char *dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+    };
+    auto fetch_item = [&](int64_t head_b, int tile, int chunk, int slot) {
+        const char *src = k_batch + head_b + (size_t)tile_first(tile) * k_row_b + chunk * 128;
+        char *dst = my_ring + slot * ITEM;
+        FCS_OPAQUE_V(k_voff[0]);
+        FCS_OPAQUE_V(k_voff[1]);
+        const char *src2 = src + (size_t)(16 * k_row_b);
+        if (NARROW) {
+            const uint32_t v0 = chunk ? k_voff_n[0] : k_voff[0], v1 = chunk ? k_voff_n[NARROW ? 1 : 0] : k_voff[1];
+            dma(src + v0, dst);
+            dma(src + v1, dst + 1024);
+            dma(src2 + v0, dst + 2048);
+            dma(src2 + v1, dst + 3072);
+        } else {
+            dma(src + k_voff[0], dst);
+            dma(src + k_voff[1], dst + 1024);
+            dma(src2 + k_voff[0], dst + 2048);
+            dma(src2 + k_voff[1], dst + 3072);
+        }
+    };
+    // the wave's 8 of a unit's 64 query rows: 4 rows x 256 bytes per instruction, position p of row r holds piece p ^ (r & 15);
+    // rows past the last one repeat it (they are given no weight)
+    auto fetch_q = [&](int head, int row0, int buf) {
+        const char *slice = q_batch + (int64_t)head * q_head_b;
+        char *dst = qtile + buf * QTILE + wave * 2048;
+        int l = lane;
+        FCS_OPAQUE_V(l);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = wave * 8 + i * 4 + (l >> 4);
+            const int piece = (l & 15) ^ (r & 15);
+            const char *src = slice + (size_t)min(row0 + r, a.Sq - 1) * q_row_b + piece * 16;
+            if (NARROW && piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_tall_zeros);
+            dma(src, dst + i * 1024);
+        }
+    };
+
+    // ---- read-back.  Lane (n, g) takes, for step tt of a chunk, piece 2 tt + g of row n.
+    uint32_t k_take = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)my_ring + (uint32_t)(n * 128 + ((g ^ ((n >> 1) & 7)) * 16));
+    uint32_t q_take = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)qtile + (uint32_t)(n * 256 + ((n >> 3) & 1) * 128 + ((g ^ (n & 7)) * 16));
+
+    float col_acc[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) col_acc[t] = 0.f;
+    float *wv_w = wv + wave * 64;
+
+    // Two orders of the items alternate between the row blocks of a key head: 0 .. STEPS-1 and (rot) back.  Step s of a row block
+    // works on item `item`, chunk item / TPW of key tile item % TPW; its scores are in acc[.][s % TPW], which is tile
+    // s % TPW or (rot) TPW - 1 - s % TPW.
+    int rot = 0;
+    auto item_of = [&](int s) { return rot ? STEPS - 1 - s : s; };
+    auto slot_of = [&](int s) { return rot ? (STEPS - 1 - s) % NS : s % NS; };
+    auto tile_of = [&](int s) { return rot ? TPW - 1 - s % TPW : s % TPW; };
+    auto chunk_of = [&](int s) { return rot ? 1 - s / TPW : s / TPW; };
+
+    int cur_rb = 0, cur_hr = 0;  // row block and head of the current unit, relative
+    auto key_off = [&](int hr) { return (int64_t)kv_head(h_begin + hr, a.kv_group, a.kv_magic) * k_head_b; };
+    int64_t k_cur = key_off(0);
+
+    fetch_q(h_begin, rb_first * 64, 0);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) fetch_item(k_cur, s % TPW, s / TPW, s);
+    FCS_WAIT_VM(0);
+    __syncthreads();
+
+    // the scale with its sign (a score of negated query rows, times c, has the very bits of the score times -c); scalar
+    const float cs = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, a.negate ? -a.c : a.c)));
+    for (int unit = 0; unit < n_units; ++unit) {
+        const int h = h_begin + cur_hr, row0 = (rb_first + cur_rb) * 64;
+        // the next unit (the last one is followed by itself)
+        int nxt_rb = cur_rb, nxt_hr = cur_hr;
+        if (unit + 1 < n_units && ++nxt_rb == rb_n) {
+            nxt_rb = 0;
+            ++nxt_hr;
+        }
+        const int64_t k_nxt = key_off(nxt_hr);
+        const int next_key_head = __builtin_amdgcn_readfirstlane(k_nxt != k_cur ? 1 : 0);
+
+        // The query rows are in their tile since the barrier before.  The first NS key items are in the ring: left behind by the
+        // unit before, or requested during its last steps.
+        half8 qf[2][NT], kf[2][NT];  // [32-row fragment]
+        FCS_OPAQUE_V(q_take);
+        FCS_OPAQUE_V(k_take);
+        const uint32_t q_at = q_take + (uint32_t)((unit & 1) * QTILE);
+        take_issue<0>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[0]);
+        take_issue<8192>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[1]);
+        FCS_WAIT_VM(0);
+        take_issue<0>(k_take + (uint32_t)(slot_of(0) * ITEM), kf[0]);
+
+        floatx16 acc[2][TPW];
+        float e[2][TPW][16];
+        auto exp_tile = [&](int nb, int t) {  // e = 2^(c s) in place, and into the row sums; a column that does not count: 2^-inf
+            const float bias = tile_of(t) <= tmax_lane ? 0.f : -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                e[nb][t][i] = fast_exp2(fmaf(acc[nb][t][i], cs, bias));
+            }
+            pin16(e[nb][t]);  // (else the exponents sink below the last MFMA)
+        };
+
+        // ---------------- phase 1
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int half = s / TPW, t = s % TPW;
+            // (the two waves of a SIMD take turns at the higher priority, as in fcs_fused.hip)
+            if (((s & 1) != 0) == (wave >= 4)) asm volatile("s_setprio 2");
+            else asm volatile("s_setprio 0");
+            if (t == 0) {
+                take_wait(qf[0]);
+                take_wait(qf[1]);
+            }
+            FCS_OPAQUE_V(k_take);  // addresses are formed where they are used
+            take_wait(kf[s & 1]);
+            if (s == 0) fetch_q(h_begin + nxt_hr, (rb_first + nxt_rb) * 64, (unit + 1) & 1);
+            // the slot is free: it takes the item of step s + NS, or the next key head's item that belongs in it
+            if (s + NS < STEPS) fetch_item(k_cur, tile_of(s + NS), chunk_of(s + NS), slot_of(s));
+            else if (next_key_head) fetch_item(k_nxt, slot_of(s) % TPW, slot_of(s) / TPW, slot_of(s));
+            // Item s + 1 has landed once at most the items requested behind it are outstanding (step s + 1 - NS requested it; the
+            // last step that requests one of this unit is STEPS - NS - 1).  The query rows, requested before all of them, have too.
+            if (s + 1 >= NS && s + 1 < STEPS) FCS_WAIT_VM((STEPS - 2 - s < NS - 1 ? STEPS - 2 - s : NS - 1) * NT);
+            if (s + 1 < STEPS) take_issue<0>(k_take + (uint32_t)(slot_of(s + 1) * ITEM), kf[(s + 1) & 1]);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if (half) c = acc[nb][t];
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) c = mfma16<BF>(qf[nb][tt], kf[s & 1][tt], c);
+                acc[nb][t] = c;
+            }
+            if (s == TPW - 1) {  // the other chunk of the query rows, behind the last chain that reads the first
+                asm volatile("" : "+v"(acc[0][t]), "+v"(acc[1][t]));
+                take_issue<0>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[0]);
+                take_issue<8192>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[1]);
+            }
+            if (half && t > 0) {  // VALU work of the tile before under this one's MFMAs
+                exp_tile(0, t - 1);
+                exp_tile(1, t - 1);
+            }
+        }
+        exp_tile(0, TPW - 1);
+        exp_tile(1, TPW - 1);
+
+        // ---------------- row sums over lanes and waves: one barrier, which also publishes the next unit's query rows
+        float *pt = part + (unit & 1) * 512;
+        // the row (of 32) whose total over this wave's keys a lane is left with, like its neighbour
+        int lane_r = lane;
+        FCS_OPAQUE_V(lane_r);  // addresses are formed here, not kept through phase 1
+        const int g_r = lane_r >> 5;
+        const int row_w = 16 * ((lane_r >> 4) & 1) + 8 * ((lane_r >> 3) & 1) + 4 * g_r + 2 * ((lane_r >> 2) & 1) + ((lane_r >> 1) & 1);
+        auto fold_rows = [&](int nb, float v) {
+            if ((lane_r & 1) == 0) pt[(nb * 32 + row_w) * 8 + wave] = v;
+        };
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            float rs[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                rs[i] = e[nb][0][i] + e[nb][1][i];
+                if (TPW == 3) rs[i] += e[nb][TPW - 1][i];
+                if (TPW == 4) rs[i] += e[nb][TPW - 2][i] + e[nb][TPW - 1][i];
+            }
+            fold_rows(nb, fold_lanes_sum(rs, lane_r));
+        }
+        __syncthreads();
+        // lane L adds up row L; every wave sees all of the rows' parts
+        bool slow;
+        {
+            const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + lane_r * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + lane_r * 8 + 4);
+            const float tot = ((f0[0] + f0[1]) + (f0[2] + f0[3])) + ((f1[0] + f1[1]) + (f1[2] + f1[3]));
+            bool ok = true;
+            float most = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                ok = ok && f0[j] < kSumHi && f1[j] < kSumHi;  // false for NaN
+                most = fmaxf(most, fmaxf(f0[j], f1[j]));
+            }
+            slow = __builtin_amdgcn_ballot_w64(!ok || !(most >= kSumLo)) != 0;
+            wv_w[lane_r] = (row0 + lane_r < a.q_rows) ? __builtin_amdgcn_rcpf(tot) : 0.f;
+            __builtin_amdgcn_wave_barrier();
+        }
+
+        if (__builtin_expect(!slow, 1)) {
+            // ---------------- phase 3: column sums of e * w, this row block's by themselves first
+            float sum[TPW];
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) sum[t] = 0.f;
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const floatx4 w4 = *reinterpret_cast<const floatx4 *>(wv_w + nb * 32 + 8 * i4 + 4 * g_r);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int t = 0; t < TPW; ++t) sum[t] = fmaf(e[nb][t][4 * i4 + j], w4[j], sum[t]);
+                }
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) col_acc[t] += rot ? sum[TPW - 1 - t] : sum[t];
+        } else {
+            // ------------ rare: the softmax with the row maximum subtracted, three passes over the keys with one score tile in
+            // registers at a time, from ordinary loads.  (From an opaque copy of the lane id: nothing of this is kept by the
+            // common path.)
+            int lane_s = lane;
+            FCS_OPAQUE_V(lane_s);
+            const int n_s = lane_s & 31, g_s = lane_s >> 5;
+            const int tmax_s = (n_s + a.Sk - 32 - kbase) >> 5;
+            const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_batch + k_cur) + g_s * 8;
+            float v16[2][16];
+            half8 qs[2 * NT];
+            auto load_rows = [&](int nb) {
+                const _Float16 *qp = reinterpret_cast<const _Float16 *>(q_batch + (int64_t)h * q_head_b) +
+                                     (int64_t)min(row0 + nb * 32 + n_s, a.Sq - 1) * a.qs_s + g_s * 8;
+#pragma unroll
+                for (int tt = 0; tt < 2 * NT; ++tt) {
+                    half8 v = kZero8;
+                    if (!NARROW || tt * 16 + g_s * 8 < a.D) v = load8(qp + tt * 16);
+                    qs[tt] = a.negate ? flip_sign(v) : v;
+                }
+            };
+            auto score_tile = [&](int t) {
+                const int krow = tile_first(t) + n_s;
+                floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int tt = 0; tt < 2 * NT; ++tt) {
+                    half8 kv = kZero8;
+                    if (!NARROW || tt * 16 + g_s * 8 < a.D) kv = load8(kp + (int64_t)krow * a.ks_s + tt * 16);
+                    c = mfma16<BF>(qs[tt], kv, c);
+                }
+                return c;
+            };
+            // row values over lanes and waves: f(the 8 waves' parts of row `lane`) goes to wv_w.  The barrier in front is for the
+            // part buffer's last readers.
+            auto reduce = [&](bool is_max, auto f) {
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) v16[nb][0] = is_max ? fold_lanes_max(v16[nb], lane_s) : fold_lanes_sum(v16[nb], lane_s);
+                __syncthreads();
+                const int rw = 16 * ((lane_s >> 4) & 1) + 8 * ((lane_s >> 3) & 1) + 4 * g_s + 2 * ((lane_s >> 2) & 1) + ((lane_s >> 1) & 1);
+                if ((lane_s & 1) == 0) {
+                    pt[rw * 8 + wave] = v16[0][0];
+                    pt[(32 + rw) * 8 + wave] = v16[1][0];
+                }
+                __syncthreads();
+                const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + lane_s * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + lane_s * 8 + 4);
+                wv_w[lane_s] = f(f0, f1);
+                __builtin_amdgcn_wave_barrier();
+            };
+            auto row_values = [&](float (&v)[16], int nb) {
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const floatx4 x = *reinterpret_cast<const floatx4 *>(wv_w + nb * 32 + 8 * i4 + 4 * g_s);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[4 * i4 + j] = x[j];
+                }
+            };
+            float rmax[2][16];
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                load_rows(nb);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v16[nb][i] = kNegBig;
+#pragma unroll 1
+                for (int t = 0; t < TPW; ++t) {
+                    const floatx16 c = score_tile(t);
+                    const bool real = t <= tmax_s;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v16[nb][i] = fmaxf(v16[nb][i], real ? c[i] : kNegBig);
+                }
+            }
+            reduce(true, [](floatx4 x, floatx4 y) {
+                return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])));
+            });
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                row_values(rmax[nb], nb);  // subtracted from the scores before the scale
+                load_rows(nb);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v16[nb][i] = 0.f;
+#pragma unroll 1
+                for (int t = 0; t < TPW; ++t) {
+                    const floatx16 c = score_tile(t);
+                    const bool real = t <= tmax_s;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v16[nb][i] += real ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f;
+                }
+            }
+            reduce(false, [&](floatx4 x, floatx4 y) {
+                const float L = ((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]));
+                return (row0 + lane_s < a.q_rows) ? __builtin_amdgcn_rcpf(L) : 0.f;
+            });
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                row_values(v16[nb], nb);
+                load_rows(nb);
+#pragma unroll 1
+                for (int t = 0; t < TPW; ++t) {
+                    const floatx16 c = score_tile(t);
+                    const bool real = t <= tmax_s;
+                    float sum = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sum = fmaf(real ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f, v16[nb][i], sum);
+#pragma unroll
+                    for (int u = 0; u < TPW; ++u)  // col_acc lives in registers: static index only
+                        if (u == t) col_acc[u] += sum;
+                }
+            }
+        }
+        rot = __builtin_amdgcn_readfirstlane(next_key_head ? 0 : (rot ^ 1));
+        k_cur = k_nxt;
+        cur_rb = nxt_rb;
+        cur_hr = nxt_hr;
+    }
+    FCS_WAIT_VM(0);  // drain the look-ahead fetches before the block's LDS is released
+
+    // ---------------- the two half-waves hold different rows of the same keys: add, then store
+    float *dst = a.partial + ((int64_t)(hgi * a.f_nwgq + qwg) * a.B + b) * a.Sk;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+        const float v = col_acc[t] + __shfl_xor(col_acc[t], 32);
+        if (g == 0 && t <= tmax_lane) dst[tile_first(t) + n] = v;
+    }
+}
+
+template <int TPW, bool BF>
+static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
+{
+    const dim3 grid(p.f_nwgq * p.B, p.f_hg);
+    if (p.D == 128) hipLaunchKernelGGL((fcs_tall_kernel<TPW, BF, false>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((fcs_tall_kernel<TPW, BF, true>), grid, dim3(512), 0, st, a);
+}
+
+hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
+{
+    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk) return hipErrorInvalidValue;
+    if (p.f_tpw == 2) p.bf16 ? launch_tpw<2, true>(p, a, st) : launch_tpw<2, false>(p, a, st);
+    else if (p.f_tpw == 3) p.bf16 ? launch_tpw<3, true>(p, a, st) : launch_tpw<3, false>(p, a, st);
+    else if (p.f_tpw == 4) p.bf16 ? launch_tpw<4, true>(p, a, st) : launch_tpw<4, false>(p, a, st);
+    else return hipErrorInvalidValue;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_finalize(a, st);
+}
+
+// (names the variant of fcs_fused.hip that serves such a call 32 rows to a wave, which it stands for)
+size_t describe_tall(const Plan &p, const Args &a, char *buf, size_t n)
+{
+    const char *bf = p.bf16 ? "true" : "false", *narrow = p.D == 128 ? "" : ",true";
+    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%s,%s> (for fcs_fused_kernel<128,%d,true,0,%s,true%s> ) grid %d x %d, %d x %d units per workgroup, %d slabs",
+                           p.f_tpw, bf, p.D == 128 ? "false" : "true", p.tall, bf, narrow, p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
+    if (r < 0) return 0;
+    const size_t len = (size_t)r;
+    return len + describe_finalize(a, false, len < n ? buf + len : nullptr, len < n ? n - len : 0);
+}
+
+}  // namespace fcs
