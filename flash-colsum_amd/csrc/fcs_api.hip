@@ -41,12 +41,12 @@ hipError_t static_scratch(void **ptr)
 // microseconds (more with many heads), so every thread remembers the plans of its last few
 // geometries.
 struct PlanKey {
-    int causal, B, H, Hk, Sq, Sk, D, cls_n, k_past;
+    int causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, raw;
     size_t within;  // non-causal: the plan for a workspace of this many bytes (0: the usual one)
     bool operator==(const PlanKey &o) const
     {
         return causal == o.causal && B == o.B && H == o.H && Hk == o.Hk && Sq == o.Sq && Sk == o.Sk && D == o.D && cls_n == o.cls_n &&
-               k_past == o.k_past && within == o.within;
+               k_past == o.k_past && raw == o.raw && within == o.within;
     }
 };
 constexpr int kPlanMemo = 8;
@@ -58,16 +58,16 @@ struct PlanMemo {
 };
 thread_local PlanMemo t_memo;
 
-bool cached_plan(fcs::Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, size_t within = 0)
+bool cached_plan(fcs::Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int raw = 0, size_t within = 0)
 {
-    const PlanKey key{causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, within};
+    const PlanKey key{causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, raw, within};
     PlanMemo &m = t_memo;
     for (int i = 0; i < kPlanMemo; ++i)
         if (m.used[i] && m.key[i] == key) {
             p = m.plan[i];
             return true;
         }
-    if (!(within ? fcs::plan_within(p, within, B, H, Hk, Sq, Sk, D, cls_n) : fcs::make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past))) return false;
+    if (!(within ? fcs::plan_within(p, within, B, H, Hk, Sq, Sk, D, cls_n) : fcs::make_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, 0, raw))) return false;
     const int slot = m.next;
     m.next = (slot + 1) % kPlanMemo;
     m.key[slot] = key;
@@ -104,9 +104,11 @@ int prepare(fcs::Plan &p, fcs::Args &a, int bf16, int causal, const void *q, con
     // mean the same and must not reach the kernels' 32-bit row arithmetic
     if (k_past > Sk) k_past = Sk;
 
-    if (!cached_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past)) return FCS_E_DIMS;
+    // (64-wide non-causal heads only: else the plan does not depend on it)
+    const int raw = !causal && D == 64 && (bf16 || fabsf(scale) > fcs::kPrescaledMaxScale);
+    if (!cached_plan(p, causal, B, H, Hk, Sq, Sk, D, cls_n, k_past, raw)) return FCS_E_DIMS;
     // (a fixed workspace, of non-causal calls: the call is laid out in it where it can be)
-    if (fit_workspace && p.total > ws_bytes && !cached_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, ws_bytes)) return FCS_E_STATIC_LIMIT;
+    if (fit_workspace && p.total > ws_bytes && !cached_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, 0, ws_bytes)) return FCS_E_STATIC_LIMIT;
     p.bf16 = bf16;
     if (need_ptrs) {
         if (ws && (reinterpret_cast<uintptr_t>(ws) & 255u)) return FCS_E_WORKSPACE;
@@ -193,6 +195,7 @@ size_t fcs_workspace_bytes(int causal, int B, int H, int Sq, int Sk, int D, int 
     const int rows = cls_n < 0 ? -1 : cls_n;
     if (!cached_plan(p, causal ? 1 : 0, B, H, H, Sq, Sk, D, rows, k_past)) return 0;
     size_t most = p.total;
+    if (!causal && D == 64 && cached_plan(p, 0, B, H, H, Sq, Sk, D, rows, 0, 1) && p.total > most) most = p.total;  // either operand
     // enough for any number of key heads: the two-pass path lays grouped heads out differently
     // (and beyond 2048 keys a call that the single-pass path serves may be one of those)
     for (int hk = 1; hk <= H / 2 && !(p.fewrows || p.small || (p.fused && Sk <= fcs::kFusedMaxKeys)); ++hk)
@@ -253,7 +256,7 @@ int fcs_colsum_noncausal_f16_static(const void *q, const void *k, float *out, vo
     // size check first: it needs no GPU, like every other argument error
     fcs::Plan p;
     if (!cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0)) return FCS_E_DIMS;
-    if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES && !cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0, FCS_STATIC_SCRATCH_BYTES))
+    if (p.total > (size_t)FCS_STATIC_SCRATCH_BYTES && !cached_plan(p, 0, B, H, H, S, S, D, cls_n < 0 ? -1 : cls_n, 0, 0, FCS_STATIC_SCRATCH_BYTES))
         return FCS_E_STATIC_LIMIT;
     if (!q || !k || !out || !q_strides || !k_strides) return FCS_E_NULL;
     void *ws = nullptr;

@@ -838,7 +838,7 @@ static FusedVariant pick_fused(const Plan &p, const Args &a, bool bf)
     // ... pre-scaled when the rounding of Q*c to fp16 cannot show in the means
     // (up to 2048 keys.  Longer calls took their exact operand from a row sum of 2^20 on while they ran in two passes, not from
     // 2^28: the scores' rounding would reach rows that it did not reach then.)
-    const bool pre = shared_q && !bf && p.Sk <= kFusedMaxKeys && (long)p.H * p.q_rows >= 4096 && fabsf(a.c) <= 0.1251f * 1.44269504f;
+    const bool pre = shared_q && !bf && p.Sk <= kFusedMaxKeys && (long)p.H * p.q_rows >= 4096 && fabsf(a.c) <= kPrescaledMaxScale * 1.44269504f;
     if (pre && whole && TPW == 8 && (p.f_kg == 8 || p.f_kg == 4)) return {8, false, p.f_kg, true};
     if (pre) return {TPW, true, p.f_kg, true};
     // ... else Q shared through LDS as it is (8 or 4 key groups).  (Two key groups that cannot be

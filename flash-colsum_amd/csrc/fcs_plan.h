@@ -11,6 +11,7 @@ constexpr int kWavesPerBlock = 4;   // 256 threads
 constexpr int kStageKeys = 64;      // keys staged in LDS per step of either pass
 constexpr int kComputeUnits = 256;  // MI355X
 constexpr int kFusedMaxKeys = 2048; // 8 waves x 8 tiles x 32 keys of fp32 scores per 32 query rows
+constexpr float kPrescaledMaxScale = 0.1251f;  // single-pass kernels: the operand is pre-scaled up to this |scale| (fp16)
 constexpr int kFusedMaxKeys64 = 2560; // 64-wide heads: ten tiles per wave
 constexpr int kFewRowsMaxRows = 4;      // few-rows path: at most this many averaged query rows per head ...
 constexpr int kFewRowsMaxScores = 12288; // ... and rows * Sk scores (48 KB of LDS)
@@ -174,10 +175,11 @@ struct Plan {
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Returns false for invalid dimensions.  cls_n <= 0 means all rows.  Hk: key heads, a divisor of H.
+// Returns false for invalid dimensions.  cls_n <= 0 means all rows.  raw: the single-pass kernels may not take a pre-scaled operand.  Hk: key heads, a divisor of H.
 // tight_stages > 0: the two-pass path with as little workspace as it can do with: row blocks are not cut, chunks are not longer
 // than that; < 0: not even slabs, a workgroup computes all of a chunk (see plan_within).
-inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight_stages = 0)
+inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight_stages = 0,
+                      int raw = 0)
 {
     if (B < 1 || H < 1 || Hk < 1 || H % Hk != 0 || Sq < 1 || Sk < 1 || D < 1 || k_past < 0) return false;
     p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
@@ -507,13 +509,19 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         //  * More groups of fewer tiles where the workgroups get two units at most, i.e. where most of the chip is idle or a
         //    unit's chain of tiles is all there is: B 2 H 4 S 512 9.3 -> 7.3, B 1 H 16 S 1024 bf16 14.1 -> 12.3, D 128
         //    18.2 -> 15.1, B 8 H 8 S 197 D 128 11.3 -> 8.7.  With three units or more it was up to 9 % slower.
-        // Heads of 65 .. 128 channels and 449 (narrower than 128: 385) .. 1024 keys: 64 query rows per wave, eight key groups (fcs_tall.hip).
-        // us per call, 32 rows -> 64: B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5; S 768 41.1 -> 36.6, S 640 32.1 -> 31.0; with two
-        // tiles per wave S 512 B 32 76.3 -> 68.2, S 480 B 16 40.2 -> 35.6, but S 448 B 8 20.2 -> 20.8, S 384 B 32 47.3 -> 54.2 (D 128; D 96,
-        // S 400 62.1 -> 51.6).  A call that leaves half of the chip idle takes the shorter blocks:
-        // B 2 H 4 S 1024 10.4 against 11.1.  So do calls of up to 32 averaged rows.
-        const bool tall = D > 64 && tiles > (narrow128 ? 12 : 14) && tiles <= 32 && tight_stages == 0 && p.q_rows > 32 &&
-                          (long)B * H * ceil_div(p.q_rows, 64) > kComputeUnits / 2;
+        // 64 query rows per wave and eight key groups (fcs_tall.hip), up to 1024 keys.  us per call, 32 rows -> 64:
+        //  * heads of 65 .. 128 channels, from 449 keys on (narrower than 128: 385): B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5;
+        //    S 768 41.1 -> 36.6, S 640 32.1 -> 31.0; with two tiles per wave S 512 B 32 76.3 -> 68.2, S 480 B 16 40.2 -> 35.6, but
+        //    S 448 B 8 20.2 -> 20.8, S 384 B 32 47.3 -> 54.2 (D 128; D 96, S 400 62.1 -> 51.6).
+        //  * 64 channels from 865 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 249.8 -> 232.1, B 16 S 900 63.6 -> 61.7,
+        //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4; fewer channels from 769 on: D 32 B 16 S 1000
+        //    68.5 -> 60.5, D 48 B 32 H 12 S 800 81.6 -> 77.7, but D 48 S 500 24.1 -> 25.8.
+        // A call that leaves half of the chip idle takes the shorter blocks (B 2 H 4 S 1024 D 128 10.4 against 11.1; up to 64 channels the
+        // splits over more waves below have calls of two units per workgroup), and so do calls of up to 32 averaged rows.
+        const long tall_units = (long)B * H * ceil_div(p.q_rows, 64);
+        const bool tall = tight_stages == 0 && p.q_rows > 32 && tiles <= 32 &&
+                          (D > 64 ? tiles > (narrow128 ? 12 : 14) && tall_units > kComputeUnits / 2
+                                  : (D < 64 ? tiles > 24 : raw && tiles > 27) && tall_units > 2 * kComputeUnits);
         double best_kg = 0.;
         bool any = false;
         for (int kg = tall ? 8 : (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {

@@ -1,18 +1,22 @@
-// Attention column means on gfx950 (MI355X): single-pass path for wide heads (65 .. 128 channels) of 513 .. 1024 keys,
-// non-causal.  A wave owns 64 query rows x up to 128 keys, where the waves of fcs_fused.hip own 32 rows x up to 256.
+// Attention column means on gfx950 (MI355X): single-pass path with 64 query rows x up to 128 keys per wave, where the waves of
+// fcs_fused.hip own 32 rows x up to 256.  Non-causal calls of up to 1024 keys: heads of 65 .. 128 channels, and those of up to 64
+// with four key tiles per wave whose operand is not pre-scaled (make_plan says where, with both sides' times).
 //
-// What bounds the 32-row tile at these head dims is moving operands, not arithmetic: every wave brings its own copy of its keys,
+// What bounds the 32-row tile at 128 channels is moving operands, not arithmetic: every wave brings its own copy of its keys,
 // so that a row block of 64 rows x 1024 keys of 128 channels takes 576 KB through the L2 -> LDS path (about 65 B/clk
 // per compute unit: 8.9 k cycles of the 15.5 k that the block took at B 8, H 16, S 1024) and as much through the LDS read port.
 // With 64 rows to a wave
 //   * no key tile is fetched twice by a workgroup (eight key groups, one group of rows), and an operand fragment that has been read
 //     back serves two MFMA chains: half of both streams;
 //   * the 64 query rows come once per workgroup, by DMA into an LDS tile that all waves read;
-//   * the ring's last three items stay for the next row block of the same key head, which walks them in the opposite order.
-// us per call, 32 rows -> 64: B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5, B 16 H 16 S 800 120.7 -> 85.1.  What is left: without
-// the key fetches it would be 7 % faster, without three of four MFMAs 14 %, without phase 3 5 %.
+//   * the ring's last three items stay for the next row block of the same key head, which walks them in the opposite order; of 64-wide
+//     heads all of them stay, and a key head is fetched once per workgroup.
+// B 8 H 16 S 1024 D 128 bf16 60.1 -> 47.7 us per call.  What is left there: without the key fetches it would be 7 % faster,
+// without three of four MFMAs 14 %, without phase 3 5 %.  64-wide heads are bound by the exponents either way: bf16 B 64 H 16 S 1024
+// 256.9 -> 239.7.  (Their pre-scaled operand was tried: 245 -> 231 at B 64, 2 .. 13 % slower with two and three tiles per wave, and
+// the rows' way through registers cannot be expressed safely in a loop with two waits; not built.)
 //
-// The scores of a wave (2 x 4 tiles) fill 128 registers as there.  Both chunks of 64 channels of the query rows would take another
+// The scores of a wave (2 x 4 tiles) fill 128 registers as there.  Both chunks of 64 channels of wide query rows would take another
 // 64, which is more than there is: all tiles take the first chunk's products, then all take the second's, and only one
 // chunk of the rows is held at a time.  The exponents run under the second chunk's MFMAs.  The row sums are added up behind
 // them: running sums in phase 1 would be 32 registers more and were 4 % slower; and the rare path is marked as such,
@@ -67,16 +71,17 @@ __device__ __forceinline__ void take_wait(half8 (&dst)[4])
 
 }  // namespace
 
-// TPW: 32-key tiles per wave.  NARROW: the head dim is less than 128.
-template <int TPW, bool BF, bool NARROW>
+// DC: chunks of 64 channels.  TPW: 32-key tiles per wave.  NARROW: the head dim is less than DC x 64.
+template <int DC, int TPW, bool BF, bool NARROW>
 __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 {
     constexpr int NT = 4;                // MFMA steps per chunk of 64 channels
-    constexpr int STEPS = 2 * TPW;       // ring items of a row block: half tiles, 32 keys x 64 channels; chunk by chunk
-    constexpr int NS = 3;                // ring slots per wave; item j of every row block lives in slot j % NS
+    constexpr int STEPS = DC * TPW;      // ring items of a row block: half tiles, 32 keys x 64 channels; chunk by chunk
+    constexpr bool KEEP_ALL = DC == 1;   // every item of a key head stays in the ring
+    constexpr int NS = KEEP_ALL ? TPW : 3;              // ring slots per wave; item j of every row block lives in slot j % NS
     constexpr int ITEM = 4096;
-    constexpr int QTILE = 64 * 256;
-    static_assert(STEPS > NS, "the waits below count on a request at the first step");
+    constexpr int QROW = DC * 128, QTILE = 64 * QROW, QI = DC;  // QI: a wave's DMA instructions for its 8 query rows
+    static_assert(KEEP_ALL || STEPS > NS, "the waits below count on a request at the first step");
     __shared__ __attribute__((aligned(256))) char ring[8 * NS * ITEM];
     __shared__ __attribute__((aligned(256))) char qtile[2 * QTILE];  // 64 rows x 128 channels, double-buffered
     __shared__ __attribute__((aligned(16))) float part[2 * 64 * 8];  // row sums per (row, wave), double-buffered
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         k_voff[i] = row + piece_b;
         // (second chunk of a narrower head: a piece past the head dim is replaced by the row's first of the chunk; the query
         // rows hold zeros there)
-        if (NARROW) k_voff_n[i % (NARROW ? 2 : 1)] = row + ((int)(64 + (piece_b >> 1)) < a.D ? piece_b : 0u);
+        if (NARROW) k_voff_n[i % (NARROW ? 2 : 1)] = row + ((int)((DC - 1) * 64 + (piece_b >> 1)) < a.D ? piece_b : 0u);
     }
     auto dma = [](const char *src, char *dst) {
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
@@ -131,7 +136,8 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         FCS_OPAQUE_V(k_voff[1]);
         const char *src2 = src + (size_t)(16 * k_row_b);
         if (NARROW) {
-            const uint32_t v0 = chunk ? k_voff_n[0] : k_voff[0], v1 = chunk ? k_voff_n[NARROW ? 1 : 0] : k_voff[1];
+            const bool last = chunk == DC - 1;
+            const uint32_t v0 = last ? k_voff_n[0] : k_voff[0], v1 = last ? k_voff_n[NARROW ? 1 : 0] : k_voff[1];
             dma(src + v0, dst);
             dma(src + v1, dst + 1024);
             dma(src2 + v0, dst + 2048);
@@ -147,13 +153,13 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     // rows past the last one repeat it (they are given no weight)
     auto fetch_q = [&](int head, int row0, int buf) {
         const char *slice = q_batch + (int64_t)head * q_head_b;
-        char *dst = qtile + buf * QTILE + wave * 2048;
+        char *dst = qtile + buf * QTILE + wave * (8 * QROW);
         int l = lane;
         FCS_OPAQUE_V(l);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int r = wave * 8 + i * 4 + (l >> 4);
-            const int piece = (l & 15) ^ (r & 15);
+        for (int i = 0; i < QI; ++i) {
+            const int r = DC == 2 ? wave * 8 + i * 4 + (l >> 4) : wave * 8 + (l >> 3);
+            const int piece = DC == 2 ? (l & 15) ^ (r & 15) : (l & 7) ^ ((r >> 1) & 7);
             const char *src = slice + (size_t)min(row0 + r, a.Sq - 1) * q_row_b + piece * 16;
             if (NARROW && piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_tall_zeros);
             dma(src, dst + i * 1024);
@@ -162,7 +168,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 
     // ---- read-back.  Lane (n, g) takes, for step tt of a chunk, piece 2 tt + g of row n.
     uint32_t k_take = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)my_ring + (uint32_t)(n * 128 + ((g ^ ((n >> 1) & 7)) * 16));
-    uint32_t q_take = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)qtile + (uint32_t)(n * 256 + ((n >> 3) & 1) * 128 + ((g ^ (n & 7)) * 16));
+    uint32_t q_take = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)qtile + (DC == 2 ? (uint32_t)(n * 256 + ((n >> 3) & 1) * 128 + ((g ^ (n & 7)) * 16)) : (uint32_t)(n * 128 + ((g ^ ((n >> 1) & 7)) * 16)));
 
     float col_acc[TPW];
 #pragma unroll
@@ -208,7 +214,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         FCS_OPAQUE_V(k_take);
         const uint32_t q_at = q_take + (uint32_t)((unit & 1) * QTILE);
         take_issue<0>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[0]);
-        take_issue<8192>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[1]);
+        take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[1]);
         FCS_WAIT_VM(0);
         take_issue<0>(k_take + (uint32_t)(slot_of(0) * ITEM), kf[0]);
 
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             else if (next_key_head) fetch_item(k_nxt, slot_of(s) % TPW, slot_of(s) / TPW, slot_of(s));
             // Item s + 1 has landed once at most the items requested behind it are outstanding (step s + 1 - NS requested it; the
             // last step that requests one of this unit is STEPS - NS - 1).  The query rows, requested before all of them, have too.
-            if (s + 1 >= NS && s + 1 < STEPS) FCS_WAIT_VM((STEPS - 2 - s < NS - 1 ? STEPS - 2 - s : NS - 1) * NT);
+            if (!KEEP_ALL && s + 1 >= NS && s + 1 < STEPS) FCS_WAIT_VM((STEPS - 2 - s < NS - 1 ? STEPS - 2 - s : NS - 1) * NT);
             if (s + 1 < STEPS) take_issue<0>(k_take + (uint32_t)(slot_of(s + 1) * ITEM), kf[(s + 1) & 1]);
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
@@ -252,18 +258,23 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                 for (int tt = 0; tt < NT; ++tt) c = mfma16<BF>(qf[nb][tt], kf[s & 1][tt], c);
                 acc[nb][t] = c;
             }
-            if (s == TPW - 1) {  // the other chunk of the query rows, behind the last chain that reads the first
+            if (DC == 2 && s == TPW - 1) {  // the other chunk of the query rows, behind the last chain that reads the first
                 asm volatile("" : "+v"(acc[0][t]), "+v"(acc[1][t]));
                 take_issue<0>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[0]);
-                take_issue<8192>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[1]);
+                take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[1]);
             }
-            if (half && t > 0) {  // VALU work of the tile before under this one's MFMAs
+            if (half == DC - 1 && t > 0) {  // VALU work of the tile before under this one's MFMAs
                 exp_tile(0, t - 1);
                 exp_tile(1, t - 1);
             }
         }
         exp_tile(0, TPW - 1);
         exp_tile(1, TPW - 1);
+
+        if (KEEP_ALL) {  // the next unit's query rows have landed: behind them is the next key head, or nothing
+            if (next_key_head) FCS_WAIT_VM(STEPS * NT);
+            else FCS_WAIT_VM(0);
+        }
 
         // ---------------- row sums over lanes and waves: one barrier, which also publishes the next unit's query rows
         float *pt = part + (unit & 1) * 512;
@@ -331,12 +342,12 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             const int tmax_s = (n_s + a.Sk - 32 - kbase) >> 5;
             const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_batch + k_cur) + g_s * 8;
             float v16[2][16];
-            half8 qs[2 * NT];
+            half8 qs[DC * NT];
             auto load_rows = [&](int nb) {
                 const _Float16 *qp = reinterpret_cast<const _Float16 *>(q_batch + (int64_t)h * q_head_b) +
                                      (int64_t)min(row0 + nb * 32 + n_s, a.Sq - 1) * a.qs_s + g_s * 8;
 #pragma unroll
-                for (int tt = 0; tt < 2 * NT; ++tt) {
+                for (int tt = 0; tt < DC * NT; ++tt) {
                     half8 v = kZero8;
                     if (!NARROW || tt * 16 + g_s * 8 < a.D) v = load8(qp + tt * 16);
                     qs[tt] = a.negate ? flip_sign(v) : v;
@@ -346,7 +357,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                 const int krow = tile_first(t) + n_s;
                 floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int tt = 0; tt < 2 * NT; ++tt) {
+                for (int tt = 0; tt < DC * NT; ++tt) {
                     half8 kv = kZero8;
                     if (!NARROW || tt * 16 + g_s * 8 < a.D) kv = load8(kp + (int64_t)krow * a.ks_s + tt * 16);
                     c = mfma16<BF>(qs[tt], kv, c);
@@ -429,7 +440,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                 }
             }
         }
-        rot = __builtin_amdgcn_readfirstlane(next_key_head ? 0 : (rot ^ 1));
+        if (!KEEP_ALL) rot = __builtin_amdgcn_readfirstlane(next_key_head ? 0 : (rot ^ 1));
         k_cur = k_nxt;
         cur_rb = nxt_rb;
         cur_hr = nxt_hr;
@@ -449,13 +460,15 @@ template <int TPW, bool BF>
 static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
 {
     const dim3 grid(p.f_nwgq * p.B, p.f_hg);
-    if (p.D == 128) hipLaunchKernelGGL((fcs_tall_kernel<TPW, BF, false>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((fcs_tall_kernel<TPW, BF, true>), grid, dim3(512), 0, st, a);
+    if (p.D == 128) hipLaunchKernelGGL((fcs_tall_kernel<2, TPW, BF, false>), grid, dim3(512), 0, st, a);
+    else if (p.D > 64) hipLaunchKernelGGL((fcs_tall_kernel<2, TPW, BF, true>), grid, dim3(512), 0, st, a);
+    else if (p.D == 64) hipLaunchKernelGGL((fcs_tall_kernel<1, 4, BF, false>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((fcs_tall_kernel<1, 4, BF, true>), grid, dim3(512), 0, st, a);
 }
 
 hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
 {
-    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk) return hipErrorInvalidValue;
+    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (p.D <= 64 && p.f_tpw != 4)) return hipErrorInvalidValue;
     if (p.f_tpw == 2) p.bf16 ? launch_tpw<2, true>(p, a, st) : launch_tpw<2, false>(p, a, st);
     else if (p.f_tpw == 3) p.bf16 ? launch_tpw<3, true>(p, a, st) : launch_tpw<3, false>(p, a, st);
     else if (p.f_tpw == 4) p.bf16 ? launch_tpw<4, true>(p, a, st) : launch_tpw<4, false>(p, a, st);
@@ -468,9 +481,9 @@ hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
 // (names the variant of fcs_fused.hip that serves such a call 32 rows to a wave, which it stands for)
 size_t describe_tall(const Plan &p, const Args &a, char *buf, size_t n)
 {
-    const char *bf = p.bf16 ? "true" : "false", *narrow = p.D == 128 ? "" : ",true";
-    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%s,%s> (for fcs_fused_kernel<128,%d,true,0,%s,true%s> ) grid %d x %d, %d x %d units per workgroup, %d slabs",
-                           p.f_tpw, bf, p.D == 128 ? "false" : "true", p.tall, bf, narrow, p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
+    const char *bf = p.bf16 ? "true" : "false", *narrow = p.D % 64 ? "true" : "false";
+    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%s,%s> (for fcs_fused_kernel<%d,%d,true,0,%s,true%s> ) grid %d x %d, %d x %d units per workgroup, %d slabs",
+                           p.Dp / 64, p.f_tpw, bf, narrow, p.Dp, p.tall, bf, p.D % 64 ? ",true" : "", p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
     if (r < 0) return 0;
     const size_t len = (size_t)r;
     return len + describe_finalize(a, false, len < n ? buf + len : nullptr, len < n ? n - len : 0);
