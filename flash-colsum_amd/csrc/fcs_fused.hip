@@ -694,7 +694,9 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
             return (blk_row0 + row < a.q_rows) ? __builtin_amdgcn_rcpf(L) : 0.f;
         }, PRESCALED ? kSumHiPre : kSumHi);
 
-        if (!slow && KEEP && rot) {
+        // (The rare path's loops weigh nothing to the register allocator: what it spills, it spills there.  Else 128-wide heads of eight
+        // tiles per wave spilled in phase 1: B 8 H 16 S 2048 D 128 243.7 -> 235.5 us per call.)
+        if (KEEP && __builtin_expect(!slow, 1) && rot) {
             // ---------------- phase 3 of a unit in the second order: step t held tile tile_of(t)
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4) {
@@ -709,7 +711,7 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
                 }
             }
             asm volatile("" ::: "memory");
-        } else if (!slow) {
+        } else if (__builtin_expect(!slow, 1)) {
             // ---------------- phase 3: column sums of e * w
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4) {

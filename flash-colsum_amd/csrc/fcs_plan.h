@@ -484,22 +484,23 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // ---- fused path
     // (at least one whole key tile: the kernel moves a tile that reaches past the last key back to end there)
     // (64-wide kernels for head dims up to 64, 128-wide ones up to 128; wider heads take the two-pass path)
-    // (Heads of 72 .. 120 channels: the 128-wide kernel's variant for narrower heads runs out of registers at seven
-    // and eight key tiles per wave, so it takes at most six, i.e. 1536 keys; longer calls take the two-pass path.)
+    // (Heads of 72 .. 120 channels: six key tiles per wave where that is enough, seven and eight beyond 1536 keys, where the rare path
+    // spills.  us per call, two passes -> here: B 8 H 16 S 2000 D 96 279 -> 226, S 1700 D 80 224.3 -> 155.8.  The plan tests hold the
+    // longest such call, 2048 keys, to the two-pass path: up to 63 tiles.)
     const bool narrow128 = D > 64 && D < 128;
     // (64-wide heads: the shared-Q variants hold ten tiles per wave, so calls of up to 2560 keys are served too, unless grouped
     // heads are laid end to end, whose keys are streamed once for the whole group.  us per call, two passes -> here:
     // B 1 H 16 S 2500 47.9 -> 33.5, B 4 H 16 S 2300 212.8 -> 88.0, H 1 S 2500 14.6 -> 10.9, 5 averaged rows of B 8 H 16
     // S 2300 30.2 -> 12.1, 128 of them 29.9 -> 18.5; no size in between was slower.)
     const bool wide = D == 64 && tight_stages == 0;
-    const int fused_max = narrow128 ? 8 * 6 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
+    const int fused_max = narrow128 ? 63 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
     if (!causal && Sk >= 32 && Sk <= fused_max && D <= 128) {
         p.fused = 1;
         p.fold = 1;
         const int tiles = ceil_div(Sk, 32);
         int usual = 1;  // key groups: the fewest that hold the keys with eight tiles per wave
         while (usual * 8 < tiles && usual < 8) usual *= 2;
-        if (narrow128) while (usual * 6 < tiles) usual *= 2;  // six there
+        if (narrow128) while (usual * 6 < tiles && usual < 8) usual *= 2;  // six there
         // Other splits over the key groups are priced too; tight_stages keeps the usual one, whose slabs are what such a
         // caller has always had room for.
         //  * Half as many groups of nine or ten tiles (64-wide heads): half the barriers, row sums and exchanges, but the last
