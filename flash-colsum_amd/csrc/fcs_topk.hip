@@ -26,7 +26,7 @@
 //      wave of words, and where more than 64 share a bin (ties, a few outliers in several parts of the row), a bitonic
 //      sort: exchanges over less than a wave's elements are DPP and lane swaps in registers, only the wider ones go through
 //      LDS.  Its 55 steps on 1024 words were 4 us of the 15, all VALU work of a single compute unit.
-// Measured, sorted, B 4, bitonic sort -> counting: S 8192, k 128 11.1 -> 10.1 us, 512 13.0 -> 10.8, 1024 14.9 -> 11.3,
+// Measured (with shuffles in place of the DPP scans, 1 us more), sorted, B 4, bitonic sort -> counting: S 8192, k 128 11.1 -> 10.1 us, 512 13.0 -> 10.8, 1024 14.9 -> 11.3,
 // 4096 31.0 -> 17.0; S 32768, k 2048 32.1 -> 26.5; S 131072, k 4096 103.8 -> 94.1.  k 64 is equal either way.  Rows with a
 // crowded bin pay for the count and the sort (S 8192, k 1024, 16.0 -> 16.8).
 // The threshold form is step 3 alone with a given threshold.
@@ -125,18 +125,31 @@ struct TopkLds {
     int crowded;
 };
 
+// A wave's running totals op(v of lane 0, .., v of this lane), in registers: within rows of 16 lanes, then the rows' last lanes to the
+// rows above (a lane without a partner takes `none`).  A step is one DPP instruction, where a shuffle is an LDS round trip.  us per
+// selection, shuffles -> this: B 4, S 8192, k 1024 11.4 -> 10.4, S 1898, k 314 8.0 -> 6.8, S 32768, k 2048 26.0 -> 24.7.
+template <typename F>
+__device__ __forceinline__ uint32_t lanes_below(uint32_t v, uint32_t none, F op)
+{
+#define FCS_SCAN_STEP(CTRL, ROWS) v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, CTRL, ROWS, 0xF, false))
+    FCS_SCAN_STEP(0x111, 0xF);  // row_shr:1
+    FCS_SCAN_STEP(0x112, 0xF);
+    FCS_SCAN_STEP(0x114, 0xF);
+    FCS_SCAN_STEP(0x118, 0xF);
+    FCS_SCAN_STEP(0x142, 0xA);  // row_bcast:15, into rows 1 and 3
+    FCS_SCAN_STEP(0x143, 0xC);  // row_bcast:31, into rows 2 and 3
+#undef FCS_SCAN_STEP
+    return v;
+}
+__device__ __forceinline__ uint32_t last_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
+
 // How many of the counted keys lie in the bins of higher threads; c: those in this thread's two.  One barrier.
 __device__ __forceinline__ int in_higher_bins(int c, TopkLds &lds, int wave, int lane)
 {
-    int run = c;  // this lane and the higher ones of its wave
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const int o = __shfl_down(run, m);
-        run += (lane + m < 64) ? o : 0;
-    }
-    if (lane == 0) lds.wsum[wave] = run;
+    const uint32_t run = lanes_below((uint32_t)c, 0u, [](uint32_t a, uint32_t b) { return a + b; }), all = last_lane(run);
+    if (lane == 0) lds.wsum[wave] = (int)all;
     __syncthreads();
-    int above = run - c;
+    int above = (int)(all - run);
 #pragma unroll
     for (int w = 0; w < kTopkWaves; ++w) above += (w > wave) ? lds.wsum[w] : 0;
     return above;
@@ -316,11 +329,8 @@ __global__ __launch_bounds__(kTopkThreads) void fcs_topk_kernel(const float *mea
         kmin = in ? min(kmin, key) : kmin;
         kmax = in ? max(kmax, key) : kmax;
     });
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, m));
-        kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, m));
-    }
+    kmin = last_lane(lanes_below(kmin, 0xffffffffu, [](uint32_t a, uint32_t b) { return min(a, b); }));
+    kmax = last_lane(lanes_below(kmax, 0u, [](uint32_t a, uint32_t b) { return max(a, b); }));
     if (lane == 0) {
         lds.wmin[wave] = kmin;
         lds.wmax[wave] = kmax;
