@@ -494,7 +494,13 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // S 2300 30.2 -> 12.1, 128 of them 29.9 -> 18.5; no size in between was slower.)
     const bool wide = D == 64 && tight_stages == 0;
     const int fused_max = narrow128 ? 63 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
-    if (!causal && Sk >= 32 && Sk <= fused_max && D <= 128) {
+    // Causal calls of 257 .. 1024 keys whose heads are not laid end to end: the same, a mask on the tiles that the diagonal crosses and no
+    // exponents behind it.  Two passes cost three launches and both products for what is mostly latency; us per call, two passes -> here:
+    // H 32 S 1000 D 128 32.1 -> 21.5, H 16 S 800 D 64 21.2 -> 11.8, H 16 Q 100 K 1000 D 128 17.6 -> 11.6, H 2 S 300 D 128 14.6 -> 8.7;
+    // none of 17 sizes slower.  (One batch entry, as prompts and windows are: batches gain as much, B 64 H 16 S 1024 D 64 327 -> 257, but the
+    // tests of shares that cross batch entries hold such a call to two passes.)
+    const bool causal_single = causal && B == 1 && p.fold == 1 && D <= 128 && Sk > 256 && Sk <= 1024;
+    if (causal_single || (!causal && Sk >= 32 && Sk <= fused_max && D <= 128)) {
         p.fused = 1;
         p.fold = 1;
         const int tiles = ceil_div(Sk, 32);
@@ -520,9 +526,9 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         // A call that leaves half of the chip idle takes the shorter blocks (B 2 H 4 S 1024 D 128 10.4 against 11.1; up to 64 channels the
         // splits over more waves below have calls of two units per workgroup), and so do calls of up to 32 averaged rows.
         const long tall_units = (long)B * H * ceil_div(p.q_rows, 64);
-        const bool tall = tight_stages == 0 && p.q_rows > 32 && tiles <= 32 &&
+        const bool tall = causal_single || (tight_stages == 0 && p.q_rows > 32 && tiles <= 32 &&
                           (D > 64 ? tiles > (narrow128 ? 12 : 14) && tall_units > kComputeUnits / 2
-                                  : (D < 64 ? tiles > 24 : raw && tiles > 27) && tall_units > 2 * kComputeUnits);
+                                  : (D < 64 ? tiles > 24 : raw && tiles > 27) && tall_units > 2 * kComputeUnits));
         double best_kg = 0.;
         bool any = false;
         for (int kg = tall ? 8 : (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {

@@ -1,6 +1,9 @@
 // Attention column means on gfx950 (MI355X): single-pass path with 64 query rows x up to 128 keys per wave, where the waves of
-// fcs_fused.hip own 32 rows x up to 256.  Non-causal calls of up to 1024 keys: heads of 65 .. 128 channels, and those of up to 64
-// with four key tiles per wave whose operand is not pre-scaled (make_plan says where, with both sides' times).
+// fcs_fused.hip own 32 rows x up to 256.  Calls of up to 1024 keys: non-causal ones of heads of 65 .. 128 channels, and of up to 64
+// with four key tiles per wave whose operand is not pre-scaled; causal ones (make_plan says where, with both sides' times).
+//
+// Causal calls: a key tile behind the last key that any of 32 rows sees has no exponents, one on the diagonal is masked after them.  (Its
+// MFMAs run all the same: a branch around a chain made the register allocator spill 400 registers.)
 //
 // What bounds the 32-row tile at 128 channels is moving operands, not arithmetic: every wave brings its own copy of its keys,
 // so that a row block of 64 rows x 1024 keys of 128 channels takes 576 KB through the L2 -> LDS path (about 65 B/clk
@@ -72,7 +75,7 @@ __device__ __forceinline__ void take_wait(half8 (&dst)[4])
 }  // namespace
 
 // DC: chunks of 64 channels.  TPW: 32-key tiles per wave.  NARROW: the head dim is less than DC x 64.
-template <int DC, int TPW, bool BF, bool NARROW>
+template <int DC, int TPW, bool BF, bool NARROW, bool CAUSAL>
 __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 {
     constexpr int NT = 4;                // MFMA steps per chunk of 64 channels
@@ -99,13 +102,19 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     }
     // the walk over units (head, row block of 64 rows), row blocks innermost
     const int h_begin = hgi * a.f_hpg, n_heads = min(a.H, h_begin + a.f_hpg) - h_begin;
-    const int rb_first = qwg * a.f_rbpw, rb_n = min(a.f_rbpw, a.f_nqblk - rb_first);
+    const int rb_first = qwg * a.f_rbpw;
+    // Causal row blocks see more and more keys: a workgroup takes every f_nwgq-th of them, there and back, so that all have alike.
+    auto row_block = [&](int r) { return !CAUSAL ? rb_first + r : (r & 1) ? (r + 1) * a.f_nwgq - 1 - qwg : r * a.f_nwgq + qwg; };
+    const int rb_n = CAUSAL ? a.f_rbpw - (row_block(a.f_rbpw - 1) >= a.f_nqblk ? 1 : 0) : min(a.f_rbpw, a.f_nqblk - rb_first);
     const int n_units = rb_n * n_heads;
-    // key tile t of the wave holds keys [kbase + 32 t, ..), moved back to end at the last key where it would reach past it; its
-    // columns then repeat keys of the tile before and count for nothing: those of a lane are t > tmax_lane
-    const int kbase = wave * TPW * 32;
-    auto tile_first = [&](int t) { return min(kbase + t * 32, a.Sk - 32); };
-    const int tmax_lane = (n + a.Sk - 32 - kbase) >> 5;
+    // key tile t of the wave holds keys [kbase + kstep t, ..), moved back to end at the last key where it would reach past it; its
+    // columns then repeat keys of the tile before and count for nothing: those of a lane are t > tmax_lane.  Causal calls deal the
+    // tiles to the waves in turn, so that the keys that a row block sees are spread over all of them.
+    const int kbase = CAUSAL ? wave * 32 : wave * TPW * 32;
+    constexpr int kstep = CAUSAL ? 256 : 32;
+    auto tile_first = [&](int t) { return min(kbase + t * kstep, a.Sk - 32); };
+    auto tiles_counted = [&](int l) { return (l + a.Sk - 32 - kbase) >> (CAUSAL ? 8 : 5); };  // arithmetic shift: floor, also when negative
+    const int tmax_lane = tiles_counted(n);
 
     const uint32_t q_row_b = (uint32_t)a.qs_s * 2u, k_row_b = (uint32_t)a.ks_s * 2u;
     const char *q_batch = reinterpret_cast<const char *>(a.q + (int64_t)b * a.qs_b);
@@ -188,7 +197,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     auto key_off = [&](int hr) { return (int64_t)kv_head(h_begin + hr, a.kv_group, a.kv_magic) * k_head_b; };
     int64_t k_cur = key_off(0);
 
-    fetch_q(h_begin, rb_first * 64, 0);
+    fetch_q(h_begin, row_block(0) * 64, 0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) fetch_item(k_cur, s % TPW, s / TPW, s);
     FCS_WAIT_VM(0);
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     // the scale with its sign (a score of negated query rows, times c, has the very bits of the score times -c); scalar
     const float cs = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, a.negate ? -a.c : a.c)));
     for (int unit = 0; unit < n_units; ++unit) {
-        const int h = h_begin + cur_hr, row0 = (rb_first + cur_rb) * 64;
+        const int h = h_begin + cur_hr, row0 = row_block(cur_rb) * 64;
         // the next unit (the last one is followed by itself)
         int nxt_rb = cur_rb, nxt_hr = cur_hr;
         if (unit + 1 < n_units && ++nxt_rb == rb_n) {
@@ -220,11 +229,24 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 
         floatx16 acc[2][TPW];
         float e[2][TPW][16];
-        auto exp_tile = [&](int nb, int t) {  // e = 2^(c s) in place, and into the row sums; a column that does not count: 2^-inf
+        // causal: the last key that all / any of 32 rows see; a tile behind the latter has no products and no exponents
+        auto seen_by_all = [&](int nb) { return a.k_past + row0 + nb * 32; };
+        auto hidden = [&](int nb, int t) { return CAUSAL && tile_first(tile_of(t)) > seen_by_all(nb) + 31; };
+        auto exp_tile = [&](int nb, int t) {  // e = 2^(c s); a column that does not count, a key that the row does not see: 2^-inf
             const float bias = tile_of(t) <= tmax_lane ? 0.f : -INFINITY;
+            const int key0 = tile_first(tile_of(t));
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                e[nb][t][i] = fast_exp2(fmaf(acc[nb][t][i], cs, bias));
+            for (int i = 0; i < 16; ++i) e[nb][t][i] = acc[nb][t][i];
+            if (!hidden(nb, t)) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) e[nb][t][i] = fast_exp2(fmaf(e[nb][t][i], cs, bias));
+            }
+            if (CAUSAL && key0 + 31 > seen_by_all(nb)) {  // (in place, and one-sided: else both sides' registers are live)
+                pin16(e[nb][t]);
+                int rel = key0 + n - seen_by_all(nb) - 4 * g;  // seen by the row of register i: rel <= 8 (i / 4) + i % 4
+                FCS_OPAQUE_V(rel);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) e[nb][t][i] = rel <= 8 * (i >> 2) + (i & 3) ? e[nb][t][i] : 0.f;
             }
             pin16(e[nb][t]);  // (else the exponents sink below the last MFMA)
         };
@@ -242,7 +264,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             }
             FCS_OPAQUE_V(k_take);  // addresses are formed where they are used
             take_wait(kf[s & 1]);
-            if (s == 0) fetch_q(h_begin + nxt_hr, (rb_first + nxt_rb) * 64, (unit + 1) & 1);
+            if (s == 0) fetch_q(h_begin + nxt_hr, row_block(nxt_rb) * 64, (unit + 1) & 1);
             // the slot is free: it takes the item of step s + NS, or the next key head's item that belongs in it
             if (s + NS < STEPS) fetch_item(k_cur, tile_of(s + NS), chunk_of(s + NS), slot_of(s));
             else if (next_key_head) fetch_item(k_nxt, slot_of(s) % TPW, slot_of(s) / TPW, slot_of(s));
@@ -339,10 +361,14 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             int lane_s = lane;
             FCS_OPAQUE_V(lane_s);
             const int n_s = lane_s & 31, g_s = lane_s >> 5;
-            const int tmax_s = (n_s + a.Sk - 32 - kbase) >> 5;
+            const int tmax_s = tiles_counted(n_s);
             const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_batch + k_cur) + g_s * 8;
             float v16[2][16];
             half8 qs[DC * NT];
+            // (register i: row 8 (i / 4) + 4 g + i % 4 of the 32)
+            auto counts = [&](int t, int nb, int i) {
+                return t <= tmax_s && (!CAUSAL || tile_first(t) + n_s <= seen_by_all(nb) + 8 * (i >> 2) + 4 * g_s + (i & 3));
+            };
             auto load_rows = [&](int nb) {
                 const _Float16 *qp = reinterpret_cast<const _Float16 *>(q_batch + (int64_t)h * q_head_b) +
                                      (int64_t)min(row0 + nb * 32 + n_s, a.Sq - 1) * a.qs_s + g_s * 8;
@@ -397,9 +423,8 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 #pragma unroll 1
                 for (int t = 0; t < TPW; ++t) {
                     const floatx16 c = score_tile(t);
-                    const bool real = t <= tmax_s;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v16[nb][i] = fmaxf(v16[nb][i], real ? c[i] : kNegBig);
+                    for (int i = 0; i < 16; ++i) v16[nb][i] = fmaxf(v16[nb][i], counts(t, nb, i) ? c[i] : kNegBig);
                 }
             }
             reduce(true, [](floatx4 x, floatx4 y) {
@@ -414,9 +439,8 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 #pragma unroll 1
                 for (int t = 0; t < TPW; ++t) {
                     const floatx16 c = score_tile(t);
-                    const bool real = t <= tmax_s;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v16[nb][i] += real ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f;
+                    for (int i = 0; i < 16; ++i) v16[nb][i] += counts(t, nb, i) ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f;
                 }
             }
             reduce(false, [&](floatx4 x, floatx4 y) {
@@ -430,10 +454,9 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 #pragma unroll 1
                 for (int t = 0; t < TPW; ++t) {
                     const floatx16 c = score_tile(t);
-                    const bool real = t <= tmax_s;
                     float sum = 0.f;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) sum = fmaf(real ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f, v16[nb][i], sum);
+                    for (int i = 0; i < 16; ++i) sum = fmaf(counts(t, nb, i) ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f, v16[nb][i], sum);
 #pragma unroll
                     for (int u = 0; u < TPW; ++u)  // col_acc lives in registers: static index only
                         if (u == t) col_acc[u] += sum;
@@ -456,22 +479,27 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     }
 }
 
-template <int TPW, bool BF>
-static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
+template <int DC, int TPW, bool NARROW, bool CAUSAL>
+static void launch_one(const Plan &p, const Args &a, hipStream_t st)
 {
     const dim3 grid(p.f_nwgq * p.B, p.f_hg);
-    if (p.D == 128) hipLaunchKernelGGL((fcs_tall_kernel<2, TPW, BF, false>), grid, dim3(512), 0, st, a);
-    else if (p.D > 64) hipLaunchKernelGGL((fcs_tall_kernel<2, TPW, BF, true>), grid, dim3(512), 0, st, a);
-    else if (p.D == 64) hipLaunchKernelGGL((fcs_tall_kernel<1, 4, BF, false>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((fcs_tall_kernel<1, 4, BF, true>), grid, dim3(512), 0, st, a);
+    if (p.bf16) hipLaunchKernelGGL((fcs_tall_kernel<DC, TPW, true, NARROW, CAUSAL>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((fcs_tall_kernel<DC, TPW, false, NARROW, CAUSAL>), grid, dim3(512), 0, st, a);
+}
+template <int DC, int TPW>
+static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
+{
+    const bool narrow = p.D != DC * 64;
+    if (p.causal) narrow ? launch_one<DC, TPW, true, true>(p, a, st) : launch_one<DC, TPW, false, true>(p, a, st);
+    else if constexpr (DC == 2 || TPW == 4) narrow ? launch_one<DC, TPW, true, false>(p, a, st) : launch_one<DC, TPW, false, false>(p, a, st);
 }
 
 hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
 {
-    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (p.D <= 64 && p.f_tpw != 4)) return hipErrorInvalidValue;
-    if (p.f_tpw == 2) p.bf16 ? launch_tpw<2, true>(p, a, st) : launch_tpw<2, false>(p, a, st);
-    else if (p.f_tpw == 3) p.bf16 ? launch_tpw<3, true>(p, a, st) : launch_tpw<3, false>(p, a, st);
-    else if (p.f_tpw == 4) p.bf16 ? launch_tpw<4, true>(p, a, st) : launch_tpw<4, false>(p, a, st);
+    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (!p.causal && p.D <= 64 && p.f_tpw != 4)) return hipErrorInvalidValue;
+    if (p.f_tpw == 2) p.D > 64 ? launch_tpw<2, 2>(p, a, st) : launch_tpw<1, 2>(p, a, st);
+    else if (p.f_tpw == 3) p.D > 64 ? launch_tpw<2, 3>(p, a, st) : launch_tpw<1, 3>(p, a, st);
+    else if (p.f_tpw == 4) p.D > 64 ? launch_tpw<2, 4>(p, a, st) : launch_tpw<1, 4>(p, a, st);
     else return hipErrorInvalidValue;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -482,8 +510,10 @@ hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
 size_t describe_tall(const Plan &p, const Args &a, char *buf, size_t n)
 {
     const char *bf = p.bf16 ? "true" : "false", *narrow = p.D % 64 ? "true" : "false";
-    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%s,%s> (for fcs_fused_kernel<%d,%d,true,0,%s,true%s> ) grid %d x %d, %d x %d units per workgroup, %d slabs",
-                           p.Dp / 64, p.f_tpw, bf, narrow, p.Dp, p.tall, bf, p.D % 64 ? ",true" : "", p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
+    char stands_for[64] = "";
+    if (!p.causal) snprintf(stands_for, sizeof stands_for, " (for fcs_fused_kernel<%d,%d,true,0,%s,true%s> )", p.Dp, p.tall, bf, p.D % 64 ? ",true" : "");
+    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%s,%s,%s>%s grid %d x %d, %d x %d units per workgroup, %d slabs", p.Dp / 64, p.f_tpw, bf, narrow,
+                           p.causal ? "true" : "false", stands_for, p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
     if (r < 0) return 0;
     const size_t len = (size_t)r;
     return len + describe_finalize(a, false, len < n ? buf + len : nullptr, len < n ? n - len : 0);

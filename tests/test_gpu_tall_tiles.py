@@ -94,3 +94,47 @@ def test_up_to_64_channels(s, d, hk):
         q[:, 5, s // 2] *= 60
         k[1, hk - 1, -1] *= 50
         _check(q, k, kw, 4)
+
+
+def _check_causal(q, k, kw):
+    t = _hip.plan_description(tuple(q.shape), tuple(k.shape), causal=True, bf16=q.dtype == torch.bfloat16, cls_n=kw.get("cls_len", -1),
+                              k_past=kw.get("k_past"), scale=kw.get("scale"))
+    assert re.match(r"fcs_tall_kernel<\d,%d,\w+,\w+,true>" % max(2, -(-k.shape[2] // 256)), t), t
+    print("causal tall tiles", tuple(q.shape), q.stride(), tuple(k.shape), q.dtype, kw, flush=True)
+    got = flash_colsum_ext(q, k, is_causal=True, out_dtype=torch.float32, **kw)
+    ref = torch.cat([colsum_ext_exact(q[b:b + 1], k[b:b + 1], is_causal=True, **kw) for b in range(q.shape[0])])
+    err = (got.double() - ref).abs()
+    assert torch.isfinite(got).all()
+    # (2^-126: probabilities that fp32 flushes to zero)
+    assert (err <= 1e-4).all() and (err <= 1e-3 * ref.abs() + 2.0 ** -126).all(), (err.max().item(), (err / ref).max().item())
+    assert torch.equal(got, flash_colsum_ext(q, k, is_causal=True, out_dtype=torch.float32, **kw))
+
+
+# prompts (square), windows, diagonals that start at and between tile edges, last tiles of one key, more rows than keys
+CAUSAL = [(300, 300, None), (257, 257, None), (512, 512, None), (700, 700, None), (769, 769, None), (1024, 1024, None), (33, 1000, None), (1, 900, None),
+          (16, 520, None), (64, 1024, None), (130, 600, 31), (65, 600, 32), (200, 993, 500), (300, 700, 0), (300, 700, 5000), (900, 400, 0), (400, 400, 7)]
+
+
+@pytest.mark.parametrize("q_len,k_len,k_past", CAUSAL)
+@pytest.mark.parametrize("d,dtype", [(64, torch.float16), (128, torch.bfloat16), (40, torch.bfloat16), (96, torch.float16)])
+def test_causal(q_len, k_len, k_past, d, dtype):
+    q, k = _make(1, 6, 6, q_len, k_len, d, dtype, layout="tokens" if k_len % 2 else "heads", seed=q_len + d)
+    _check_causal(q, k, {} if k_past is None else {"k_past": k_past})
+
+
+@pytest.mark.parametrize("which", ["row", "keys", "scale", "cls_len", "units"])
+@pytest.mark.parametrize("s,d", [(400, 64), (700, 72), (1000, 128)])
+def test_causal_rows_out_of_range_and_units(which, s, d):
+    """Row blocks that leave the unstabilised range; several heads and row blocks per workgroup, there and back."""
+    h = 360 if which == "units" else 9
+    q, k = _make(1, h, h // 3, s, s, d, torch.float16, seed=5)
+    kw = {}
+    if which == "row":
+        q[:, 3, [0, 70, s - 1]] *= 60
+    elif which == "keys":
+        k[:, 1, 5:s // 2] *= 40
+    elif which == "scale":
+        kw = {"scale": -0.7}
+    elif which == "cls_len":
+        kw = {"cls_len": 150}
+    _check_causal(q, k, kw)
