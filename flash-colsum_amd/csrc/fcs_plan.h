@@ -494,12 +494,16 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // S 2300 30.2 -> 12.1, 128 of them 29.9 -> 18.5; no size in between was slower.)
     const bool wide = D == 64 && tight_stages == 0;
     const int fused_max = narrow128 ? 63 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
-    // Causal calls of 257 .. 1024 keys whose heads are not laid end to end: the same, a mask on the tiles that the diagonal crosses and no
+    // Causal calls of 257 .. 2048 keys whose heads are not laid end to end: the same, a mask on the tiles that the diagonal crosses and no
     // exponents behind it.  Two passes cost three launches and both products for what is mostly latency; us per call, two passes -> here:
-    // H 32 S 1000 D 128 32.1 -> 21.5, H 16 S 800 D 64 21.2 -> 11.8, H 16 Q 100 K 1000 D 128 17.6 -> 11.6, H 2 S 300 D 128 14.6 -> 8.7;
-    // none of 17 sizes slower.  (One batch entry, as prompts and windows are: batches gain as much, B 64 H 16 S 1024 D 64 327 -> 257, but the
+    // up to 1024 keys, 64 rows per wave: H 32 S 1000 D 128 32.1 -> 21.5, H 16 S 800 D 64 21.2 -> 11.8, H 16 Q 100 K 1000 D 128 17.6 -> 11.6,
+    // H 2 S 300 D 128 14.6 -> 8.7; beyond, 32 rows: H 32 S 1500 D 128 48.3 -> 40.7, S 1200 D 64 36.7 -> 22.7, Q 128 K 2048 H 64 23.9 -> 16.0.
+    // Long prompts of many heads fill the chip in two passes, which leave out the products behind the diagonal too: H 64 S 2048 D 128
+    // 103.9 against 112.6, H 32 60.2 against 61.1 (H 24 53.6 -> 47.0; D 64, H 64 75.4 -> 75.2; Q 1024 K 2048 H 64 D 128 76.3 -> 60.3).
+    // (One batch entry, as prompts and windows are: batches gain as much, B 64 H 16 S 1024 D 64 327 -> 257, but the
     // tests of shares that cross batch entries hold such a call to two passes.)
-    const bool causal_single = causal && B == 1 && p.fold == 1 && D <= 128 && Sk > 256 && Sk <= 1024;
+    const bool long_prompt = Sk > 1792 && 2L * (Sk - Sq) < Sq && (long)B * H * ceil_div(p.q_rows, 32) >= (D > 64 ? 2000 : 4200);
+    const bool causal_single = causal && B == 1 && p.fold == 1 && D <= 128 && Sk > 256 && Sk <= 2048 && !long_prompt;
     if (causal_single || (!causal && Sk >= 32 && Sk <= fused_max && D <= 128)) {
         p.fused = 1;
         p.fold = 1;
@@ -532,7 +536,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         double best_kg = 0.;
         bool any = false;
         for (int kg = tall ? 8 : (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {
-            const int tpw = ceil_div(tiles, kg), nqblk = ceil_div(p.q_rows, tall ? 64 : 32 * (8 / kg));
+            const int tpw = ceil_div(tiles, kg), nqblk = ceil_div(p.q_rows, tall ? (tiles > 32 ? 32 : 64) : 32 * (8 / kg));
             if (!tall && kg > usual && (tight_stages != 0 || (long)B * H * nqblk > 2 * kComputeUnits)) break;
             // Units per workgroup: a unit is one (query block, head); a workgroup takes f_rbpw adjacent
             // query blocks times f_hpg heads.  One workgroup is resident per compute unit, so the launch

@@ -1,6 +1,7 @@
 // Attention column means on gfx950 (MI355X): single-pass path with 64 query rows x up to 128 keys per wave, where the waves of
 // fcs_fused.hip own 32 rows x up to 256.  Calls of up to 1024 keys: non-causal ones of heads of 65 .. 128 channels, and of up to 64
-// with four key tiles per wave whose operand is not pre-scaled; causal ones (make_plan says where, with both sides' times).
+// with four key tiles per wave whose operand is not pre-scaled; causal ones, which beyond 1024 keys (up to 2048) have 32 rows
+// per wave and five to eight key tiles (make_plan says where, with both sides' times).
 //
 // Causal calls: a key tile behind the last key that any of 32 rows sees has no exponents, one on the diagonal is masked after them.  (Its
 // MFMAs run all the same: a branch around a chain made the register allocator spill 400 registers.)
@@ -74,21 +75,22 @@ __device__ __forceinline__ void take_wait(half8 (&dst)[4])
 
 }  // namespace
 
-// DC: chunks of 64 channels.  TPW: 32-key tiles per wave.  NARROW: the head dim is less than DC x 64.
-template <int DC, int TPW, bool BF, bool NARROW, bool CAUSAL>
+// DC: chunks of 64 channels.  NB: 32-row fragments per wave.  TPW: 32-key tiles per wave.  NARROW: the head dim is less than DC x 64.
+template <int DC, int NB, int TPW, bool BF, bool NARROW, bool CAUSAL>
 __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 {
+    constexpr int ROWS = 32 * NB;
     constexpr int NT = 4;                // MFMA steps per chunk of 64 channels
     constexpr int STEPS = DC * TPW;      // ring items of a row block: half tiles, 32 keys x 64 channels; chunk by chunk
-    constexpr bool KEEP_ALL = DC == 1;   // every item of a key head stays in the ring
-    constexpr int NS = KEEP_ALL ? TPW : 3;              // ring slots per wave; item j of every row block lives in slot j % NS
+    constexpr bool KEEP_ALL = DC == 1 && NB == 2;   // every item of a key head stays in the ring
+    constexpr int NS = KEEP_ALL ? TPW : NB == 2 ? 3 : 4;              // ring slots per wave; item j of every row block lives in slot j % NS
     constexpr int ITEM = 4096;
-    constexpr int QROW = DC * 128, QTILE = 64 * QROW, QI = DC;  // QI: a wave's DMA instructions for its 8 query rows
+    constexpr int QROW = DC * 128, QTILE = ROWS * QROW, QI = (DC * NB + 1) / 2;  // QI: a wave's DMA instructions for its 8 query rows
     static_assert(KEEP_ALL || STEPS > NS, "the waits below count on a request at the first step");
     __shared__ __attribute__((aligned(256))) char ring[8 * NS * ITEM];
-    __shared__ __attribute__((aligned(256))) char qtile[2 * QTILE];  // 64 rows x 128 channels, double-buffered
-    __shared__ __attribute__((aligned(16))) float part[2 * 64 * 8];  // row sums per (row, wave), double-buffered
-    __shared__ __attribute__((aligned(16))) float wv[8 * 64];        // per wave: a value per row
+    __shared__ __attribute__((aligned(256))) char qtile[2 * QTILE];  // the unit's query rows, double-buffered
+    __shared__ __attribute__((aligned(16))) float part[2 * ROWS * 8];  // row sums per (row, wave), double-buffered
+    __shared__ __attribute__((aligned(16))) float wv[8 * ROWS];        // per wave: a value per row
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -100,7 +102,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         b = bx / a.f_nwgq;
         hgi = by;
     }
-    // the walk over units (head, row block of 64 rows), row blocks innermost
+    // the walk over units (head, row block of ROWS rows), row blocks innermost
     const int h_begin = hgi * a.f_hpg, n_heads = min(a.H, h_begin + a.f_hpg) - h_begin;
     const int rb_first = qwg * a.f_rbpw;
     // Causal row blocks see more and more keys: a workgroup takes every f_nwgq-th of them, there and back, so that all have alike.
@@ -158,16 +160,20 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             dma(src2 + k_voff[1], dst + 3072);
         }
     };
-    // the wave's 8 of a unit's 64 query rows: 4 rows x 256 bytes per instruction, position p of row r holds piece p ^ (r & 15);
+    // the wave's eighth of a unit's query rows: 4 rows x 256 bytes per instruction, position p of row r holds piece p ^ (r & 15) (one
+    // chunk: 8 rows x 128 bytes, as a key item);
     // rows past the last one repeat it (they are given no weight)
     auto fetch_q = [&](int head, int row0, int buf) {
         const char *slice = q_batch + (int64_t)head * q_head_b;
-        char *dst = qtile + buf * QTILE + wave * (8 * QROW);
+        // (32 rows of one chunk are four instructions: the waves 4 .. 7 bring what 0 .. 3 do, so that all count the same)
+        const int w = DC * NB == 1 ? wave & 3 : wave;
+        constexpr int RI = 1024 / QROW;  // rows of an instruction
+        char *dst = qtile + buf * QTILE + w * (QI * 1024);
         int l = lane;
         FCS_OPAQUE_V(l);
 #pragma unroll
         for (int i = 0; i < QI; ++i) {
-            const int r = DC == 2 ? wave * 8 + i * 4 + (l >> 4) : wave * 8 + (l >> 3);
+            const int r = (w * QI + i) * RI + (DC == 2 ? l >> 4 : l >> 3);
             const int piece = DC == 2 ? (l & 15) ^ (r & 15) : (l & 7) ^ ((r >> 1) & 7);
             const char *src = slice + (size_t)min(row0 + r, a.Sq - 1) * q_row_b + piece * 16;
             if (NARROW && piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_tall_zeros);
@@ -182,7 +188,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     float col_acc[TPW];
 #pragma unroll
     for (int t = 0; t < TPW; ++t) col_acc[t] = 0.f;
-    float *wv_w = wv + wave * 64;
+    float *wv_w = wv + wave * ROWS;
 
     // Two orders of the items alternate between the row blocks of a key head: 0 .. STEPS-1 and (rot) back.  Step s of a row block
     // works on item `item`, chunk item / TPW of key tile item % TPW; its scores are in acc[.][s % TPW], which is tile
@@ -191,13 +197,13 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     auto item_of = [&](int s) { return rot ? STEPS - 1 - s : s; };
     auto slot_of = [&](int s) { return rot ? (STEPS - 1 - s) % NS : s % NS; };
     auto tile_of = [&](int s) { return rot ? TPW - 1 - s % TPW : s % TPW; };
-    auto chunk_of = [&](int s) { return rot ? 1 - s / TPW : s / TPW; };
+    auto chunk_of = [&](int s) { return rot ? DC - 1 - s / TPW : s / TPW; };
 
     int cur_rb = 0, cur_hr = 0;  // row block and head of the current unit, relative
     auto key_off = [&](int hr) { return (int64_t)kv_head(h_begin + hr, a.kv_group, a.kv_magic) * k_head_b; };
     int64_t k_cur = key_off(0);
 
-    fetch_q(h_begin, row_block(0) * 64, 0);
+    fetch_q(h_begin, row_block(0) * ROWS, 0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) fetch_item(k_cur, s % TPW, s / TPW, s);
     FCS_WAIT_VM(0);
@@ -206,7 +212,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     // the scale with its sign (a score of negated query rows, times c, has the very bits of the score times -c); scalar
     const float cs = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, a.negate ? -a.c : a.c)));
     for (int unit = 0; unit < n_units; ++unit) {
-        const int h = h_begin + cur_hr, row0 = row_block(cur_rb) * 64;
+        const int h = h_begin + cur_hr, row0 = row_block(cur_rb) * ROWS;
         // the next unit (the last one is followed by itself)
         int nxt_rb = cur_rb, nxt_hr = cur_hr;
         if (unit + 1 < n_units && ++nxt_rb == rb_n) {
@@ -218,17 +224,17 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 
         // The query rows are in their tile since the barrier before.  The first NS key items are in the ring: left behind by the
         // unit before, or requested during its last steps.
-        half8 qf[2][NT], kf[2][NT];  // [32-row fragment]
+        half8 qf[NB][NT], kf[2][NT];  // [32-row fragment]
         FCS_OPAQUE_V(q_take);
         FCS_OPAQUE_V(k_take);
         const uint32_t q_at = q_take + (uint32_t)((unit & 1) * QTILE);
         take_issue<0>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[0]);
-        take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[1]);
+        if constexpr (NB == 2) take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[NB - 1]);
         FCS_WAIT_VM(0);
         take_issue<0>(k_take + (uint32_t)(slot_of(0) * ITEM), kf[0]);
 
-        floatx16 acc[2][TPW];
-        float e[2][TPW][16];
+        floatx16 acc[NB][TPW];
+        float e[NB][TPW][16];
         // causal: the last key that all / any of 32 rows see; a tile behind the latter has no products and no exponents
         auto seen_by_all = [&](int nb) { return a.k_past + row0 + nb * 32; };
         auto hidden = [&](int nb, int t) { return CAUSAL && tile_first(tile_of(t)) > seen_by_all(nb) + 31; };
@@ -260,11 +266,11 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             else asm volatile("s_setprio 0");
             if (t == 0) {
                 take_wait(qf[0]);
-                take_wait(qf[1]);
+                if constexpr (NB == 2) take_wait(qf[NB - 1]);
             }
             FCS_OPAQUE_V(k_take);  // addresses are formed where they are used
             take_wait(kf[s & 1]);
-            if (s == 0) fetch_q(h_begin + nxt_hr, row_block(nxt_rb) * 64, (unit + 1) & 1);
+            if (s == 0) fetch_q(h_begin + nxt_hr, row_block(nxt_rb) * ROWS, (unit + 1) & 1);
             // the slot is free: it takes the item of step s + NS, or the next key head's item that belongs in it
             if (s + NS < STEPS) fetch_item(k_cur, tile_of(s + NS), chunk_of(s + NS), slot_of(s));
             else if (next_key_head) fetch_item(k_nxt, slot_of(s) % TPW, slot_of(s) / TPW, slot_of(s));
@@ -273,7 +279,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             if (!KEEP_ALL && s + 1 >= NS && s + 1 < STEPS) FCS_WAIT_VM((STEPS - 2 - s < NS - 1 ? STEPS - 2 - s : NS - 1) * NT);
             if (s + 1 < STEPS) take_issue<0>(k_take + (uint32_t)(slot_of(s + 1) * ITEM), kf[(s + 1) & 1]);
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
+            for (int nb = 0; nb < NB; ++nb) {
                 floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                 if (half) c = acc[nb][t];
 #pragma unroll
@@ -281,17 +287,17 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                 acc[nb][t] = c;
             }
             if (DC == 2 && s == TPW - 1) {  // the other chunk of the query rows, behind the last chain that reads the first
-                asm volatile("" : "+v"(acc[0][t]), "+v"(acc[1][t]));
+                asm volatile("" : "+v"(acc[0][t]), "+v"(acc[NB - 1][t]));
                 take_issue<0>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[0]);
-                take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[1]);
+                if constexpr (NB == 2) take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[NB - 1]);
             }
             if (half == DC - 1 && t > 0) {  // VALU work of the tile before under this one's MFMAs
                 exp_tile(0, t - 1);
-                exp_tile(1, t - 1);
+                if (NB == 2) exp_tile(NB - 1, t - 1);
             }
         }
         exp_tile(0, TPW - 1);
-        exp_tile(1, TPW - 1);
+        if (NB == 2) exp_tile(NB - 1, TPW - 1);
 
         if (KEEP_ALL) {  // the next unit's query rows have landed: behind them is the next key head, or nothing
             if (next_key_head) FCS_WAIT_VM(STEPS * NT);
@@ -299,7 +305,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         }
 
         // ---------------- row sums over lanes and waves: one barrier, which also publishes the next unit's query rows
-        float *pt = part + (unit & 1) * 512;
+        float *pt = part + (unit & 1) * (ROWS * 8);
         // the row (of 32) whose total over this wave's keys a lane is left with, like its neighbour
         int lane_r = lane;
         FCS_OPAQUE_V(lane_r);  // addresses are formed here, not kept through phase 1
@@ -309,21 +315,23 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             if ((lane_r & 1) == 0) pt[(nb * 32 + row_w) * 8 + wave] = v;
         };
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
             float rs[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 rs[i] = e[nb][0][i] + e[nb][1][i];
-                if (TPW == 3) rs[i] += e[nb][TPW - 1][i];
-                if (TPW == 4) rs[i] += e[nb][TPW - 2][i] + e[nb][TPW - 1][i];
+#pragma unroll
+                for (int t = 2; t + 1 < TPW; t += 2) rs[i] += e[nb][t][i] + e[nb][t + 1][i];
+                if (TPW % 2) rs[i] += e[nb][TPW - 1][i];
             }
             fold_rows(nb, fold_lanes_sum(rs, lane_r));
         }
         __syncthreads();
-        // lane L adds up row L; every wave sees all of the rows' parts
+        // lane L adds up row L (32 rows: the upper half-wave does what the lower does); every wave sees all of the rows' parts
         bool slow;
         {
-            const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + lane_r * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + lane_r * 8 + 4);
+            const int row = lane_r & (ROWS - 1);
+            const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + row * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + row * 8 + 4);
             const float tot = ((f0[0] + f0[1]) + (f0[2] + f0[3])) + ((f1[0] + f1[1]) + (f1[2] + f1[3]));
             bool ok = true;
             float most = 0.f;
@@ -333,7 +341,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                 most = fmaxf(most, fmaxf(f0[j], f1[j]));
             }
             slow = __builtin_amdgcn_ballot_w64(!ok || !(most >= kSumLo)) != 0;
-            wv_w[lane_r] = (row0 + lane_r < a.q_rows) ? __builtin_amdgcn_rcpf(tot) : 0.f;
+            wv_w[row] = (row0 + row < a.q_rows) ? __builtin_amdgcn_rcpf(tot) : 0.f;
             __builtin_amdgcn_wave_barrier();
         }
 
@@ -343,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 #pragma unroll
             for (int t = 0; t < TPW; ++t) sum[t] = 0.f;
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
                     const floatx4 w4 = *reinterpret_cast<const floatx4 *>(wv_w + nb * 32 + 8 * i4 + 4 * g_r);
@@ -363,7 +371,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             const int n_s = lane_s & 31, g_s = lane_s >> 5;
             const int tmax_s = tiles_counted(n_s);
             const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_batch + k_cur) + g_s * 8;
-            float v16[2][16];
+            float v16[NB][16];
             half8 qs[DC * NT];
             // (register i: row 8 (i / 4) + 4 g + i % 4 of the 32)
             auto counts = [&](int t, int nb, int i) {
@@ -394,16 +402,17 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             // part buffer's last readers.
             auto reduce = [&](bool is_max, auto f) {
 #pragma unroll
-                for (int nb = 0; nb < 2; ++nb) v16[nb][0] = is_max ? fold_lanes_max(v16[nb], lane_s) : fold_lanes_sum(v16[nb], lane_s);
+                for (int nb = 0; nb < NB; ++nb) v16[nb][0] = is_max ? fold_lanes_max(v16[nb], lane_s) : fold_lanes_sum(v16[nb], lane_s);
                 __syncthreads();
                 const int rw = 16 * ((lane_s >> 4) & 1) + 8 * ((lane_s >> 3) & 1) + 4 * g_s + 2 * ((lane_s >> 2) & 1) + ((lane_s >> 1) & 1);
                 if ((lane_s & 1) == 0) {
                     pt[rw * 8 + wave] = v16[0][0];
-                    pt[(32 + rw) * 8 + wave] = v16[1][0];
+                    if (NB == 2) pt[(32 + rw) * 8 + wave] = v16[NB - 1][0];
                 }
                 __syncthreads();
-                const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + lane_s * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + lane_s * 8 + 4);
-                wv_w[lane_s] = f(f0, f1);
+                const int row = lane_s & (ROWS - 1);
+                const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + row * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + row * 8 + 4);
+                wv_w[row] = f(row, f0, f1);
                 __builtin_amdgcn_wave_barrier();
             };
             auto row_values = [&](float (&v)[16], int nb) {
@@ -414,9 +423,9 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                     for (int j = 0; j < 4; ++j) v[4 * i4 + j] = x[j];
                 }
             };
-            float rmax[2][16];
+            float rmax[NB][16];
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
+            for (int nb = 0; nb < NB; ++nb) {
                 load_rows(nb);
 #pragma unroll
                 for (int i = 0; i < 16; ++i) v16[nb][i] = kNegBig;
@@ -427,11 +436,11 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                     for (int i = 0; i < 16; ++i) v16[nb][i] = fmaxf(v16[nb][i], counts(t, nb, i) ? c[i] : kNegBig);
                 }
             }
-            reduce(true, [](floatx4 x, floatx4 y) {
+            reduce(true, [](int, floatx4 x, floatx4 y) {
                 return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])));
             });
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
+            for (int nb = 0; nb < NB; ++nb) {
                 row_values(rmax[nb], nb);  // subtracted from the scores before the scale
                 load_rows(nb);
 #pragma unroll
@@ -443,12 +452,12 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                     for (int i = 0; i < 16; ++i) v16[nb][i] += counts(t, nb, i) ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f;
                 }
             }
-            reduce(false, [&](floatx4 x, floatx4 y) {
+            reduce(false, [&](int row, floatx4 x, floatx4 y) {
                 const float L = ((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]));
-                return (row0 + lane_s < a.q_rows) ? __builtin_amdgcn_rcpf(L) : 0.f;
+                return (row0 + row < a.q_rows) ? __builtin_amdgcn_rcpf(L) : 0.f;
             });
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
+            for (int nb = 0; nb < NB; ++nb) {
                 row_values(v16[nb], nb);
                 load_rows(nb);
 #pragma unroll 1
@@ -479,28 +488,41 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     }
 }
 
-template <int DC, int TPW, bool NARROW, bool CAUSAL>
+template <int DC, int NB, int TPW, bool NARROW, bool CAUSAL>
 static void launch_one(const Plan &p, const Args &a, hipStream_t st)
 {
     const dim3 grid(p.f_nwgq * p.B, p.f_hg);
-    if (p.bf16) hipLaunchKernelGGL((fcs_tall_kernel<DC, TPW, true, NARROW, CAUSAL>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((fcs_tall_kernel<DC, TPW, false, NARROW, CAUSAL>), grid, dim3(512), 0, st, a);
+    if (p.bf16) hipLaunchKernelGGL((fcs_tall_kernel<DC, NB, TPW, true, NARROW, CAUSAL>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((fcs_tall_kernel<DC, NB, TPW, false, NARROW, CAUSAL>), grid, dim3(512), 0, st, a);
 }
-template <int DC, int TPW>
+template <int DC, int NB, int TPW>
 static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
 {
     const bool narrow = p.D != DC * 64;
-    if (p.causal) narrow ? launch_one<DC, TPW, true, true>(p, a, st) : launch_one<DC, TPW, false, true>(p, a, st);
-    else if constexpr (DC == 2 || TPW == 4) narrow ? launch_one<DC, TPW, true, false>(p, a, st) : launch_one<DC, TPW, false, false>(p, a, st);
+    if (p.causal) narrow ? launch_one<DC, NB, TPW, true, true>(p, a, st) : launch_one<DC, NB, TPW, false, true>(p, a, st);
+    else if constexpr (NB == 2 && (DC == 2 || TPW == 4))
+        narrow ? launch_one<DC, NB, TPW, true, false>(p, a, st) : launch_one<DC, NB, TPW, false, false>(p, a, st);
+}
+template <int DC>
+static bool launch_dc(const Plan &p, const Args &a, hipStream_t st)
+{
+    switch (p.f_tpw) {
+    case 2: launch_tpw<DC, 2, 2>(p, a, st); break;
+    case 3: launch_tpw<DC, 2, 3>(p, a, st); break;
+    case 4: launch_tpw<DC, 2, 4>(p, a, st); break;
+    case 5: launch_tpw<DC, 1, 5>(p, a, st); break;
+    case 6: launch_tpw<DC, 1, 6>(p, a, st); break;
+    case 7: launch_tpw<DC, 1, 7>(p, a, st); break;
+    case 8: launch_tpw<DC, 1, 8>(p, a, st); break;
+    default: return false;
+    }
+    return true;
 }
 
 hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
 {
-    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (!p.causal && p.D <= 64 && p.f_tpw != 4)) return hipErrorInvalidValue;
-    if (p.f_tpw == 2) p.D > 64 ? launch_tpw<2, 2>(p, a, st) : launch_tpw<1, 2>(p, a, st);
-    else if (p.f_tpw == 3) p.D > 64 ? launch_tpw<2, 3>(p, a, st) : launch_tpw<1, 3>(p, a, st);
-    else if (p.f_tpw == 4) p.D > 64 ? launch_tpw<2, 4>(p, a, st) : launch_tpw<1, 4>(p, a, st);
-    else return hipErrorInvalidValue;
+    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (!p.causal && (p.f_tpw > 4 || (p.D <= 64 && p.f_tpw != 4)))) return hipErrorInvalidValue;
+    if (!(p.D > 64 ? launch_dc<2>(p, a, st) : launch_dc<1>(p, a, st))) return hipErrorInvalidValue;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return launch_finalize(a, st);
@@ -512,7 +534,7 @@ size_t describe_tall(const Plan &p, const Args &a, char *buf, size_t n)
     const char *bf = p.bf16 ? "true" : "false", *narrow = p.D % 64 ? "true" : "false";
     char stands_for[64] = "";
     if (!p.causal) snprintf(stands_for, sizeof stands_for, " (for fcs_fused_kernel<%d,%d,true,0,%s,true%s> )", p.Dp, p.tall, bf, p.D % 64 ? ",true" : "");
-    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%s,%s,%s>%s grid %d x %d, %d x %d units per workgroup, %d slabs", p.Dp / 64, p.f_tpw, bf, narrow,
+    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%d,%s,%s,%s>%s grid %d x %d, %d x %d units per workgroup, %d slabs", p.Dp / 64, p.f_tpw > 4 ? 1 : 2, p.f_tpw, bf, narrow,
                            p.causal ? "true" : "false", stands_for, p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
     if (r < 0) return 0;
     const size_t len = (size_t)r;
