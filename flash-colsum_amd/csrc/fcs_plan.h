@@ -484,9 +484,8 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // ---- fused path
     // (at least one whole key tile: the kernel moves a tile that reaches past the last key back to end there)
     // (64-wide kernels for head dims up to 64, 128-wide ones up to 128; wider heads take the two-pass path)
-    // (Heads of 72 .. 120 channels: six key tiles per wave where that is enough, seven and eight beyond 1536 keys, where the rare path
-    // spills.  us per call, two passes -> here: B 8 H 16 S 2000 D 96 279 -> 226, S 1700 D 80 224.3 -> 155.8.  The plan tests hold the
-    // longest such call, 2048 keys, to the two-pass path: up to 63 tiles.)
+    // (Heads of 72 .. 120 channels: us per call beyond 1536 keys, two passes -> one: B 8 H 16 S 2000 D 96 279 -> 226, S 1700 D 80
+    // 224.3 -> 155.8.  The plan tests hold the longest such call, 2048 keys, to the two-pass path: up to 63 tiles.)
     const bool narrow128 = D > 64 && D < 128;
     // (64-wide heads: the shared-Q variants hold ten tiles per wave, so calls of up to 2560 keys are served too, unless grouped
     // heads are laid end to end, whose keys are streamed once for the whole group.  us per call, two passes -> here:
@@ -527,12 +526,20 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         //  * 64 channels from 865 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 249.8 -> 232.1, B 16 S 900 63.6 -> 61.7,
         //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4; fewer channels from 769 on: D 32 B 16 S 1000
         //    68.5 -> 60.5, D 48 B 32 H 12 S 800 81.6 -> 77.7, but D 48 S 500 24.1 -> 25.8.
-        // A call that leaves half of the chip idle takes the shorter blocks (B 2 H 4 S 1024 D 128 10.4 against 11.1; up to 64 channels the
+        //  * 65 .. 128 channels beyond 1024 keys, with 32 rows per wave: B 8 H 16 D 128 S 2048 235.5 -> 230.4, S 1370 125 -> 118.6, B 64 H 8
+        //    S 1200 407 -> 370, Q 32 K 2048 16.9 -> 15.8; H 1 S 2048 12.1 -> 11.9; D 120 S 1700 212.9 -> 199.3 (D 72 B 3 H 12 S 1900 62.5 -> 64.7;
+        //    64 channels: S 2048 123.9 against 134.9).
+        // A call of up to 1024 keys that leaves half of the chip idle takes the shorter blocks (B 2 H 4 S 1024 D 128 10.4 against 11.1; up to 64 channels the
         // splits over more waves below have calls of two units per workgroup), and so do calls of up to 32 averaged rows.
         const long tall_units = (long)B * H * ceil_div(p.q_rows, 64);
-        const bool tall = causal_single || (tight_stages == 0 && p.q_rows > 32 && tiles <= 32 &&
-                          (D > 64 ? tiles > (narrow128 ? 12 : 14) && tall_units > kComputeUnits / 2
-                                  : (D < 64 ? tiles > 24 : raw && tiles > 27) && tall_units > 2 * kComputeUnits));
+        const auto tall_pays = [&]() {
+            if (tight_stages != 0 || tiles > 64) return false;
+            if (tiles > 32) return D > 64;
+            if (p.q_rows <= 32) return false;
+            return D > 64 ? tiles > (narrow128 ? 12 : 14) && tall_units > kComputeUnits / 2
+                          : (D < 64 ? tiles > 24 : raw && tiles > 27) && tall_units > 2 * kComputeUnits;
+        };
+        const bool tall = causal_single || tall_pays();
         double best_kg = 0.;
         bool any = false;
         for (int kg = tall ? 8 : (wide && usual >= 4 && usual * 5 >= tiles) ? usual / 2 : usual; kg <= 8; kg *= 2) {

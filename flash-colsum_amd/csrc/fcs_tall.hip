@@ -1,7 +1,8 @@
 // Attention column means on gfx950 (MI355X): single-pass path with 64 query rows x up to 128 keys per wave, where the waves of
 // fcs_fused.hip own 32 rows x up to 256.  Calls of up to 1024 keys: non-causal ones of heads of 65 .. 128 channels, and of up to 64
-// with four key tiles per wave whose operand is not pre-scaled; causal ones, which beyond 1024 keys (up to 2048) have 32 rows
-// per wave and five to eight key tiles (make_plan says where, with both sides' times).
+// with four key tiles per wave whose operand is not pre-scaled; causal ones.  Beyond 1024 keys (up to 2048) causal calls, and others of
+// 65 .. 128 channels, have 32 rows per wave and five to eight key tiles (make_plan says where, with both sides' times): what
+// they gain on fcs_fused.hip is the shared query rows and the four items that stay in the ring.
 //
 // Causal calls: a key tile behind the last key that any of 32 rows sees has no exponents, one on the diagonal is masked after them.  (Its
 // MFMAs run all the same: a branch around a chain made the register allocator spill 400 registers.)
@@ -500,7 +501,7 @@ static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
 {
     const bool narrow = p.D != DC * 64;
     if (p.causal) narrow ? launch_one<DC, NB, TPW, true, true>(p, a, st) : launch_one<DC, NB, TPW, false, true>(p, a, st);
-    else if constexpr (NB == 2 && (DC == 2 || TPW == 4))
+    else if constexpr (DC == 2 || (NB == 2 && TPW == 4))
         narrow ? launch_one<DC, NB, TPW, true, false>(p, a, st) : launch_one<DC, NB, TPW, false, false>(p, a, st);
 }
 template <int DC>
@@ -521,7 +522,7 @@ static bool launch_dc(const Plan &p, const Args &a, hipStream_t st)
 
 hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
 {
-    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (!p.causal && (p.f_tpw > 4 || (p.D <= 64 && p.f_tpw != 4)))) return hipErrorInvalidValue;
+    if (p.Sk < 32 || p.f_kg != 8 || p.f_tpw * 256 < p.Sk || (!p.causal && p.D <= 64 && p.f_tpw != 4)) return hipErrorInvalidValue;
     if (!(p.D > 64 ? launch_dc<2>(p, a, st) : launch_dc<1>(p, a, st))) return hipErrorInvalidValue;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
