@@ -16,16 +16,17 @@
 //   * the 64 query rows come once per workgroup, by DMA into an LDS tile that all waves read;
 //   * the ring's last three items stay for the next row block of the same key head, which walks them in the opposite order; of 64-wide
 //     heads all of them stay, and a key head is fetched once per workgroup.
-// B 8 H 16 S 1024 D 128 bf16 60.1 -> 47.7 us per call.  What is left there: without the key fetches it would be 7 % faster,
+// B 8 H 16 S 1024 D 128 bf16 60.1 -> 47.2 us per call.  What is left there: without the key fetches it would be 7 % faster,
 // without three of four MFMAs 14 %, without phase 3 5 %.  64-wide heads are bound by the exponents either way: bf16 B 64 H 16 S 1024
 // 256.9 -> 239.7.  (Their pre-scaled operand was tried: 245 -> 231 at B 64, 2 .. 13 % slower with two and three tiles per wave, and
 // the rows' way through registers cannot be expressed safely in a loop with two waits; not built.)
 //
-// The scores of a wave (2 x 4 tiles) fill 128 registers as there.  Both chunks of 64 channels of wide query rows would take another
-// 64, which is more than there is: all tiles take the first chunk's products, then all take the second's, and only one
-// chunk of the rows is held at a time.  The exponents run under the second chunk's MFMAs.  The row sums are added up behind
-// them: running sums in phase 1 would be 32 registers more and were 4 % slower; and the rare path is marked as such,
-// since the register allocator otherwise spilled a tile's exponentials to spare it (67 us at B 8, H 16, S 1024).
+// The scores of a wave (2 x 4 tiles) fill 128 registers as there, both chunks of 64 channels of wide query rows 64, two half tiles of
+// keys 32.  A tile's exponents run under the next tile's MFMAs, a 32-row fragment under each chunk's.  (All tiles' first chunks, then all
+// second ones, with one chunk of the rows in registers at a time, has MFMAs alone in its first half: S 1024 D 96 52.0 against
+// 49.5 us, D 128 52.5 against 51.8, S 1300 D 128 113.3 against 109.1.)  What makes room: the row sums are added up behind
+// phase 1 (running sums would be 32 registers more; they spilled, or were 4 % slower), and the rare path is marked as such,
+// since the register allocator otherwise spilled a tile's exponentials to spare it (67 us at B 8, H 16, S 1024, D 128).
 //
 // The rest is fcs_fused.hip's: e = 2^(c s) without max subtraction while every row sum lands in [2^-80, 2^120), in-lane
 // column sums, one barrier per row block, a slab of column sums per workgroup; a row block outside the range is redone
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 {
     constexpr int ROWS = 32 * NB;
     constexpr int NT = 4;                // MFMA steps per chunk of 64 channels
-    constexpr int STEPS = DC * TPW;      // ring items of a row block: half tiles, 32 keys x 64 channels; chunk by chunk
+    constexpr int STEPS = DC * TPW;      // ring items of a row block: (half) tiles, 32 keys x 64 channels; the chunks of a tile one after the other
     constexpr bool KEEP_ALL = DC == 1 && NB == 2;   // every item of a key head stays in the ring
     constexpr int NS = KEEP_ALL ? TPW : NB == 2 ? 3 : 4;              // ring slots per wave; item j of every row block lives in slot j % NS
     constexpr int ITEM = 4096;
@@ -191,14 +192,13 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     for (int t = 0; t < TPW; ++t) col_acc[t] = 0.f;
     float *wv_w = wv + wave * ROWS;
 
-    // Two orders of the items alternate between the row blocks of a key head: 0 .. STEPS-1 and (rot) back.  Step s of a row block
-    // works on item `item`, chunk item / TPW of key tile item % TPW; its scores are in acc[.][s % TPW], which is tile
-    // s % TPW or (rot) TPW - 1 - s % TPW.
+    // Two orders of the items alternate between the row blocks of a key head: 0 .. STEPS-1 and (rot) back.  Item j is chunk j % DC of key
+    // tile j / DC; the scores of step s are in acc[.][s / DC], which is tile s / DC or (rot) TPW - 1 - s / DC.
     int rot = 0;
-    auto item_of = [&](int s) { return rot ? STEPS - 1 - s : s; };
     auto slot_of = [&](int s) { return rot ? (STEPS - 1 - s) % NS : s % NS; };
-    auto tile_of = [&](int s) { return rot ? TPW - 1 - s % TPW : s % TPW; };
-    auto chunk_of = [&](int s) { return rot ? DC - 1 - s / TPW : s / TPW; };
+    auto tile_of = [&](int s) { return rot ? TPW - 1 - s / DC : s / DC; };  // of step s
+    auto chunk_of = [&](int s) { return rot ? DC - 1 - s % DC : s % DC; };
+    auto tile_at = [&](int t) { return rot ? TPW - 1 - t : t; };  // of accumulator t
 
     int cur_rb = 0, cur_hr = 0;  // row block and head of the current unit, relative
     auto key_off = [&](int hr) { return (int64_t)kv_head(h_begin + hr, a.kv_group, a.kv_magic) * k_head_b; };
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 
     fetch_q(h_begin, row_block(0) * ROWS, 0);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) fetch_item(k_cur, s % TPW, s / TPW, s);
+    for (int s = 0; s < NS; ++s) fetch_item(k_cur, s / DC, s % DC, s);
     FCS_WAIT_VM(0);
     __syncthreads();
 
@@ -225,12 +225,15 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 
         // The query rows are in their tile since the barrier before.  The first NS key items are in the ring: left behind by the
         // unit before, or requested during its last steps.
-        half8 qf[NB][NT], kf[2][NT];  // [32-row fragment]
+        half8 qf[DC][NB][NT], kf[2][NT];  // [chunk][32-row fragment]
         FCS_OPAQUE_V(q_take);
         FCS_OPAQUE_V(k_take);
         const uint32_t q_at = q_take + (uint32_t)((unit & 1) * QTILE);
-        take_issue<0>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[0]);
-        if constexpr (NB == 2) take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(0) * 128), qf[NB - 1]);
+#pragma unroll
+        for (int dc = 0; dc < DC; ++dc) {
+            take_issue<0>(q_at ^ (uint32_t)(chunk_of(dc) * 128), qf[dc][0]);
+            if constexpr (NB == 2) take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(dc) * 128), qf[dc][NB - 1]);
+        }
         FCS_WAIT_VM(0);
         take_issue<0>(k_take + (uint32_t)(slot_of(0) * ITEM), kf[0]);
 
@@ -238,10 +241,10 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         float e[NB][TPW][16];
         // causal: the last key that all / any of 32 rows see; a tile behind the latter has no products and no exponents
         auto seen_by_all = [&](int nb) { return a.k_past + row0 + nb * 32; };
-        auto hidden = [&](int nb, int t) { return CAUSAL && tile_first(tile_of(t)) > seen_by_all(nb) + 31; };
+        auto hidden = [&](int nb, int t) { return CAUSAL && tile_first(tile_at(t)) > seen_by_all(nb) + 31; };
         auto exp_tile = [&](int nb, int t) {  // e = 2^(c s); a column that does not count, a key that the row does not see: 2^-inf
-            const float bias = tile_of(t) <= tmax_lane ? 0.f : -INFINITY;
-            const int key0 = tile_first(tile_of(t));
+            const float bias = tile_at(t) <= tmax_lane ? 0.f : -INFINITY;
+            const int key0 = tile_first(tile_at(t));
 #pragma unroll
             for (int i = 0; i < 16; ++i) e[nb][t][i] = acc[nb][t][i];
             if (!hidden(nb, t)) {
@@ -261,20 +264,23 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         // ---------------- phase 1
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
-            const int half = s / TPW, t = s % TPW;
+            const int dc = s % DC, t = s / DC;
             // (the two waves of a SIMD take turns at the higher priority, as in fcs_fused.hip)
             if (((s & 1) != 0) == (wave >= 4)) asm volatile("s_setprio 2");
             else asm volatile("s_setprio 0");
-            if (t == 0) {
-                take_wait(qf[0]);
-                if constexpr (NB == 2) take_wait(qf[NB - 1]);
+            if (s == 0) {
+#pragma unroll
+                for (int dc = 0; dc < DC; ++dc) {
+                    take_wait(qf[dc][0]);
+                    if constexpr (NB == 2) take_wait(qf[dc][NB - 1]);
+                }
             }
             FCS_OPAQUE_V(k_take);  // addresses are formed where they are used
             take_wait(kf[s & 1]);
             if (s == 0) fetch_q(h_begin + nxt_hr, row_block(nxt_rb) * ROWS, (unit + 1) & 1);
             // the slot is free: it takes the item of step s + NS, or the next key head's item that belongs in it
             if (s + NS < STEPS) fetch_item(k_cur, tile_of(s + NS), chunk_of(s + NS), slot_of(s));
-            else if (next_key_head) fetch_item(k_nxt, slot_of(s) % TPW, slot_of(s) / TPW, slot_of(s));
+            else if (next_key_head) fetch_item(k_nxt, slot_of(s) / DC, slot_of(s) % DC, slot_of(s));
             // Item s + 1 has landed once at most the items requested behind it are outstanding (step s + 1 - NS requested it; the
             // last step that requests one of this unit is STEPS - NS - 1).  The query rows, requested before all of them, have too.
             if (!KEEP_ALL && s + 1 >= NS && s + 1 < STEPS) FCS_WAIT_VM((STEPS - 2 - s < NS - 1 ? STEPS - 2 - s : NS - 1) * NT);
@@ -282,19 +288,14 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                if (half) c = acc[nb][t];
+                if (dc) c = acc[nb][t];
 #pragma unroll
-                for (int tt = 0; tt < NT; ++tt) c = mfma16<BF>(qf[nb][tt], kf[s & 1][tt], c);
+                for (int tt = 0; tt < NT; ++tt) c = mfma16<BF>(qf[dc][nb][tt], kf[s & 1][tt], c);
                 acc[nb][t] = c;
             }
-            if (DC == 2 && s == TPW - 1) {  // the other chunk of the query rows, behind the last chain that reads the first
-                asm volatile("" : "+v"(acc[0][t]), "+v"(acc[NB - 1][t]));
-                take_issue<0>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[0]);
-                if constexpr (NB == 2) take_issue<32 * QROW>(q_at ^ (uint32_t)(chunk_of(TPW) * 128), qf[NB - 1]);
-            }
-            if (half == DC - 1 && t > 0) {  // VALU work of the tile before under this one's MFMAs
-                exp_tile(0, t - 1);
-                if (NB == 2) exp_tile(NB - 1, t - 1);
+            if (t > 0) {  // VALU work of the tile before under this one's MFMAs, spread over its steps
+                if (dc == 0) exp_tile(0, t - 1);
+                if (NB == 2 && dc == DC - 1) exp_tile(NB - 1, t - 1);
             }
         }
         exp_tile(0, TPW - 1);
