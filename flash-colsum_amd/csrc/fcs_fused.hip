@@ -1,6 +1,8 @@
 // Attention column means on gfx950 (MI355X): fused single-kernel path for non-causal
 // calls whose whole key range fits in one workgroup's registers (32 <= S_k <= 2560, head dims up to 128:
-// 64 channels natively, 128 as two 64-channel chunks, anything narrower on one of those two with zeros in Q).
+// 64 channels natively, 128 as two 64-channel chunks, anything narrower on one of those two with zeros in Q).  Most calls of 65 .. 128
+// channels, and 64-wide ones near 1024 keys that are not pre-scaled, go to fcs_tall.hip; of wide heads, calls of up to 448 keys and small ones
+// of up to 1024 stay here.
 //
 // One workgroup = 8 waves.  The waves form a (query group) x (key group) grid; a wave
 // computes the 32 x (32 * tiles) block of scores  S = Q_tile * K_tile^T  for its 32 query

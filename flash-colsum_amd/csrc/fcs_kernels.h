@@ -70,7 +70,7 @@ __device__ __forceinline__ void fetch_args(const Args &a)
 // Enqueues every kernel of one call on `stream`; returns 0 or the hipError_t of a failed launch.
 int launch_colsum(const Plan &p, const Args &a, void *stream);
 
-// fused path, defined in fcs_fused.hip
+// fused path, defined in fcs_fused.hip, and (p.tall) fcs_tall.hip
 hipError_t launch_fused(const Plan &p, const Args &a, hipStream_t st);
 hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st);
 // few-rows path (fcs_fewrows.hip): p.fewrows == 1

@@ -1,4 +1,6 @@
 // Attention column means on gfx950 (MI355X): the kernels of the general two-pass path.  The column pass comes first.
+// (Causal calls of one batch entry and up to 2048 keys are mostly served by fcs_tall.hip; where such a size is quoted below, it was
+// measured here.)
 // (Templates; fcs_stream_{rows,cols}.hip and fcs_stream_{rows,cols}_grouped.hip instantiate one pass each, so that the
 // four compile side by side.)
 //
