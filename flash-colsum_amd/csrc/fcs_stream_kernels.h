@@ -301,6 +301,10 @@ __device__ __forceinline__ half8 prescale(half8 v, float cs)
 template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD, bool ONE>
 __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args a)
 {
+    // A workgroup with one chunk of one unit streams the stages that all its rows see backwards: pass 1 has just read the same keys forwards on the
+    // same XCD, and its last ones are what the L2 still holds.  us per call on changing keys, forwards -> backwards: H 32 Q 128 K 16384 D 128
+    // 68.2 -> 65.6, 4 x 32 heads on 8, Q 64 K 8192 64.2 -> 61.7; same bits (a key's sums do not depend on the stages' order).
+    constexpr bool REV = ONE && !PRE;
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
     constexpr int THREADS = 64 * WAVES;
     constexpr int NT = D / 16;                 // MFMA steps along the head dim
@@ -426,6 +430,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
             else continue;
         }
         const int n_whole = (D == 64 || a.D == D) ? min(nst, (a.Sk - c0) / KT) : 0;  // stages inside the tensor, of rows as wide as compiled (64: or not)
+        // REV: the stages that all rows of the block see are streamed backwards, [0, n_rev)
+        const int n_rev = !REV ? 0 : plain_stages(c0, nst, a.causal ? min(a.k_past + rows_first<FOLD>(a, row0, BLOCK_ROWS), a.Sk - 1) : a.Sk - 1);
+        auto pos = [&](int st) { return REV && st < n_rev ? n_rev - 1 - st : st; };
         if constexpr (!ONE) {  // what derives from these is formed anew, not kept from unit to unit
 #pragma unroll
             for (int t = 0; t < NTA; ++t) asm volatile("" : "+v"(take[t]));
@@ -481,10 +488,11 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
         };
         auto fetch_stage = [&](int st, int slot) __attribute__((always_inline)) {
             if (__builtin_expect(st < n_whole, 1)) {
+                if (REV) k_src = kp + (int64_t)(c0 + pos(st) * KT) * k_row_b;
                 fetch_whole(slot);
                 return;
             }
-            const int kb = c0 + st * KT;
+            const int kb = c0 + pos(st) * KT;
             char *dst = ring_w + slot * STAGE_BYTES;
             if (D == 256 && kb + KT <= a.Sk) {  // narrower rows, as in the row pass (the smaller kernels are no faster with it)
                 const char *base = kp + kb * k_row_b;
@@ -804,7 +812,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 // one stage, in ring slot SLOT (compile-time; the phase's first stage is in slot 0)
                 auto stage = [&](int st, auto slot_c) {
                     constexpr int SLOT = decltype(slot_c)::value;
-                    const int kb = c0 + st * KT;
+                    const int kb = c0 + pos(st) * KT;
                     const bool first = SLOT == 0 && st == s0;
                     if (!first) enter(st, s1);
                     if (NS == 3) fetch_ahead(st, s1, (SLOT + NS - 1) % NS);
@@ -821,7 +829,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                             else take_frag(std::integral_constant<int, ((SLOT + 1) % NS) * STAGE_BYTES>{}, kf);
                         }
                         // the tile before: in this stage, or the last one of the previous stage
-                        const int p_kb = (q > 0) ? kb : kb - KT;
+                        const int p_kb = (q > 0) ? kb : REV ? c0 + pos(st - 1) * KT : kb - KT;
                         const int p_na = (q > 0) ? (q - 1) / NB : NA - 1, p_nb = (q > 0) ? (q - 1) % NB : NB - 1;
                         if (q > 0 || !first) {
                             drain_begin(p_kb, p_na, p_nb);
@@ -839,7 +847,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
                 }
                 static_assert(NS <= 4, "unrolled above");
                 frag_wait(kf);  // (the first fragment of the next stage, if there is one)
-                drain_begin(c0 + (sp - 1) * KT, NA - 1, NB - 1);
+                drain_begin(c0 + pos(sp - 1) * KT, NA - 1, NB - 1);
                 drain_plain(acc[(TILES - 1) & 1], NB - 1);
                 drain_end(NB - 1);
             }
