@@ -301,9 +301,11 @@ __device__ __forceinline__ half8 prescale(half8 v, float cs)
 template <int D, int NB, int WAVES, bool BF, bool PRE, bool FOLD, bool ONE>
 __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args a)
 {
-    // A workgroup with one chunk of one unit streams the stages that all its rows see backwards: pass 1 has just read the same keys forwards on the
-    // same XCD, and its last ones are what the L2 still holds.  us per call on changing keys, forwards -> backwards: H 32 Q 128 K 16384 D 128
-    // 68.2 -> 65.6, 4 x 32 heads on 8, Q 64 K 8192 64.2 -> 61.7; same bits (a key's sums do not depend on the stages' order).
+    // A workgroup with one chunk of one unit streams the stages that all its rows see backwards: pass 1 has just read the same keys forwards, and
+    // its last ones are what the Infinity Cache surely still holds.  (The L2s hold nothing from kernel to kernel: their fetch traffic is all of the
+    // keys either way.)  us per call on changing keys, forwards -> backwards: H 32 Q 128 K 16384 D 128 68.2 -> 65.6, 4 x 32 heads on 8, Q 64
+    // K 8192 64.2 -> 61.7; same bits (a key's sums do not depend on the stages' order).  Alternating directions over the units of a walk
+    // gained nothing (S 4096 167.9 and 167.8, S 8192 D 64 bf16 353 and 357).
     constexpr bool REV = ONE && !PRE;
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
     constexpr int THREADS = 64 * WAVES;
