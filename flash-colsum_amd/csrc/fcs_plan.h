@@ -492,7 +492,9 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // B 1 H 16 S 2500 47.9 -> 33.5, B 4 H 16 S 2300 212.8 -> 88.0, H 1 S 2500 14.6 -> 10.9, 5 averaged rows of B 8 H 16
     // S 2300 30.2 -> 12.1, 128 of them 29.9 -> 18.5; no size in between was slower.)
     const bool wide = D == 64 && tight_stages == 0;
-    const int fused_max = narrow128 ? 63 * 32 : (wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys;
+    // (tight_stages: in two passes beyond 1536 keys.  The single pass has the same slabs in every layout, and the row statistics that two
+    // passes can do with are mostly less: B 32 H 16 S 1537 D 96 10.5 MiB and 8.)
+    const int fused_max = !narrow128 ? ((wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys) : tight_stages == 0 ? 63 * 32 : 48 * 32;
     // Causal calls of 257 .. 2048 keys whose heads are not laid end to end: the same, a mask on the tiles that the diagonal crosses and no
     // exponents behind it.  Two passes cost three launches and both products for what is mostly latency; us per call, two passes -> here:
     // up to 1024 keys, 64 rows per wave: H 32 S 1000 D 128 32.1 -> 21.5, H 16 S 800 D 64 21.2 -> 11.8, H 16 Q 100 K 1000 D 128 17.6 -> 11.6,

@@ -79,12 +79,13 @@ def _static(q, k):
     return out
 
 
-@pytest.mark.parametrize("b,h,s,d", [(352, 23, 27, 256), (568, 14, 2, 72), (172, 47, 13, 200)])
+@pytest.mark.parametrize("b,h,s,d", [(352, 23, 27, 256), (568, 14, 2, 72), (172, 47, 13, 200), (64, 8, 1537, 96), (256, 1, 1700, 80)])
 def test_static_scratch_without_room_for_slabs(b, h, s, d):
     g = torch.Generator(device="cuda").manual_seed(2)
     q, k = (torch.randn(b, h, s, d, generator=g, device="cuda").half() for _ in range(2))
     out, usual = _static(q, k), flash_colsum_ext(q, k, is_causal=False, out_dtype=torch.float32)
-    assert ((out - usual).abs() <= 2e-6 * usual).all()  # the same terms in another grouping: up to 47 x 13 of them
+    # the same terms in another grouping: up to 47 x 13 of them (the last two: a single pass otherwise)
+    assert ((out - usual).abs() <= 2e-6 * usual).all()
 
 
 def test_static_scratch_lays_out_what_the_usual_plan_does_not_fit():

@@ -299,6 +299,19 @@ def test_static_scratch_takes_calls_whose_row_statistics_fit(b, h, s, d):
     assert b"static scratch" in lib.fcs_strerror(rc)
 
 
+@pytest.mark.parametrize("b,h,s,d", [(32, 16, 1537, 96), (64, 8, 1537, 96), (256, 1, 1700, 96), (192, 2, 2000, 80), (256, 2, 2016, 120), (512, 1, 1600, 72)])
+def test_static_scratch_takes_narrow_heads_beyond_1536_keys(b, h, s, d):
+    """The single pass that serves them otherwise does not fit, the two passes do; and so wherever the row statistics fit."""
+    static = _hip.lib().fcs_colsum_noncausal_f16_static
+    assert _hip.workspace_bytes(False, b, h, s, s, d) > 8 << 20
+    assert static(None, None, None, None, b, h, s, d, None, None, ctypes.c_float(0.1), -1, None) == -1  # the size is looked at before the pointers
+    rng = random.Random(s)
+    for _ in range(100):
+        s2, h2 = rng.randint(1537, 2016), rng.choice([1, 2, 3, 8])
+        b2 = (8 << 20) // (8 * h2 * -(-s2 // 512) * 512)  # rows in blocks of up to 512
+        assert static(None, None, None, None, b2, h2, s2, d, None, None, ctypes.c_float(0.1), -1, None) == -1, (b2, h2, s2, d)
+
+
 def test_shares_of_uneven_row_blocks_are_equal():
     """The triangle of a prompt against itself: 32 heads x (8 + 16 + .. + 64) stages over 256 workgroups."""
     t = _hip.plan_description((1, 32, 4096, 128), (1, 32, 4096, 128), causal=True)
