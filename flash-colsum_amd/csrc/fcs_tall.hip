@@ -164,7 +164,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     };
     // the wave's eighth of a unit's query rows: 4 rows x 256 bytes per instruction, position p of row r holds piece p ^ (r & 15) (one
     // chunk: 8 rows x 128 bytes, as a key item);
-    // rows past the last one repeat it (they are given no weight)
+    // rows past the last averaged one repeat it (they are given no weight, which would not do for a NaN in a row that is not averaged)
     auto fetch_q = [&](int head, int row0, int buf) {
         const char *slice = q_batch + (int64_t)head * q_head_b;
         // (32 rows of one chunk are four instructions: the waves 4 .. 7 bring what 0 .. 3 do, so that all count the same)
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         for (int i = 0; i < QI; ++i) {
             const int r = (w * QI + i) * RI + (DC == 2 ? l >> 4 : l >> 3);
             const int piece = DC == 2 ? (l & 15) ^ (r & 15) : (l & 7) ^ ((r >> 1) & 7);
-            const char *src = slice + (size_t)min(row0 + r, a.Sq - 1) * q_row_b + piece * 16;
+            const char *src = slice + (size_t)min(row0 + r, a.q_rows - 1) * q_row_b + piece * 16;
             if (NARROW && piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_tall_zeros);
             dma(src, dst + i * 1024);
         }
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             };
             auto load_rows = [&](int nb) {
                 const _Float16 *qp = reinterpret_cast<const _Float16 *>(q_batch + (int64_t)h * q_head_b) +
-                                     (int64_t)min(row0 + nb * 32 + n_s, a.Sq - 1) * a.qs_s + g_s * 8;
+                                     (int64_t)min(row0 + nb * 32 + n_s, a.q_rows - 1) * a.qs_s + g_s * 8;
 #pragma unroll
                 for (int tt = 0; tt < DC * NT; ++tt) {
                     half8 v = kZero8;

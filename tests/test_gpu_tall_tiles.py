@@ -141,3 +141,18 @@ def test_causal_rows_out_of_range_and_units(which, s, d):
     elif which == "cls_len":
         kw = {"cls_len": 150}
     _check_causal(q, k, kw)
+
+
+@pytest.mark.parametrize("q_len,k_len,d,cls_len,causal", [(1024, 1024, 96, 96, False), (600, 600, 128, 65, False), (900, 1000, 128, 127, False), (1000, 1000, 64, 70, False),
+                                                          (700, 1700, 128, 5, False), (400, 400, 64, 33, True), (1024, 1024, 128, 63, True), (1500, 1500, 72, 40, True)])
+def test_rows_that_are_not_averaged_are_not_read(q_len, k_len, d, cls_len, causal):
+    """NaN and infinities in the rows behind the averaged ones, the first of them in the same row block."""
+    q, k = _make(1 if causal else 12, 16 if causal else 32, 16, q_len, k_len, d, torch.bfloat16, seed=q_len)
+    kw = {"cls_len": cls_len, "is_causal": causal}
+    t = _hip.plan_description(tuple(q.shape), tuple(k.shape), causal=causal, bf16=True, cls_n=cls_len)
+    print("rows not averaged", tuple(q.shape), tuple(k.shape), kw, t, flush=True)
+    assert t.startswith("fcs_tall_kernel<")
+    want = flash_colsum_ext(q, k, out_dtype=torch.float32, **kw)
+    q[:, ::2, cls_len:] = float("nan")
+    q[:, 1::2, cls_len:] = float("inf")
+    assert torch.isfinite(want).all() and torch.equal(flash_colsum_ext(q, k, out_dtype=torch.float32, **kw), want)
