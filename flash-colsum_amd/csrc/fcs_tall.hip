@@ -375,9 +375,11 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
             const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_batch + k_cur) + g_s * 8;
             float v16[NB][16];
             half8 qs[DC * NT];
-            // (register i: row 8 (i / 4) + 4 g + i % 4 of the 32)
+            // (register i: row 8 (i / 4) + 4 g + i % 4 of the 32; causal: rows past the averaged ones see nothing, or a NaN in a key
+            // that none of those sees would reach its mean)
+            const int seen_by_last = a.k_past + a.q_rows - 1;
             auto counts = [&](int t, int nb, int i) {
-                return t <= tmax_s && (!CAUSAL || tile_first(t) + n_s <= seen_by_all(nb) + 8 * (i >> 2) + 4 * g_s + (i & 3));
+                return t <= tmax_s && (!CAUSAL || tile_first(t) + n_s <= min(seen_by_all(nb) + 8 * (i >> 2) + 4 * g_s + (i & 3), seen_by_last));
             };
             auto load_rows = [&](int nb) {
                 const _Float16 *qp = reinterpret_cast<const _Float16 *>(q_batch + (int64_t)h * q_head_b) +
@@ -467,7 +469,10 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
                     const floatx16 c = score_tile(t);
                     float sum = 0.f;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) sum = fmaf(counts(t, nb, i) ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f, v16[nb][i], sum);
+                    for (int i = 0; i < 16; ++i) {  // (a row's weight may be NaN: then it must not reach the keys that the row does not see)
+                        const float with = fmaf(fast_exp2((c[i] - rmax[nb][i]) * a.c), v16[nb][i], sum);
+                        sum = counts(t, nb, i) ? with : sum;
+                    }
 #pragma unroll
                     for (int u = 0; u < TPW; ++u)  // col_acc lives in registers: static index only
                         if (u == t) col_acc[u] += sum;

@@ -156,3 +156,35 @@ def test_rows_that_are_not_averaged_are_not_read(q_len, k_len, d, cls_len, causa
     q[:, ::2, cls_len:] = float("nan")
     q[:, 1::2, cls_len:] = float("inf")
     assert torch.isfinite(want).all() and torch.equal(flash_colsum_ext(q, k, out_dtype=torch.float32, **kw), want)
+
+
+def _means_of_seen(q, k, scale, k_past, rows):
+    """float64 means whose probabilities are 0, and not what a NaN makes of them, at keys that a row does not see."""
+    s = q[:, :, :rows].double() @ k.double().transpose(2, 3) * scale
+    seen = torch.arange(k.shape[2], device=q.device)[None, :] <= k_past + torch.arange(rows, device=q.device)[:, None]
+    e = torch.where(seen, torch.exp(s - torch.where(seen, s, -torch.inf).amax(3, keepdim=True)), 0.0)
+    return torch.where(seen, e / e.sum(3, keepdim=True), 0.0).mean((1, 2))
+
+
+@pytest.mark.parametrize("q_len,k_len,d,k_past,cls_len", [(805, 805, 96, 0, None), (400, 400, 64, 0, 70), (58, 1282, 128, 844, None), (1000, 1427, 120, 427, 49),
+                                                          (33, 978, 48, 548, 12), (1100, 1100, 128, 0, 700), (737, 707, 72, 193, 464), (1, 2048, 128, 700, None)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["row", "key", "keys that no row sees"])
+def test_causal_not_a_number_stays_where_it_is_seen(q_len, k_len, d, k_past, cls_len, value, where):
+    q, k = _make(1, 4, 4, q_len, k_len, d, torch.bfloat16, seed=k_len)
+    rows = q_len if cls_len is None else cls_len
+    last = k_past + rows  # the first key that no averaged row sees
+    if where == "row":
+        q[:, 1, rows // 3] = value
+    elif where == "key":
+        k[:, 2, k_past + rows // 2] = value
+    elif last < k_len:
+        k[:, :, last:] = value
+    print(where, value, tuple(q.shape), tuple(k.shape), k_past, cls_len, flush=True)
+    t = _hip.plan_description(tuple(q.shape), tuple(k.shape), causal=True, bf16=True, k_past=k_past, cls_n=rows)
+    assert t.startswith("fcs_tall_kernel<")
+    got = flash_colsum_ext(q, k, is_causal=True, k_past=k_past, cls_len=cls_len, out_dtype=torch.float32).double()
+    ref = _means_of_seen(q, k, d ** -0.5, k_past, rows)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and (got[:, last:] == 0).all()
+    fine = ~torch.isnan(ref)
+    assert ((got - ref).abs()[fine] <= 1e-4).all() and ((got - ref).abs()[fine] <= 1e-3 * ref[fine] + 1e-12).all()
