@@ -120,7 +120,8 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
     auto tiles_counted = [&](int l) { return (l + a.Sk - 32 - kbase) >> (CAUSAL ? 8 : 5); };  // arithmetic shift: floor, also when negative
     const int tmax_lane = tiles_counted(n);
 
-    const uint32_t q_row_b = (uint32_t)a.qs_s * 2u, k_row_b = (uint32_t)a.ks_s * 2u;
+    const int64_t q_row_b = a.qs_s * 2;  // (of either sign, as on the two-pass path)
+    const uint32_t k_row_b = (uint32_t)a.ks_s * 2u;
     const char *q_batch = reinterpret_cast<const char *>(a.q + (int64_t)b * a.qs_b);
     const char *k_batch = reinterpret_cast<const char *>(a.k + (int64_t)b * a.ks_b);
     const int64_t q_head_b = a.qs_h * 2, k_head_b = a.ks_h * 2;
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
         for (int i = 0; i < QI; ++i) {
             const int r = (w * QI + i) * RI + (DC == 2 ? l >> 4 : l >> 3);
             const int piece = DC == 2 ? (l & 15) ^ (r & 15) : (l & 7) ^ ((r >> 1) & 7);
-            const char *src = slice + (size_t)min(row0 + r, a.q_rows - 1) * q_row_b + piece * 16;
+            const char *src = slice + min(row0 + r, a.q_rows - 1) * q_row_b + piece * 16;
             if (NARROW && piece * 8 >= a.D) src = reinterpret_cast<const char *>(g_tall_zeros);
             dma(src, dst + i * 1024);
         }

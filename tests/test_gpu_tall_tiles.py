@@ -1,5 +1,6 @@
 """Single-pass path with 64 query rows per wave (up to 1024 keys).  Error bar as everywhere: max 1e-4, element-wise
 relative 1e-3, of the fp32 means against float64."""
+import ctypes
 import re
 
 import pytest
@@ -188,3 +189,21 @@ def test_causal_not_a_number_stays_where_it_is_seen(q_len, k_len, d, k_past, cls
     assert torch.equal(torch.isnan(got), torch.isnan(ref)) and (got[:, last:] == 0).all()
     fine = ~torch.isnan(ref)
     assert ((got - ref).abs()[fine] <= 1e-4).all() and ((got - ref).abs()[fine] <= 1e-3 * ref[fine] + 1e-12).all()
+
+
+@pytest.mark.parametrize("h,q_len,k_len,d,causal", [(8, 100, 1000, 128, True), (4, 700, 700, 64, True), (16, 1300, 1300, 96, True), (4, 300, 1700, 96, False)])
+def test_query_rows_stored_backwards(h, q_len, k_len, d, causal):
+    """The C entry point takes query rows of a negative stride: these calls had been served by the two passes, which do."""
+    q, k = _make(1, h, h, q_len, k_len, d, torch.float16, seed=k_len)
+    back = q.flip(2).contiguous()
+    i64x4 = ctypes.c_int64 * 4
+    ws = torch.empty(_hip.workspace_bytes(causal, 1, h, q_len, k_len, d), dtype=torch.uint8, device="cuda")
+    out = torch.empty(1, k_len, device="cuda")
+    assert _hip.plan_description(tuple(q.shape), tuple(k.shape), causal=causal).startswith("fcs_tall_kernel<")
+    last_row = back.data_ptr() + (q_len - 1) * d * 2  # row r of head i is at last_row + 2 (i q_len d - r d)
+    print("backwards", tuple(q.shape), tuple(k.shape), causal, flush=True)
+    rc = _hip.lib().fcs_colsum_general(0, int(causal), last_row, k.data_ptr(), out.data_ptr(), None, ws.data_ptr(), ws.numel(), 1, h, h, q_len, k_len, d, -1,
+                                       max(0, k_len - q_len) if causal else 0, i64x4(h * q_len * d, q_len * d, -d, 1), i64x4(*k.stride()),
+                                       ctypes.c_float(d ** -0.5), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(out, flash_colsum_ext(q, k, is_causal=causal, out_dtype=torch.float32))
