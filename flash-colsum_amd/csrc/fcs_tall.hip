@@ -75,6 +75,24 @@ __device__ __forceinline__ void take_wait(half8 (&dst)[4])
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(dst[0]), "+v"(dst[1]), "+v"(dst[2]), "+v"(dst[3])::"memory");
 }
 
+// this lane's number, from no register
+__device__ __forceinline__ int lane_number()
+{
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+// both at once, where nothing is to be done in between
+__device__ __forceinline__ void take_now(uint32_t at, half8 (&dst)[4])
+{
+    const uint32_t a1 = at ^ 32u, a2 = at ^ 64u, a3 = at ^ 96u;
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(dst[0]), "=&v"(dst[1]), "=&v"(dst[2]), "=&v"(dst[3])
+                 : "v"(at), "v"(a1), "v"(a2), "v"(a3)
+                 : "memory");
+}
+
 }  // namespace
 
 // DC: chunks of 64 channels.  NB: 32-row fragments per wave.  TPW: 32-key tiles per wave.  NARROW: the head dim is less than DC x 64.
@@ -366,117 +384,157 @@ __global__ __launch_bounds__(512, 2) void fcs_tall_kernel(const Args a)
 #pragma unroll
             for (int t = 0; t < TPW; ++t) col_acc[t] += rot ? sum[TPW - 1 - t] : sum[t];
         } else {
-            // ------------ rare: the softmax with the row maximum subtracted, three passes over the keys with one score tile in
-            // registers at a time, from ordinary loads.  (From an opaque copy of the lane id: nothing of this is kept by the
-            // common path.)
+            // ------------ rare: the softmax with the row maximum subtracted, 32 rows after the other, two sweeps over the keys that the
+            // block sees with one score tile in registers at a time: row maxima and sums, then column sums.  The keys come through the
+            // ring as in phase 1; what the ring held for the next unit is requested again behind the sweeps.
+            // What bounds it is VALU work, up to 22 instructions a score, and that all of a unit's waves go through it for one row.  us per
+            // call with every row out of range, of scores formed three times over from ordinary loads (64 lanes to 32 rows), this, and
+            // the kernel that served the call before: causal H 32 S 1000 D 128 194, 66, 53; Q 128 K 2048 73, 35, 31; H 24 S 2048 393, 125,
+            // 97; H 32 S 1500 D 64 160, 76, 64; B 8 H 16 S 1024 D 128 541, 227, 425, S 1000 D 96 435, 240, 260, S 1800 D 96 1114, 898, 505.
+            // With a hundredth of the rows so it is the quickest of the three but for Q 128 K 2048 (72, 34, 31).
+            // From an opaque copy of the lane id: nothing of this is kept by the common path.
             int lane_s = lane;
             FCS_OPAQUE_V(lane_s);
             const int n_s = lane_s & 31, g_s = lane_s >> 5;
-            const int tmax_s = tiles_counted(n_s);
-            const _Float16 *kp = reinterpret_cast<const _Float16 *>(k_batch + k_cur) + g_s * 8;
-            float v16[NB][16];
-            half8 qs[DC * NT];
-            // (register i: row 8 (i / 4) + 4 g + i % 4 of the 32; causal: rows past the averaged ones see nothing, or a NaN in a key
-            // that none of those sees would reach its mean)
-            const int seen_by_last = a.k_past + a.q_rows - 1;
-            auto counts = [&](int t, int nb, int i) {
-                return t <= tmax_s && (!CAUSAL || tile_first(t) + n_s <= min(seen_by_all(nb) + 8 * (i >> 2) + 4 * g_s + (i & 3), seen_by_last));
-            };
-            auto load_rows = [&](int nb) {
-                const _Float16 *qp = reinterpret_cast<const _Float16 *>(q_batch + (int64_t)h * q_head_b) +
-                                     (int64_t)min(row0 + nb * 32 + n_s, a.q_rows - 1) * a.qs_s + g_s * 8;
+            const int seen_by_last = a.k_past + a.q_rows - 1;  // causal: rows past the averaged ones see what the last of those sees
+            // the wave's tiles that any row of the block sees
+            const int past = CAUSAL ? min(a.Sk, min(a.k_past + row0 + ROWS - 1, seen_by_last) + 1) : a.Sk;
+            const int tiles = past > kbase ? min(TPW, (past - kbase + kstep - 1) / kstep) : 0, n_items = DC * tiles;
+            const bool gone = !KEEP_ALL || next_key_head;  // the ring does not hold all of this key head
+            FCS_WAIT_VM(0);
+            if (KEEP_ALL && gone) {
 #pragma unroll
-                for (int tt = 0; tt < DC * NT; ++tt) {
-                    half8 v = kZero8;
-                    if (!NARROW || tt * 16 + g_s * 8 < a.D) v = load8(qp + tt * 16);
-                    qs[tt] = a.negate ? flip_sign(v) : v;
-                }
-            };
-            auto score_tile = [&](int t) {
-                const int krow = tile_first(t) + n_s;
-                floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int tt = 0; tt < DC * NT; ++tt) {
-                    half8 kv = kZero8;
-                    if (!NARROW || tt * 16 + g_s * 8 < a.D) kv = load8(kp + (int64_t)krow * a.ks_s + tt * 16);
-                    c = mfma16<BF>(qs[tt], kv, c);
-                }
-                return c;
-            };
-            // row values over lanes and waves: f(the 8 waves' parts of row `lane`) goes to wv_w.  The barrier in front is for the
-            // part buffer's last readers.
-            auto reduce = [&](bool is_max, auto f) {
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) v16[nb][0] = is_max ? fold_lanes_max(v16[nb], lane_s) : fold_lanes_sum(v16[nb], lane_s);
-                __syncthreads();
-                const int rw = 16 * ((lane_s >> 4) & 1) + 8 * ((lane_s >> 3) & 1) + 4 * g_s + 2 * ((lane_s >> 2) & 1) + ((lane_s >> 1) & 1);
-                if ((lane_s & 1) == 0) {
-                    pt[rw * 8 + wave] = v16[0][0];
-                    if (NB == 2) pt[(32 + rw) * 8 + wave] = v16[NB - 1][0];
-                }
-                __syncthreads();
-                const int row = lane_s & (ROWS - 1);
-                const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + row * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + row * 8 + 4);
-                wv_w[row] = f(row, f0, f1);
-                __builtin_amdgcn_wave_barrier();
-            };
-            auto row_values = [&](float (&v)[16], int nb) {
-#pragma unroll
-                for (int i4 = 0; i4 < 4; ++i4) {
-                    const floatx4 x = *reinterpret_cast<const floatx4 *>(wv_w + nb * 32 + 8 * i4 + 4 * g_s);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) v[4 * i4 + j] = x[j];
-                }
-            };
-            float rmax[NB][16];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                load_rows(nb);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) v16[nb][i] = kNegBig;
-#pragma unroll 1
-                for (int t = 0; t < TPW; ++t) {
-                    const floatx16 c = score_tile(t);
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) v16[nb][i] = fmaxf(v16[nb][i], counts(t, nb, i) ? c[i] : kNegBig);
-                }
+                for (int s = 0; s < STEPS; ++s) fetch_item(k_cur, s, 0, s);
+                FCS_WAIT_VM(0);
             }
-            reduce(true, [](int, floatx4 x, floatx4 y) {
-                return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])));
-            });
+            // The query rows are kept, or where registers do not suffice read again for each tile (what a loop spills costs more: a
+            // reload waits for all fetches).
+            constexpr bool KEEP_Q = NB * TPW < (DC == 2 ? 6 : CAUSAL ? 8 : 9);
+            auto take_rows = [&](int nb, int dc, half8 (&q)[NT]) __attribute__((always_inline)) {
+                take_now((q_at ^ (uint32_t)(dc * 128)) + (uint32_t)(nb * 32 * QROW), q);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                row_values(rmax[nb], nb);  // subtracted from the scores before the scale
-                load_rows(nb);
+                for (int tt = 0; tt < NT; ++tt) q[tt] = a.negate ? flip_sign(q[tt]) : q[tt];
+            };
+            // f(t, the scores of tile t, which of them count), for all of them
+            auto sweep = [&](int nb, half8 (&qs)[DC][NT], auto f) __attribute__((always_inline)) {
+                if (tiles == 0) return;
+                if (!KEEP_ALL) {
+                    FCS_WAIT_VM(0);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v16[nb][i] = 0.f;
-#pragma unroll 1
-                for (int t = 0; t < TPW; ++t) {
-                    const floatx16 c = score_tile(t);
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) v16[nb][i] += counts(t, nb, i) ? fast_exp2((c[i] - rmax[nb][i]) * a.c) : 0.f;
+                    for (int j = 0; j < NS; ++j) fetch_item(k_cur, min(j, n_items - 1) / DC, min(j, n_items - 1) % DC, j);
                 }
-            }
-            reduce(false, [&](int row, floatx4 x, floatx4 y) {
-                const float L = ((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]));
-                return (row0 + row < a.q_rows) ? __builtin_amdgcn_rcpf(L) : 0.f;
-            });
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                row_values(v16[nb], nb);
-                load_rows(nb);
+                int slot = 0;
 #pragma unroll 1
-                for (int t = 0; t < TPW; ++t) {
-                    const floatx16 c = score_tile(t);
+                for (int t = 0; t < tiles; ++t) {
+                    floatx16 c = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int dc = 0; dc < DC; ++dc) {
+                        half8 kv[NT];
+                        if (!KEEP_Q) take_rows(nb, dc, qs[dc]);
+                        if (!KEEP_ALL) FCS_WAIT_VM((NS - 1) * NT);
+                        take_now(k_take + (uint32_t)(slot * ITEM), kv);
+                        if (!KEEP_ALL) {
+                            const int ahead = min(DC * t + dc + NS, n_items - 1);  // (the last one again at the end: the waits count on a request)
+                            fetch_item(k_cur, ahead / DC, ahead % DC, slot);
+                        }
+                        slot = slot + 1 == NS ? 0 : slot + 1;
+#pragma unroll
+                        for (int tt = 0; tt < NT; ++tt) {
+                            // (the pieces past the head dim repeat others: an infinity there, times 0)
+                            if (NARROW && dc == DC - 1 && dc * 64 + tt * 16 + (lane_number() >> 5) * 8 >= a.D) kv[tt] = kZero8;
+                            c = mfma16<BF>(qs[dc][tt], kv[tt], c);
+                        }
+                    }
+                    const int first = kbase + t * kstep;
+                    if (first <= a.Sk - 32 && (!CAUSAL || first + 31 <= min(seen_by_all(nb), seen_by_last))) {
+                        f(t, c, [](int) { return true; });
+                    } else {
+                        // the row of register i, 8 (i / 4) + 4 g + i % 4 of the 32, counts this lane's key: rel <= 8 (i / 4) + i % 4
+                        // (from the lane number formed anew: a register that is kept for it is spilled, and a reload waits for all fetches)
+                        const int lane_t = lane_number(), n_t = lane_t & 31, key = tile_first(t) + n_t;
+                        const int rel = t > tiles_counted(n_t) || (CAUSAL && key > seen_by_last) ? 1 << 20 : CAUSAL ? key - seen_by_all(nb) - 4 * (lane_t >> 5) : -1;
+                        f(t, c, [rel](int i) { return rel <= 8 * (i >> 2) + (i & 3); });
+                    }
+                }
+            };
+#pragma unroll 1
+            for (int nb = 0; nb < NB; ++nb) {
+                half8 qs[DC][NT];
+#pragma unroll
+                for (int dc = 0; dc < DC; ++dc)
+                    if (KEEP_Q) take_rows(nb, dc, qs[dc]);
+                // row values over lanes and waves: f(the 8 waves' parts of a row) goes to wv_w, and from there to v.  The barrier in
+                // front is for the part buffer's last readers.
+                const int row = nb * 32 + n_s;
+                auto reduce = [&](float mine, float (&v)[16], auto f) {
+                    __syncthreads();
+                    const int rw = 16 * ((lane_s >> 4) & 1) + 8 * ((lane_s >> 3) & 1) + 4 * g_s + 2 * ((lane_s >> 2) & 1) + ((lane_s >> 1) & 1);
+                    if ((lane_s & 1) == 0) pt[(nb * 32 + rw) * 8 + wave] = mine;
+                    __syncthreads();
+                    const floatx4 f0 = *reinterpret_cast<const floatx4 *>(pt + row * 8), f1 = *reinterpret_cast<const floatx4 *>(pt + row * 8 + 4);
+                    wv_w[row] = f(f0, f1);
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        const floatx4 x = *reinterpret_cast<const floatx4 *>(wv_w + nb * 32 + 8 * i4 + 4 * g_s);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) v[4 * i4 + j] = x[j];
+                    }
+                };
+                auto exponent = [&](float s, float most) {  // (the maximum is subtracted before the scale)
+                    float e = fast_exp2((s - most) * a.c);
+                    FCS_OPAQUE_V(e);  // (else it is branched around, register by register)
+                    return e;
+                };
+                float most[16], v[16];  // of this lane's keys so far: maximum, and sum relative to it
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    most[i] = kNegBig;
+                    v[i] = 0.f;
+                }
+                sweep(nb, qs, [&](int, const floatx16 &c, auto counts) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const float m = fmaxf(most[i], counts(i) ? c[i] : kNegBig), e = exponent(c[i], m);
+                        v[i] = fmaf(v[i], exponent(most[i], m), counts(i) ? e : 0.f);
+                        most[i] = m;
+                    }
+                });
+                float rmax[16];
+                {
+                    float m[16];
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) m[i] = most[i];
+                    reduce(fold_lanes_max(m, lane_s), rmax, [](floatx4 x, floatx4 y) {
+                        return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])));
+                    });
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] *= exponent(most[i], rmax[i]);
+                reduce(fold_lanes_sum(v, lane_s), v, [&](floatx4 x, floatx4 y) {
+                    const float L = ((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]));
+                    return (row0 + row < a.q_rows) ? __builtin_amdgcn_rcpf(L) : 0.f;
+                });
+                sweep(nb, qs, [&](int t, const floatx16 &c, auto counts) {
                     float sum = 0.f;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {  // (a row's weight may be NaN: then it must not reach the keys that the row does not see)
-                        const float with = fmaf(fast_exp2((c[i] - rmax[nb][i]) * a.c), v16[nb][i], sum);
-                        sum = counts(t, nb, i) ? with : sum;
+                        const float with = fmaf(exponent(c[i], rmax[i]), v[i], sum);
+                        sum = counts(i) ? with : sum;
                     }
 #pragma unroll
                     for (int u = 0; u < TPW; ++u)  // col_acc lives in registers: static index only
                         if (u == t) col_acc[u] += sum;
+                });
+            }
+            __syncthreads();  // the query rows are read no more: their tile may be rewritten
+            FCS_WAIT_VM(0);
+            if (gone) {
+                const int rot_n = KEEP_ALL || next_key_head ? 0 : rot ^ 1;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const int j = rot_n ? STEPS - 1 - s : s;
+                    fetch_item(k_nxt, j / DC, j % DC, j % NS);
                 }
             }
         }

@@ -207,3 +207,23 @@ def test_query_rows_stored_backwards(h, q_len, k_len, d, causal):
                                        ctypes.c_float(d ** -0.5), torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     assert torch.equal(out, flash_colsum_ext(q, k, is_causal=causal, out_dtype=torch.float32))
+
+
+@pytest.mark.parametrize("b,h,s,d,dtype,causal", [(8, 16, 1024, 128, torch.bfloat16, False), (4, 24, 1000, 96, torch.float16, False), (16, 16, 1000, 32, torch.bfloat16, False),
+                                                  (2, 24, 1800, 96, torch.float16, False), (4, 12, 2048, 128, torch.bfloat16, False), (1, 64, 600, 64, torch.float16, True),
+                                                  (1, 48, 300, 128, torch.bfloat16, True), (1, 40, 1000, 128, torch.float16, True), (1, 40, 1500, 64, torch.float16, True),
+                                                  (1, 30, 2040, 72, torch.float16, True)])
+@pytest.mark.parametrize("every", [1, 3])
+def test_units_out_of_range_between_others(b, h, s, d, dtype, causal, every):
+    """A row block outside the unstabilised range takes the ring for itself: the units behind it, of the same head and of the next
+    one, find it as they expect it."""
+    q, k = _make(b, h, h, s, s, d, dtype, seed=s)
+    for i in range(0, h, every):
+        q[:, i, (37 * i) % s::128] *= 40
+    print("units out of range", tuple(q.shape), dtype, causal, every, flush=True)
+    assert _hip.plan_description(tuple(q.shape), tuple(k.shape), causal=causal, bf16=dtype == torch.bfloat16).startswith("fcs_tall_kernel<")
+    got = flash_colsum_ext(q, k, is_causal=causal, out_dtype=torch.float32).double()
+    ref = torch.cat([colsum_ext_exact(q[i:i + 1], k[i:i + 1], is_causal=causal) for i in range(b)])
+    err = (got - ref).abs()
+    # (2^-126: probabilities that fp32 flushes to zero)
+    assert torch.isfinite(got).all() and (err <= 1e-4).all() and (err <= 1e-3 * ref + 2.0 ** -126).all(), (err.max(), (err / ref).max())
