@@ -197,8 +197,9 @@ size_t fcs_workspace_bytes(int causal, int B, int H, int Sq, int Sk, int D, int 
     size_t most = p.total;
     if (!causal && D == 64 && cached_plan(p, 0, B, H, H, Sq, Sk, D, rows, 0, 1) && p.total > most) most = p.total;  // either operand
     // enough for any number of key heads: the two-pass path lays grouped heads out differently
-    // (and beyond 2048 keys a call that the single-pass path serves may be one of those)
-    for (int hk = 1; hk <= H / 2 && (causal || !(p.fewrows || p.small || (p.fused && Sk <= fcs::kFusedMaxKeys))); ++hk)
+    // (and beyond 2048 keys, or 1536 of 72 .. 120 channels, a call that the single-pass path serves may be one of those)
+    const int alike = (D > 64 && D < 128) ? fcs::kFusedMaxKeysNarrow : fcs::kFusedMaxKeys;
+    for (int hk = 1; hk <= H / 2 && (causal || !(p.fewrows || p.small || (p.fused && Sk <= alike))); ++hk)
         if (H % hk == 0 && fcs::make_plan(p, causal ? 1 : 0, B, H, hk, Sq, Sk, D, rows, k_past) && p.total > most) most = p.total;
     return most;
 }

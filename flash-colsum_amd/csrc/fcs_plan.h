@@ -13,6 +13,7 @@ constexpr int kComputeUnits = 256;  // MI355X
 constexpr int kFusedMaxKeys = 2048; // 8 waves x 8 tiles x 32 keys of fp32 scores per 32 query rows
 constexpr float kPrescaledMaxScale = 0.1251f;  // single-pass kernels: the operand is pre-scaled up to this |scale| (fp16)
 constexpr int kFusedMaxKeys64 = 2560; // 64-wide heads: ten tiles per wave
+constexpr int kFusedMaxKeysNarrow = 1536; // heads of 72 .. 120 channels: in every layout and whatever the number of key heads
 constexpr int kFewRowsMaxRows = 4;      // few-rows path: at most this many averaged query rows per head ...
 constexpr int kFewRowsMaxScores = 12288; // ... and rows * Sk scores (48 KB of LDS)
 constexpr int kSmallMaxTiles = 9;        // short-sequence path: one wave holds the scores of 32 rows x (32 x 9) keys
@@ -177,9 +178,9 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Returns false for invalid dimensions.  cls_n <= 0 means all rows.  raw: the single-pass kernels may not take a pre-scaled operand.  Hk: key heads, a divisor of H.
 // tight_stages > 0: the two-pass path with as little workspace as it can do with: row blocks are not cut, chunks are not longer
-// than that; < 0: not even slabs, a workgroup computes all of a chunk (see plan_within).
+// than that; < 0: not even slabs, a workgroup computes all of a chunk (see plan_within).  one_pass: in one pass also where two are quicker.
 inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight_stages = 0,
-                      int raw = 0)
+                      int raw = 0, bool one_pass = false)
 {
     if (B < 1 || H < 1 || Hk < 1 || H % Hk != 0 || Sq < 1 || Sk < 1 || D < 1 || k_past < 0) return false;
     p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
@@ -492,9 +493,22 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // B 1 H 16 S 2500 47.9 -> 33.5, B 4 H 16 S 2300 212.8 -> 88.0, H 1 S 2500 14.6 -> 10.9, 5 averaged rows of B 8 H 16
     // S 2300 30.2 -> 12.1, 128 of them 29.9 -> 18.5; no size in between was slower.)
     const bool wide = D == 64 && tight_stages == 0;
-    // (tight_stages: in two passes beyond 1536 keys.  The single pass has the same slabs in every layout, and the row statistics that two
-    // passes can do with are mostly less: B 32 H 16 S 1537 D 96 10.5 MiB and 8.)
-    const int fused_max = !narrow128 ? ((wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys) : tight_stages == 0 ? 63 * 32 : 48 * 32;
+    // Heads of 72 .. 120 channels beyond 1536 keys, in two passes:
+    //  * with tight_stages.  The single pass has the same slabs in every layout, and the row statistics that two passes can do with are
+    //    mostly less: B 32 H 16 S 1537 D 96 10.5 MiB and 8.
+    //  * many more (batch entry, head) pairs than compute units, with few rows each.  Each unit then reads a key head of its own, and those
+    //    that an XCD reads at a time are many times its L2.  us per call, two passes against one, K 1600, D 120 unless stated: B 32 H 32
+    //    Q 64 134 against 92, Q 128 182 against 197, Q 256 271 against 326, Q 512 476 against 529 (D 96 Q 128 0.93 of two passes' time, Q 256
+    //    1.09, Q 512 0.99; D 72 Q 256 0.95; half as many pairs Q 256 1.20, Q 512 1.10).
+    //    Rows laid end to end read a key head once for all its query heads: 32 on 8 heads B 32 Q 32 52.6 against 50.6, Q 64 76 against
+    //    88, Q 128 125 against 162 (D 96 119 against 131, D 72 0.91; 32 on 16 Q 32 0.69, Q 64 1.04, 32 on 4 Q 4 1.57, D 72 1.28; with half as
+    //    many pairs Q 4 1.00, Q 128 0.96).  Beyond 128 rows they are not laid so, and one pass is quicker: Q 256 0.84.
+    const long pairs = (long)B * H;
+    const bool crowded = narrow128 && !one_pass && pairs > kComputeUnits &&
+                         (p.fold > 1 ? pairs > 2 * kComputeUnits && (p.q_rows > 32 ? D > 80 : p.fold > 2)
+                                     : Hk == H && p.q_rows >= 128 && p.q_rows <= 512 && D > (p.q_rows % 256 == 0 ? 80 : 96));
+    const int fused_max = !narrow128 ? ((wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys)
+                          : tight_stages == 0 && !crowded ? 63 * 32 : kFusedMaxKeysNarrow;
     // Causal calls of 257 .. 2048 keys whose heads are not laid end to end: the same, a mask on the tiles that the diagonal crosses and no
     // exponents behind it.  Two passes cost three launches and both products for what is mostly latency; us per call, two passes -> here:
     // up to 1024 keys, 64 rows per wave: H 32 S 1000 D 128 32.1 -> 21.5, H 16 S 800 D 64 21.2 -> 11.8, H 16 Q 100 K 1000 D 128 17.6 -> 11.6,
@@ -627,7 +641,8 @@ inline bool plan_within(Plan &p, size_t bytes, int B, int H, int Hk, int Sq, int
         if (!make_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, stages)) return false;
         if (p.total <= bytes) return true;
     }
-    return false;
+    // (slabs may fit where row statistics do not: B 487 H 19 S 1884 D 104, 153 averaged rows, 3.5 MiB and 18)
+    return make_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, 0, 0, true) && p.total <= bytes;
 }
 
 }  // namespace fcs

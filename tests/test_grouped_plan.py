@@ -103,3 +103,23 @@ def test_workspace_serves_every_number_of_key_heads(plan):
                 assert p["stats"] % 256 == 0 and p["slabs"] % 256 == 0
                 assert p["stats"] <= p["stats_end"] <= p["slabs"] <= p["slabs_end"] <= p["total"]
     assert grouped_needs_more > 0  # else the shapes above would not show a bound that forgets the grouped layouts
+
+
+def test_narrow_heads_beyond_1536_keys(plan):
+    """In one pass, but for many heads of few rows each; what fcs_workspace_bytes() promises holds for both."""
+    d = _hip.plan_description
+    for b, h, hk, q_len, s_k, dim, one in [(8, 16, 16, 2000, 2000, 96, True), (8, 32, 32, 256, 1600, 120, True), (16, 32, 32, 256, 1600, 120, False), (32, 32, 32, 127, 1600, 120, True),
+                                           (32, 32, 32, 512, 1600, 112, False), (32, 32, 32, 513, 1600, 112, True), (32, 32, 32, 256, 1600, 88, False),
+                                           (32, 32, 32, 300, 1600, 96, True), (32, 32, 32, 256, 1536, 120, True), (32, 32, 8, 128, 1600, 96, False), (32, 32, 8, 128, 1600, 80, True),
+                                           (16, 32, 8, 128, 1600, 96, True), (32, 32, 16, 32, 1600, 120, True), (32, 32, 8, 32, 1600, 72, False), (32, 32, 8, 129, 1600, 120, True)]:
+        t = d((b, h, q_len, dim), (b, hk, s_k, dim))
+        assert t.startswith("fcs_tall_kernel<" if one else "fcs_rowstream_kernel<128,"), (b, h, hk, q_len, s_k, dim, t)
+    rng = random.Random(12)
+    for _ in range(200):
+        b, h, sq, sk, dim = rng.choice([1, 8, 32, 64, 300]), rng.choice([4, 12, 32]), rng.choice([1, 33, 128, 256, 512, 700]), rng.randint(1500, 2050), rng.choice([72, 88, 96, 120])
+        n = _hip.workspace_bytes(False, b, h, sq, sk, dim)
+        for hk in [x for x in range(1, h + 1) if h % x == 0]:
+            assert plan(False, b, h, hk, sq, sk, dim)["total"] <= n, (b, h, hk, sq, sk, dim)
+    # the static scratch holds the slabs of one pass where it does not hold the row statistics of two
+    rc = _hip.lib().fcs_colsum_noncausal_f16_static(None, None, None, None, 487, 19, 1884, 104, None, None, ctypes.c_float(0.1), 153, None)
+    assert _hip.lib().fcs_strerror(rc) == b"a required pointer is NULL"
