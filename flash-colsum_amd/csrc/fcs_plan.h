@@ -178,9 +178,10 @@ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Returns false for invalid dimensions.  cls_n <= 0 means all rows.  raw: the single-pass kernels may not take a pre-scaled operand.  Hk: key heads, a divisor of H.
 // tight_stages > 0: the two-pass path with as little workspace as it can do with: row blocks are not cut, chunks are not longer
-// than that; < 0: not even slabs, a workgroup computes all of a chunk (see plan_within).  one_pass: in one pass also where two are quicker.
+// than that; < 0: not even slabs, a workgroup computes all of a chunk (see plan_within).  few_slabs: in one pass, and 64 rows per wave, also
+// where something else is quicker.
 inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk, int D, int cls_n, int k_past, int tight_stages = 0,
-                      int raw = 0, bool one_pass = false)
+                      int raw = 0, bool few_slabs = false)
 {
     if (B < 1 || H < 1 || Hk < 1 || H % Hk != 0 || Sq < 1 || Sk < 1 || D < 1 || k_past < 0) return false;
     p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
@@ -504,7 +505,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     //    88, Q 128 125 against 162 (D 96 119 against 131, D 72 0.91; 32 on 16 Q 32 0.69, Q 64 1.04, 32 on 4 Q 4 1.57, D 72 1.28; with half as
     //    many pairs Q 4 1.00, Q 128 0.96).  Beyond 128 rows they are not laid so, and one pass is quicker: Q 256 0.84.
     const long pairs = (long)B * H;
-    const bool crowded = narrow128 && !one_pass && pairs > kComputeUnits &&
+    const bool crowded = narrow128 && !few_slabs && pairs > kComputeUnits &&
                          (p.fold > 1 ? pairs > 2 * kComputeUnits && (p.q_rows > 32 ? D > 80 : p.fold > 2)
                                      : Hk == H && p.q_rows >= 128 && p.q_rows <= 512 && D > (p.q_rows % 256 == 0 ? 80 : 96));
     const int fused_max = !narrow128 ? ((wide && p.fold == 1) ? kFusedMaxKeys64 : kFusedMaxKeys)
@@ -539,21 +540,26 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         //  * heads of 65 .. 128 channels, from 449 keys on (narrower than 128: 385): B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5;
         //    S 768 41.1 -> 36.6, S 640 32.1 -> 31.0; with two tiles per wave S 512 B 32 76.3 -> 68.2, S 480 B 16 40.2 -> 35.6, but
         //    S 448 B 8 20.2 -> 20.8, S 384 B 32 47.3 -> 54.2 (D 128; D 96, S 400 62.1 -> 51.6).
-        //  * 64 channels from 865 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 249.8 -> 232.1, B 16 S 900 63.6 -> 61.7,
-        //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4; fewer channels from 769 on: D 32 B 16 S 1000
+        //  * 64 channels from 897 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 249.8 -> 232.1, B 16 S 900 63.6 -> 61.7,
+        //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4, B 21 H 4 S 887 23.1 -> 23.2; fewer channels from 769 on: D 32 B 16 S 1000
         //    68.5 -> 60.5, D 48 B 32 H 12 S 800 81.6 -> 77.7, but D 48 S 500 24.1 -> 25.8.
         //  * 65 .. 128 channels beyond 1024 keys, with 32 rows per wave: B 8 H 16 D 128 S 2048 235.5 -> 230.4, S 1370 125 -> 118.6, B 64 H 8
         //    S 1200 407 -> 370, Q 32 K 2048 16.9 -> 15.8; H 1 S 2048 12.1 -> 11.9; D 120 S 1700 212.9 -> 199.3 (D 72 B 3 H 12 S 1900 62.5 -> 64.7;
         //    64 channels: S 2048 123.9 against 134.9).
-        // A call of up to 1024 keys that leaves half of the chip idle takes the shorter blocks (B 2 H 4 S 1024 D 128 10.4 against 11.1; up to 64 channels the
-        // splits over more waves below have calls of two units per workgroup), and so do calls of up to 32 averaged rows.
-        const long tall_units = (long)B * H * ceil_div(p.q_rows, 64);
+        // Up to 1024 keys, one generation of row blocks of 64 has to stand for nearly one and a half of the shorter ones at least, or those fill
+        // the chip better: B 2 H 4 S 1024 D 128 10.4 against 11.1, B 8 H 12 Q 147 K 753 (288 blocks, 480 shorter ones) 13.3 against 14.5, but
+        // B 12 H 6 Q 255 K 578 (288, 576) 15.0 -> 13.8, B 9 H 24 Q 69 K 598 (432, 648) 16.5 -> 15.1.  (Up to 64 channels the splits over more waves
+        // below have calls of two units per workgroup.)  Up to 64 channels what is gained is the keys, fetched once for a workgroup's row
+        // blocks: not with one of them (B 31 H 32 Q 50 K 792 D 48 23.1 against 24.7), and below 897 keys not with few
+        // (B 40 H 8 Q 153 K 806 D 48 20.6 against 21.9; B 8 H 12 S 785 D 32 0.93 of the shorter blocks' time, B 14 H 8 S 811 D 48 0.97).
+        const auto generations = [&](int rows) { return ((long)B * H * ceil_div(p.q_rows, rows) + kComputeUnits - 1) / kComputeUnits; };
         const auto tall_pays = [&]() {
             if (tight_stages != 0 || tiles > 64) return false;
             if (tiles > 32) return D > 64;
             if (p.q_rows <= 32) return false;
-            return D > 64 ? tiles > (narrow128 ? 12 : 14) && tall_units > kComputeUnits / 2
-                          : (D < 64 ? tiles > 24 : raw && tiles > 27) && tall_units > 2 * kComputeUnits;
+            if (D > 64) return tiles > (narrow128 ? 12 : 14) && (few_slabs || 10 * generations(32) >= 14 * generations(64));
+            if (few_slabs) return D < 64 && tiles > 24;
+            return (D < 64 || raw) && p.q_rows > 64 && generations(64) > 2 && (tiles > 28 || (D < 64 && tiles > 24 && p.q_rows > 384));
         };
         const bool tall = causal_single || tall_pays();
         double best_kg = 0.;
@@ -641,7 +647,8 @@ inline bool plan_within(Plan &p, size_t bytes, int B, int H, int Hk, int Sq, int
         if (!make_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, stages)) return false;
         if (p.total <= bytes) return true;
     }
-    // (slabs may fit where row statistics do not: B 487 H 19 S 1884 D 104, 153 averaged rows, 3.5 MiB and 18)
+    // (slabs may fit where row statistics do not: B 487 H 19 S 1884 D 104, 153 averaged rows, 3.5 MiB and 18; B 159 H 16
+    // S 868 D 8, 126 of them, 4.2 and 8.4 with the shorter blocks)
     return make_plan(p, 0, B, H, Hk, Sq, Sk, D, cls_n, 0, 0, 0, true) && p.total <= bytes;
 }
 

@@ -56,7 +56,8 @@ def test_lengths(s, d, tiles, dtype):
 def test_rows_and_key_heads(q_len, cls_len, hk):
     """Row blocks that end inside 64 rows, rows that are not averaged, and units that do or do not change the key head."""
     for k_len, d, tiles in [(500, 128, 2), (700, 88, 3), (1000, 128, 4)]:
-        q, k = _make(12, 12, hk, q_len, k_len, d, torch.float16, seed=q_len)
+        # (65 rows, two blocks or three of 32: from 384 blocks on)
+        q, k = _make(16 if q_len == 65 else 12, 12, hk, q_len, k_len, d, torch.float16, seed=q_len)
         if q_len == 1:
             tiles = 0  # 32 averaged rows or fewer
         _check(q, k, {"cls_len": cls_len} if cls_len else {}, tiles)
@@ -85,7 +86,7 @@ def test_scales():
         _check(q, k, {"scale": scale}, 3)
 
 
-@pytest.mark.parametrize("s,d", [(865, 64), (1000, 64), (1024, 64), (800, 8), (993, 48), (1024, 32)])
+@pytest.mark.parametrize("s,d", [(897, 64), (1000, 64), (1024, 64), (800, 8), (993, 48), (1024, 32)])
 @pytest.mark.parametrize("hk", [16, 4])
 def test_up_to_64_channels(s, d, hk):
     """Keys that stay in the ring through a key head's row blocks; operands that are not pre-scaled."""

@@ -123,3 +123,15 @@ def test_narrow_heads_beyond_1536_keys(plan):
     # the static scratch holds the slabs of one pass where it does not hold the row statistics of two
     rc = _hip.lib().fcs_colsum_noncausal_f16_static(None, None, None, None, 487, 19, 1884, 104, None, None, ctypes.c_float(0.1), 153, None)
     assert _hip.lib().fcs_strerror(rc) == b"a required pointer is NULL"
+
+
+@pytest.mark.parametrize("b,h,q_len,s_k,d,tall", [
+    # 65 .. 128 channels: a generation of 64-row blocks for one and a half of 32-row ones
+    (4, 12, 132, 762, 128, False), (8, 4, 484, 484, 128, True), (3, 12, 219, 713, 128, False), (8, 12, 147, 753, 128, False), (12, 6, 255, 578, 80, True),
+    (9, 24, 69, 598, 96, True), (8, 4, 448, 448, 128, False), (8, 16, 1024, 1024, 128, True), (64, 16, 32, 1024, 128, False),
+    # up to 64: more than one block per head, and below 897 keys more than six
+    (31, 32, 50, 900, 48, False), (31, 32, 65, 897, 48, True), (40, 8, 153, 806, 48, False), (8, 12, 785, 785, 32, True), (64, 16, 896, 896, 64, False), (64, 16, 897, 897, 64, True),
+    (64, 16, 768, 768, 32, False), (64, 16, 385, 769, 32, True), (64, 16, 384, 769, 32, False), (8, 8, 512, 1000, 64, False)])
+def test_which_calls_take_64_rows_per_wave(b, h, q_len, s_k, d, tall):
+    t = _hip.plan_description((b, h, q_len, d), (b, h, s_k, d), bf16=True)
+    assert t.startswith("fcs_tall_kernel<" if tall else "fcs_fused_kernel<"), t
