@@ -156,7 +156,7 @@ struct Plan {
     int small;       // 1: short-sequence path (non-causal, Sk <= 288, D <= 64): grid = B * f_hg, slabs = f_hg,
                      //    f_tpw key tiles, f_nqblk row tiles of 32 rows per head
     int fused;       // 1: use it (then the two-pass fields above are unused)
-    int tall;        // with fused: 64 query rows per wave (fcs_tall.hip) in place of 32 rows with this many key tiles; else 0
+    int tall;        // with fused: 1: shared query rows (fcs_tall.hip), 64 of them per wave up to four key tiles per wave, 32 beyond
     int f_kg, f_qg;  // waves along keys / along queries, f_kg * f_qg == 8
     int f_tpw;       // 32-key tiles per wave
     int f_nqblk;     // query blocks of 32 * f_qg rows
@@ -614,7 +614,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
                 p.f_rbpw = best_rbpw;
             }
         }
-        p.tall = tall ? ceil_div(tiles, usual) : 0;
+        p.tall = tall;
         p.f_hg = ceil_div(H, p.f_hpg);
         p.f_nwgq = ceil_div(p.f_nqblk, p.f_rbpw);
         p.n_partials = p.f_hg * p.f_nwgq * p.f_qg;

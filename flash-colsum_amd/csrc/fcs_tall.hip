@@ -594,14 +594,11 @@ hipError_t launch_tall(const Plan &p, const Args &a, hipStream_t st)
     return launch_finalize(a, st);
 }
 
-// (names the variant of fcs_fused.hip that serves such a call 32 rows to a wave, which it stands for)
 size_t describe_tall(const Plan &p, const Args &a, char *buf, size_t n)
 {
-    const char *bf = p.bf16 ? "true" : "false", *narrow = p.D % 64 ? "true" : "false";
-    char stands_for[64] = "";
-    if (!p.causal) snprintf(stands_for, sizeof stands_for, " (for fcs_fused_kernel<%d,%d,true,0,%s,true%s> )", p.Dp, p.tall, bf, p.D % 64 ? ",true" : "");
-    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%d,%s,%s,%s>%s grid %d x %d, %d x %d units per workgroup, %d slabs", p.Dp / 64, p.f_tpw > 4 ? 1 : 2, p.f_tpw, bf, narrow,
-                           p.causal ? "true" : "false", stands_for, p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
+    const char *bf = p.bf16 ? "true" : "false", *narrow = p.D % 64 ? "true" : "false", *causal = p.causal ? "true" : "false";
+    const int r = snprintf(buf, n, "fcs_tall_kernel<%d,%d,%d,%s,%s,%s> grid %d x %d, %d x %d units per workgroup, %d slabs", p.Dp / 64, p.f_tpw > 4 ? 1 : 2, p.f_tpw, bf,
+                           narrow, causal, p.f_nwgq * p.B, p.f_hg, p.f_hpg, p.f_rbpw, p.n_partials);
     if (r < 0) return 0;
     const size_t len = (size_t)r;
     return len + describe_finalize(a, false, len < n ? buf + len : nullptr, len < n ? n - len : 0);

@@ -434,16 +434,16 @@ def test_other_head_dims(d):
 
 
 @pytest.mark.parametrize("shape,kw,bf16,boost", [
-    ((8, 16, 1024, 128), {}, False, 0.0),                 # 128-wide heads, eight tiles x four key groups
-    ((2, 4, 2048, 128), {"scale": -0.0884}, False, 0.0),  # eight key groups, the sign on the Q chunks
+    ((8, 16, 1024, 128), {}, False, 0.0),                 # 128-wide heads, 64 query rows per wave
+    ((2, 4, 2048, 128), {"scale": -0.0884}, False, 0.0),  # 32, eight tiles; the sign with the scale
     ((3, 5, 333, 128), {}, True, 0.0),                    # ragged, bf16, two key groups
-    ((2, 3, 1500, 128), {"cls_len": 700}, False, 0.0),    # six tiles per wave (static ring slots)
+    ((2, 3, 1500, 128), {"cls_len": 700}, False, 0.0),    # six tiles per wave
     ((2, 6, 1792, 128), {}, False, 0.0),                  # seven tiles per wave
     ((4, 4, 100, 128), {}, False, 0.0),                   # one key group, four tiles
     ((4, 8, 577, 80), {}, False, 0.0),                    # ViT-H: 80 channels, the upper chunk's last 48 read as zeros
     ((2, 8, 730, 72), {}, True, 0.0),                     # SigLIP: 72 channels
     ((2, 4, 1024, 96), {}, False, 0.0),
-    ((2, 4, 1536, 112), {"scale": 0.05}, False, 0.0),      # the longest a 72 .. 120-channel head takes on this path
+    ((2, 4, 1536, 112), {"scale": 0.05}, False, 0.0),      # six tiles of 72 .. 120 channels
     ((2, 8, 600, 32), {}, False, 0.0),                    # narrow heads past the short-sequence kernel: 64-wide fused kernel
     ((2, 8, 1200, 48), {}, True, 0.0),
     ((3, 4, 300, 8), {"scale": 0.3}, False, 0.0),
@@ -465,7 +465,7 @@ def test_fused_path_for_head_dims_other_than_64(shape, kw, bf16, boost):
     q, k = (q.bfloat16(), k.bfloat16()) if bf16 else (q.half(), k.half())
     text = _hip.plan_description(shape, shape, cls_n=kw.get("cls_len", -1), scale=kw.get("scale"), bf16=bf16)
     print("fused, other head dim", shape, kw, text, flush=True)
-    assert "fcs_fused_kernel" in text
+    assert text.startswith(("fcs_fused_kernel<", "fcs_tall_kernel<"))  # the latter: most of 65 .. 128 channels
     ref = _oracle(q.float(), k.float(), **kw)
     out = _run(q, k, **kw)
     _assert_close(out, ref, f"fused D={shape[3]} {shape} {kw} bf16={bf16} boost={boost}")
@@ -473,6 +473,31 @@ def test_fused_path_for_head_dims_other_than_64(shape, kw, bf16, boost):
     qs = q.cuda().permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)  # (B,S,H,D) storage
     ks = k.cuda().permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
     assert torch.equal(out, _run(qs, ks, **kw))
+
+
+@pytest.mark.parametrize("shape,rows,name,boost", [
+    ((64, 16, 500, 128), 16, "128,8,true,0,false,true", 0.0), ((64, 16, 600, 128), 16, "128,5,true,0,false,true", 0.0), ((64, 16, 700, 128), 20, "128,6,true,0,false,true", 0.0),
+    ((256, 8, 448, 128), 64, "128,7,true,0,false,true", 0.0), ((64, 16, 1024, 128), 32, "128,8,true,0,false,true", 0.0), ((32, 16, 1024, 128), 5, "128,4,true,0,false,true", 0.0),
+    ((64, 16, 640, 96), 5, "128,5,true,0,false,true,true", 0.0), ((64, 16, 768, 80), 32, "128,6,true,0,false,true,true", 0.0), ((128, 16, 1000, 72), 17, "128,4,true,0,false,true,true", 0.0),
+    ((64, 16, 700, 128), 20, "128,6,true,0,false,true", 40.0), ((64, 16, 990, 128), 32, "128,8,true,0,false,true", 40.0), ((64, 16, 768, 120), 32, "128,6,true,0,false,true,true", 40.0),
+])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_wide_heads_with_few_averaged_rows(shape, rows, name, boost, bf16):
+    """65 .. 128 channels on blocks of 32 query rows, private to a wave: up to 32 averaged rows, or not many keys."""
+    from flash_colsum import _hip, flash_colsum_f32
+
+    b, h, s, d = shape
+    g = torch.Generator(device="cuda").manual_seed(s)
+    q, k = (torch.randn(shape, generator=g, device="cuda") for _ in range(2))
+    if boost:
+        q[:, ::3, :4] *= boost
+    q, k = (x.to(torch.bfloat16 if bf16 else torch.float16) for x in (q, k))
+    text = _hip.plan_description(shape, shape, cls_n=rows, bf16=bf16)
+    print("few averaged rows", shape, rows, text, flush=True)
+    assert text.startswith(f"fcs_fused_kernel<{name.replace('0,false', '0,true') if bf16 else name}> grid ")
+    out = flash_colsum_f32(q, k, cls_len=rows)
+    p = torch.softmax((q[:, :, :rows].double() @ k.double().transpose(2, 3)) * d ** -0.5, dim=-1)
+    _assert_close(out, p.mean((1, 2)), f"few averaged rows {shape} {rows} bf16={bf16} boost={boost}")
 
 
 def test_head_dims_the_library_rejects():

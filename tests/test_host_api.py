@@ -235,8 +235,13 @@ def test_plan_description_and_k_past_clamp():
     assert "fcs_fused_kernel" in d((6, 24, 197, 64), (6, 24, 197, 64), cls_n=33)  # two row tiles per head: too many heads per step
     assert "fcs_fused_kernel" in d((2, 4, 289, 64), (2, 4, 289, 64))
     # head dims other than 64 on the single-pass kernels: 128-wide ones above 64 channels, zeros past the head dim
-    assert "fcs_fused_kernel<128,8,true,0,false,true> " in d((8, 16, 1024, 128), (8, 16, 1024, 128))
-    assert "fcs_fused_kernel<128,4,true,0,false,true,true>" in d((8, 16, 1024, 96), (8, 16, 1024, 96))
+    assert d((8, 16, 1024, 128), (8, 16, 1024, 128)).startswith("fcs_tall_kernel<2,2,4,false,false,false> grid ")
+    assert d((8, 16, 1024, 96), (8, 16, 1024, 96)).startswith("fcs_tall_kernel<2,2,4,false,true,false> grid ")
+    assert d((2, 8, 1700, 128), (2, 8, 1700, 128), bf16=True).startswith("fcs_tall_kernel<2,1,7,true,false,false> grid ")
+    assert d((1, 8, 700, 64), (1, 8, 700, 64), causal=True).startswith("fcs_tall_kernel<1,2,3,false,false,true> grid ")
+    assert d((64, 16, 1024, 128), (64, 16, 1024, 128), cls_n=16).startswith("fcs_fused_kernel<128,8,true,0,false,true> grid ")  # few averaged rows
+    assert d((2, 4, 1024, 96), (2, 4, 1024, 96)).startswith("fcs_fused_kernel<128,4,true,0,false,true,true> grid ")  # few heads
+    assert "fused" not in d((8, 16, 1024, 128), (8, 16, 1024, 128)) and "tall" not in d((2, 4, 1024, 96), (2, 4, 1024, 96))  # nothing but what is launched
     assert "fcs_fused_kernel<64,8,true,0,true,true,true>" in d((8, 16, 2048, 32), (8, 16, 2048, 32), bf16=True)
     assert "fcs_rowstream_kernel<128" in d((8, 16, 2048, 96), (8, 16, 2048, 96))     # 72 .. 120 channels stop at 1536 keys
     assert "fcs_rowstream_kernel<256" in d((8, 16, 1024, 160), (8, 16, 1024, 160))
