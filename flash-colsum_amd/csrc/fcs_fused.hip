@@ -697,7 +697,7 @@ __global__ __launch_bounds__(512, 2) void fcs_fused_kernel(const Args a)
         }, PRESCALED ? kSumHiPre : kSumHi);
 
         // (The rare path's loops weigh nothing to the register allocator: what it spills, it spills there.  Else 128-wide heads of eight
-        // tiles per wave spilled in phase 1: B 8 H 16 S 2048 D 128 243.7 -> 235.5 us per call.)
+        // tiles per wave spill in phase 1: B 64 H 16 S 1024 D 128, 32 averaged rows, 76.2 -> 67.8 us per call; 64-wide ones are the same either way.)
         if (KEEP && __builtin_expect(!slow, 1) && rot) {
             // ---------------- phase 3 of a unit in the second order: step t held tile tile_of(t)
 #pragma unroll
@@ -878,8 +878,8 @@ static void launch_tpw(const Plan &p, const Args &a, hipStream_t st)
     const FusedVariant v = pick_fused(p, a, BF);
     if (p.Dp == 128 && p.D == 128)
         hipLaunchKernelGGL((fcs_fused_kernel<128, TPW, true, 0, BF>), grid, dim3(512), 0, st, a);
-    else if (p.Dp == 128)
-        hipLaunchKernelGGL((fcs_fused_kernel<128, TPW, true, 0, BF, true, true>), grid, dim3(512), 0, st, a);
+    else if (p.Dp == 128)  // (up to 1536 keys: more of them are fcs_tall.hip's, or in two passes)
+        hipLaunchKernelGGL((fcs_fused_kernel<128, (TPW <= 6 ? TPW : 6), true, 0, BF, true, true>), grid, dim3(512), 0, st, a);
     else if (p.D != 64)
         hipLaunchKernelGGL((fcs_fused_kernel<64, TPW, true, 0, BF, true, true>), grid, dim3(512), 0, st, a);
     else if (v.pre == 8 && v.qs && !v.ragged)
@@ -935,7 +935,7 @@ static bool launch_fused_t(const Plan &p, const Args &a, hipStream_t st)
 
 hipError_t launch_fused(const Plan &p, const Args &a, hipStream_t st)
 {
-    if (p.Sk < 32) return hipErrorInvalidValue;  // the ragged kernel fetches whole key tiles that end at the last key
+    if (p.Sk < 32 || (p.D > 64 && p.D < 128 && p.f_tpw > 6)) return hipErrorInvalidValue;  // the ragged kernel fetches whole key tiles that end at the last key
     if (!(p.bf16 ? launch_fused_t<true>(p, a, st) : launch_fused_t<false>(p, a, st))) return hipErrorInvalidValue;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
