@@ -486,8 +486,9 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
     // ---- fused path
     // (at least one whole key tile: the kernel moves a tile that reaches past the last key back to end there)
     // (64-wide kernels for head dims up to 64, 128-wide ones up to 128; wider heads take the two-pass path)
-    // (Heads of 72 .. 120 channels: us per call beyond 1536 keys, two passes -> one: B 8 H 16 S 2000 D 96 279 -> 226, S 1700 D 80
-    // 224.3 -> 155.8.  The plan tests hold the longest such call, 2048 keys, to the two-pass path: up to 63 tiles.)
+    // (Heads of 72 .. 120 channels: us per call beyond 1536 keys, two passes -> one: B 8 H 16 S 2000 D 96 299 -> 219, S 1700 D 80 230 -> 155,
+    // D 120 260 -> 201, B 3 H 12 S 1900 D 72 87 -> 60.  Up to 63 tiles: 2017 .. 2048 keys would gain as much, S 2048 D 96 287 against 230, and
+    // have not been moved yet.)
     const bool narrow128 = D > 64 && D < 128;
     // (64-wide heads: the shared-Q variants hold ten tiles per wave, so calls of up to 2560 keys are served too, unless grouped
     // heads are laid end to end, whose keys are streamed once for the whole group.  us per call, two passes -> here:
@@ -512,12 +513,14 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
                           : tight_stages == 0 && !crowded ? 63 * 32 : kFusedMaxKeysNarrow;
     // Causal calls of 257 .. 2048 keys whose heads are not laid end to end: the same, a mask on the tiles that the diagonal crosses and no
     // exponents behind it.  Two passes cost three launches and both products for what is mostly latency; us per call, two passes -> here:
-    // up to 1024 keys, 64 rows per wave: H 32 S 1000 D 128 32.1 -> 21.5, H 16 S 800 D 64 21.2 -> 11.8, H 16 Q 100 K 1000 D 128 17.6 -> 11.6,
-    // H 2 S 300 D 128 14.6 -> 8.7; beyond, 32 rows: H 32 S 1500 D 128 48.3 -> 40.7, S 1200 D 64 36.7 -> 22.7, Q 128 K 2048 H 64 23.9 -> 16.0.
-    // Long prompts of many heads fill the chip in two passes, which leave out the products behind the diagonal too: H 64 S 2048 D 128
-    // 103.9 against 112.6, H 32 60.2 against 61.1 (H 24 53.6 -> 47.0; D 64, H 64 75.4 -> 75.2; Q 1024 K 2048 H 64 D 128 76.3 -> 60.3).
-    // (One batch entry, as prompts and windows are: batches gain as much, B 64 H 16 S 1024 D 64 327 -> 257, but the
-    // tests of shares that cross batch entries hold such a call to two passes.)
+    // up to 1024 keys, 64 rows per wave: H 32 S 1000 D 128 31.7 -> 20.7, H 16 S 800 D 64 21.1 -> 12.0, H 16 Q 100 K 1000 D 128 17.6 -> 12.1,
+    // H 2 S 300 D 128 14.8 -> 10.5; beyond, 32 rows: H 32 S 1500 D 128 47.6 -> 38.9, S 1200 D 64 36.2 -> 22.6, Q 128 K 2048 H 64 24.8 -> 17.0,
+    // H 64 S 1700 97.5 -> 86.8, H 96 S 1536 101.9 -> 99.8.  With rows out of range: see the rare path of fcs_tall.hip.
+    // Long prompts of many heads fill the chip in two passes, which leave out the products behind the diagonal too, two passes against one:
+    // D 128, S 2048 H 96 153 against 173, H 64 106 against 111, H 48 86 and 86, H 32 60.2 against 61.4, H 24 54.3 against 48.0; S 1900 H 64
+    // 103.5 against 107.8, H 32 60.9 against 59.3; D 64, H 96 106 against 111, H 64 75.9 and 75.6; Q 1024 K 2048 H 64 79.8 against 62.1.
+    // (One batch entry, as prompts and windows are.  Batches would gain as much, two passes against one: B 64 H 16 S 1024 D 64 336 against
+    // 265, B 16 H 12 S 700 D 80 86 against 47, though not B 4 H 32 S 2048 D 128, 191 against 227; they have not been moved yet.)
     const bool long_prompt = Sk > 1792 && 2L * (Sk - Sq) < Sq && (long)B * H * ceil_div(p.q_rows, 32) >= (D > 64 ? 2000 : 4200);
     const bool causal_single = causal && B == 1 && p.fold == 1 && D <= 128 && Sk > 256 && Sk <= 2048 && !long_prompt;
     if (causal_single || (!causal && Sk >= 32 && Sk <= fused_max && D <= 128)) {
@@ -537,15 +540,15 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         //    unit's chain of tiles is all there is: B 2 H 4 S 512 9.3 -> 7.3, B 1 H 16 S 1024 bf16 14.1 -> 12.3, D 128
         //    18.2 -> 15.1, B 8 H 8 S 197 D 128 11.3 -> 8.7.  With three units or more it was up to 9 % slower.
         // 64 query rows per wave and eight key groups (fcs_tall.hip), up to 1024 keys.  us per call, 32 rows -> 64:
-        //  * heads of 65 .. 128 channels, from 449 keys on (narrower than 128: 385): B 8 H 16 S 1024 D 128 67.3 -> 54.4, D 96 76.8 -> 56.5;
-        //    S 768 41.1 -> 36.6, S 640 32.1 -> 31.0; with two tiles per wave S 512 B 32 76.3 -> 68.2, S 480 B 16 40.2 -> 35.6, but
+        //  * heads of 65 .. 128 channels, from 449 keys on (narrower than 128: 385): B 8 H 16 S 1024 D 128 67.2 -> 53.0, D 96 72.1 -> 50.8;
+        //    S 768 40.3 -> 33.5, S 640 31.2 -> 29.1; with two tiles per wave S 512 B 32 75.2 -> 65.5, S 480 B 16 37.7 -> 33.2, but
         //    S 448 B 8 20.2 -> 20.8, S 384 B 32 47.3 -> 54.2 (D 128; D 96, S 400 62.1 -> 51.6).
-        //  * 64 channels from 897 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 249.8 -> 232.1, B 16 S 900 63.6 -> 61.7,
-        //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4, B 21 H 4 S 887 23.1 -> 23.2; fewer channels from 769 on: D 32 B 16 S 1000
-        //    68.5 -> 60.5, D 48 B 32 H 12 S 800 81.6 -> 77.7, but D 48 S 500 24.1 -> 25.8.
-        //  * 65 .. 128 channels beyond 1024 keys, with 32 rows per wave: B 8 H 16 D 128 S 2048 235.5 -> 230.4, S 1370 125 -> 118.6, B 64 H 8
-        //    S 1200 407 -> 370, Q 32 K 2048 16.9 -> 15.8; H 1 S 2048 12.1 -> 11.9; D 120 S 1700 212.9 -> 199.3 (D 72 B 3 H 12 S 1900 62.5 -> 64.7;
-        //    64 channels: S 2048 123.9 against 134.9).
+        //  * 64 channels from 897 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 252 -> 236, B 16 S 900 63.0 -> 60.1,
+        //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4, B 21 H 4 S 887 23.1 -> 23.2; fewer channels from 769 on: D 32
+        //    B 16 S 1000 68.8 -> 61.1, D 48 B 32 H 12 S 800 81.6 -> 78.7, but D 48 S 500 24.1 -> 25.8.
+        //  * 65 .. 128 channels beyond 1024 keys, with 32 rows per wave: B 8 H 16 D 128 S 2048 248 -> 226, S 1370 128 -> 118, B 64 H 8
+        //    S 1200 407 -> 376, Q 32 K 2048 18.6 -> 16.8; H 1 S 2048 13.5 -> 12.8; against the narrow variant of the shorter blocks D 120 S 1700
+        //    212.9 -> 199.3, but D 72 B 3 H 12 S 1900 62.5 -> 64.7, B 12 H 32 Q 145 K 1433 D 80 62.7 -> 64.7 (64 channels: S 2048 123.9 against 134.9).
         // Up to 1024 keys, one generation of row blocks of 64 has to stand for nearly one and a half of the shorter ones at least, or those fill
         // the chip better: B 2 H 4 S 1024 D 128 10.4 against 11.1, B 8 H 12 Q 147 K 753 (288 blocks, 480 shorter ones) 13.3 against 14.5, but
         // B 12 H 6 Q 255 K 578 (288, 576) 15.0 -> 13.8, B 9 H 24 Q 69 K 598 (432, 648) 16.5 -> 15.1.  (Up to 64 channels the splits over more waves

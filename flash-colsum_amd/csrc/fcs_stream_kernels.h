@@ -303,9 +303,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void fcs_colstream_kernel(const Args
 {
     // A workgroup with one chunk of one unit streams the stages that all its rows see backwards: pass 1 has just read the same keys forwards, and
     // its last ones are what the Infinity Cache surely still holds.  (The L2s hold nothing from kernel to kernel: their fetch traffic is all of the
-    // keys either way.)  us per call on changing keys, forwards -> backwards: H 32 Q 128 K 16384 D 128 68.2 -> 65.6, 4 x 32 heads on 8, Q 64
-    // K 8192 64.2 -> 61.7; same bits (a key's sums do not depend on the stages' order).  Alternating directions over the units of a walk
-    // gained nothing (S 4096 167.9 and 167.8, S 8192 D 64 bf16 353 and 357).
+    // keys either way.)  us per call on changing keys, forwards -> backwards, D 128: H 32 Q 128 K 16384 69.5 -> 68.0 (bf16 61.7 -> 60.6), K 8192 35.3 -> 34.1,
+    // K 32768 114.3 -> 113.8, 4 x 32 heads on 8, Q 64 K 8192 51.7 -> 49.6 (it varies by 2 % from box to box); same bits (a key's sums do not depend on the
+    // stages' order).  Alternating directions over the units of a walk gained nothing (S 4096 167.9 and 167.8, S 8192 D 64 bf16 353 and 357).
     constexpr bool REV = ONE && !PRE;
     static_assert(!PRE || (!BF && D == 64), "the pre-scaled variant exists for fp16 operands and 64-wide heads");
     constexpr int THREADS = 64 * WAVES;
