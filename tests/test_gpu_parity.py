@@ -465,7 +465,9 @@ def test_fused_path_for_head_dims_other_than_64(shape, kw, bf16, boost):
     q, k = (q.bfloat16(), k.bfloat16()) if bf16 else (q.half(), k.half())
     text = _hip.plan_description(shape, shape, cls_n=kw.get("cls_len", -1), scale=kw.get("scale"), bf16=bf16)
     print("fused, other head dim", shape, kw, text, flush=True)
-    assert text.startswith(("fcs_fused_kernel<", "fcs_tall_kernel<"))  # the latter: most of 65 .. 128 channels
+    # 65 .. 128 channels beyond 1024 keys, or with heads and rows enough: the kernel with shared query rows
+    tall = shape in [(8, 16, 1024, 128), (4, 8, 577, 80), (2, 8, 730, 72)] or (shape[3] > 64 and shape[2] > 1024)
+    assert text.startswith("fcs_tall_kernel<" if tall else "fcs_fused_kernel<"), text
     ref = _oracle(q.float(), k.float(), **kw)
     out = _run(q, k, **kw)
     _assert_close(out, ref, f"fused D={shape[3]} {shape} {kw} bf16={bf16} boost={boost}")
