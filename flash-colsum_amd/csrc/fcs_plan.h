@@ -543,7 +543,7 @@ inline bool make_plan(Plan &p, int causal, int B, int H, int Hk, int Sq, int Sk,
         //  * heads of 65 .. 128 channels, from 449 keys on (narrower than 128: 385): B 8 H 16 S 1024 D 128 67.2 -> 53.0, D 96 72.1 -> 50.8;
         //    S 768 40.3 -> 33.5, S 640 31.2 -> 29.1; with two tiles per wave S 512 B 32 75.2 -> 65.5, S 480 B 16 37.7 -> 33.2, but
         //    S 448 B 8 20.2 -> 20.8, S 384 B 32 47.3 -> 54.2 (D 128; D 96, S 400 62.1 -> 51.6).
-        //  * 64 channels from 897 keys on where the operand is not pre-scaled: bf16 B 64 H 16 S 1024 252 -> 236, B 16 S 900 63.0 -> 60.1,
+        //  * 64 channels from 897 keys on where type or scale keep the operand from being pre-scaled: bf16 B 64 H 16 S 1024 252 -> 236, B 16 S 900 63.0 -> 60.1,
         //    but S 800 52.5 -> 53.7, S 577 33.1 -> 35.3, S 512 B 32 40.4 -> 46.4, B 21 H 4 S 887 23.1 -> 23.2; fewer channels from 769 on: D 32
         //    B 16 S 1000 68.8 -> 61.1, D 48 B 32 H 12 S 800 81.6 -> 78.7, but D 48 S 500 24.1 -> 25.8.
         //  * 65 .. 128 channels beyond 1024 keys, with 32 rows per wave: B 8 H 16 D 128 S 2048 248 -> 226, S 1370 128 -> 118, B 64 H 8
